@@ -56,7 +56,7 @@ __host__ __device__ inline uint32_t spread_at(int counter, uint32_t slot) {
 }
 enum Ctr : int {
     C_ACTIVE = 0, C_FIT, C_VO, C_FO, C_FV, C_VERTS, C_FACES, C_FACEVERTS, C_B1, C_B2, C_B3, C_B5, C_BX, C_DEGEN,
-    C_Q2, C_Q3, C_Q5, C_ABORT, C_TETFACES, C_RECW, C_DFAIL, C_CUTK3, C_CUTW3, C_CUTK5, C_CUTW5, C_E3, C_E5, C_E3B, C_N
+    C_Q2, C_Q3, C_Q5, C_ABORT, C_TETFACES, C_RECW, C_CUTK3, C_CUTW3, C_CUTK5, C_CUTW5, C_E3, C_E5, C_E3B, C_N
 };
 
 struct K1Entry {
@@ -1720,11 +1720,11 @@ struct Workspace {
     DBuf<uint32_t> fq_a, fq_vs, fve;
     DBuf<uint16_t> fq_l;
     DBuf<uint8_t> fq_fn, fq_bnd;
-    DBuf<uint32_t> first, vid, vrank, first_occ, mo, fail;
+    DBuf<uint32_t> first, vid, vrank, first_occ, mo;
     DBuf<uint32_t> tile_first;  // star path: first occurrences per tile of occurrences
     DBuf<uint32_t> star_head;  // star tables of the regular grid (k_dedup_star)
     DBuf<uint8_t> star_ent;
-    // vertex dedup hash table (zero between runs) and each occurrence's slot
+    // explicit meshes: vertex dedup hash table (zero between runs) and each occurrence's slot
     DBuf<unsigned long long> hkey;
     DBuf<uint32_t> hmx, hslot;
     int hbits = 0;
@@ -1928,7 +1928,7 @@ void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
     W.okey.alloc(m, c.vo + 1);
     W.oa.alloc(m, c.vo + 1);
     W.oj.alloc(m, c.vo + 1);
-    for (auto* b : {&W.first, &W.vid, &W.vrank, &W.first_occ, &W.hslot, &W.mo, &W.fail}) b->alloc(m, c.vo + 1);
+    for (auto* b : {&W.first, &W.vrank, &W.first_occ, &W.mo}) b->alloc(m, c.vo + 1);
     W.tile_first.alloc(m, (c.vo + kDedupTile - 1) / kDedupTile + 1);
     {
         const StarTables& ST = star_tables();
@@ -1937,13 +1937,17 @@ void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
         RIN_HIP(hipMemcpyAsync(W.star_head.p, ST.head.data(), 4 * ST.head.size(), hipMemcpyHostToDevice, s));
         RIN_HIP(hipMemcpyAsync(W.star_ent.p, ST.ent.data(), ST.ent.size(), hipMemcpyHostToDevice, s));
     }
-    W.hbits = 10;
-    while (W.hbits < 31 && (1ull << W.hbits) < 2ull * c.vo) ++W.hbits;
-    W.hkey.alloc(m, 1ull << W.hbits);
-    W.hmx.alloc(m, 1ull << W.hbits);
-    RIN_HIP(hipMemsetAsync(W.hkey.p, 0, 8ull << W.hbits, s));
-    RIN_HIP(hipMemsetAsync(W.hmx.p, 0, 4ull << W.hbits, s));
-    W.hash_dirty = false;
+    if (!g.view.regular) {
+        W.vid.alloc(m, c.vo + 1);
+        W.hslot.alloc(m, c.vo + 1);
+        W.hbits = 10;
+        while (W.hbits < 31 && (1ull << W.hbits) < 2ull * c.vo) ++W.hbits;
+        W.hkey.alloc(m, 1ull << W.hbits);
+        W.hmx.alloc(m, 1ull << W.hbits);
+        RIN_HIP(hipMemsetAsync(W.hkey.p, 0, 8ull << W.hbits, s));
+        RIN_HIP(hipMemsetAsync(W.hmx.p, 0, 4ull << W.hbits, s));
+        W.hash_dirty = false;
+    }
     W.fq_a.alloc(m, c.fo + 1);
     W.fq_vs.alloc(m, c.fo + 1);
     W.fq_l.alloc(m, c.fo + 1);
@@ -2296,12 +2300,8 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
     const Count NVO(ctr + C_VO, c.vo, abort), NFO(ctr + C_FO, c.fo, abort), NV(ctr + C_VERTS, c.vo, abort),
         NF(ctr + C_FACES, c.fo, abort);
     if (part & REST_DEDUP) {
-        // regular grids: star tables, then the hash path for what they leave;
-        // explicit meshes: the hash path for every occurrence
+        // regular grids: star tables; explicit meshes: the hash path
         const bool star = g.view.regular != 0;
-        const Count NH = star ? Count(ctr + C_DFAIL, c.vo, abort) : NVO;
-        const uint32_t* list = star ? W.fail.p : nullptr;
-        const unsigned hgrid = star ? std::min(nblk(c.vo), 1024u) : nblk(c.vo);
         const unsigned tgrid = (unsigned)((c.vo + kDedupTile - 1) / kDedupTile);
         if (star) {
             StarArgs S;
@@ -2315,30 +2315,23 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
             S.star_ent = W.star_ent.p;
             S.first = W.first.p;
             S.mo = W.mo.p;
-            S.fail = W.fail.p;
-            S.n_fail = ctr + C_DFAIL;
-            S.cap_fail = c.vo;
             S.n_active = ctr + C_ACTIVE;
             S.tile_first = W.tile_first.p;
             hipLaunchKernelGGL(k_dedup_star, dim3(tgrid), dim3(256), 0, s, NVO, S);
         }
         if (star) {
-            // the fallback and the scan of the star pass's tile counts in one
-            // workgroup, then ranks per tile
-            hipLaunchKernelGGL(k_dedup_fallback_scan, dim3(1), dim3(1024), 0, s, NH, list, (const uint64_t*)W.okey.p,
-                               W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p, W.first.p, W.mo.p, NVO,
-                               W.tile_first.p, ctr + C_VERTS);
+            hipLaunchKernelGGL(k_dedup_tile_scan, dim3(1), dim3(1024), 0, s, NVO, W.tile_first.p, ctr + C_VERTS);
             hipLaunchKernelGGL(k_dedup_rank, dim3(tgrid), dim3(256), 0, s, NVO, (const uint32_t*)W.first.p,
-                               (const uint32_t*)W.tile_first.p, W.vrank.p, W.first_occ.p, NH, list,
-                               (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p);
+                               (const uint32_t*)W.tile_first.p, W.vrank.p, W.first_occ.p);
         } else {
-            hipLaunchKernelGGL(k_hash_insert, dim3(hgrid), dim3(256), 0, s, NH, list, (const uint64_t*)W.okey.p,
+            const uint32_t* list = nullptr;
+            hipLaunchKernelGGL(k_hash_insert, dim3(nblk(c.vo)), dim3(256), 0, s, NVO, list, (const uint64_t*)W.okey.p,
                                W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p);
-            hipLaunchKernelGGL(k_hash_first, dim3(hgrid), dim3(256), 0, s, NH, list, (const uint32_t*)W.hslot.p,
+            hipLaunchKernelGGL(k_hash_first, dim3(nblk(c.vo)), dim3(256), 0, s, NVO, list, (const uint32_t*)W.hslot.p,
                                (const uint32_t*)W.hmx.p, W.first.p, W.mo.p);
             scan_u32(m, W.first.p, W.vrank.p, NVO, ctr + C_VERTS, s);
             hipLaunchKernelGGL(k_dedup_assign, dim3(cgrid(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.mo.p,
-                               (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p, NH,
+                               (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p, NVO,
                                list, (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p, true);
         }
     }
@@ -2805,7 +2798,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         read_back(false);
         w.ctr_clear = true;  // the run's closing kernel cleared them
         const uint32_t e = errors();
-        if (e) w.hash_dirty = true;
+        if (e && w.hkey.p) w.hash_dirty = true;
         if (e & ERR_OVERFLOW) {
             w.drop_graphs();
             w.exec = false;

@@ -1171,9 +1171,15 @@ __global__ void k_patch_keys_pid(Count nf, const uint32_t* __restrict__ order, c
 // host-built table lists the star of each simplex shape (the lattice
 // directions from its lowest vertex, by that vertex's parity) as cube offsets
 // and tets, in tet order; the first in-grid entry is that lowest tet, whose
-// occurrences are searched for the key.  Interior keys are unique.  A key
-// whose lowest star tet does not hold it (only degenerate inputs) goes, with
-// every other occurrence of it, to the hash path below.
+// occurrences are searched for the key.  Interior keys are unique.  Where a
+// function vanishes on a simplex, the star's lowest tets need not hold the
+// key (only degenerate inputs): the lane then walks the star's later tets in
+// order, up to its own, which holds it, so every key is decided without a
+// table.  Measured at 33^3 vertices and 18 dyadic planes: a hash table filled
+// by one workgroup for those keys took 445 us of a 0.83 ms run; the walk
+// takes the run to 0.33 ms.
+//
+// Explicit meshes take the hash path.
 //
 // Hash path: the table holds key + 1 (0: empty) and ~(smallest occurrence
 // index) (0: none) per slot, linear probing; it is zero between runs (the
@@ -1209,8 +1215,7 @@ struct StarArgs {
     const uint32_t *oa, *act, *rank, *voff;
     const uint32_t* star_head;  // [2][kStarShapes]: first entry << 8 | entry count
     const uint8_t* star_ent;    // (di+1) | (dj+1) << 2 | (dk+1) << 4 with di.. in {-1, 0}, then q
-    uint32_t *first, *mo, *fail, *n_fail;
-    uint32_t cap_fail;
+    uint32_t *first, *mo;
     const uint32_t* n_active;
     uint32_t* tile_first;  // first occurrences per tile of kDedupTile occurrences
 };
@@ -1222,32 +1227,64 @@ struct StarArgs {
 constexpr int kDedupU = 2;  // measured against 1, 4 and 8 occurrences a lane
 constexpr uint32_t kDedupTile = 256u * kDedupU;
 
-// lowest tet of the star of key K's simplex inside the grid (~0: none)
-__device__ inline uint64_t star_lowest_tet(const StarArgs& A, uint32_t R, uint32_t N, uint64_t K) {
-    const uint32_t type = (uint32_t)(K & 3);
-    uint32_t a, shape;
-    if (type == 0) {
-        a = (uint32_t)(K >> 2);
-        shape = 0;
-    } else if (type == 1) {
-        const uint64_t e = K >> 8;
-        a = (uint32_t)(e / 27);
-        shape = 1 + (uint32_t)(e % 27);
-    } else {
-        const uint64_t fc = K >> 14;
-        a = (uint32_t)(fc / 729);
-        shape = 28 + (uint32_t)(fc % 729);
+// The star of key K's simplex: its tets inside the grid, in tet order.
+struct StarWalk {
+    uint32_t ai, aj, ak, e, end;
+    __device__ StarWalk(const StarArgs& A, uint32_t N, uint64_t K) {
+        const uint32_t type = (uint32_t)(K & 3);
+        uint32_t a, shape;
+        if (type == 0) {
+            a = (uint32_t)(K >> 2);
+            shape = 0;
+        } else if (type == 1) {
+            const uint64_t x = K >> 8;
+            a = (uint32_t)(x / 27);
+            shape = 1 + (uint32_t)(x % 27);
+        } else {
+            const uint64_t fc = K >> 14;
+            a = (uint32_t)(fc / 729);
+            shape = 28 + (uint32_t)(fc % 729);
+        }
+        ai = a / (N * N);
+        const uint32_t ar = a - ai * N * N;
+        aj = ar / N;
+        ak = ar - aj * N;
+        const uint32_t head = A.star_head[((ai + aj + ak) & 1u) * kStarShapes + shape];
+        e = head >> 8;
+        end = e + (head & 255u);
     }
-    const uint32_t ai = a / (N * N), ar = a - ai * N * N, aj = ar / N, ak = ar - aj * N;
-    const uint32_t head = A.star_head[((ai + aj + ak) & 1u) * kStarShapes + shape];
-    for (uint32_t e = head >> 8, end = (head >> 8) + (head & 255u); e < end; e += 2) {
-        const uint32_t d = A.star_ent[e];
-        const int ci = (int)ai + (int)(d & 3u) - 1, cj = (int)aj + (int)((d >> 2) & 3u) - 1,
-                  ck = (int)ak + (int)((d >> 4) & 3u) - 1;
-        if (ci < 0 || cj < 0 || ck < 0 || ci >= (int)R || cj >= (int)R || ck >= (int)R) continue;
-        return (((uint64_t)ci * R + cj) * R + ck) * 5 + A.star_ent[e + 1];
+    // the next tet (~0: none left)
+    __device__ uint64_t next(const StarArgs& A, uint32_t R) {
+        for (; e < end; e += 2) {
+            const uint32_t d = A.star_ent[e];
+            const int ci = (int)ai + (int)(d & 3u) - 1, cj = (int)aj + (int)((d >> 2) & 3u) - 1,
+                      ck = (int)ak + (int)((d >> 4) & 3u) - 1;
+            if (ci < 0 || cj < 0 || ck < 0 || ci >= (int)R || cj >= (int)R || ck >= (int)R) continue;
+            const uint64_t t = (((uint64_t)ci * R + cj) * R + ck) * 5 + A.star_ent[e + 1];
+            e += 2;
+            return t;
+        }
+        return ~0ull;
     }
-    return ~0ull;
+};
+
+// The first occurrence of key K, held by tet t at occurrence o, among the
+// star's tets after the lowest (which does not hold it) and up to t.
+__device__ __forceinline__ uint32_t star_walk_first(const StarArgs& A, uint32_t NA, uint32_t NO, uint64_t K, uint32_t t,
+                                                 uint32_t o) {
+    const uint32_t R = (uint32_t)A.res;
+    StarWalk S(A, R + 1, K);
+    (void)S.next(A, R);
+    for (;;) {
+        const uint64_t ts = S.next(A, R);
+        if (ts >= t) return o;
+        const uint32_t a = A.rank[ts];
+        if (a >= NA || A.act[a] != (uint32_t)ts) continue;
+        uint32_t hi = a + 1 < NA ? A.voff[a + 1] : NO;
+        hi = hi < NO ? hi : NO;
+        for (uint32_t p = A.voff[a]; p < hi; ++p)
+            if (A.okey[p] == K) return p;
+    }
 }
 
 __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
@@ -1272,7 +1309,7 @@ __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
     for (int u = 0; u < kDedupU; ++u) {
         const bool inner = (K[u] & 3) == 3;
         t[u] = inner ? 0u : A.act[oa[u]];
-        ts[u] = inner ? ~0ull : star_lowest_tet(A, R, N, K[u]);
+        ts[u] = inner ? ~0ull : StarWalk(A, N, K[u]).next(A, R);
     }
 #pragma unroll
     for (int u = 0; u < kDedupU; ++u) {
@@ -1303,24 +1340,12 @@ __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
 #pragma unroll
     for (int u = 0; u < kDedupU; ++u) {
         const bool in = o[u] < NO;
-        const bool fail = in && found[u] == ~0u;
+        if (in && found[u] == ~0u) found[u] = star_walk_first(A, NA, NO, K[u], t[u], o[u]);
         if (in) {
             A.first[o[u]] = found[u] == o[u];
-            if (!fail) A.mo[o[u]] = found[u];
+            A.mo[o[u]] = found[u];
         }
         nfirst += in && found[u] == o[u];
-        // failures: one counter update per wave
-        const uint64_t m = __ballot(fail);
-        if (m) {
-            const int leader = __ffsll((unsigned long long)m) - 1;
-            uint32_t b0 = 0;
-            if (lane == leader) b0 = atomicAdd(A.n_fail, (uint32_t)__popcll(m));
-            b0 = __shfl(b0, leader, 64);
-            if (fail) {
-                const uint32_t slot = b0 + (uint32_t)__popcll(m & ((1ull << lane) - 1));
-                if (slot < A.cap_fail) A.fail[slot] = o[u];
-            }
-        }
     }
     __shared__ uint32_t red[256 / 64];
     for (int d = 32; d > 0; d >>= 1) nfirst += __shfl_xor(nfirst, d, 64);
@@ -1376,29 +1401,9 @@ __device__ inline void scan_tiles_block(uint32_t nt, uint32_t* __restrict__ x, i
     }
 }
 
-// Star path, after the star pass, in one workgroup: the hash fallback for
-// the occurrences the star tables left (only degenerate inputs leave any; a
-// long list is taken in passes), their first occurrences joining the tile
-// counts, then the scan of the tile counts (*total: the vertex count).
-__global__ void __launch_bounds__(1024) k_dedup_fallback_scan(Count n_fail, const uint32_t* __restrict__ list,
-                                                              const uint64_t* __restrict__ okey,
-                                                              unsigned long long* __restrict__ hkey,
-                                                              uint32_t* __restrict__ hmx, int bits,
-                                                              uint32_t* __restrict__ hslot, uint32_t* __restrict__ errs,
-                                                              uint32_t* __restrict__ first, uint32_t* __restrict__ mo,
-                                                              Count n, uint32_t* __restrict__ tile_first,
-                                                              uint32_t* __restrict__ total) {
-    const uint32_t nf = (uint32_t)count_of(n_fail);
-    for (uint32_t i = threadIdx.x; i < nf; i += blockDim.x) hash_insert_one(list[i], okey, hkey, hmx, bits, hslot, errs);
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < nf; i += blockDim.x) {
-        const uint32_t o = list[i];
-        const uint32_t m = ~__hip_atomic_load(&hmx[hslot[o]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        first[o] = m == o;
-        mo[o] = m;
-        if (m == o) atomicAdd(&tile_first[o / kDedupTile], 1u);
-    }
-    __syncthreads();
+// The scan of the star pass's tile counts, one workgroup (*total: the vertex count).
+__global__ void __launch_bounds__(1024) k_dedup_tile_scan(Count n, uint32_t* __restrict__ tile_first,
+                                                          uint32_t* __restrict__ total) {
     const TileTotals tt = {{total, nullptr, nullptr, nullptr}};
     scan_tiles_block((uint32_t)((count_of(n) + kDedupTile - 1) / kDedupTile), tile_first, 1, 1, tt);
 }
@@ -1544,22 +1549,9 @@ __global__ void __launch_bounds__(256) k_bucket_fill(Count nc, const uint8_t* __
 // occurrences, in occurrence order) from its tile's prefix, written where
 // the id lookups read it (vrank at first occurrences: the id of occurrence o
 // is vrank[mo[o]]), and first_occ.
-// It also clears the hash slots the fallback used (one per distinct key:
-// that of its first occurrence), leaving the table zero for the next run.
 __global__ void __launch_bounds__(256) k_dedup_rank(Count n, const uint32_t* __restrict__ first,
                                                     const uint32_t* __restrict__ tile_first,
-                                                    uint32_t* __restrict__ vrank, uint32_t* __restrict__ first_occ,
-                                                    Count n_hash, const uint32_t* __restrict__ list,
-                                                    const uint32_t* __restrict__ hslot,
-                                                    unsigned long long* __restrict__ hkey, uint32_t* __restrict__ hmx) {
-    GRID_STRIDE(i, n_hash) {
-        const uint32_t o = list[i];
-        if (first[o]) {
-            const uint32_t h = hslot[o];
-            hkey[h] = 0;
-            hmx[h] = 0;
-        }
-    }
+                                                    uint32_t* __restrict__ vrank, uint32_t* __restrict__ first_occ) {
     const uint32_t NO = (uint32_t)count_of(n);
     const uint32_t nt = (NO + kDedupTile - 1) / kDedupTile;
     if (blockIdx.x >= nt) return;
