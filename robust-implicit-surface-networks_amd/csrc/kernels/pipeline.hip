@@ -1205,59 +1205,32 @@ void compute_patches(DevMem& mem, RunOut& r, hipStream_t s) {
         r.have_patches = true;
         return;
     }
-    DBuf<uint32_t> adj(mem, NO + 1), parent(mem, NF), seed(mem, NF + 1), srank(mem, NF + 1), pid(mem, NF),
-        level(mem, NF), fa(mem, NF), fb(mem, NF), order(mem, NF), cnt(mem, 2);
+    DBuf<uint32_t> adj(mem, NO + 1), parent(mem, NF), seed(mem, NF + 1), srank(mem, NF + 1), seeds(mem, NF),
+        size(mem, NF + 1), err(mem, 1);
     DBuf<unsigned long long> claim(mem, NF);
-    DBuf<uint64_t> key(mem, NF);
+    DBuf<uint4> rows(mem, 2 * NF);
     hipLaunchKernelGGL(k_face_adj, dim3(nblk(NO)), dim3(256), 0, s, Count(NO), (const uint32_t*)r.e_of_occ.p,
                        (const uint32_t*)r.e_start.p, (const uint32_t*)r.e_occ.p, (const uint32_t*)r.e_face_of.p,
                        adj.p);
+    hipLaunchKernelGGL(k_face_rows, dim3(nblk(NF)), dim3(256), 0, s, Count(NF), (const uint32_t*)r.view.f_vstart,
+                       (const uint32_t*)adj.p, rows.p);
     iota_u32(parent.p, Count(NF), s);
+    fill_u32(size.p, 0, NF + 1, s);
+    fill_u32(err.p, 0, 1, s);
     hipLaunchKernelGGL(k_uf_hook, dim3(nblk(NO)), dim3(256), 0, s, Count(NO), (const uint32_t*)r.e_face_of.p,
                        (const uint32_t*)adj.p, parent.p);
     hipLaunchKernelGGL(k_uf_roots, dim3(nblk(NF)), dim3(256), 0, s, Count(NF), parent.p, seed.p);
     scan_u32(mem, seed.p, srank.p, Count(NF), srank.p + NF, s);
     hipLaunchKernelGGL(k_patch_seeds, dim3(nblk(NF)), dim3(256), 0, s, Count(NF), (const uint32_t*)parent.p,
-                       (const uint32_t*)seed.p, (const uint32_t*)srank.p, pid.p, level.p, fa.p, claim.p);
+                       (const uint32_t*)seed.p, (const uint32_t*)srank.p, seeds.p, claim.p, size.p);
     const uint64_t NP = read1(srank.p + NF, s);
     r.n_patches = NP;
-    copy_u32(order.p, fa.p, Count(NP), s);
-    // breadth-first levels over every patch at once
-    uint32_t* front = fa.p;
-    uint32_t* next = fb.p;
-    uint64_t nfront = NP, base = NP;
-    uint32_t lv = 1;
-    DBuf<uint32_t> sorted(mem, NF);
-    while (nfront) {
-        fill_u32(cnt.p, (uint32_t)nfront, 1, s);
-        fill_u32(cnt.p + 1, 0, 1, s);
-        hipLaunchKernelGGL(k_patch_claim, dim3(nblk(nfront)), dim3(256), 0, s, (const uint32_t*)cnt.p,
-                           (const uint32_t*)front, (const uint32_t*)r.view.f_vstart, (const uint32_t*)adj.p,
-                           (const uint32_t*)level.p, claim.p, next, cnt.p + 1);
-        const uint64_t nn = read1(cnt.p + 1, s);
-        if (nn == 0) break;
-        if (base + nn > NF) throw std::runtime_error("patch search listed a face twice");
-        hipLaunchKernelGGL(k_patch_keys, dim3(nblk(nn)), dim3(256), 0, s, (const uint32_t*)(cnt.p + 1),
-                           (const uint32_t*)next, (const unsigned long long*)claim.p, key.p, sorted.p);
-        sort_pairs(mem, key.p, sorted.p, Count(nn), 16 + bits_for(nfront), s);
-        hipLaunchKernelGGL(k_patch_level, dim3(nblk(nn)), dim3(256), 0, s, (const uint32_t*)(cnt.p + 1),
-                           (const uint32_t*)sorted.p, lv, level.p, order.p, (uint32_t)base);
-        copy_u32(front, sorted.p, Count(nn), s);
-        base += nn;
-        nfront = nn;
-        ++lv;  // front holds the new frontier in order; next takes the next offers
-    }
-    if (base != NF) throw std::runtime_error("patch search did not reach every face");
-    // faces by patch, each patch in its breadth-first order (stable placement)
-    DBuf<uint32_t> pc(mem, NP + 1);
-    fill_u32(pc.p, 0, NP + 1, s);
-    hipLaunchKernelGGL(k_patch_count, dim3(nblk(NF)), dim3(256), 0, s, Count(NF), (const uint32_t*)pid.p, pc.p);
-    scan_u32(mem, pc.p, r.p_start.p, Count(NP), r.p_start.p + NP, s);
-    hipLaunchKernelGGL(k_patch_keys_pid, dim3(nblk(NF)), dim3(256), 0, s, Count(NF), (const uint32_t*)order.p,
-                       (const uint32_t*)pid.p, key.p, r.p_faces.p);
-    sort_pairs(mem, key.p, r.p_faces.p, Count(NF), bits_for(NP), s);
+    scan_u32(mem, size.p, r.p_start.p, Count(NP), r.p_start.p + NP, s);
+    hipLaunchKernelGGL(k_patch_walk, dim3((unsigned)NP), dim3(kPatchLanes), 0, s, (const uint32_t*)seeds.p,
+                       (const uint32_t*)r.p_start.p, (const uint32_t*)r.view.f_vstart, (const uint32_t*)adj.p,
+                       (const uint4*)rows.p, claim.p, r.p_faces.p, err.p);
     RIN_HIP(hipGetLastError());
-    RIN_HIP(hipStreamSynchronize(s));
+    if (read1(err.p, s) != 0) throw std::runtime_error("patch search did not reach every face");
     r.have_patches = true;
 }
 
@@ -1274,7 +1247,7 @@ void compute_chains(DevMem& mem, RunOut& r, hipStream_t s) {
         r.have_chains = true;
         return;
     }
-    DBuf<uint32_t> vdeg(mem, NV + 1), vslot(mem, 2 * NV + 2), nb(mem, 2 * NE), parent(mem, NE), seen(mem, NE),
+    DBuf<uint32_t> vdeg(mem, NV + 1), vslot(mem, 2 * NV + 2), nb(mem, 2 * NE), parent(mem, NE),
         seed(mem, NE + 1), srank(mem, NE + 1), size(mem, NE + 1), seeds(mem, NE + 1), err(mem, 1);
     fill_u32(vdeg.p, 0, NV + 1, s);
     fill_u32(err.p, 0, 1, s);
@@ -1282,7 +1255,7 @@ void compute_chains(DevMem& mem, RunOut& r, hipStream_t s) {
     const uint32_t* es = r.e_start.p;
     hipLaunchKernelGGL(k_chain_vert, dim3(nblk(NE)), dim3(256), 0, s, Count(NE), v12, es, vdeg.p, vslot.p);
     hipLaunchKernelGGL(k_chain_links, dim3(nblk(NE)), dim3(256), 0, s, Count(NE), v12, es, (const uint32_t*)vdeg.p,
-                       (const uint32_t*)vslot.p, nb.p, parent.p, seen.p);
+                       (const uint32_t*)vslot.p, nb.p, parent.p);
     hipLaunchKernelGGL(k_chain_hook, dim3(nblk(2 * NE)), dim3(256), 0, s, Count(2 * NE), (const uint32_t*)nb.p,
                        parent.p);
     hipLaunchKernelGGL(k_chain_roots, dim3(nblk(NE)), dim3(256), 0, s, Count(NE), es, parent.p, seed.p);
@@ -1300,7 +1273,7 @@ void compute_chains(DevMem& mem, RunOut& r, hipStream_t s) {
                        (const uint32_t*)seed.p, (const uint32_t*)srank.p, size.p, seeds.p);
     scan_u32(mem, size.p, r.c_start.p, Count(NC), r.c_start.p + NC, s);
     hipLaunchKernelGGL(k_chain_walk, dim3(nblk(NC)), dim3(256), 0, s, Count(NC), (const uint32_t*)seeds.p,
-                       (const uint32_t*)r.c_start.p, (const uint32_t*)nb.p, seen.p, r.c_edges.p, err.p);
+                       (const uint32_t*)r.c_start.p, (const uint2*)nb.p, r.c_edges.p, err.p);
     RIN_HIP(hipGetLastError());
     if (read1(err.p, s) != 0) throw std::runtime_error("chain walk did not cover its component");
     RIN_HIP(hipStreamSynchronize(s));
