@@ -42,9 +42,8 @@ enum MICtr : uint32_t {
     M_ABORT,       // a count exceeded its capacity: later stages process nothing
     M_N
 };
-// kMiHuge: a tet has more than 8 materials (the large-capacity cut takes it)
+// kMiHuge: a tet has more than 8 materials (the wide cut takes it)
 constexpr uint32_t kMiOverflow = 1u << 8, kMiPlain = 1u << 9, kMiHuge = 1u << 10;
-constexpr unsigned kHugeBlocks = 4;  // lanes of the large-capacity cut: 4 x 64
 constexpr int kMiPub = 32;
 static_assert(M_N <= kMiPub, "published counters");
 
@@ -175,7 +174,7 @@ struct MIWorkspace {
     DBuf<uint16_t> rec;
     DBuf<uint64_t> emask;
     unsigned cut_blocks[2] = {0, 0};
-    DBuf<uint8_t> ws_huge;  // the large-capacity cut's complexes, once a run needs them
+    bool wide = false;  // the path holds the cut of more than 8 materials, once a run needs it
     // per complex face, occurrence, face
     DBuf<uint16_t> fl, fw, oj, fq_l;
     DBuf<uint64_t> ft, okey;
@@ -330,7 +329,7 @@ void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev
     const uint64_t V = G.V, T = G.T;
     const uint32_t F = val.F;
     MICaps c = W.cap;
-    c.huge = W.ws_huge.p ? 1u : 0u;
+    c.huge = W.wide ? 1u : 0u;
     uint32_t* ctr = W.ctr.p;
     const uint32_t* abort = ctr + M_ABORT;
     const double* vals = val.vals.p;
@@ -401,18 +400,20 @@ void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev
         hipLaunchKernelGGL((k_cut_group<CMed, 64, true>), dim3(g1), dim3(64), 0, s, G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, (const uint32_t*)bl[1], n1, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, 0, m3s);
+                           W.cnt.p, W.errs.p, 0, (uint32_t)0, m3s);
         hipLaunchKernelGGL((k_cut_group<CBig, 64, true>), dim3(g2), dim3(64), 0, s, G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, (const uint32_t*)bl[2], n2, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, 0, m3s);
+                           W.cnt.p, W.errs.p, 0, (uint32_t)0, m3s);
     }
-    if (W.ws_huge.p)
-        hipLaunchKernelGGL(k_cut_huge<true>, dim3(kHugeBlocks), dim3(64), 0, s, G, vals, (const uint32_t*)W.act.p,
-                           (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p, (const uint8_t*)W.fit.p,
-                           (const uint32_t*)bl[3], Count(ctr + M_LIST + 3, c.active, abort), (uint32_t)0,
-                           (const uint32_t*)W.rec_off.p, W.rec.p, W.cnt.p, W.errs.p, W.ws_huge.p,
-                           (const uint32_t*)nullptr, (uint32_t)0);
+    if (W.wide) {
+        const MI3Snap none{nullptr, nullptr, nullptr};
+        hipLaunchKernelGGL((k_cut_group<CWideMI, 64, true>), dim3((unsigned)std::min<uint64_t>(c.active + 1, 512)),
+                           dim3(64), 0, s, G, vals, (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p,
+                           (const uint32_t*)W.csr_off.p, (const uint8_t*)W.fit.p, (const uint32_t*)bl[3],
+                           Count(ctr + M_LIST + 3, c.active, abort), (const uint32_t*)W.rec_off.p, W.rec.p, W.cnt.p,
+                           W.errs.p, 0, (uint32_t)0, none);
+    }
     // extraction (src/extract_mesh.cpp:569-986): boundary-face pairing, then
     // occurrences in the reference's creation order
     MIArgs A;
@@ -595,12 +596,11 @@ void run_batched_mi(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t 
         std::memcpy(pub, w.pub_h, sizeof(pub));
         uint32_t e = pub[kMiPub];
         // a stopped or failed run may leave table entries
-        if ((e & ~kMiHuge) || ((e & kMiHuge) && !w.ws_huge.p)) w.hash_dirty = true;
+        if ((e & ~kMiHuge) || ((e & kMiHuge) && !w.wide)) w.hash_dirty = true;
         if (e & kMiPlain) throw NeedsPlainForm("a tet has more materials than the device cut holds");
-        if ((e & kMiHuge) && !w.ws_huge.p) {
-            // first run with such tets: room for the large-capacity cut, and
-            // the path captured again with its launch
-            w.ws_huge.alloc(w.mem, LaneCut<CHuge>::stride * 64 * kHugeBlocks);
+        if ((e & kMiHuge) && !w.wide) {
+            // first run with such tets: the path captured again with the wide cut
+            w.wide = true;
             w.drop_graph();
             continue;
         }

@@ -724,8 +724,8 @@ __device__ __forceinline__ int wave_mi_record(WaveMI<C>& X, int k, uint16_t* out
     const int lane = W::lane();
     const int L = 4 + k, nv = X.nv, nf = X.nf, nc = X.nc;
     // face word offsets: fpe is free after the insertions
-    static_assert(4 + C::MFV < 16, "face words fit four bits");
-    const uint32_t fwords = wave_prefix<G, 4>(
+    static_assert(4 + C::MFV < 32, "face words fit five bits");
+    const uint32_t fwords = wave_prefix<G, (4 + C::MFV < 16 ? 4 : 5)>(
         nf, [&](int f) { return (uint32_t)(4 + X.fn[f]); }, [&](int f, uint32_t o) { X.fpe[f] = (uint16_t)o; });
     const int total = 8 + 4 * nv + (int)fwords + nc + (X.dup ? L : 0);
     for (int v = lane; v < nv; v += G) X.used[v] = 0;

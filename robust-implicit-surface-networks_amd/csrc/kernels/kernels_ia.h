@@ -14,9 +14,14 @@ namespace {
 using dev::Complex;
 using CMed = dev::Caps<40, 64, 8, 8>;      // up to 4 active functions
 using CBig = dev::Caps<132, 284, 10, 12>;  // up to 8 active functions
-// more than 8 active functions (degenerate inputs: ties, coincident
-// functions; many functions on coarse grids) and complexes beyond a bucket's
-// capacities: up to 28 functions, 16-bit ids, the complex in device memory
+// more than 8 active functions (ties, coincident functions; many functions on
+// coarse grids): a wavefront a tet with the complex in LDS.  The functions of
+// a tet rarely all meet inside it, so 8-bit ids hold nearly every such
+// complex (all of them at 33^3 vertices and 32 functions)
+using CWide = dev::Caps<254, 640, 15, 32>;
+using CWideMI = dev::Caps<254, 360, 15, 32>;  // interfaces have fewer faces
+// complexes beyond those capacities: 16-bit ids, a lane a tet with the complex
+// in device memory
 using CHuge = dev::Caps<1023, 1500, 32, 32, uint16_t>;
 constexpr int kMaskWords = (CHuge::MV + 63) / 64;  // vertex masks of any record
 constexpr int kMaxHuge = CHuge::MP - 4;
@@ -60,9 +65,6 @@ __device__ inline uint32_t xcd_tile(uint32_t b, uint32_t n) {
 // [i * stride, (i + 1) * stride).  Kept out of the private segment, so the
 // runtime's per-queue scratch stays small and several queues can run cuts
 // at once.
-// lanes of a plain-form thread-cut launch (the grid strides beyond)
-constexpr uint64_t kCutLanes = 16384;
-
 template <class C>
 struct LaneCut {
     static constexpr size_t stride =
@@ -343,26 +345,7 @@ __device__ inline void cut_tet(const GridView& g, const double* __restrict__ val
     cnt[3 * a + 2] = a2;
 }
 
-template <class C, bool MI>
-__global__ void __launch_bounds__(64) k_cut(GridView g, const double* __restrict__ vals, const uint32_t* __restrict__ act,
-                                            const uint8_t* __restrict__ act_k, const uint32_t* __restrict__ csr_off,
-                                            const uint8_t* __restrict__ fit, Count n_active, int kmin, int kmax,
-                                            uint32_t flags, const uint32_t* __restrict__ rec_off,
-                                            uint16_t* __restrict__ rec, uint32_t* __restrict__ cnt,
-                                            uint32_t* __restrict__ errs, const uint32_t* __restrict__ list,
-                                            uint8_t* __restrict__ ws) {
-    const uint64_t lane = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    Complex<C>& X = LaneCut<C>::X(ws, lane);
-    dev::InsertTemps<C>& Tm = LaneCut<C>::T(ws, lane);
-    GRID_STRIDE(i, n_active) {
-        const uint64_t a = list ? list[i] : i;
-        const int k = act_k[a];
-        if (k < kmin || k > kmax) continue;
-        cut_tet<C, MI>(g, vals, act, csr_off, fit, a, k, flags, rec_off, rec, cnt, errs, X, Tm);
-    }
-}
-
-// The same with each lane's complex and working arrays in LDS (LANES lanes a
+// The thread cut with each lane's complex and working arrays in LDS (LANES lanes a
 // block, blockDim.x == LANES): for short lists, where one lane's latency
 // through its cut is the kernel's time and LDS answers several times faster
 // than the device-memory workspace.
@@ -566,6 +549,12 @@ __device__ __forceinline__ bool mi3_start(dev::WaveMI<C>& X, const MI3Snap& S, i
     return true;
 }
 
+// The plain form's cuts beyond the tables (and the batched material
+// interfaces'): a lane group a tet.  The -R check's counts come from here too
+// (RUN_CUT_ONLY: vertices, faces and cells, no record; RUN_REVERSE: the rows
+// in descending order): at 50^3 vertices and 8 functions one pass of that
+// check takes 0.25 ms of cuts, and took 4.7 ms a lane a tet, 1.4 ms of them
+// for a single tet of five functions.
 template <class C, int G, bool MI>
 __global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __restrict__ vals,
                                                   const uint32_t* __restrict__ act, const uint8_t* __restrict__ act_k,
@@ -573,7 +562,7 @@ __global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __re
                                                   const uint8_t* __restrict__ fit, const uint32_t* __restrict__ list,
                                                   Count nlist, const uint32_t* __restrict__ rec_off,
                                                   uint16_t* __restrict__ rec, uint32_t* __restrict__ cnt,
-                                                  uint32_t* __restrict__ errs, int retry,
+                                                  uint32_t* __restrict__ errs, int retry, uint32_t flags,
                                                   typename std::conditional<MI, MI3Snap, K2Snap>::type snap) {
     constexpr int NG = 64 / G;
     using Cx = typename std::conditional<MI, dev::WaveMI<C>, dev::WaveIA<C>>::type;
@@ -586,11 +575,14 @@ __global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __re
         const uint32_t a = list[i];
         const int k = act_k[a];
         const uint32_t t = act[a], s0 = csr_off[t];
-        if (lane < 4 * k && 4 + k <= C::MP) {
+        if (4 + k <= C::MP) {
             uint32_t v[4];
             dev::tet_corners(g, t, v);
-            const uint32_t f = fit[s0 + (lane >> 2)];
-            X.P[lane >> 2][lane & 3] = vals[(uint64_t)f * V + v[lane & 3]];
+            for (int q = lane; q < 4 * k; q += G) {
+                const int row = q >> 2;
+                const uint32_t f = fit[s0 + ((flags & RUN_REVERSE) ? k - 1 - row : row)];
+                X.P[row][q & 3] = vals[(uint64_t)f * V + v[q & 3]];
+            }
         }
         __syncthreads();
         if constexpr (MI) {
@@ -604,7 +596,12 @@ __global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __re
         const int cap = (int)(rec_off[a + 1] - rec_off[a]);
         uint32_t a0 = 0, a1 = 0, a2 = 0;
         int len = -1;
-        if (!X.err) {
+        if (!X.err && (flags & RUN_CUT_ONLY)) {
+            len = 0;
+            a0 = (uint32_t)X.nv;
+            a1 = (uint32_t)X.nf;
+            a2 = (uint32_t)X.nc;
+        } else if (!X.err) {
             if constexpr (MI)
                 len = dev::wave_mi_record<C, G>(X, k, out, cap, a0, a1, a2);
             else

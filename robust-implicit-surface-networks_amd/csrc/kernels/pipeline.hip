@@ -670,13 +670,12 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         RIN_HIP(hipGetLastError());
     }
     // the cuts beyond the tables: lane groups with the complex in LDS (the
-    // -R check's counts and reversed order take the thread cut)
-    const bool groups = !(flags & (RUN_REVERSE | RUN_CUT_ONLY));
+    // -R check's reversed order reverses a tet's rows)
     // the implicit-arrangement lane groups start from the k = 2 table's
     // complex after two planes (RIN_K2_START=0: they insert every plane)
     K2Snap k2s{nullptr, nullptr, nullptr};
     const char* ks = std::getenv("RIN_K2_START");
-    if (!MI && groups && !(ks && !std::strcmp(ks, "0"))) {
+    if (!MI && !(ks && !std::strcmp(ks, "0"))) {
         const void* pat = nullptr;
         plain_k2_snapshots(s, &pat, &k2s.off, &k2s.bytes);
         k2s.pat = static_cast<const K2Pat*>(pat);
@@ -685,11 +684,14 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     // complex after three materials (RIN_MI3_START=0: they insert every one)
     MI3Snap m3s{nullptr, nullptr, nullptr};
     const char* ms = std::getenv("RIN_MI3_START");
-    if (MI && groups && !(ms && !std::strcmp(ms, "0"))) {
+    if (MI && !(ms && !std::strcmp(ms, "0"))) {
         const MITablesDev TT = mi_tables_dev(s);
         m3s = MI3Snap{TT.pat3, TT.snap_off3, TT.snap3};
     }
-    for (int q = 0; q < 2 && NA && groups; ++q) {
+    // list 3 (more than 8 functions) by a wavefront a tet as well: a lane a
+    // tet took 6 to 45 ms for some hundred tets of 9..13 functions (33^3
+    // vertices, 32 functions), this takes 0.2 ms
+    for (int q = 2; q >= 0 && NA; --q) {
         const uint64_t nl = bcnt[1 + q];
         if (!nl) continue;
         auto go = [&](auto kernel, int per_wave, auto snap) {
@@ -698,46 +700,17 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
                                (const uint32_t*)out.act.p, (const uint8_t*)out.act_k.p,
                                (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p,
                                (const uint32_t*)blist[1 + q], Count(nl), (const uint32_t*)out.rec_off.p, out.rec.p,
-                               cnt.p, errs.p, 1, snap);
+                               cnt.p, errs.p, 1, flags, snap);
         };
         if (q == 0)
             MI ? go(k_cut_group<CMed, 64, true>, 1, m3s) : go(k_cut_group<CMed, 16, false>, 4, k2s);
-        else
+        else if (q == 1)
             MI ? go(k_cut_group<CBig, 64, true>, 1, m3s) : go(k_cut_group<CBig, 64, false>, 1, k2s);
-        RIN_HIP(hipGetLastError());
-    }
-    // each thread-per-tet cut kernel runs over its own k range only
-    DBuf<uint8_t> ws_cut[2];
-    for (int q = 0; q < 2 && NA && !groups; ++q) {
-        const uint64_t nl = bcnt[1 + q];
-        if (!nl) continue;
-        // lanes per workgroup (one wavefront): a lane runs a whole cut, whose
-        // loops diverge between lanes, so a short list runs faster with few
-        // lanes per wavefront as long as its wavefronts all fit on the GPU
-        // at once (about 2048 of these)
-        unsigned lanes = 2;
-        while (lanes < 64 && nl > (uint64_t)lanes * 2048) lanes *= 2;
-        // each lane's complex and working arrays in a device workspace; the
-        // grid strides over the list beyond kCutLanes lanes
-        const uint64_t nb = (nl + lanes - 1) / lanes;
-        const unsigned blocks = (unsigned)std::min<uint64_t>(nb, kCutLanes / lanes);
-        const int kmin = q == 0 ? 1 : 5, kmax = q == 0 ? 4 : 8;
-        const size_t stride = q == 0 ? LaneCut<CMed>::stride : LaneCut<CBig>::stride;
-        ws_cut[q].alloc(mem, stride * blocks * lanes);
-        auto go = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(lanes), 0, s, g.view, (const double*)val.vals.p,
-                               (const uint32_t*)out.act.p, (const uint8_t*)out.act_k.p,
-                               (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p, Count(nl), kmin, kmax, flags,
-                               (const uint32_t*)out.rec_off.p, out.rec.p, cnt.p, errs.p,
-                               (const uint32_t*)blist[1 + q], ws_cut[q].p);
-        };
-        if (q == 0)
-            MI ? go(k_cut<CMed, true>) : go(k_cut<CMed, false>);
         else
-            MI ? go(k_cut<CBig, true>) : go(k_cut<CBig, false>);
+            MI ? go(k_cut_group<CWideMI, 64, true>, 1, m3s) : go(k_cut_group<CWide, 64, false>, 1, k2s);
         RIN_HIP(hipGetLastError());
     }
-    // rare tets: one lane each, complexes in device memory; list: device
+    // complexes that outgrew those: one lane each, in device memory; list: device
     auto cut_large = [&](const uint32_t* list, uint64_t nl, const uint32_t* loc, uint32_t fixed_cap) {
         // ~200 KB of complex per lane: a few blocks
         const unsigned blocks = (unsigned)std::min<uint64_t>((nl + 63) / 64, 4);
@@ -753,7 +726,6 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         RIN_HIP(hipGetLastError());
         RIN_HIP(hipStreamSynchronize(s));  // the workspace returns to the pool
     };
-    if (bcnt[3]) cut_large(blist[3], bcnt[3], nullptr, 0);
     // record location of every active tet: its slot, or (after a retry) a slot
     // appended for a large complex
     out.rec_loc.alloc(mem, NA + 1);
