@@ -362,11 +362,15 @@ const K2Plans& k2_plans() {
     return P;
 }
 
-__device__ inline int bucket_of(int k) { return k <= 1 ? 0 : (k == 2 ? 1 : (k <= 4 ? 2 : (k <= 8 ? 3 : 4))); }
+// kbig: the most functions the last bucket takes (8, or kMaxHuge once a value
+// set has shown tets of more)
+__device__ inline int bucket_of(int k, int kbig) {
+    return k <= 1 ? 0 : (k == 2 ? 1 : (k <= 4 ? 2 : (k <= kbig ? 3 : 4)));
+}
 
 // per tet: active count and bucket histogram
 __global__ void k_filter_count(GridView g, const uint64_t* __restrict__ pos, const uint64_t* __restrict__ neg,
-                               uint64_t full, uint32_t* __restrict__ kcnt, uint32_t* __restrict__ isact,
+                               uint64_t full, int kbig, uint32_t* __restrict__ kcnt, uint32_t* __restrict__ isact,
                                uint32_t* __restrict__ ctr) {
     __shared__ uint32_t hist[8];
     if (threadIdx.x < 8) hist[threadIdx.x] = 0;
@@ -380,7 +384,8 @@ __global__ void k_filter_count(GridView g, const uint64_t* __restrict__ pos, con
         const uint32_t k = (uint32_t)__popcll(m);
         kcnt[t] = k;
         isact[t] = k != 0;
-        if (k) atomicAdd(&hist[bucket_of((int)k)], 1u);
+        if (k) atomicAdd(&hist[bucket_of((int)k, kbig)], 1u);
+        if (k > 8 && k <= (uint32_t)kbig) atomicAdd(&hist[4], 1u);  // the last field counts every tet of more than 8
     }
     __syncthreads();
     if (threadIdx.x < 5 && hist[threadIdx.x]) atomicAdd(&ctr[C_B1 + threadIdx.x], hist[threadIdx.x]);
@@ -397,7 +402,8 @@ struct FillArgs {
     uint32_t* act_off;  // CSR offset by active rank
     uint8_t* act_k;
     const K1Entry* k1;
-    uint32_t* list[3];      // buckets k=2, 3..4, 5..8
+    int kbig;
+    uint32_t* list[3];      // buckets k=2, 3..4, 5..kbig
     uint64_t* lts[3];       // per slot: CSR offset << 32 | tet
     uint32_t cap[3];
     uint32_t rec_base[3];   // word offsets of each bucket's slots
@@ -453,7 +459,7 @@ __global__ void k_fill_batched(FillArgs A) {
                     A.cnt[3 * r + 2] = E.nfv;
                     A.rec_loc[r] = K1_FLAG | (uint32_t)pat;
                 } else {
-                    b = k == 2 ? 0 : (k <= 4 ? 1 : (k <= 8 ? 2 : -1));
+                    b = k == 2 ? 0 : (k <= 4 ? 1 : (k <= A.kbig ? 2 : -1));
                     if (b < 0) A.errs[lane] |= 1;  // more active functions than the device cut supports
                 }
             }
@@ -562,7 +568,7 @@ __device__ inline void cube_masks(const GridView& g, uint32_t cube, const uint64
 }
 
 // Per tile of cubes: active functions, active tets and tets per bucket
-// (k = 1, 2, 3..4, 5..8, > 8).  No atomics: the tile scan below turns the
+// (k = 1, 2, 3..4, 5..kbig; and every tet with k > 8).  No atomics: the tile scan below turns the
 // tile sums into prefixes (the CSR offsets and the bucket-list slots of each
 // tile) and writes the totals, so the bucket lists come out in tet order.
 constexpr int kTileFields = 8;
@@ -590,7 +596,7 @@ struct EarlyEntry {
 // are contiguous and in tet order (the back part reversed).
 template <int TILE>
 __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const uint64_t* __restrict__ pos,
-                                                          const uint64_t* __restrict__ neg, uint64_t full,
+                                                          const uint64_t* __restrict__ neg, uint64_t full, int kbig,
                                                           TileSums* __restrict__ tile_sums, EarlyEntry* early3,
                                                           EarlyEntry* early5, uint32_t early_cap3,
                                                           uint32_t early_cap5, uint32_t* ctr) {
@@ -608,7 +614,11 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const uint64_t*
             const int k = __popcll(m[q]);
             v[TF_FIT] += (uint32_t)k;
             v[TF_ACTIVE] += k != 0;
-            if (k) v[TF_B1 + bucket_of(k)]++;
+            v[TF_B1] += k == 1;
+            v[TF_B2] += k == 2;
+            v[TF_B3] += k == 3 || k == 4;
+            v[TF_B5] += k >= 5 && k <= kbig;
+            v[TF_BX] += k > 8;
             n4 += k == 4;
         }
     }
@@ -671,7 +681,7 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const uint64_t*
                     const uint32_t back = ebase[2] + b3++;
                     if (back < early_cap3) early3[early_cap3 - 1 - back] = {t, tile, lo, lr | rank << 16};
                 }
-            } else if (k >= 5 && k <= 8 && early5) {
+            } else if (k >= 5 && k <= kbig && early5) {
                 const uint32_t at = ebase[1] + b5;
                 if (at < early_cap5) early5[at] = {t, tile, lo, lr | b5 << 16};
                 ++b5;
@@ -779,7 +789,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
         const int k = __popcll(m[q]);
         ks += (uint32_t)k;
         as += k != 0;
-        if (k >= 2 && k <= 8) bp += 1u << (10 * (k == 2 ? 0 : (k <= 4 ? 1 : 2)));
+        if (k >= 2 && k <= A.kbig) bp += 1u << (10 * (k == 2 ? 0 : (k <= 4 ? 1 : 2)));
     }
     // bucket slots: the tile's prefix, the waves before this one, the lanes
     // before this one (a wave holds at most 320 tets of a list)
@@ -832,7 +842,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
                     A.cnt[3 * r + 1] = E.nif;
                     A.cnt[3 * r + 2] = E.nfv;
                     A.rec_loc[r] = K1_FLAG | (uint32_t)pat[q];
-                } else if (k <= 8) {
+                } else if (k <= A.kbig) {
                     const int qq = k == 2 ? 0 : (k <= 4 ? 1 : 2);
                     const uint32_t slot = bnext[qq]++;
                     if (slot < A.cap[qq]) {
@@ -887,6 +897,7 @@ struct CutArgs {
     uint64_t full;
     uint32_t rec_base, cap_active;
     int tf;
+    int kmin, kmax;  // the tets of the list that this launch cuts
     K2Snap k2s;  // lane-group forms: the complexes after two planes (off null: none)
 };
 
@@ -905,6 +916,7 @@ __global__ void __launch_bounds__(64) k_cut_bucket(CutArgs A) {
         if (i >= n) continue;
         const uint32_t r = A.list[i];
         const int k = A.act_k[r];
+        if (k < A.kmin || k > A.kmax) continue;
         const uint32_t t = A.act[r];
         uint32_t v[4];
         dev::tet_corners(A.g, t, v);
@@ -977,13 +989,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
         const uint64_t m = A.full & ~((A.pos[v[0]] & A.pos[v[1]] & A.pos[v[2]] & A.pos[v[3]]) |
                                       (A.neg[v[0]] & A.neg[v[1]] & A.neg[v[2]] & A.neg[v[3]]));
         k = __popcll(m);
-        if (lane < 4 * (C::MP - 4)) {
+        if (k < A.kmin || k > A.kmax) return;
+        for (int e4 = lane; e4 < 4 * (C::MP - 4); e4 += G) {
             // row q: the q-th active function (rows past k load function 0, unused)
             uint64_t mm = m;
-            for (int q = lane >> 2; q > 0 && mm; --q) mm &= mm - 1;
+            for (int q = e4 >> 2; q > 0 && mm; --q) mm &= mm - 1;
             const uint32_t f = mm ? (uint32_t)(__ffsll((unsigned long long)mm) - 1) : 0u;
-            const double x = A.vals[(uint64_t)f * A.g.V + v[lane & 3]];
-            if (lane < 4 * k && 4 + k <= C::MP) X.P[lane >> 2][lane & 3] = x;
+            const double x = A.vals[(uint64_t)f * A.g.V + v[e4 & 3]];
+            if (e4 < 4 * k && 4 + k <= C::MP) X.P[e4 >> 2][e4 & 3] = x;
         }
     } else {
         const uint32_t n = *A.abort ? 0u : min(*A.n, A.cap);
@@ -991,18 +1004,19 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
         r = A.list[i];
         const uint64_t ts = A.lts[i];
         k = A.act_k[r];
+        if (k < A.kmin || k > A.kmax) return;
         rec_at = 0;
         // corner values: the loads need not wait for k (rows past the tet's
         // functions read the CSR's next entries, inside its head-room of 64,
         // with the function id clamped into range; their values go unused)
-        if (lane < 4 * (C::MP - 4)) {
-            const uint32_t t = (uint32_t)ts, s0 = (uint32_t)(ts >> 32);
-            uint32_t v[4];
-            dev::tet_corners(A.g, t, v);
-            const uint32_t fr = A.fit[s0 + (lane >> 2)];
+        const uint32_t t = (uint32_t)ts, s0 = (uint32_t)(ts >> 32);
+        uint32_t v[4];
+        dev::tet_corners(A.g, t, v);
+        for (int e4 = lane; e4 < 4 * (C::MP - 4); e4 += G) {
+            const uint32_t fr = A.fit[s0 + (e4 >> 2)];
             const uint32_t f = fr < A.F ? fr : 0u;
-            const double x = A.vals[(uint64_t)f * A.g.V + v[lane & 3]];
-            if (lane < 4 * k && 4 + k <= C::MP) X.P[lane >> 2][lane & 3] = x;
+            const double x = A.vals[(uint64_t)f * A.g.V + v[e4 & 3]];
+            if (e4 < 4 * k && 4 + k <= C::MP) X.P[e4 >> 2][e4 & 3] = x;
         }
     }
     int start = 0;
@@ -1431,9 +1445,9 @@ __global__ void k_extract_records(ExtractArgs A) { extract_rec_role(A, blockIdx.
 // the iso flags, so many waves stay resident to cover the loads.
 // Occurrences and face rows come out in the order one lane per tet gives.
 struct WaveExtractLds {
-    uint16_t fo[CBig::MF];
-    uint32_t isov[(CBig::MV + 31) / 32];
-    uint8_t isof[CBig::MF];
+    uint16_t fo[CWide::MF];
+    uint32_t isov[(CWide::MV + 31) / 32];
+    uint8_t isof[CWide::MF];
 };
 
 __device__ inline void extract_wave_role(const ExtractArgs& A, WaveExtractLds& S, uint32_t blk) {
@@ -1453,7 +1467,7 @@ __device__ inline void extract_wave_role(const ExtractArgs& A, WaveExtractLds& S
     if (W[0] != 1) return;
     const uint32_t len = W[6];
     const int nv = W[2], nf = W[3], L = W[1];
-    if (nv > CBig::MV || nf > CBig::MF || len < 8u + 4u * nv) {
+    if (nv > CWide::MV || nf > CWide::MF || len < 8u + 4u * nv) {
         if (lane == 0) A.errs[0] |= ERR_RECORD;
         return;
     }
@@ -1703,6 +1717,11 @@ struct Workspace {
     // words per record slot: the largest record a bucket's capacity allows
     // (header, vertices, faces with their cycles, coincidence groups)
     uint32_t slot[3] = {rec_words<CK2>(), rec_words<CMed>(), rec_words<CBig>()};
+    // value sets of this plan have tets of more than 8 functions: they join
+    // the last bucket, whose slots grow, and the wide cut takes them (such a
+    // run was handed to the plain form: 3.9 ms against 2.8 ms for a job of 32
+    // functions at 33^3 vertices, 1.9 ms of either the copies to the host)
+    bool wide = false;
     bool wave_cut[3] = {false, false, false};  // bucket cut by the wave form (records carry face offsets)
     DBuf<uint64_t> pos, neg;
     DBuf<uint32_t> kcnt, isact, csr_off, rank, act, rec_loc, cnt, list[3];
@@ -1759,8 +1778,8 @@ struct Workspace {
     hipGraphExec_t whole = nullptr;
     // side branches of the whole graph (the cut kernels beside each other and
     // beside the fill pass): streams to capture them on, fork and join events
-    hipStream_t side = nullptr, side2 = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr;
+    hipStream_t side = nullptr, side2 = nullptr, side3 = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr, join3 = nullptr;
     // pinned, device-mapped summary the closing kernel of a run writes (counters
     // and error flags), read by the host after the stream synchronises
     uint32_t* pub_h = nullptr;
@@ -1794,6 +1813,8 @@ struct Workspace {
         if (fork) (void)hipEventDestroy(fork);
         if (join) (void)hipEventDestroy(join);
         if (join2) (void)hipEventDestroy(join2);
+        if (join3) (void)hipEventDestroy(join3);
+        if (side3) (void)hipStreamDestroy(side3);
         if (side2) (void)hipStreamDestroy(side2);
         if (side) (void)hipStreamDestroy(side);
         if (pub_h) (void)hipHostFree(pub_h);
@@ -1805,6 +1826,7 @@ struct Plan {
     std::vector<std::shared_ptr<Workspace>> ws;
     int blocks_per_cu[3] = {0, 0, 0};  // autotuned grid of each bucket's cut kernel
     int cube_tile = 0;                  // autotuned cube tile of the count and fill passes (0: not yet)
+    bool wide = false;                  // new workspaces start wide
     uint32_t hint_b[5] = {0, 0, 0, 0, 0};
 };
 
@@ -1894,6 +1916,7 @@ unsigned cube_tiles(const Grid& g, int tile = kCubeTile) {
 
 void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
     W.cap = c;
+    W.slot[2] = W.wide ? rec_words<CWide>() : rec_words<CBig>();
     DevMem& m = W.mem;
     const uint64_t V = g.view.V, T = g.view.T;
     W.pos.alloc(m, V);
@@ -2019,11 +2042,12 @@ void stage_count(Workspace& W, const Grid& g, const Values& val, hipStream_t s, 
     hipLaunchKernelGGL(k_signs_count, dim3(nblk(V, 1024)), dim3(1024), 0, s, (const double*)val.vals.p, V, F, W.pos.p,
                        W.neg.p, W.ctr.p);
     const uint64_t full = (F == 64) ? ~0ull : ((1ull << F) - 1);
+    const int kbig = W.wide ? kMaxHuge : 8;
     if (g.view.regular) {
         const int tile = W.cube_tile;
         auto count = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, g.view, (const uint64_t*)W.pos.p,
-                               (const uint64_t*)W.neg.p, full, W.tile_sums.p, early3 ? W.early[1].p : nullptr,
+                               (const uint64_t*)W.neg.p, full, kbig, W.tile_sums.p, early3 ? W.early[1].p : nullptr,
                                early5 ? W.early[2].p : nullptr, W.cap.b[1], W.cap.b[2], W.ctr.p);
         };
         if (tile == 256)
@@ -2037,7 +2061,7 @@ void stage_count(Workspace& W, const Grid& g, const Values& val, hipStream_t s, 
         return;
     }
     hipLaunchKernelGGL(k_filter_count, dim3(nblk(T)), dim3(256), 0, s, g.view, (const uint64_t*)W.pos.p,
-                       (const uint64_t*)W.neg.p, full, W.kcnt.p, W.isact.p, W.ctr.p);
+                       (const uint64_t*)W.neg.p, full, kbig, W.kcnt.p, W.isact.p, W.ctr.p);
     scan_u32(W.mem, W.kcnt.p, W.csr_off.p, Count(T), W.ctr.p + C_FIT, s);
     scan_u32(W.mem, W.isact.p, W.rank.p, Count(T), W.ctr.p + C_ACTIVE, s);
 }
@@ -2089,9 +2113,18 @@ void launch_cut(Workspace& W, const Grid& g, const Values& val, int q, int grid,
     A.cnt = W.cnt.p;
     A.errs = W.errs.p;
     A.ctr = W.ctr.p;
+    A.kmin = 0;
+    A.kmax = q == 2 ? 8 : kMaxHuge;
     A.stat_k = q == 1 ? SP_CUTK3 : (q == 2 ? SP_CUTK5 : -1);
     A.stat_w = q == 1 ? SP_CUTW3 : (q == 2 ? SP_CUTW5 : -1);
     A.k2s = W.k2_start ? K2Snap{W.k2pat.p, W.k2snap_off.p, W.k2snap.p} : K2Snap{nullptr, nullptr, nullptr};
+    if (W.wide && q == 2) {  // the list's tets of more than 8 functions
+        CutArgs B = A;
+        B.kmin = 9;
+        B.kmax = kMaxHuge;
+        B.stat_k = B.stat_w = -1;
+        hipLaunchKernelGGL((k_cut_wave<CWide, 64>), dim3(W.cap.b[q]), dim3(64), 0, s, B);
+    }
     if (grid == -2) {  // k = 2 table
         K2Args K = k2_args(W, g, val);
         K.n = A.n;
@@ -2125,7 +2158,9 @@ void launch_cut(Workspace& W, const Grid& g, const Values& val, int q, int grid,
 // the k = 3..4 (q = 1) or 5..8 (q = 2) cut from the count pass's list,
 // beside the fill pass (regular grids, lane-group forms: grid -1, or -3 for
 // four tets a wavefront)
-void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int grid, hipStream_t s) {
+// wide: the tets of the last list with more than 8 functions
+void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int grid, hipStream_t s,
+                      bool wide = false) {
     CutArgs A = {};
     A.g = g.view;
     A.vals = val.vals.p;
@@ -2136,8 +2171,10 @@ void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int
     A.cnt = W.cnt.p;
     A.errs = W.errs.p;
     A.ctr = W.ctr.p;
-    A.stat_k = q == 1 ? SP_CUTK3 : SP_CUTK5;
-    A.stat_w = q == 1 ? SP_CUTW3 : SP_CUTW5;
+    A.kmin = wide ? 9 : 0;
+    A.kmax = wide ? kMaxHuge : 8;
+    A.stat_k = wide ? -1 : (q == 1 ? SP_CUTK3 : SP_CUTK5);
+    A.stat_w = wide ? -1 : (q == 1 ? SP_CUTW3 : SP_CUTW5);
     A.early = W.early[q].p;
     A.n_early = W.ctr.p + (q == 1 ? C_E3 : C_E5);
     A.n_back = q == 1 ? W.ctr.p + C_E3B : nullptr;
@@ -2150,7 +2187,9 @@ void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int
     A.tf = q == 1 ? TF_B3 : TF_B5;
     A.k2s = W.k2_start ? K2Snap{W.k2pat.p, W.k2snap_off.p, W.k2snap.p} : K2Snap{nullptr, nullptr, nullptr};
     const uint32_t cap = W.cap.b[q];
-    if (q == 2)
+    if (wide)
+        hipLaunchKernelGGL((k_cut_wave<CWide, 64, true>), dim3(cap), dim3(64), 0, s, A);
+    else if (q == 2)
         hipLaunchKernelGGL((k_cut_wave<CBig, 64, true>), dim3(cap), dim3(64), 0, s, A);
     else if (grid == -3)
         hipLaunchKernelGGL((k_cut_wave<CMed, 16, true>), dim3((cap + 3) / 4), dim3(64), 0, s, A);
@@ -2181,6 +2220,7 @@ void stage_fill(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
     A.cnt = W.cnt.p;
     A.act_k = W.act_k.p;
     A.k1 = W.k1.p;
+    A.kbig = W.wide ? kMaxHuge : 8;
     for (int q = 0; q < 3; ++q) {
         A.list[q] = W.list[q].p;
         A.lts[q] = W.lts[q].p;
@@ -2411,8 +2451,8 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
 
 // conservative per-tet output bounds by active count (maxima of the cut's
 // vertex / face counts, see the capacities of the bucket kernels)
-void caps_from_counts(const uint32_t* ctr, Caps_& c) {
-    const uint64_t b1 = ctr[C_B1], b2 = ctr[C_B2], b3 = ctr[C_B3], b5 = ctr[C_B5];
+void caps_from_counts(const uint32_t* ctr, bool wide, Caps_& c) {
+    const uint64_t b1 = ctr[C_B1], b2 = ctr[C_B2], b3 = ctr[C_B3], bx = wide ? ctr[C_BX] : 0, b5 = ctr[C_B5] - bx;
     auto clamp = [](uint64_t x) -> uint32_t {
         if (x >= (1ull << 31)) throw std::runtime_error("workspace capacity exceeds 2^31 entries");
         return (uint32_t)x;
@@ -2421,10 +2461,10 @@ void caps_from_counts(const uint32_t* ctr, Caps_& c) {
     c.fit = clamp(ctr[C_FIT] + 64);
     c.b[0] = clamp(b2 + 64);
     c.b[1] = clamp(b3 + 64);
-    c.b[2] = clamp(b5 + 64);
-    c.vo = clamp(4 * b1 + 16 * b2 + 40 * b3 + 132 * b5 + 64);
-    c.fo = clamp(1 * b1 + 24 * b2 + 64 * b3 + 284 * b5 + 64);
-    c.fv = clamp(4 * b1 + 24 * 6 * b2 + 64 * 8 * b3 + 284 * 10 * b5 + 64);
+    c.b[2] = clamp(b5 + bx + 64);
+    c.vo = clamp(4 * b1 + 16 * b2 + 40 * b3 + 132 * b5 + (uint64_t)CWide::MV * bx + 64);
+    c.fo = clamp(1 * b1 + 24 * b2 + 64 * b3 + 284 * b5 + (uint64_t)CWide::MF * bx + 64);
+    c.fv = clamp(4 * b1 + 24 * 6 * b2 + 64 * 8 * b3 + 284 * 10 * b5 + (uint64_t)CWide::MF * CWide::MFV * bx + 64);
 }
 
 bool caps_ok(const Caps_& have, const Caps_& need) {
@@ -2516,6 +2556,10 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         RIN_HIP(hipStreamCreateWithFlags(&w.side2, hipStreamNonBlocking));
         RIN_HIP(hipEventCreateWithFlags(&w.join2, hipEventDisableTiming));
     }
+    if (w.wide && !w.side3) {
+        RIN_HIP(hipStreamCreateWithFlags(&w.side3, hipStreamNonBlocking));
+        RIN_HIP(hipEventCreateWithFlags(&w.join3, hipEventDisableTiming));
+    }
     hipGraph_t gr = nullptr;
     RIN_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
     // regular grids with lane-group cuts start them right after the counts,
@@ -2535,6 +2579,11 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
             RIN_HIP(hipStreamWaitEvent(w.side, w.fork, 0));
             launch_cut_early(w, g, val, 2, w.grid[2], w.side);
             RIN_HIP(hipEventRecord(w.join, w.side));
+            if (w.wide) {
+                RIN_HIP(hipStreamWaitEvent(w.side3, w.fork, 0));
+                launch_cut_early(w, g, val, 2, w.grid[2], w.side3, true);
+                RIN_HIP(hipEventRecord(w.join3, w.side3));
+            }
         }
         RIN_HIP(hipStreamWaitEvent(w.side2, w.fork, 0));
         stage_fill(w, g, val, w.side2);
@@ -2543,6 +2592,7 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         if (w.cap.b[0]) launch_cut<CK2>(w, g, val, 0, w.grid[0], w.side2);
         RIN_HIP(hipEventRecord(w.join2, w.side2));
         if (e5) RIN_HIP(hipStreamWaitEvent(s, w.join, 0));
+        if (e5 && w.wide) RIN_HIP(hipStreamWaitEvent(s, w.join3, 0));
         RIN_HIP(hipStreamWaitEvent(s, w.join2, 0));
     } else {
         stage_fill(w, g, val, s);
@@ -2636,6 +2686,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         }
     if (!W) {
         W = std::make_shared<Workspace>();
+        W->wide = P.wide;
         P.ws.push_back(W);
     }
     Workspace& w = *W;
@@ -2658,7 +2709,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
     };
     auto errors = [&] { return herr; };
     bool ran = false;
-    for (int attempt = 0; attempt < 3 && !ran; ++attempt) {
+    for (int attempt = 0; attempt < 4 && !ran; ++attempt) {
         if (!w.exec) {
             w.ctr_clear = false;  // the eager passes below use the counters
             // size the workspace from an eager counting pass
@@ -2671,9 +2722,15 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             }
             stage_count(w, g, val, s);
             read_back(true);
-            if (hctr[C_BX]) throw NeedsPlainForm("a tet has more than 8 active functions");
+            if (hctr[C_BX] && !w.wide) {
+                // larger slots for the last bucket, and the counts with it
+                w.wide = P.wide = true;
+                w.cap = Caps_{};
+                stage_count(w, g, val, s);
+                read_back(true);
+            }
             Caps_ need;
-            caps_from_counts(hctr, need);
+            caps_from_counts(hctr, w.wide, need);
             if (!caps_ok(w.cap, need)) {
                 // grow with head-room, keeping the k=1 table
                 Caps_ grow = need;
@@ -2804,6 +2861,11 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             w.exec = false;
             continue;
         }
+        if (e && hctr[C_BX] && !w.wide) {  // the first value set with tets of more than 8 functions
+            w.drop_graphs();
+            w.exec = false;
+            continue;
+        }
         if (e) {
             out.err = e;
             throw NeedsPlainForm("a complex exceeds the bucket capacities or the predicate range");
@@ -2842,7 +2904,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
     out.n_face_occ = hctr[C_FO];
     out.n_face_occ_verts = hctr[C_FV];
     out.n_cut34 = hctr[C_B3];
-    out.n_cut58 = hctr[C_B5];
+    out.n_cut58 = hctr[C_B5] - (w.wide ? hctr[C_BX] : 0u);
     out.n_rec_words = hctr[C_RECW];
     out.cut_k_sum[0] = hctr[C_CUTK3];
     out.cut_k_sum[1] = hctr[C_CUTK5];

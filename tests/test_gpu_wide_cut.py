@@ -28,21 +28,32 @@ CASES = [(0, 9, 0.8), (0, 12, 0.8), (0, 16, 0.9), (0, 24, 0.9), (1, 9, 0.1), (1,
 
 
 @pytest.mark.parametrize("mi,F,spread", CASES)
-def test_more_than_eight(ctx, mi, F, spread):
+@pytest.mark.parametrize("regular", [True, False])
+def test_more_than_eight(ctx, mi, F, spread, regular):
     import rin
 
     res = 2
-    g = ctx.grid_regular(res)
+    pts, tets = S.grid(res)
+    g = ctx.grid_regular(res) if regular else ctx.grid_explicit(pts, tets)
     fs = _set(mi, F, spread)
     vals = g.eval(*fs.arrays())
-    pts, tets = S.grid(res)
     ref = S.OracleRun(mi, pts, tets, S.evaluate(*fs.arrays(), pts))
     assert np.diff(ref.start_index.astype(np.int64)).max() > 8
     base = rin.FLAG_MI if mi else 0
     for flags in (0, rin.FLAG_NO_LOOKUP, rin.FLAG_BATCHED, rin.FLAG_BATCHED):
         dev = vals.run(base | flags)
         _compare(dev, ref)
+        if flags == rin.FLAG_BATCHED and not mi:  # the batched form hands over what outgrows the LDS complex only
+            assert (dev.stage_times()[0][0] == "batched path (one graph)") == (F < 24)
         dev.release()
+    # another value set of the same plan, all of its tets with 8 functions or fewer
+    few = S.evaluate(*fs.arrays(), pts)
+    few[:, 8:] = -9.0 if mi else 1.0
+    v2 = g.upload(few)
+    dev = v2.run(base | rin.FLAG_BATCHED)
+    _compare(dev, S.OracleRun(mi, pts, tets, few))
+    dev.release()
+    v2.release()
     vals.release()
     g.release()
 
