@@ -173,9 +173,8 @@ def d2h_ms(res_obj, reps=3):
 def fresh_values_leg(ctx, res, n_sets, steps):
     """Batched runs that switch value sets every step: n_sets seeded function
     sets of the headline shape (6 planes, 6 spheres, 4 cylinders, 4 tori) on
-    one grid, values resident; each switch re-records the captured graph and
-    updates it in place.  Also the first run on a new grid (counting pass,
-    tuning, capture)."""
+    one grid, values resident (one captured graph serves them all).  Also the
+    first run on a new grid (counting pass, tuning, capture)."""
     import numpy as np
 
     import rin

@@ -492,7 +492,9 @@ __global__ void k_fill_batched(FillArgs A) {
 // caches 37.6 us against 40.6 us at 256; streaming loads, as ordinary loads
 // took 72 us when the caches held other kernels' dirty lines)
 __global__ void __launch_bounds__(1024) k_signs_count(const double* __restrict__ vals, uint64_t V, uint32_t F, uint64_t* __restrict__ pos,
-                              uint64_t* __restrict__ neg, uint32_t* __restrict__ ctr) {
+                              uint64_t* __restrict__ neg, uint32_t* __restrict__ ctr, const double** __restrict__ slot) {
+    // the later kernels, captured once per workspace, find the values here
+    if (blockIdx.x == 0 && threadIdx.x == 0) *slot = vals;
     uint32_t z = 0;
     GRID_STRIDE(v, V) {
         uint64_t p = 0, n = 0;
@@ -873,7 +875,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
 
 struct CutArgs {
     GridView g;
-    const double* vals;
+    const double* const* vals;  // where the signs pass left the run's values
     const uint32_t *act, *csr_off, *list, *rec_loc;
     const uint64_t* lts;  // per slot: CSR offset << 32 | tet
     const uint8_t *act_k, *fit;
@@ -924,7 +926,7 @@ __global__ void __launch_bounds__(64) k_cut_bucket(CutArgs A) {
         double P[C::MP - 4][4];
         for (int q = 0; q < k; ++q) {
             const uint32_t f = A.fit[s0 + q];
-            for (int c = 0; c < 4; ++c) P[q][c] = A.vals[(uint64_t)f * V + v[c]];
+            for (int c = 0; c < 4; ++c) P[q][c] = (*A.vals)[(uint64_t)f * V + v[c]];
         }
         const uint64_t slot = (uint64_t)blockIdx.x * 64 + lane;
         dev::Complex<C>& X = LaneCut<C>::X(A.ws, slot);
@@ -966,6 +968,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
     __shared__ dev::WaveIA<C> Xs[NG];
     const int gid = threadIdx.x / G, lane = threadIdx.x & (G - 1);
     dev::WaveIA<C>& X = Xs[gid];
+    const double* __restrict__ vals = *A.vals;
     const uint32_t i = blockIdx.x * NG + gid;
     uint32_t r, rec_at;
     int k;
@@ -995,7 +998,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
             uint64_t mm = m;
             for (int q = e4 >> 2; q > 0 && mm; --q) mm &= mm - 1;
             const uint32_t f = mm ? (uint32_t)(__ffsll((unsigned long long)mm) - 1) : 0u;
-            const double x = A.vals[(uint64_t)f * A.g.V + v[e4 & 3]];
+            const double x = vals[(uint64_t)f * A.g.V + v[e4 & 3]];
             if (e4 < 4 * k && 4 + k <= C::MP) X.P[e4 >> 2][e4 & 3] = x;
         }
     } else {
@@ -1015,7 +1018,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
         for (int e4 = lane; e4 < 4 * (C::MP - 4); e4 += G) {
             const uint32_t fr = A.fit[s0 + (e4 >> 2)];
             const uint32_t f = fr < A.F ? fr : 0u;
-            const double x = A.vals[(uint64_t)f * A.g.V + v[e4 & 3]];
+            const double x = vals[(uint64_t)f * A.g.V + v[e4 & 3]];
             if (e4 < 4 * k && 4 + k <= C::MP) X.P[e4 >> 2][e4 & 3] = x;
         }
     }
@@ -1052,7 +1055,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
 
 struct K2Args {
     GridView g;
-    const double* vals;
+    const double* const* vals;  // where the signs pass left the run's values
     const uint64_t *pos, *neg;
     uint64_t full;  // the functions' bits
     const uint32_t *act, *csr_off, *list;
@@ -1074,6 +1077,7 @@ struct K2Args {
 __device__ __forceinline__ uint32_t k2_table_slot(const K2Args& A, const K2Pat* pats, const uint32_t* v, uint32_t fa,
                                                   uint32_t fb) {
     const uint64_t V = A.g.V;
+    const double* __restrict__ vals = *A.vals;
     int pa = 0, sB[4];
     for (int c = 0, w = 1; c < 4; ++c, w *= 3) {
         const uint64_t p = A.pos[v[c]], q = A.neg[v[c]];
@@ -1089,8 +1093,8 @@ __device__ __forceinline__ uint32_t k2_table_slot(const K2Args& A, const K2Pat* 
         int sg;
         if (sB[c1] * sB[c2] < 0) {
             // second plane at the point of edge c1 c2 where the first vanishes
-            sg = dev::orient_ia_edge(A.vals[(uint64_t)fa * V + v[c1]], A.vals[(uint64_t)fa * V + v[c2]],
-                                     A.vals[(uint64_t)fb * V + v[c1]], A.vals[(uint64_t)fb * V + v[c2]], err);
+            sg = dev::orient_ia_edge(vals[(uint64_t)fa * V + v[c1]], vals[(uint64_t)fa * V + v[c2]],
+                                     vals[(uint64_t)fb * V + v[c1]], vals[(uint64_t)fb * V + v[c2]], err);
         } else {
             sg = sB[c1] == sB[c2] ? sB[c1] : (sB[c1] != 0 ? sB[c1] : sB[c2]);
         }
@@ -1723,6 +1727,7 @@ struct Workspace {
     // functions at 33^3 vertices, 1.9 ms of either the copies to the host)
     bool wide = false;
     bool wave_cut[3] = {false, false, false};  // bucket cut by the wave form (records carry face offsets)
+    DBuf<const double*> vals_at;  // the run's values, left by its signs pass for the captured kernels
     DBuf<uint64_t> pos, neg;
     DBuf<uint32_t> kcnt, isact, csr_off, rank, act, rec_loc, cnt, list[3];
     DBuf<uint64_t> lts[3];  // per bucket slot: CSR offset << 32 | tet
@@ -1786,9 +1791,8 @@ struct Workspace {
     uint32_t* pub_d = nullptr;
     bool exec = false;  // graphs captured for the current capacities
     int grid[3] = {0, 0, 0};  // cut kernels' grids the graphs were captured with
-    // the values the whole graph and the per-stage graphs read (a run with
-    // other values of the same size re-records the graph and updates it in place)
-    const double* bound_whole = nullptr;
+    // the values the per-stage graphs' signs pass reads (a run with others
+    // records them again)
     const double* bound_parts = nullptr;
     bool ctr_clear = false;  // counters and error flags are zero (left so by the last run)
     bool in_use = false;
@@ -1805,7 +1809,6 @@ struct Workspace {
         if (whole_graph) (void)hipGraphDestroy(whole_graph);
         whole = nullptr;
         whole_graph = nullptr;
-        bound_whole = nullptr;
     }
     ~Workspace() {
         drop_graphs();
@@ -1919,6 +1922,7 @@ void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
     W.slot[2] = W.wide ? rec_words<CWide>() : rec_words<CBig>();
     DevMem& m = W.mem;
     const uint64_t V = g.view.V, T = g.view.T;
+    W.vals_at.alloc(m, 1);
     W.pos.alloc(m, V);
     W.neg.alloc(m, V);
     if (g.view.regular) {
@@ -2031,16 +2035,21 @@ void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
 }
 
 // stage 1 (also run eagerly to size the workspace): signs, filter, and
-// either the per-tile sums (regular grids) or the per-tet CSR scans; zero:
-// clear the counters first (the whole-path graph leaves them clear instead)
+// either the per-tile sums (regular grids) or the per-tet CSR scans.  The
+// signs pass is launched for each run, before the path's graph: it is the one
+// kernel that is given the values, and runs while the host launches the
+// graph; zero: clear the counters first (a whole run leaves them clear)
 // early3, early5: list the k = 3..4 / 5..8 tets for launch_cut_early (regular grids)
-void stage_count(Workspace& W, const Grid& g, const Values& val, hipStream_t s, bool zero = true,
-                 bool early3 = false, bool early5 = false) {
-    const uint64_t V = g.view.V, T = g.view.T;
-    const uint32_t F = val.F;
+void stage_signs(Workspace& W, const Grid& g, const Values& val, hipStream_t s, bool zero) {
     if (zero) hipLaunchKernelGGL(k_zero_ctr, dim3(1), dim3(64), 0, s, W.ctr.p, (int)C_N, W.errs.p);
-    hipLaunchKernelGGL(k_signs_count, dim3(nblk(V, 1024)), dim3(1024), 0, s, (const double*)val.vals.p, V, F, W.pos.p,
-                       W.neg.p, W.ctr.p);
+    hipLaunchKernelGGL(k_signs_count, dim3(nblk(g.view.V, 1024)), dim3(1024), 0, s, (const double*)val.vals.p, g.view.V,
+                       val.F, W.pos.p, W.neg.p, W.ctr.p, W.vals_at.p);
+}
+
+void stage_filter(Workspace& W, const Grid& g, const Values& val, hipStream_t s, bool early3 = false,
+                  bool early5 = false) {
+    const uint64_t T = g.view.T;
+    const uint32_t F = val.F;
     const uint64_t full = (F == 64) ? ~0ull : ((1ull << F) - 1);
     const int kbig = W.wide ? kMaxHuge : 8;
     if (g.view.regular) {
@@ -2066,12 +2075,17 @@ void stage_count(Workspace& W, const Grid& g, const Values& val, hipStream_t s, 
     scan_u32(W.mem, W.isact.p, W.rank.p, Count(T), W.ctr.p + C_ACTIVE, s);
 }
 
+void stage_count(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
+    stage_signs(W, g, val, s, true);
+    stage_filter(W, g, val, s);
+}
+
 // the k = 2 table lookups' arguments (the bucket list's size and the abort
 // flag are the caller's)
 K2Args k2_args(Workspace& W, const Grid& g, const Values& val) {
     K2Args K = {};
     K.g = g.view;
-    K.vals = val.vals.p;
+    K.vals = W.vals_at.p;
     K.pos = W.pos.p;
     K.neg = W.neg.p;
     K.full = (val.F == 64) ? ~0ull : ((1ull << val.F) - 1);
@@ -2095,7 +2109,7 @@ template <class C>
 void launch_cut(Workspace& W, const Grid& g, const Values& val, int q, int grid, hipStream_t s) {
     CutArgs A;
     A.g = g.view;
-    A.vals = val.vals.p;
+    A.vals = W.vals_at.p;
     A.act = W.act.p;
     A.csr_off = W.csr_off.p;
     A.list = W.list[q].p;
@@ -2163,7 +2177,7 @@ void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int
                       bool wide = false) {
     CutArgs A = {};
     A.g = g.view;
-    A.vals = val.vals.p;
+    A.vals = W.vals_at.p;
     A.cap = W.cap.b[q];
     A.slot = W.slot[q];
     A.F = val.F;
@@ -2377,7 +2391,7 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
     }
     VertFieldArgs VF;
     VF.g = g.view;
-    VF.vals = (const double*)val.vals.p;
+    VF.vals = ValsRef{nullptr, W.vals_at.p};
     VF.act = W.act.p;
     VF.off = W.act_off.p;
     VF.per_rank = true;
@@ -2566,7 +2580,7 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
     // beside the fill pass; the k = 2 lookups follow the fill pass
     const bool e3 = g.view.regular && w.cap.b[1] && w.grid[1] < 0;
     const bool e5 = g.view.regular && w.cap.b[2] && w.grid[2] < 0;
-    stage_count(w, g, val, s, false, e3, e5);
+    stage_filter(w, g, val, s, e3, e5);
     if (e3 || e5) {
         // the k = 3..4 cut, captured first on the capturing stream, starts
         // a few microseconds before the other branches: its wavefronts (all
@@ -2609,26 +2623,13 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
     stage_rest(w, g, val, s, REST_DEDUP);
     stage_rest(w, g, val, s, REST_XYZ | REST_FACES);
     RIN_HIP(hipStreamEndCapture(s, &gr));
-    bool updated = false;
-    if (w.whole) {
-        hipGraphNode_t bad = nullptr;
-        hipGraphExecUpdateResult res;
-        updated = hipGraphExecUpdate(w.whole, gr, &bad, &res) == hipSuccess && res == hipGraphExecUpdateSuccess;
-        if (!updated) {
-            (void)hipGetLastError();
-            (void)hipGraphExecDestroy(w.whole);
-            w.whole = nullptr;
-        }
-    }
-    if (!updated) RIN_HIP(hipGraphInstantiate(&w.whole, gr, nullptr, nullptr, 0));
-    if (w.whole_graph) (void)hipGraphDestroy(w.whole_graph);
+    RIN_HIP(hipGraphInstantiate(&w.whole, gr, nullptr, nullptr, 0));
     w.whole_graph = gr;
     while (w.ev.size() < 2) {
         hipEvent_t e;
         RIN_HIP(hipEventCreate(&e));
         w.ev.push_back(e);
     }
-    w.bound_whole = val.vals.p;
 }
 
 // the same path as one graph per stage, for per-stage device times
@@ -2732,14 +2733,16 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             Caps_ need;
             caps_from_counts(hctr, w.wide, need);
             if (!caps_ok(w.cap, need)) {
-                // grow with head-room, keeping the k=1 table
-                Caps_ grow = need;
-                grow.active = need.active + need.active / 8;
-                grow.fit = need.fit + need.fit / 8;
-                for (int q = 0; q < 3; ++q) grow.b[q] = need.b[q] + need.b[q] / 8;
-                grow.vo = need.vo + need.vo / 8;
-                grow.fo = need.fo + need.fo / 8;
-                grow.fv = need.fv + need.fv / 8;
+                // grow with head-room; what is there already stays, so that
+                // value sets that alternate settle on one capacity
+                auto more = [](uint32_t have, uint32_t n) { return std::max(have, n + n / 8); };
+                Caps_ grow;
+                grow.active = more(w.cap.active, need.active);
+                grow.fit = more(w.cap.fit, need.fit);
+                for (int q = 0; q < 3; ++q) grow.b[q] = more(w.cap.b[q], need.b[q]);
+                grow.vo = more(w.cap.vo, need.vo);
+                grow.fo = more(w.cap.fo, need.fo);
+                grow.fv = more(w.cap.fv, need.fv);
                 alloc_ws(w, g, grow, s);
                 stage_count(w, g, val, s);
             }
@@ -2768,7 +2771,8 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
                         // cuts: listing the k = 3..8 tets (the lists go unused here)
                         for (int rep = 0; rep < 2; ++rep)  // the second pass, caches warm
                             ms = time_ms(s, [&] {
-                                stage_count(w, g, val, s, true, w.cap.b[1] != 0, w.cap.b[2] != 0);
+                                stage_signs(w, g, val, s, true);
+                                stage_filter(w, g, val, s, w.cap.b[1] != 0, w.cap.b[2] != 0);
                                 stage_fill(w, g, val, s);
                             });
                         if (ms < best) {
@@ -2830,10 +2834,10 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             RIN_HIP(hipStreamSynchronize(s));
             w.exec = true;
         }
-        // (re-)record the graphs for these values: a new workspace capacity
-        // drops them; new values of the same size re-record the whole graph
-        // and update the instantiated one in place
-        if (w.bound_whole != val.vals.p) record_whole(w, g, val, s);
+        // the graph is recorded once per workspace capacity; it holds no
+        // pointer to the values (re-recording it for each value set and
+        // updating it in place took the host 60 to 120 us a run)
+        if (!w.whole) record_whole(w, g, val, s);
         if (staged && w.bound_parts != val.vals.p) record_parts(w, g, val, P, s);
         if (w.hash_dirty) {
             RIN_HIP(hipMemsetAsync(w.hkey.p, 0, 8ull << w.hbits, s));
@@ -2843,6 +2847,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         if (!w.ctr_clear) hipLaunchKernelGGL(k_zero_ctr, dim3(1), dim3(64), 0, s, w.ctr.p, (int)C_N, w.errs.p);
         w.ctr_clear = false;
         RIN_HIP(hipEventRecord(w.ev[0], s));
+        if (!staged) stage_signs(w, g, val, s, false);
         if (staged) {
             for (size_t i = 0; i < w.parts.size(); ++i) {
                 RIN_HIP(hipGraphLaunch(w.parts[i].second, s));

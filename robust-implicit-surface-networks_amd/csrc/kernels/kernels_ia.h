@@ -1723,9 +1723,16 @@ __global__ void k_dedup_assign(Count n, const uint32_t* __restrict__ mo, const u
 
 // vertex records and coordinates (src/extract_mesh.cpp:95-228, 1446-1538)
 // off: CSR offsets by tet (per_rank false) or by active rank (per_rank true)
+// the values themselves, or where a captured path's run left them
+struct ValsRef {
+    const double* p;
+    const double* const* at;
+    __device__ const double* get() const { return at ? *at : p; }
+};
+
 struct VertFieldArgs {
     GridView g;
-    const double* vals;
+    ValsRef vals;
     const uint32_t* act;
     const uint32_t* off;  // CSR offsets by tet (per_rank false) or by active rank (per_rank true)
     bool per_rank;
@@ -1748,7 +1755,7 @@ struct VertFieldArgs {
 // as a workgroup role: blk of nblk workgroups
 __device__ inline void vert_fields_ia_role(const VertFieldArgs& P, uint32_t blk, uint32_t nblk) {
     const GridView& g = P.g;
-    const double* __restrict__ vals = P.vals;
+    const double* __restrict__ vals = P.vals.get();
     const uint32_t* __restrict__ act = P.act;
     const uint32_t* __restrict__ off = P.off;
     const bool per_rank = P.per_rank;

@@ -830,7 +830,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     {
         VertFieldArgs VF;
         VF.g = g.view;
-        VF.vals = (const double*)val.vals.p;
+        VF.vals = ValsRef{(const double*)val.vals.p, nullptr};
         VF.act = out.act.p;
         VF.off = out.csr_off.p;
         VF.per_rank = false;
