@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "devmem.h"
+#include "kernels/fetch.h"
 #include "kernels/pipeline.h"
 #include "rin.h"
 
@@ -17,6 +18,7 @@ struct rin_ctx {
     void* scratch = nullptr;  // the allocation-free path's array on this device
     hipStream_t stream = nullptr;
     rin::DevMem mem;
+    rin::HostStage stage;
     std::mutex mu;
     std::string err;
 };
@@ -61,21 +63,22 @@ int guarded(rin_ctx* c, F&& f) {
     }
 }
 
-template <class T, class U>
-void widen(const rin::DBuf<T>& d, size_t n, std::vector<U>& h, hipStream_t s) {
-    std::vector<T> tmp(n);
-    if (n) RIN_HIP(hipMemcpyAsync(tmp.data(), d.p, n * sizeof(T), hipMemcpyDeviceToHost, s));
-    RIN_HIP(hipStreamSynchronize(s));
-    h.assign(tmp.begin(), tmp.end());
+// an output array: `words` 64-bit words at dst
+rin::PackCol col(rin::PackKind kind, uint64_t words, void* dst, const void* p0, const void* p1 = nullptr,
+                 const void* p2 = nullptr, const void* p3 = nullptr, const void* p4 = nullptr) {
+    rin::PackCol c;
+    c.kind = kind;
+    c.words = words;
+    c.dst = dst;
+    c.p[0] = p0;
+    c.p[1] = p1;
+    c.p[2] = p2;
+    c.p[3] = p3;
+    c.p[4] = p4;
+    return c;
 }
 
-template <class T>
-std::vector<T> fetch(const T* d, size_t n, hipStream_t s) {
-    std::vector<T> h(n);
-    if (n) RIN_HIP(hipMemcpyAsync(h.data(), d, n * sizeof(T), hipMemcpyDeviceToHost, s));
-    RIN_HIP(hipStreamSynchronize(s));
-    return h;
-}
+void fetch(rin_ctx* c, const std::vector<rin::PackCol>& cols) { c->stage.fetch(c->device, cols, c->stream); }
 
 }  // namespace
 
@@ -122,6 +125,7 @@ int rin_destroy(rin_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     c->mem.trim();
+    c->stage.release();
     (void)hipStreamDestroy(c->stream);
     delete c;
     return RIN_OK;
@@ -201,10 +205,10 @@ int rin_eval_points_noalloc(rin_ctx* c, const double* pts, uint64_t n, const rin
 int rin_values_download(rin_ctx* c, const rin_values* v, double* rm) {
     if (!v || !rm) return fail(c, RIN_ERR_ARG, "null argument");
     return guarded(c, [&] {
-        const uint64_t V = v->v.V, F = v->v.F;
-        auto h = fetch(v->v.vals.p, V * F, c->stream);
-        for (uint64_t f = 0; f < F; ++f)
-            for (uint64_t i = 0; i < V; ++i) rm[i * F + f] = h[f * V + i];
+        rin::PackCol x = col(rin::PACK_ROWMAJOR, v->v.V * v->v.F, rm, v->v.vals.p);
+        x.rows = v->v.F;
+        x.stride = v->v.V;
+        fetch(c, {x});
     });
 }
 
@@ -272,33 +276,18 @@ int rin_result_csr(rin_ctx* c, const rin_result* res, uint64_t* fit, uint64_t* s
     if (!res || !fit || !start) return fail(c, RIN_ERR_ARG, "null argument");
     return guarded(c, [&] {
         const auto& r = res->r;
-        auto a = fetch(r.view.fit, r.n_fit, c->stream);
-        auto b = fetch(r.view.csr_off, r.T + 1, c->stream);
-        for (uint64_t i = 0; i < r.n_fit; ++i) fit[i] = a[i];
-        for (uint64_t i = 0; i <= r.T; ++i) start[i] = b[i];
+        rin::PackCol f = col(rin::PACK_U8, r.n_fit, fit, r.view.fit);
+        fetch(c, {f, col(rin::PACK_U32, r.T + 1, start, r.view.csr_off)});
     });
 }
 
 int rin_result_verts(rin_ctx* c, const rin_result* res, uint64_t* rec11, double* xyz) {
     if (!res || !rec11 || !xyz) return fail(c, RIN_ERR_ARG, "null argument");
     return guarded(c, [&] {
-        const auto& r = res->r;
-        const uint64_t n = r.n_verts;
-        auto tet = fetch(r.view.v_tet, n, c->stream);
-        auto j = fetch(r.view.v_j, n, c->stream);
-        auto ss = fetch(r.view.v_ss, n, c->stream);
-        auto sv = fetch(r.view.v_sv, 4 * n, c->stream);
-        auto fn = fetch(r.view.v_fn, 4 * n, c->stream);
-        auto x = fetch(r.view.xyz, 3 * n, c->stream);
-        for (uint64_t i = 0; i < n; ++i) {
-            uint64_t* o = rec11 + 11 * i;
-            o[0] = tet[i];
-            o[1] = j[i];
-            o[2] = ss[i];
-            for (int q = 0; q < 4; ++q) o[3 + q] = sv[4 * i + q] == 0xFFFFFFFFu ? UINT64_MAX : sv[4 * i + q];
-            for (int q = 0; q < 4; ++q) o[7 + q] = fn[4 * i + q] == 0xFF ? UINT64_MAX : fn[4 * i + q];
-        }
-        std::memcpy(xyz, x.data(), 24 * n);
+        const auto& w = res->r.view;
+        const uint64_t n = res->r.n_verts;
+        fetch(c, {col(rin::PACK_VERT, 11 * n, rec11, w.v_tet, w.v_j, w.v_ss, w.v_sv, w.v_fn),
+                  col(rin::PACK_F64, 3 * n, xyz, w.xyz)});
     });
 }
 
@@ -307,23 +296,12 @@ int rin_result_faces(rin_ctx* c, const rin_result* res, uint64_t* vstart, uint64
     if (!res || !vstart || !verts || !tfstart || !tf || !func) return fail(c, RIN_ERR_ARG, "null argument");
     return guarded(c, [&] {
         const auto& r = res->r;
+        const auto& w = r.view;
         const uint64_t nf = r.n_faces;
-        auto a = fetch(r.view.f_vstart, nf + 1, c->stream);
-        auto b = fetch(r.view.f_verts, r.n_face_verts, c->stream);
-        auto d = fetch(r.view.f_tfstart, nf + 1, c->stream);
-        auto e = fetch(r.view.f_tf_tet, r.n_tet_faces, c->stream);
-        auto f = fetch(r.view.f_tf_local, r.n_tet_faces, c->stream);
-        auto g = fetch(r.view.f_func, 2 * nf, c->stream);
-        for (uint64_t i = 0; i <= nf; ++i) {
-            vstart[i] = a[i];
-            tfstart[i] = d[i];
-        }
-        for (uint64_t i = 0; i < r.n_face_verts; ++i) verts[i] = b[i];
-        for (uint64_t i = 0; i < r.n_tet_faces; ++i) {
-            tf[2 * i] = e[i];
-            tf[2 * i + 1] = f[i];
-        }
-        for (uint64_t i = 0; i < 2 * nf; ++i) func[i] = g[i] == 0xFF ? UINT64_MAX : g[i];
+        fetch(c, {col(rin::PACK_U32, nf + 1, vstart, w.f_vstart), col(rin::PACK_U32, r.n_face_verts, verts, w.f_verts),
+                  col(rin::PACK_U32, nf + 1, tfstart, w.f_tfstart),
+                  col(rin::PACK_TET_FACE, 2 * r.n_tet_faces, tf, w.f_tf_tet, w.f_tf_local),
+                  col(rin::PACK_U8_NONE, 2 * nf, func, w.f_func)});
     });
 }
 
@@ -342,21 +320,10 @@ int rin_result_edges(rin_ctx* c, const rin_result* res, uint64_t* v12, uint64_t*
     return guarded(c, [&] {
         auto& r = const_cast<rin_result*>(res)->r;
         rin::compute_edges(c->mem, r, c->stream);
-        const uint64_t NE = r.n_edges, NO = r.n_face_verts, NF = r.n_faces;
-        auto a = fetch(r.e_v12.p, 2 * NE, c->stream);
-        auto b = fetch(r.e_start.p, NE + 1, c->stream);
-        auto o = fetch(r.e_occ.p, NO, c->stream);
-        auto e = fetch(r.e_of_occ.p, NO, c->stream);
-        auto f = fetch(r.e_face_of.p, NO, c->stream);
-        auto vs = fetch(r.view.f_vstart, NF + 1, c->stream);
-        for (uint64_t i = 0; i < 2 * NE; ++i) v12[i] = a[i];
-        for (uint64_t i = 0; i <= NE; ++i) start[i] = b[i];
-        for (uint64_t i = 0; i < NO; ++i) {
-            const uint32_t x = o[i], face = f[x];
-            occ[2 * i] = face;
-            occ[2 * i + 1] = x - vs[face];
-            edge_of[i] = e[i];
-        }
+        const uint64_t NE = r.n_edges, NO = r.n_face_verts;
+        fetch(c, {col(rin::PACK_U32, 2 * NE, v12, r.e_v12.p), col(rin::PACK_U32, NE + 1, start, r.e_start.p),
+                  col(rin::PACK_EDGE_OCC, 2 * NO, occ, r.e_occ.p, r.e_face_of.p, r.view.f_vstart),
+                  col(rin::PACK_U32, NO, edge_of, r.e_of_occ.p)});
     });
 }
 
@@ -374,10 +341,8 @@ int rin_result_patches(rin_ctx* c, const rin_result* res, uint64_t* start, uint6
     return guarded(c, [&] {
         auto& r = const_cast<rin_result*>(res)->r;
         rin::compute_patches(c->mem, r, c->stream);
-        auto a = fetch(r.p_start.p, r.n_patches + 1, c->stream);
-        auto b = fetch(r.p_faces.p, r.n_faces, c->stream);
-        for (uint64_t i = 0; i <= r.n_patches; ++i) start[i] = a[i];
-        for (uint64_t i = 0; i < r.n_faces; ++i) faces[i] = b[i];
+        fetch(c, {col(rin::PACK_U32, r.n_patches + 1, start, r.p_start.p),
+                  col(rin::PACK_U32, r.n_faces, faces, r.p_faces.p)});
     });
 }
 
@@ -395,12 +360,10 @@ int rin_result_chains(rin_ctx* c, const rin_result* res, uint64_t* start, uint64
     return guarded(c, [&] {
         auto& r = const_cast<rin_result*>(res)->r;
         rin::compute_chains(c->mem, r, c->stream);
-        auto a = fetch(r.c_start.p, r.n_chains + 1, c->stream);
-        const uint64_t n = a[r.n_chains];
+        fetch(c, {col(rin::PACK_U32, r.n_chains + 1, start, r.c_start.p)});
+        const uint64_t n = start[r.n_chains];
         if (n && !edges) throw std::invalid_argument("null argument");
-        auto b = fetch(r.c_edges.p, n, c->stream);
-        for (uint64_t i = 0; i <= r.n_chains; ++i) start[i] = a[i];
-        for (uint64_t i = 0; i < n; ++i) edges[i] = b[i];
+        if (n) fetch(c, {col(rin::PACK_U32, n, edges, r.c_edges.p)});
     });
 }
 
@@ -419,8 +382,7 @@ int rin_result_cut_counts(rin_ctx* c, const rin_result* res, uint64_t* counts) {
     return guarded(c, [&] {
         const auto& r = res->r;
         if (!r.view.cut_counts) throw std::invalid_argument("run was not RIN_FLAG_CUT_ONLY");
-        auto h = fetch(r.view.cut_counts, 3 * r.n_active, c->stream);
-        for (uint64_t i = 0; i < 3 * r.n_active; ++i) counts[i] = h[i];
+        fetch(c, {col(rin::PACK_U32, 3 * r.n_active, counts, r.view.cut_counts)});
     });
 }
 
