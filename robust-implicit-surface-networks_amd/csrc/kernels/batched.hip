@@ -1912,6 +1912,18 @@ const StarTables& star_tables() {
     return T;
 }
 
+}  // namespace
+
+void upload_star_tables(DevMem& m, DBuf<uint32_t>& head, DBuf<uint8_t>& ent, hipStream_t s) {
+    const StarTables& ST = star_tables();
+    head.alloc(m, ST.head.size());
+    ent.alloc(m, ST.ent.size());
+    RIN_HIP(hipMemcpyAsync(head.p, ST.head.data(), 4 * ST.head.size(), hipMemcpyHostToDevice, s));
+    RIN_HIP(hipMemcpyAsync(ent.p, ST.ent.data(), ST.ent.size(), hipMemcpyHostToDevice, s));
+}
+
+namespace {
+
 unsigned cube_tiles(const Grid& g, int tile = kCubeTile) {
     const uint64_t cubes = g.view.T / 5;
     return (unsigned)std::max<uint64_t>(1, (cubes + tile - 1) / tile);
@@ -1957,13 +1969,7 @@ void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
     W.oj.alloc(m, c.vo + 1);
     for (auto* b : {&W.first, &W.vrank, &W.first_occ, &W.mo}) b->alloc(m, c.vo + 1);
     W.tile_first.alloc(m, (c.vo + kDedupTile - 1) / kDedupTile + 1);
-    {
-        const StarTables& ST = star_tables();
-        W.star_head.alloc(m, ST.head.size());
-        W.star_ent.alloc(m, ST.ent.size());
-        RIN_HIP(hipMemcpyAsync(W.star_head.p, ST.head.data(), 4 * ST.head.size(), hipMemcpyHostToDevice, s));
-        RIN_HIP(hipMemcpyAsync(W.star_ent.p, ST.ent.data(), ST.ent.size(), hipMemcpyHostToDevice, s));
-    }
+    upload_star_tables(m, W.star_head, W.star_ent, s);
     if (!g.view.regular) {
         W.vid.alloc(m, c.vo + 1);
         W.hslot.alloc(m, c.vo + 1);
@@ -2360,6 +2366,9 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
         if (star) {
             StarArgs S;
             S.res = g.view.res;
+            S.edge_shift = 8;
+            S.face_shift = 14;
+            S.own = 0;
             S.okey = W.okey.p;
             S.oa = W.oa.p;
             S.act = W.act.p;

@@ -1,18 +1,17 @@
 // Batched form of the material-interface path (src/material_interface.cpp:53-447).
 //
 // The plain form's stages (highest material, filter, CSR, cut lists, the
-// per-tet cut by table or by the thread cut, boundary-face pairing,
-// extraction, radix-sort dedup, coordinates, faces) with every size kept on
+// per-tet cut by table or lane group, boundary-face pairing, extraction,
+// dedup, coordinates, faces) with every size kept on
 // the device: buffers are allocated to capacities, launches are sized by the
 // capacities and read the live counts from device memory (clamped, and
-// skipped once a count overflowed), scans run over the zero-padded
-// capacity.  So the whole path is one captured graph per workspace, replayed
-// on every run; an overflow grows the workspace and captures again, and new
-// values of the same size re-record the graph and update it in place.  The
-// closing kernel publishes the counters into pinned host memory, so a replay
-// needs no copies.  Tets the batched cut does not take (more than 8
-// materials, or a complex beyond the thread cut's capacity) send the run to
-// the plain form.
+// skipped once a count overflowed).  So the path after the first kernel is one
+// captured graph per workspace, replayed on every run and for any values: the
+// first kernel, launched with the values, leaves their address for it.  An
+// overflow grows the workspace and captures again.  The closing kernel
+// publishes the counters into pinned host memory and clears them, so a replay
+// needs no copies.  A complex beyond the lane-group cut's capacity sends the
+// run to the plain form.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -35,7 +34,6 @@ enum MICtr : uint32_t {
     M_ACTIVE,      // active tets
     M_LIST,        // cut list sizes [4], histogram [3], 3..4 / 5..8 counts, largest count (k_bucket_scan)
     M_WORDS = M_LIST + 10,  // record words
-    M_NFT,         // faces of the active tets' complexes
     M_VO, M_FO, M_FV,  // vertex occurrences, faces, face corners
     M_NV,          // vertices after dedup
     M_FIT,         // active (tet, material) entries: the CSR's total
@@ -48,7 +46,7 @@ constexpr int kMiPub = 32;
 static_assert(M_N <= kMiPub, "published counters");
 
 struct MICaps {
-    uint32_t active = 0, fit = 0, words = 0, nft = 0, vo = 0, fo = 0, fv = 0;
+    uint32_t active = 0, fit = 0, words = 0, vo = 0, fo = 0, fv = 0;
     uint32_t huge = 0;  // the captured path holds the large-capacity cut
 };
 
@@ -57,21 +55,164 @@ __global__ void k_mi_zero(uint32_t* ctr, uint32_t* errs) {
     if (threadIdx.x < 64) errs[threadIdx.x] = 0;
 }
 
-// after each counting stage: a count beyond its capacity stops the later
-// stages (and asks the host to grow the workspace); the cut lists' sizes are
-// zeroed then, so the cut kernels read nothing out of range
-__global__ void k_mi_check(uint32_t* ctr, const uint32_t* csr_off, uint64_t T, MICaps c, uint32_t* errs) {
-    if (threadIdx.x != 0) return;
-    ctr[M_FIT] = csr_off[T];
-    bool over = ctr[M_ACTIVE] > c.active || csr_off[T] > c.fit || ctr[M_WORDS] > c.words ||
-                ctr[M_NFT] > c.nft || ctr[M_VO] > c.vo || ctr[M_FO] > c.fo || ctr[M_FV] > c.fv;
+// Filter, CSR, active list, cut lists and record slots by tiles of 1280 tets
+// (a workgroup of 256 lanes, five consecutive tets a lane: a cube of a regular
+// grid): a count pass leaves each tet's material mask and each tile's sums,
+// one workgroup turns the sums into prefixes and totals and checks the
+// capacities, a fill pass places the tile's tets.  Three launches for what
+// took thirteen (a scan of three fields over every tet, the lists' count,
+// scan and fill, the slots' bounds and scan, checks and copies): 41 us at 65^3
+// vertices and 8 materials, from 100.
+constexpr uint32_t kMiLanes = 256, kMiTile = 5 * kMiLanes;
+enum MITileField {
+    MT_FIT = 0, MT_ACTIVE, MT_LIST, MT_WORDS = MT_LIST + 4,  // prefixes: the CSR, active tets, four lists, slot words
+    MT_HIST,                     // totals: two, three and more materials
+    MT_N34 = MT_HIST + 3, MT_N58, MT_KMAX, MT_N = 16
+};
+constexpr int kMiPrefixes = MT_WORDS + 1;
+struct MITile {
+    uint32_t v[MT_N];
+};
+
+// a tet's place among the cut lists (bucket_of_k) and its slot's words
+__device__ inline uint32_t mi_slot_words(int k) {
+    constexpr uint32_t wide = 8 + 4 * CWideMI::MV + CWideMI::MF * (4 + CWideMI::MFV) + 2 * CWideMI::MP;
+    return k > 8 ? wide : rec_bound(1, k);
+}
+
+// The highest materials at a tet's corners are active; so is every material
+// above the lowest of those at two corners or more
+// (src/material_interface.cpp:94-152).  Few tets have two materials among
+// their corners' highest, so each lane finds its own tets' and the workgroup
+// then takes those together, a lane a corner, the loads of eight materials in
+// flight (a lane a tet left one lane in twenty busy through 4 F dependent
+// loads: 102 us at 100^3 vertices and 18 materials against 65).
+__global__ void __launch_bounds__(kMiLanes) k_mi_count_tiles(GridView g, const double* const* vref, uint32_t F,
+                                                             const uint64_t* __restrict__ hm, int tables,
+                                                             uint64_t* __restrict__ amask,
+                                                             MITile* __restrict__ tiles) {
+    const double* __restrict__ vals = *vref;
+    __shared__ uint64_t s_mask[kMiTile];
+    __shared__ uint16_t s_list[kMiTile];
+    __shared__ uint32_t s_n;
+    const uint64_t V = g.V;
+    const uint32_t t0 = blockIdx.x * kMiTile, tid = threadIdx.x;
+    if (tid == 0) s_n = 0;
+    __syncthreads();
+    auto put = [&](uint32_t local, uint64_t u) {
+        s_mask[local] = u;
+        if (__popcll(u) >= 2) s_list[atomicAdd(&s_n, 1u)] = (uint16_t)local;
+    };
+    if (g.regular) {
+        const uint32_t cube = blockIdx.x * kMiLanes + tid;
+        if ((uint64_t)cube * 5 < g.T) {
+            const uint32_t R = (uint32_t)g.res, N = R + 1;
+            const uint32_t i = cube / (R * R), rem = cube - i * (R * R), j = rem / R, k = rem - j * R;
+            const uint32_t b = i * N * N + j * N + k;
+            const uint32_t c[8] = {b, b + N * N, b + N * N + N, b + N, b + 1, b + N * N + 1, b + N * N + N + 1, b + N + 1};
+            uint64_t h[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) h[q] = hm[c[q]];
+            const bool even = ((i + j + k) & 1u) == 0;
+            for (int q = 0; q < 5; ++q) {
+                const uint8_t* t = even ? dev::kCubeTetEven[q] : dev::kCubeTetOdd[q];
+                put(5 * tid + q, h[t[0]] | h[t[1]] | h[t[2]] | h[t[3]]);
+            }
+        }
+    } else {
+        for (uint32_t q = tid; q < kMiTile; q += kMiLanes) {
+            const uint64_t t = (uint64_t)t0 + q;
+            if (t >= g.T) continue;
+            uint32_t v[4];
+            dev::tet_corners(g, t, v);
+            put(q, hm[v[0]] | hm[v[1]] | hm[v[2]] | hm[v[3]]);
+        }
+    }
+    __syncthreads();
+    const uint32_t n = s_n;
+    for (uint32_t x = tid >> 2; x < n; x += kMiLanes / 4) {
+        const uint32_t local = s_list[x], c = tid & 3;
+        uint32_t v[4];
+        dev::tet_corners(g, (uint64_t)t0 + local, v);
+        const double* at = vals + (c == 0 ? v[0] : (c == 1 ? v[1] : (c == 2 ? v[2] : v[3])));
+        const uint64_t u = s_mask[local];
+        double mn = 1.79769313486231570815e308;
+        for (uint64_t m = u; m; m &= m - 1) {
+            const double y = at[(uint64_t)(__ffsll((unsigned long long)m) - 1) * V];
+            if (y < mn) mn = y;
+        }
+        uint64_t above = 0;
+        for (uint32_t j0 = 0; j0 < F; j0 += 8) {
+            double y[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) y[q] = at[(uint64_t)(j0 + q < F ? j0 + q : 0) * V];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) above |= (uint64_t)(j0 + q < F && y[q] > mn) << (j0 + q);
+        }
+        // materials above at two corners or more, over the tet's four lanes
+        const uint64_t p = __shfl_xor(above, 1, 64), both = above & p, any = above | p;
+        const uint64_t both2 = __shfl_xor(both, 2, 64), any2 = __shfl_xor(any, 2, 64);
+        if (c == 0) s_mask[local] = u | both | both2 | (any & any2);
+    }
+    __syncthreads();
+    uint32_t s[MT_N];
+#pragma unroll
+    for (int f = 0; f < MT_N; ++f) s[f] = 0;
+    for (uint32_t q = 0; q < 5; ++q) {
+        const uint32_t local = 5 * tid + q;
+        const uint64_t t = (uint64_t)t0 + local;
+        if (t >= g.T) continue;
+        const uint64_t m = s_mask[local];
+        const int k = __popcll(m);
+        if (k < 2) continue;
+        s[MT_FIT] += (uint32_t)k;
+        s[MT_ACTIVE] += 1;
+        const int b = bucket_of_k(k, tables);
+#pragma unroll
+        for (int z = 0; z < 4; ++z) s[MT_LIST + z] += b == z;
+        s[MT_WORDS] += mi_slot_words(k);
+        s[MT_HIST] += k == 2;
+        s[MT_HIST + 1] += k == 3;
+        s[MT_HIST + 2] += k > 3;
+        s[MT_N34] += k == 3 || k == 4;
+        s[MT_N58] += k >= 5 && k <= 8;
+        s[MT_KMAX] = max(s[MT_KMAX], (uint32_t)k);
+    }
+    for (uint32_t q = tid; q < kMiTile; q += kMiLanes) {
+        const uint64_t t = (uint64_t)t0 + q;
+        if (t < g.T) amask[t] = s_mask[q];
+    }
+    __shared__ uint32_t red[kMiLanes / 64][MT_N];
+#pragma unroll
+    for (int f = 0; f < MT_N; ++f) {
+        uint32_t x = s[f];
+        for (int d = 32; d > 0; d >>= 1) {
+            const uint32_t y = __shfl_xor(x, d, 64);
+            x = f == MT_KMAX ? max(x, y) : x + y;
+        }
+        if ((tid & 63) == 0) red[tid >> 6][f] = x;
+    }
+    __syncthreads();
+    if (tid < MT_N) {
+        uint32_t x = red[0][tid];
+        for (uint32_t w = 1; w < kMiLanes / 64; ++w) x = tid == MT_KMAX ? max(x, red[w][tid]) : x + red[w][tid];
+        tiles[blockIdx.x].v[tid] = x;
+    }
+}
+
+// a count beyond its capacity stops the later stages (and asks the host to
+// grow the workspace); the cut lists' sizes are zeroed then, so the cut
+// kernels read nothing out of range
+__device__ inline void mi_check(uint32_t* ctr, const MICaps& c, uint32_t* errs) {
+    bool over = ctr[M_ACTIVE] > c.active || ctr[M_FIT] > c.fit || ctr[M_WORDS] > c.words || ctr[M_VO] > c.vo ||
+                ctr[M_FO] > c.fo || ctr[M_FV] > c.fv;
     if (over) {
         ctr[M_ABORT] = 1;
         errs[0] |= kMiOverflow;
     }
-    // tets beyond 8 materials take the large-capacity cut (a path captured
-    // without it stops here and is captured again with it); beyond its
-    // capacity the plain form reports them
+    // tets beyond 8 materials take the wide cut (a path captured without it
+    // stops here and is captured again with it); beyond its capacity the
+    // plain form reports them
     if (ctr[M_LIST + 9] > 8) {
         errs[0] |= kMiHuge;
         if (!c.huge) ctr[M_ABORT] = 1;
@@ -80,58 +221,164 @@ __global__ void k_mi_check(uint32_t* ctr, const uint32_t* csr_off, uint64_t T, M
     if (ctr[M_ABORT])
         for (int q = 0; q < 4; ++q) ctr[M_LIST + q] = 0;
 }
-
-// the CSR, active list and counts (k_fill with the capacity check)
-__global__ void k_mi_fill(uint64_t T, const uint64_t* __restrict__ amask, const uint32_t* __restrict__ csr_off,
-                          const uint32_t* __restrict__ rank, const uint32_t* __restrict__ abort,
-                          uint8_t* __restrict__ fit, uint32_t* __restrict__ act, uint8_t* __restrict__ act_k) {
-    if (*abort) return;
-    GRID_STRIDE(t, T) {
-        uint64_t m = amask[t];
-        if (!m) continue;
-        uint32_t o = csr_off[t];
-        const uint32_t r = rank[t];
-        act[r] = (uint32_t)t;
-        act_k[r] = (uint8_t)__popcll(m);
-        for (; m; m &= m - 1) fit[o++] = (uint8_t)(__ffsll((unsigned long long)m) - 1);
-    }
+__global__ void k_mi_check(uint32_t* ctr, MICaps c, uint32_t* errs) {
+    if (threadIdx.x == 0) mi_check(ctr, c, errs);
 }
 
-// record slot bounds over the whole capacity (zero past the active tets)
-__global__ void k_mi_rec_bound(uint64_t cap, const uint32_t* __restrict__ n_active,
-                               const uint32_t* __restrict__ abort, const uint8_t* __restrict__ act_k,
-                               uint32_t* __restrict__ b) {
-    const uint64_t n = *abort ? 0 : *n_active;
-    GRID_STRIDE(a, cap + 1) b[a] = a < n ? rec_bound(1, act_k[a]) : 0u;
-}
-
-// per active tet its complex's face count; zero past the active tets
-__global__ void k_mi_nf_padded(MIArgs A, uint64_t cap, uint32_t* __restrict__ nf) {
-    const uint64_t n = count_of(A.n_active);
-    GRID_STRIDE(a, cap + 1) {
-        uint32_t x = 0;
-        if (a < n) {
-            const uint16_t* r = A.rec + A.rec_loc[a];
-            x = r[0] == 2 ? r[3] : 0u;
+// The tile sums into exclusive prefixes (the first kMiPrefixes fields), the
+// totals into the counters, and the capacity check; one workgroup, a wavefront
+// a field, 16 consecutive tiles a lane.
+__global__ void __launch_bounds__(1024) k_mi_tile_scan(MITile* __restrict__ ts, uint32_t n, uint64_t T, uint32_t* ctr,
+                                                       MICaps c, uint32_t* errs, uint32_t* __restrict__ csr_off,
+                                                       uint32_t* __restrict__ rec_off) {
+    constexpr int P = 1024 + 1024 / 16;  // a pad word every 16 against bank conflicts
+    __shared__ uint32_t sm[MT_N][P];
+    __shared__ uint32_t tot[MT_N];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    static_assert(MT_N == 16, "a wavefront a field");
+    if (threadIdx.x < MT_N) tot[threadIdx.x] = 0;
+    for (uint32_t base = 0; base < n; base += 1024) {
+        const uint32_t i = base + threadIdx.x;
+        const int pi = threadIdx.x + threadIdx.x / 16;
+        MITile x = {};
+        if (i < n) x = ts[i];
+        for (int f = 0; f < MT_N; ++f) sm[f][pi] = x.v[f];
+        __syncthreads();
+        {
+            const int f = wave, e0 = 16 * lane, p0 = e0 + e0 / 16;
+            uint32_t sum = 0;
+            for (int e = 0; e < 16; ++e) sum = f == MT_KMAX ? max(sum, sm[f][p0 + e]) : sum + sm[f][p0 + e];
+            if (f < kMiPrefixes) {
+                uint32_t inc = sum;
+                for (int d = 1; d < 64; d <<= 1) {
+                    const uint32_t o = __shfl_up(inc, d, 64);
+                    if (lane >= d) inc += o;
+                }
+                uint32_t run = tot[f] + inc - sum;
+                for (int e = 0; e < 16; ++e) {
+                    const uint32_t v = sm[f][p0 + e];
+                    sm[f][p0 + e] = run;
+                    run += v;
+                }
+                sum = __shfl(inc, 63, 64);
+            } else {
+                for (int d = 32; d > 0; d >>= 1) {
+                    const uint32_t y = __shfl_xor(sum, d, 64);
+                    sum = f == MT_KMAX ? max(sum, y) : sum + y;
+                }
+            }
+            if (lane == 0) tot[f] = f == MT_KMAX ? max(tot[f], sum) : tot[f] + sum;
         }
-        nf[a] = x;
+        __syncthreads();
+        if (i < n)
+            for (int f = 0; f < kMiPrefixes; ++f) ts[i].v[f] = sm[f][pi];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        ctr[M_FIT] = tot[MT_FIT];
+        ctr[M_ACTIVE] = tot[MT_ACTIVE];
+        for (int q = 0; q < 4; ++q) ctr[M_LIST + q] = tot[MT_LIST + q];
+        for (int q = 0; q < 3; ++q) ctr[M_LIST + 4 + q] = tot[MT_HIST + q];
+        ctr[M_LIST + 7] = tot[MT_N34];
+        ctr[M_LIST + 8] = tot[MT_N58];
+        ctr[M_LIST + 9] = tot[MT_KMAX];
+        ctr[M_WORDS] = tot[MT_WORDS];
+        csr_off[T] = tot[MT_FIT];
+        mi_check(ctr, c, errs);
+        if (!ctr[M_ABORT]) rec_off[tot[MT_ACTIVE]] = tot[MT_WORDS];
     }
 }
 
-// the three per-tet output counts, zero past the active tets
-__global__ void k_mi_split_padded(Count n, uint64_t cap, const uint32_t* __restrict__ cnt, uint32_t* a,
-                                  uint32_t* b, uint32_t* c) {
-    const uint64_t na = count_of(n);
-    GRID_STRIDE(i, cap + 1) {
-        const bool in = i < na;
-        a[i] = in ? cnt[3 * i] : 0u;
-        b[i] = in ? cnt[3 * i + 1] : 0u;
-        c[i] = in ? cnt[3 * i + 2] : 0u;
+__global__ void __launch_bounds__(kMiLanes) k_mi_fill_tiles(uint64_t T, const uint64_t* __restrict__ amask,
+                                                            const MITile* __restrict__ tiles,
+                                                            const uint32_t* __restrict__ abort, int tables,
+                                                            uint32_t* __restrict__ csr_off, uint32_t* __restrict__ rank,
+                                                            uint8_t* __restrict__ fit, uint32_t* __restrict__ act,
+                                                            uint8_t* __restrict__ act_k, uint32_t* __restrict__ rec_off,
+                                                            uint32_t* __restrict__ rec_loc, uint32_t* __restrict__ l0,
+                                                            uint32_t* __restrict__ l1, uint32_t* __restrict__ l2,
+                                                            uint32_t* __restrict__ l3) {
+    if (*abort) return;
+    __shared__ uint64_t s_mask[kMiTile];
+    __shared__ uint32_t s_off[kMiTile], s_rank[kMiTile];
+    __shared__ uint64_t w0[kMiLanes / 64], w1[kMiLanes / 64];
+    __shared__ uint32_t w2[kMiLanes / 64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint64_t t0 = (uint64_t)blockIdx.x * kMiTile;
+    const MITile pre = tiles[blockIdx.x];
+    for (uint32_t q = tid; q < kMiTile; q += kMiLanes) s_mask[q] = t0 + q < T ? amask[t0 + q] : 0;
+    __syncthreads();
+    // per lane: active materials and tets (20 bits each is enough: a tile
+    // holds 1280 tets of at most 64), the four lists' tets, the slot words
+    uint64_t a = 0, b = 0;
+    uint32_t w = 0;
+    for (uint32_t q = 0; q < 5; ++q) {
+        const int k = __popcll(s_mask[5 * tid + q]);
+        if (k < 2) continue;
+        a += (uint64_t)k | 1ull << 32;
+        b += 1ull << (16 * bucket_of_k(k, tables));
+        w += mi_slot_words(k);
     }
+    uint64_t ia = a, ib = b;
+    uint32_t iw = w;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t oa = __shfl_up(ia, d, 64), ob = __shfl_up(ib, d, 64);
+        const uint32_t ow = __shfl_up(iw, d, 64);
+        if ((int)lane >= d) {
+            ia += oa;
+            ib += ob;
+            iw += ow;
+        }
+    }
+    if (lane == 63) {
+        w0[wave] = ia;
+        w1[wave] = ib;
+        w2[wave] = iw;
+    }
+    __syncthreads();
+    ia -= a;
+    ib -= b;
+    iw -= w;
+    for (uint32_t x = 0; x < wave; ++x) {
+        ia += w0[x];
+        ib += w1[x];
+        iw += w2[x];
+    }
+    uint32_t o = pre.v[MT_FIT] + (uint32_t)ia, r = pre.v[MT_ACTIVE] + (uint32_t)(ia >> 32), at = pre.v[MT_WORDS] + iw;
+    uint32_t p[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = pre.v[MT_LIST + q] + ((uint32_t)(ib >> (16 * q)) & 0xffffu);
+    for (uint32_t q = 0; q < 5; ++q) {
+        const uint32_t local = 5 * tid + q;
+        uint64_t m = s_mask[local];
+        const int k = __popcll(m);
+        s_off[local] = o;
+        s_rank[local] = r;
+        if (k < 2) continue;
+        act[r] = (uint32_t)(t0 + local);
+        act_k[r] = (uint8_t)k;
+        rec_off[r] = at;
+        rec_loc[r] = at;
+        const int z = bucket_of_k(k, tables);
+        if (z == 0) l0[p[0]++] = r;
+        if (z == 1) l1[p[1]++] = r;
+        if (z == 2) l2[p[2]++] = r;
+        if (z == 3) l3[p[3]++] = r;
+        for (uint32_t x = o; m; m &= m - 1) fit[x++] = (uint8_t)(__ffsll((unsigned long long)m) - 1);
+        o += (uint32_t)k;
+        ++r;
+        at += mi_slot_words(k);
+    }
+    __syncthreads();
+    for (uint32_t q = tid; q < kMiTile; q += kMiLanes)
+        if (t0 + q < T) {
+            csr_off[t0 + q] = s_off[q];
+            rank[t0 + q] = s_rank[q];
+        }
 }
 
 // closes the face arrays, publishes the counters and the union of the error
-// flags into pinned host memory
+// flags into pinned host memory, and clears both for the next run
 __global__ void k_mi_close(uint32_t* ctr, uint32_t* errs, uint32_t cap_fo, uint32_t* f_vstart, uint32_t* f_tfstart,
                            uint32_t* pub) {
     const uint32_t nf = ctr[M_FO] < cap_fo ? ctr[M_FO] : cap_fo;
@@ -144,6 +391,9 @@ __global__ void k_mi_close(uint32_t* ctr, uint32_t* errs, uint32_t cap_fo, uint3
     for (int d = 32; d > 0; d >>= 1) e |= __shfl_xor(e, d, 64);
     if (threadIdx.x == 0) pub[kMiPub] = e;
     __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x < M_N) ctr[threadIdx.x] = 0;
+    errs[threadIdx.x] = 0;
 }
 
 unsigned blocks_for(uint64_t n) { return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, 65535)); }
@@ -161,11 +411,13 @@ struct MIWorkspace {
     MICaps cap;
     bool in_use = false;
     // per vertex / tet (fixed by the grid)
+    DBuf<const double*> vals_at;  // the run's values, left by its first kernel for the captured ones
     DBuf<uint64_t> hm, amask;
-    DBuf<uint32_t> kcnt, isact, csr_off, rank, tscan;
+    DBuf<MITile> tiles;
+    DBuf<uint32_t> csr_off, rank;
     // per active tet
     DBuf<uint8_t> fit, act_k;
-    DBuf<uint32_t> act, blists, bc, rbound, rec_off, cnt, fb;
+    DBuf<uint32_t> act, blists, rec_off, cnt, labels;
     // each active tet's record location: its slot (rec_off), or for a table
     // tet the table's record, whose words follow the slots in rec (at
     // tab_base2 and tab_base3)
@@ -175,14 +427,15 @@ struct MIWorkspace {
     DBuf<uint64_t> emask;
     unsigned cut_blocks[2] = {0, 0};
     bool wide = false;  // the path holds the cut of more than 8 materials, once a run needs it
-    // per complex face, occurrence, face
-    DBuf<uint16_t> fl, fw, oj, fq_l;
-    DBuf<uint64_t> ft, okey;
-    DBuf<uint32_t> cv, cf, cfv, tv, tf, tfv, oa, fq_a, fq_vs, fve;
+    // per occurrence, face
+    DBuf<uint16_t> oj, fq_l;
+    DBuf<uint64_t> okey;
+    DBuf<uint32_t> cv, cf, cfv, oa, fq_a, fq_vs, fve;
     DBuf<uint8_t> fq_m;
     // dedup
-    DBuf<uint32_t> first, mo, hslot, vrank, vid, first_occ;
-    // first-occurrence hash table (key + 1, ~smallest occurrence), zero
+    DBuf<uint32_t> first, mo, hslot, vrank, vid, first_occ, tile_first, star_head;
+    DBuf<uint8_t> star_ent;
+    // explicit meshes: first-occurrence hash table (key + 1, ~smallest occurrence), zero
     // between runs: the assign pass clears the slots a run used
     DBuf<unsigned long long> hkey;
     DBuf<uint32_t> hmx;
@@ -198,16 +451,26 @@ struct MIWorkspace {
     uint32_t* pub_d = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    const double* bound = nullptr;  // the values the graph reads
+    // side branches of the graph: the cuts run beside each other
+    hipStream_t side[3] = {nullptr, nullptr, nullptr};
+    hipEvent_t fork = nullptr, join[3] = {nullptr, nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    bool ctr_clear = false;  // counters and error flags are zero (left so by the last run)
     void drop_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
         exec = nullptr;
         graph = nullptr;
-        bound = nullptr;
     }
     ~MIWorkspace() {
         drop_graph();
+        for (int q = 0; q < 3; ++q) {
+            if (join[q]) (void)hipEventDestroy(join[q]);
+            if (side[q]) (void)hipStreamDestroy(side[q]);
+        }
+        if (fork) (void)hipEventDestroy(fork);
+        for (auto e : ev)
+            if (e) (void)hipEventDestroy(e);
         if (pub_h) (void)hipHostFree(pub_h);
     }
 };
@@ -240,9 +503,8 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     if (!W.hm.p) {
         W.hm.alloc(m, V);
         W.amask.alloc(m, T);
-        W.kcnt.alloc(m, T);
-        W.isact.alloc(m, T);
-        W.tscan.alloc(m, T + 1);
+        W.vals_at.alloc(m, 1);
+        W.tiles.alloc(m, T / kMiTile + 1);
         W.csr_off.alloc(m, T + 1);
         W.rank.alloc(m, T + 1);
         W.ctr.alloc(m, 64);
@@ -253,9 +515,6 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     W.act_k.alloc(m, A + 1);
     W.act.alloc(m, A + 1);
     W.blists.alloc(m, 4 * (A + 1));
-    const uint64_t nch = (A + kBucketChunk - 1) / kBucketChunk + 1;
-    W.bc.alloc(m, (uint64_t)kBucketWords * nch + kBucketWords);
-    W.rbound.alloc(m, A + 2);
     W.rec_off.alloc(m, A + 2);
     W.rec_loc.alloc(m, A + 2);
     {
@@ -270,22 +529,16 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
         RIN_HIP(hipMemcpyAsync(W.rec.p + W.tab_base3, TR.w3, 2 * TR.n_w3, hipMemcpyDeviceToDevice, s));
     }
     W.cnt.alloc(m, 3 * A + 3);
-    W.fb.alloc(m, A + 2);
+    W.labels.alloc(m, A + 1);
     W.emask.alloc(m, A + 1);
     W.cv.alloc(m, A + 2);
     W.cf.alloc(m, A + 2);
     W.cfv.alloc(m, A + 2);
-    W.tv.alloc(m, A + 2);
-    W.tf.alloc(m, A + 2);
-    W.tfv.alloc(m, A + 2);
     // thread cuts (four and five to eight materials): a lane per tet with
     // its complex in LDS, two lanes (one for the larger complexes) a
     // wavefront, grids striding over their lists
     W.cut_blocks[0] = (unsigned)std::min<uint64_t>((A + 1) / 2 + 1, 4096);
     W.cut_blocks[1] = (unsigned)std::min<uint64_t>(A + 1, 2048);
-    W.fl.alloc(m, c.nft + 1);
-    W.fw.alloc(m, c.nft + 1);
-    W.ft.alloc(m, 3 * (uint64_t)c.nft + 3);
     W.okey.alloc(m, c.vo + 1);
     W.oa.alloc(m, c.vo + 1);
     W.oj.alloc(m, c.vo + 1);
@@ -294,15 +547,22 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     W.fq_m.alloc(m, 2 * (uint64_t)c.fo + 2);
     W.fq_vs.alloc(m, c.fo + 1);
     W.fve.alloc(m, c.fv + 1);
-    for (auto* b : {&W.first, &W.mo, &W.hslot, &W.vrank, &W.vid, &W.first_occ}) b->alloc(m, c.vo + 1);
-    // a table of at least twice the occurrence capacity, cleared once here
-    W.hbits = 10;
-    while ((1ull << W.hbits) < 2ull * (c.vo + 1)) ++W.hbits;
-    W.hkey.alloc(m, 1ull << W.hbits);
-    W.hmx.alloc(m, 1ull << W.hbits);
-    RIN_HIP(hipMemsetAsync(W.hkey.p, 0, 8ull << W.hbits, s));
-    RIN_HIP(hipMemsetAsync(W.hmx.p, 0, 4ull << W.hbits, s));
-    W.hash_dirty = false;
+    for (auto* b : {&W.first, &W.mo, &W.vrank, &W.first_occ}) b->alloc(m, c.vo + 1);
+    if (g.view.regular) {
+        W.tile_first.alloc(m, (c.vo + kDedupTile - 1) / kDedupTile + 1);
+        upload_star_tables(m, W.star_head, W.star_ent, s);
+    } else {
+        // a table of at least twice the occurrence capacity, cleared once here
+        W.vid.alloc(m, c.vo + 1);
+        W.hslot.alloc(m, c.vo + 1);
+        W.hbits = 10;
+        while ((1ull << W.hbits) < 2ull * (c.vo + 1)) ++W.hbits;
+        W.hkey.alloc(m, 1ull << W.hbits);
+        W.hmx.alloc(m, 1ull << W.hbits);
+        RIN_HIP(hipMemsetAsync(W.hkey.p, 0, 8ull << W.hbits, s));
+        RIN_HIP(hipMemsetAsync(W.hmx.p, 0, 4ull << W.hbits, s));
+        W.hash_dirty = false;
+    }
     W.v_tet.alloc(m, c.vo + 1);
     W.v_j.alloc(m, c.vo + 1);
     W.v_ss.alloc(m, c.vo + 1);
@@ -324,33 +584,14 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
 
 // the whole path on stream s; every launch is sized by capacities and reads
 // the live counts from the workspace
-void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev& TT, int kbits, hipStream_t s) {
+void mi_path(MIWorkspace& W, const Grid& g, uint32_t F, const MITablesDev& TT, hipStream_t s) {
     const GridView& G = g.view;
-    const uint64_t V = G.V, T = G.T;
-    const uint32_t F = val.F;
+    const uint64_t T = G.T;
     MICaps c = W.cap;
     c.huge = W.wide ? 1u : 0u;
     uint32_t* ctr = W.ctr.p;
     const uint32_t* abort = ctr + M_ABORT;
-    const double* vals = val.vals.p;
-    hipLaunchKernelGGL(k_mi_zero, dim3(1), dim3(64), 0, s, ctr, W.errs.p);
-    // highest material and filter (src/material_interface.cpp:53-152)
-    hipLaunchKernelGGL(k_highest_mi, dim3(blocks_for(V)), dim3(256), 0, s, vals, V, F, W.hm.p, (uint32_t*)nullptr,
-                       ctr + M_DEGEN);
-    hipLaunchKernelGGL(k_filter_mi, dim3(blocks_for(T)), dim3(256), 0, s, G, vals, F, (const uint64_t*)W.hm.p,
-                       W.amask.p, W.kcnt.p, W.isact.p);
-    {
-        // CSR offsets and active ranks in one pass (the third field is unused)
-        const uint32_t* in[3] = {W.kcnt.p, W.isact.p, W.isact.p};
-        uint32_t* out[3] = {W.csr_off.p, W.rank.p, W.tscan.p};
-        uint32_t* tot[3] = {W.csr_off.p + T, ctr + M_ACTIVE, nullptr};
-        scan3_u32(W.mem, in, 1, out, Count(T), tot, s);
-    }
-    hipLaunchKernelGGL(k_mi_check, dim3(1), dim3(64), 0, s, ctr, (const uint32_t*)W.csr_off.p, T, c, W.errs.p);
-    hipLaunchKernelGGL(k_mi_fill, dim3(blocks_for(T)), dim3(256), 0, s, T, (const uint64_t*)W.amask.p,
-                       (const uint32_t*)W.csr_off.p, (const uint32_t*)W.rank.p, abort, W.fit.p, W.act.p,
-                       W.act_k.p);
-    const Count NA(ctr + M_ACTIVE, c.active, abort);
+    const ValsRef vals{nullptr, W.vals_at.p};
     // cut lists: the tables take two and three materials, lane groups four
     // to eight.  RIN_CUT_FORM=wave or thread turns the tables off and cuts
     // every tet up to eight materials by lane groups or by a lane each.
@@ -360,34 +601,36 @@ void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev
     const int tables = (all_thread || all_wave) ? 0 : 1;
     uint32_t* bl[4];
     for (int q = 0; q < 4; ++q) bl[q] = W.blists.p + (uint64_t)q * (c.active + 1);
-    const uint32_t nch = (uint32_t)((c.active + kBucketChunk - 1) / kBucketChunk) + 1;
-    hipLaunchKernelGGL(k_bucket_count, dim3(nch), dim3(256), 0, s, NA, (const uint8_t*)W.act_k.p, 1, tables,
-                       W.bc.p);
-    hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, s, nch, W.bc.p, ctr + M_LIST);
-    hipLaunchKernelGGL(k_bucket_fill, dim3(nch), dim3(256), 0, s, NA, (const uint8_t*)W.act_k.p, tables,
-                       (const uint32_t*)W.bc.p, bl[0], bl[1], bl[2], bl[3]);
-    // record slots
-    hipLaunchKernelGGL(k_mi_rec_bound, dim3(blocks_for(c.active + 1)), dim3(256), 0, s, (uint64_t)c.active,
-                       (const uint32_t*)(ctr + M_ACTIVE), abort, (const uint8_t*)W.act_k.p, W.rbound.p);
-    scan_u32(W.mem, W.rbound.p, W.rec_off.p, Count((uint64_t)c.active + 1), ctr + M_WORDS, s);
-    hipLaunchKernelGGL(k_mi_check, dim3(1), dim3(64), 0, s, ctr, (const uint32_t*)W.csr_off.p, T, c, W.errs.p);
-    // the cut: tables for two and three materials, thread cuts beyond
-    // record locations: each tet's slot, then table tets point at the table's record
-    copy_u32(W.rec_loc.p, W.rec_off.p, NA, s);
+    // filter, CSR, lists and slots (src/material_interface.cpp:94-152)
+    const uint32_t ntiles = (uint32_t)((T + kMiTile - 1) / kMiTile);
+    hipLaunchKernelGGL(k_mi_count_tiles, dim3(ntiles), dim3(kMiLanes), 0, s, G, W.vals_at.p, F,
+                       (const uint64_t*)W.hm.p, tables, W.amask.p, W.tiles.p);
+    hipLaunchKernelGGL(k_mi_tile_scan, dim3(1), dim3(1024), 0, s, W.tiles.p, ntiles, T, ctr, c, W.errs.p, W.csr_off.p,
+                       W.rec_off.p);
+    hipLaunchKernelGGL(k_mi_fill_tiles, dim3(ntiles), dim3(kMiLanes), 0, s, T, (const uint64_t*)W.amask.p,
+                       (const MITile*)W.tiles.p, abort, tables, W.csr_off.p, W.rank.p, W.fit.p, W.act.p, W.act_k.p,
+                       W.rec_off.p, W.rec_loc.p, bl[0], bl[1], bl[2], bl[3]);
+    const Count NA(ctr + M_ACTIVE, c.active, abort);
+    // The cuts beside each other, each list on a branch of its own: the
+    // tables (table tets point at the table's record), four materials, five
+    // to eight, more.  One after another they took 59 + 65 + 34 us at 65^3
+    // vertices and 8 materials, each the latency of its longest tet.
+    RIN_HIP(hipEventRecord(W.fork, s));
+    for (int q = 0; q < (W.wide ? 3 : 2); ++q) RIN_HIP(hipStreamWaitEvent(W.side[q], W.fork, 0));
     hipLaunchKernelGGL(k_mi_table, dim3(blocks_for(c.active)), dim3(256), 0, s, G, vals, (const uint32_t*)W.act.p,
                        (const uint32_t*)W.csr_off.p, (const uint8_t*)W.fit.p, (const uint32_t*)bl[0],
                        (uint64_t)c.active, (const uint32_t*)(ctr + M_LIST), (uint32_t)0, (const uint32_t*)W.rec_off.p,
-                       W.rec.p, W.cnt.p, W.errs.p, TT, W.rec_loc.p, W.tab_base2, W.tab_base3);
+                       W.rec.p, W.cnt.p, W.errs.p, TT, W.labels.p, W.rec_loc.p, W.tab_base2, W.tab_base3);
     const Count n1(ctr + M_LIST + 1, c.active, abort), n2(ctr + M_LIST + 2, c.active, abort);
     if (all_thread) {
-        hipLaunchKernelGGL((k_cut_lds<CMed, true, 2>), dim3(W.cut_blocks[0]), dim3(2), 0, s, G, vals,
+        hipLaunchKernelGGL((k_cut_lds<CMed, true, 2>), dim3(W.cut_blocks[0]), dim3(2), 0, W.side[0], G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, n1, 1, 4, (uint32_t)0, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, (const uint32_t*)bl[1]);
-        hipLaunchKernelGGL((k_cut_lds<CBig, true, 1>), dim3(W.cut_blocks[1]), dim3(1), 0, s, G, vals,
+                           W.cnt.p, W.errs.p, (const uint32_t*)bl[1], W.labels.p);
+        hipLaunchKernelGGL((k_cut_lds<CBig, true, 1>), dim3(W.cut_blocks[1]), dim3(1), 0, W.side[1], G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, n2, 5, 8, (uint32_t)0, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, (const uint32_t*)bl[2]);
+                           W.cnt.p, W.errs.p, (const uint32_t*)bl[2], W.labels.p);
     } else {
         // a wavefront per tet: these lists are short and each tet's latency
         // is the kernel's time; the cuts start from the 3-material table's
@@ -397,22 +640,26 @@ void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev
                                                           : MI3Snap{TT.pat3, TT.snap_off3, TT.snap3};
         const unsigned g1 = (unsigned)std::min<uint64_t>(c.active + 1, 2048);
         const unsigned g2 = (unsigned)std::min<uint64_t>(c.active + 1, 1024);
-        hipLaunchKernelGGL((k_cut_group<CMed, 64, true>), dim3(g1), dim3(64), 0, s, G, vals,
+        hipLaunchKernelGGL((k_cut_group<CMed, 64, true>), dim3(g1), dim3(64), 0, W.side[0], G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, (const uint32_t*)bl[1], n1, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, 0, (uint32_t)0, m3s);
-        hipLaunchKernelGGL((k_cut_group<CBig, 64, true>), dim3(g2), dim3(64), 0, s, G, vals,
+                           W.cnt.p, W.errs.p, 0, (uint32_t)0, W.labels.p, m3s);
+        hipLaunchKernelGGL((k_cut_group<CBig, 64, true>), dim3(g2), dim3(64), 0, W.side[1], G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, (const uint32_t*)bl[2], n2, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, 0, (uint32_t)0, m3s);
+                           W.cnt.p, W.errs.p, 0, (uint32_t)0, W.labels.p, m3s);
     }
     if (W.wide) {
         const MI3Snap none{nullptr, nullptr, nullptr};
         hipLaunchKernelGGL((k_cut_group<CWideMI, 64, true>), dim3((unsigned)std::min<uint64_t>(c.active + 1, 512)),
-                           dim3(64), 0, s, G, vals, (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p,
+                           dim3(64), 0, W.side[2], G, vals, (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p,
                            (const uint32_t*)W.csr_off.p, (const uint8_t*)W.fit.p, (const uint32_t*)bl[3],
                            Count(ctr + M_LIST + 3, c.active, abort), (const uint32_t*)W.rec_off.p, W.rec.p, W.cnt.p,
-                           W.errs.p, 0, (uint32_t)0, none);
+                           W.errs.p, 0, (uint32_t)0, W.labels.p, none);
+    }
+    for (int q = 0; q < (W.wide ? 3 : 2); ++q) {
+        RIN_HIP(hipEventRecord(W.join[q], W.side[q]));
+        RIN_HIP(hipStreamWaitEvent(s, W.join[q], 0));
     }
     // extraction (src/extract_mesh.cpp:569-986): boundary-face pairing, then
     // occurrences in the reference's creation order
@@ -426,43 +673,57 @@ void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev
     A.fit = W.fit.p;
     A.rec = W.rec.p;
     A.n_active = NA;
-    hipLaunchKernelGGL(k_mi_nf_padded, dim3(blocks_for(c.active + 1)), dim3(256), 0, s, A, (uint64_t)c.active, W.fb.p);
-    scan_u32(W.mem, W.fb.p, W.fb.p, Count((uint64_t)c.active + 1), ctr + M_NFT, s);
-    hipLaunchKernelGGL(k_mi_check, dim3(1), dim3(64), 0, s, ctr, (const uint32_t*)W.csr_off.p, T, c, W.errs.p);
-    MIFaceKeys K;
-    K.fb = W.fb.p;
-    K.fl = W.fl.p;
-    K.fw = W.fw.p;
-    K.ft = W.ft.p;
-    const unsigned nbl = blocks_for((uint64_t)c.active * kBfaceLanes);
-    hipLaunchKernelGGL(k_mi_face_keys, dim3(nbl), dim3(256), 0, s, A, K);
-    hipLaunchKernelGGL(k_mi_bface, dim3(nbl), dim3(256), 0, s, A, K, W.emask.p);
-    hipLaunchKernelGGL(k_mi_count, dim3(blocks_for(c.active)), dim3(256), 0, s, A, (const uint64_t*)W.emask.p,
-                       W.cnt.p);
-    hipLaunchKernelGGL(k_mi_split_padded, dim3(blocks_for(c.active + 1)), dim3(256), 0, s, NA, (uint64_t)c.active,
-                       (const uint32_t*)W.cnt.p, W.tv.p, W.tf.p, W.tfv.p);
+    hipLaunchKernelGGL(k_mi_pair, dim3(blocks_for(c.active)), dim3(256), 0, s, A, (const uint32_t*)W.labels.p,
+                       W.emask.p, W.cnt.p);
     {
-        const uint32_t* in[3] = {W.tv.p, W.tf.p, W.tfv.p};
+        const uint32_t* in[3] = {W.cnt.p, W.cnt.p + 1, W.cnt.p + 2};
         uint32_t* out[3] = {W.cv.p, W.cf.p, W.cfv.p};
         uint32_t* tot[3] = {ctr + M_VO, ctr + M_FO, ctr + M_FV};
-        scan3_u32(W.mem, in, 1, out, Count((uint64_t)c.active + 1), tot, s);
+        scan3_u32(W.mem, in, 3, out, NA, tot, s);
     }
-    hipLaunchKernelGGL(k_mi_check, dim3(1), dim3(64), 0, s, ctr, (const uint32_t*)W.csr_off.p, T, c, W.errs.p);
+    hipLaunchKernelGGL(k_mi_check, dim3(1), dim3(64), 0, s, ctr, c, W.errs.p);
     hipLaunchKernelGGL(k_mi_extract, dim3(blocks_for(c.active)), dim3(256), 0, s, A, (const uint64_t*)W.emask.p,
                        (const uint32_t*)W.cv.p, (const uint32_t*)W.cf.p, (const uint32_t*)W.cfv.p, W.okey.p, W.oa.p,
                        W.oj.p, W.fq_a.p, W.fq_l.p, W.fq_m.p, W.fq_vs.p, W.fve.p);
-    // vertex dedup: each key's smallest occurrence by an atomic hash table,
-    // ids by a scan of the first-occurrence flags (the table is left empty)
+    // vertex dedup: on regular grids each key's first occurrence by its
+    // simplex's star, on explicit meshes by an atomic hash table (left empty);
+    // ids in the order of the first occurrences
     const Count NVO(ctr + M_VO, c.vo, abort);
-    (void)kbits;
-    hipLaunchKernelGGL(k_hash_insert, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)nullptr,
-                       (const uint64_t*)W.okey.p, W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p);
-    hipLaunchKernelGGL(k_hash_first, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)nullptr,
-                       (const uint32_t*)W.hslot.p, (const uint32_t*)W.hmx.p, W.first.p, W.mo.p);
-    scan_u32(W.mem, W.first.p, W.vrank.p, NVO, ctr + M_NV, s);
-    hipLaunchKernelGGL(k_dedup_assign, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.mo.p,
-                       (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p, NVO,
-                       (const uint32_t*)nullptr, (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p, true);
+    const uint32_t *vid = W.vid.p, *mo = nullptr;
+    if (G.regular) {
+        const unsigned tgrid = (unsigned)((c.vo + kDedupTile - 1) / kDedupTile);
+        StarArgs S;
+        S.res = G.res;
+        S.edge_shift = 14;
+        S.face_shift = 20;
+        S.own = 1;
+        S.okey = W.okey.p;
+        S.oa = W.oa.p;
+        S.act = W.act.p;
+        S.rank = W.rank.p;
+        S.voff = W.cv.p;
+        S.star_head = W.star_head.p;
+        S.star_ent = W.star_ent.p;
+        S.first = W.first.p;
+        S.mo = W.mo.p;
+        S.n_active = ctr + M_ACTIVE;
+        S.tile_first = W.tile_first.p;
+        hipLaunchKernelGGL(k_dedup_star, dim3(tgrid), dim3(256), 0, s, NVO, S);
+        hipLaunchKernelGGL(k_dedup_tile_scan, dim3(1), dim3(1024), 0, s, NVO, W.tile_first.p, ctr + M_NV);
+        hipLaunchKernelGGL(k_dedup_rank, dim3(tgrid), dim3(256), 0, s, NVO, (const uint32_t*)W.first.p,
+                           (const uint32_t*)W.tile_first.p, W.vrank.p, W.first_occ.p);
+        vid = W.vrank.p;
+        mo = W.mo.p;
+    } else {
+        hipLaunchKernelGGL(k_hash_insert, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)nullptr,
+                           (const uint64_t*)W.okey.p, W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p);
+        hipLaunchKernelGGL(k_hash_first, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)nullptr,
+                           (const uint32_t*)W.hslot.p, (const uint32_t*)W.hmx.p, W.first.p, W.mo.p);
+        scan_u32(W.mem, W.first.p, W.vrank.p, NVO, ctr + M_NV, s);
+        hipLaunchKernelGGL(k_dedup_assign, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.mo.p,
+                           (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p, NVO,
+                           (const uint32_t*)nullptr, (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p, true);
+    }
     // coordinates and faces
     const Count NV(ctr + M_NV, c.vo, abort), NF(ctr + M_FO, c.fo, abort), NFV(ctr + M_FV, c.fv, abort);
     hipLaunchKernelGGL(k_vert_fields_mi, dim3(blocks_for(c.vo)), dim3(256), 0, s, G, vals, (const uint32_t*)W.act.p,
@@ -471,7 +732,7 @@ void mi_path(MIWorkspace& W, const Grid& g, const Values& val, const MITablesDev
                        (const uint16_t*)W.oj.p, NV, W.v_tet.p, W.v_j.p, W.v_ss.p, W.v_sv.p, W.v_fn.p, W.xyz.p);
     hipLaunchKernelGGL(k_mi_face_out, dim3(blocks_for(c.fo)), dim3(256), 0, s, NF, (const uint32_t*)W.act.p,
                        (const uint32_t*)W.fq_a.p, (const uint16_t*)W.fq_l.p, (const uint8_t*)W.fq_m.p,
-                       (const uint32_t*)W.fq_vs.p, (const uint32_t*)W.fve.p, (const uint32_t*)W.vid.p, NFV,
+                       (const uint32_t*)W.fq_vs.p, (const uint32_t*)W.fve.p, vid, mo, NFV,
                        W.f_vstart.p, W.f_verts.p, W.f_tfstart.p, W.f_tf_tet.p, W.f_tf_local.p, W.f_func.p);
     hipLaunchKernelGGL(k_mi_close, dim3(1), dim3(64), 0, s, ctr, W.errs.p, c.fo, W.f_vstart.p, W.f_tfstart.p,
                        W.pub_d);
@@ -490,7 +751,6 @@ MICaps grow_caps(const MICaps& have, const uint32_t* pub, uint64_t T) {
     c.active = g(have.active, pub[M_ACTIVE]);
     c.fit = g(have.fit, pub[M_FIT]);
     c.words = g(have.words, pub[M_WORDS]);
-    c.nft = g(have.nft, pub[M_NFT]);
     c.vo = g(have.vo, pub[M_VO]);
     c.fo = g(have.fo, pub[M_FO]);
     c.fv = g(have.fv, pub[M_FV]);
@@ -498,7 +758,6 @@ MICaps grow_caps(const MICaps& have, const uint32_t* pub, uint64_t T) {
         // later stages did not count: make room in proportion to the tets
         c.fit = std::max<uint32_t>(c.fit, 3 * c.active);
         c.words = std::max<uint32_t>(c.words, 160 * c.active);
-        c.nft = std::max<uint32_t>(c.nft, 12 * c.active);
         c.vo = std::max<uint32_t>(c.vo, 8 * c.active);
         c.fo = std::max<uint32_t>(c.fo, 4 * c.active);
         c.fv = std::max<uint32_t>(c.fv, 16 * c.active);
@@ -540,63 +799,59 @@ void run_batched_mi(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t 
             c0.active = (uint32_t)std::min<uint64_t>(T, 1024 + T / 16);
             c0.fit = 3 * c0.active;
             c0.words = 160 * c0.active;
-            c0.nft = 12 * c0.active;
             c0.vo = 8 * c0.active;
             c0.fo = 4 * c0.active;
             c0.fv = 16 * c0.active;
             alloc_mi(w, g, c0, s);
         }
-        if (w.bound != val.vals.p) {
-            // (re-)record the path for these values; update the graph in place
+        if (!w.exec) {
+            // recorded once per workspace capacity: the graph holds no pointer
+            // to the values, which the first kernel of a run leaves for it
             const int kbits = 2 + std::max({bits_of(g.view.V), bits_of(g.view.n_edge_ids) + 12,
                                             bits_of(g.view.n_face_ids) + 18, bits_of(w.cap.active) + 10});
             if (kbits > 63) throw NeedsPlainForm("simplex keys exceed 63 bits for this mesh");
+            if (!w.fork) {
+                RIN_HIP(hipEventCreateWithFlags(&w.fork, hipEventDisableTiming));
+                for (int q = 0; q < 3; ++q) {
+                    RIN_HIP(hipStreamCreateWithFlags(&w.side[q], hipStreamNonBlocking));
+                    RIN_HIP(hipEventCreateWithFlags(&w.join[q], hipEventDisableTiming));
+                }
+                for (auto& e : w.ev) RIN_HIP(hipEventCreate(&e));
+            }
             hipGraph_t gr = nullptr;
             RIN_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
             try {
-                mi_path(w, g, val, TT, kbits, s);
+                mi_path(w, g, val.F, TT, s);
             } catch (...) {
                 (void)hipStreamEndCapture(s, &gr);
                 if (gr) (void)hipGraphDestroy(gr);
                 throw;
             }
             RIN_HIP(hipStreamEndCapture(s, &gr));
-            bool updated = false;
-            if (w.exec) {
-                hipGraphNode_t bad = nullptr;
-                hipGraphExecUpdateResult res;
-                updated = hipGraphExecUpdate(w.exec, gr, &bad, &res) == hipSuccess && res == hipGraphExecUpdateSuccess;
-                if (!updated) {
-                    (void)hipGetLastError();
-                    (void)hipGraphExecDestroy(w.exec);
-                    w.exec = nullptr;
-                }
-            }
-            if (!updated) RIN_HIP(hipGraphInstantiate(&w.exec, gr, nullptr, nullptr, 0));
-            if (w.graph) (void)hipGraphDestroy(w.graph);
             w.graph = gr;
-            w.bound = val.vals.p;
+            RIN_HIP(hipGraphInstantiate(&w.exec, gr, nullptr, nullptr, 0));
         }
-        hipEvent_t e0, e1;
-        RIN_HIP(hipEventCreate(&e0));
-        RIN_HIP(hipEventCreate(&e1));
         if (w.hash_dirty) {
             RIN_HIP(hipMemsetAsync(w.hkey.p, 0, 8ull << w.hbits, s));
             RIN_HIP(hipMemsetAsync(w.hmx.p, 0, 4ull << w.hbits, s));
             w.hash_dirty = false;
         }
-        RIN_HIP(hipEventRecord(e0, s));
+        if (!w.ctr_clear) hipLaunchKernelGGL(k_mi_zero, dim3(1), dim3(64), 0, s, w.ctr.p, w.errs.p);
+        w.ctr_clear = false;
+        RIN_HIP(hipEventRecord(w.ev[0], s));
+        // highest materials (src/material_interface.cpp:53-92), with the values
+        hipLaunchKernelGGL(k_highest_mi, dim3(blocks_for(g.view.V)), dim3(256), 0, s, (const double*)val.vals.p,
+                           g.view.V, val.F, w.hm.p, (uint32_t*)nullptr, w.ctr.p + M_DEGEN, w.vals_at.p);
         RIN_HIP(hipGraphLaunch(w.exec, s));
-        RIN_HIP(hipEventRecord(e1, s));
+        RIN_HIP(hipEventRecord(w.ev[1], s));
         RIN_HIP(hipStreamSynchronize(s));
+        w.ctr_clear = true;  // the run's closing kernel cleared them
         float ms = 0;
-        RIN_HIP(hipEventElapsedTime(&ms, e0, e1));
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        RIN_HIP(hipEventElapsedTime(&ms, w.ev[0], w.ev[1]));
         std::memcpy(pub, w.pub_h, sizeof(pub));
         uint32_t e = pub[kMiPub];
         // a stopped or failed run may leave table entries
-        if ((e & ~kMiHuge) || ((e & kMiHuge) && !w.wide)) w.hash_dirty = true;
+        if (w.hkey.p && ((e & ~kMiHuge) || ((e & kMiHuge) && !w.wide))) w.hash_dirty = true;
         if (e & kMiPlain) throw NeedsPlainForm("a tet has more materials than the device cut holds");
         if ((e & kMiHuge) && !w.wide) {
             // first run with such tets: the path captured again with the wide cut
@@ -624,10 +879,7 @@ void run_batched_mi(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t 
     out.F = val.F;
     out.num_degenerate = pub[M_DEGEN];
     out.n_active = out.num_intersecting = pub[M_ACTIVE];
-    uint32_t fit_total = 0;
-    RIN_HIP(hipMemcpyAsync(&fit_total, w.csr_off.p + T, 4, hipMemcpyDeviceToHost, s));
-    RIN_HIP(hipStreamSynchronize(s));
-    out.n_fit = fit_total;
+    out.n_fit = pub[M_FIT];
     for (int q = 0; q < 3; ++q) out.nb[q] = pub[M_LIST + 4 + q];
     out.n_cut34 = pub[M_LIST + 7];
     out.n_cut58 = pub[M_LIST + 8];

@@ -44,6 +44,13 @@ __device__ inline uint64_t count_of(const Count& n) { return n.get(); }
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, i##_end = count_of(n); i < i##_end; \
          i += (uint64_t)gridDim.x * blockDim.x)
 
+// the values themselves, or where a captured path's run left them
+struct ValsRef {
+    const double* p;
+    const double* const* at;
+    __device__ const double* get() const { return at ? *at : p; }
+};
+
 __device__ inline void flag_error(uint32_t* errs, uint32_t bit) { errs[threadIdx.x & 63] |= bit; }
 
 // The chip's 8 XCDs each have their own L2, and a launch's workgroups go to
@@ -153,7 +160,10 @@ __global__ void k_filter_ia(GridView g, const uint64_t* __restrict__ pos, const 
 // degen: per vertex (null: not written); total (null: not counted): the
 // number of tied vertices added per workgroup
 __global__ void k_highest_mi(const double* __restrict__ vals, uint64_t V, uint32_t F, uint64_t* __restrict__ hm,
-                             uint32_t* __restrict__ degen, uint32_t* __restrict__ total) {
+                             uint32_t* __restrict__ degen, uint32_t* __restrict__ total,
+                             const double** __restrict__ slot) {
+    // a captured path's later kernels find the values here
+    if (slot && blockIdx.x == 0 && threadIdx.x == 0) *slot = vals;
     uint32_t ties = 0;
     GRID_STRIDE(v, V) {
         double mx = vals[v];
@@ -291,13 +301,28 @@ __host__ __device__ inline void mi_counts(const Complex<C>& X, uint32_t& niv, ui
     for (int w = 0; w < W; ++w) niv += (uint32_t)__builtin_popcountll(iso[w]);
 }
 
+// Material labels on the tet faces: bit 8 l + b when a face on tet face l has
+// label 4 + b below it; kLabelsAsk when the labels alone cannot answer for
+// the face pairing (coincident materials, or a label beyond the eighth).
+constexpr uint32_t kLabelsAsk = 0xFFFFFFFFu;
+template <class C>
+__host__ __device__ inline uint32_t mi_face_labels(const Complex<C>& X) {
+    uint32_t m = X.dup ? kLabelsAsk : 0u;
+    for (int f = 0; f < X.nf; ++f) {
+        if (X.fa[f] > 3) continue;
+        const int b = (int)X.fb[f] - 4;
+        m |= b < 8 ? 1u << (8 * X.fa[f] + b) : kLabelsAsk;
+    }
+    return m;
+}
+
 // One active tet's cut into its record slot.
 template <class C, bool MI>
 __device__ inline void cut_tet(const GridView& g, const double* __restrict__ vals, const uint32_t* __restrict__ act,
                                const uint32_t* __restrict__ csr_off, const uint8_t* __restrict__ fit, uint64_t a, int k,
                                uint32_t flags, const uint32_t* __restrict__ rec_off, uint16_t* __restrict__ rec,
                                uint32_t* __restrict__ cnt, uint32_t* __restrict__ errs, Complex<C>& X,
-                               dev::InsertTemps<C>& Tm) {
+                               dev::InsertTemps<C>& Tm, uint32_t* __restrict__ labels) {
     const uint64_t V = g.V;
     const uint32_t t = act[a];
     uint32_t v[4];
@@ -318,6 +343,7 @@ __device__ inline void cut_tet(const GridView& g, const double* __restrict__ val
         cnt[3 * a] = CNT_RETRY;
         cnt[3 * a + 1] = cnt[3 * a + 2] = 0;
         rec[rec_off[a]] = 0;
+        if (MI && labels) labels[a] = kLabelsAsk;
         return;
     }
     const int cap = (int)(rec_off[a + 1] - rec_off[a]);
@@ -328,6 +354,7 @@ __device__ inline void cut_tet(const GridView& g, const double* __restrict__ val
         cnt[3 * a] = CNT_RETRY;
         cnt[3 * a + 1] = cnt[3 * a + 2] = 0;
         rec[rec_off[a]] = 0;
+        if (MI && labels) labels[a] = kLabelsAsk;
         return;
     }
     uint32_t a0, a1, a2;
@@ -337,6 +364,7 @@ __device__ inline void cut_tet(const GridView& g, const double* __restrict__ val
         a2 = X.nc;
     } else if (MI) {
         mi_counts<C>(X, a0, a1, a2);
+        if (labels) labels[a] = mi_face_labels<C>(X);
     } else {
         ia_counts<C>(X, a0, a1, a2);
     }
@@ -350,13 +378,14 @@ __device__ inline void cut_tet(const GridView& g, const double* __restrict__ val
 // through its cut is the kernel's time and LDS answers several times faster
 // than the device-memory workspace.
 template <class C, bool MI, int LANES>
-__global__ void __launch_bounds__(64) k_cut_lds(GridView g, const double* __restrict__ vals,
+__global__ void __launch_bounds__(64) k_cut_lds(GridView g, ValsRef vref,
                                                 const uint32_t* __restrict__ act, const uint8_t* __restrict__ act_k,
                                                 const uint32_t* __restrict__ csr_off, const uint8_t* __restrict__ fit,
                                                 Count n_active, int kmin, int kmax, uint32_t flags,
                                                 const uint32_t* __restrict__ rec_off, uint16_t* __restrict__ rec,
                                                 uint32_t* __restrict__ cnt, uint32_t* __restrict__ errs,
-                                                const uint32_t* __restrict__ list) {
+                                                const uint32_t* __restrict__ list, uint32_t* __restrict__ labels) {
+    const double* __restrict__ vals = vref.get();
     __shared__ Complex<C> Xs[LANES];
     __shared__ dev::InsertTemps<C> Ts[LANES];
     const int l = threadIdx.x < LANES ? threadIdx.x : 0;
@@ -368,7 +397,7 @@ __global__ void __launch_bounds__(64) k_cut_lds(GridView g, const double* __rest
         const uint64_t a = list ? list[i] : i;
         const int k = act_k[a];
         if (k < kmin || k > kmax) continue;
-        cut_tet<C, MI>(g, vals, act, csr_off, fit, a, k, flags, rec_off, rec, cnt, errs, X, Tm);
+        cut_tet<C, MI>(g, vals, act, csr_off, fit, a, k, flags, rec_off, rec, cnt, errs, X, Tm, labels);
     }
 }
 
@@ -556,14 +585,15 @@ __device__ __forceinline__ bool mi3_start(dev::WaveMI<C>& X, const MI3Snap& S, i
 // check takes 0.25 ms of cuts, and took 4.7 ms a lane a tet, 1.4 ms of them
 // for a single tet of five functions.
 template <class C, int G, bool MI>
-__global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __restrict__ vals,
+__global__ void __launch_bounds__(64) k_cut_group(GridView g, ValsRef vref,
                                                   const uint32_t* __restrict__ act, const uint8_t* __restrict__ act_k,
                                                   const uint32_t* __restrict__ csr_off,
                                                   const uint8_t* __restrict__ fit, const uint32_t* __restrict__ list,
                                                   Count nlist, const uint32_t* __restrict__ rec_off,
                                                   uint16_t* __restrict__ rec, uint32_t* __restrict__ cnt,
                                                   uint32_t* __restrict__ errs, int retry, uint32_t flags,
-                                                  typename std::conditional<MI, MI3Snap, K2Snap>::type snap) {
+                                                  uint32_t* __restrict__ labels, typename std::conditional<MI, MI3Snap, K2Snap>::type snap) {
+    const double* __restrict__ vals = vref.get();
     constexpr int NG = 64 / G;
     using Cx = typename std::conditional<MI, dev::WaveMI<C>, dev::WaveIA<C>>::type;
     __shared__ Cx Xs[NG];
@@ -602,9 +632,17 @@ __global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __re
             a1 = (uint32_t)X.nf;
             a2 = (uint32_t)X.nc;
         } else if (!X.err) {
-            if constexpr (MI)
+            if constexpr (MI) {
                 len = dev::wave_mi_record<C, G>(X, k, out, cap, a0, a1, a2);
-            else
+                uint32_t m = X.dup ? kLabelsAsk : 0u;
+                for (int f = lane; f < X.nf; f += G) {
+                    if (X.fa[f] > 3) continue;
+                    const int b = (int)X.fb[f] - 4;
+                    m |= b < 8 ? 1u << (8 * X.fa[f] + b) : kLabelsAsk;
+                }
+                for (int d = G / 2; d > 0; d >>= 1) m |= __shfl_xor(m, d, G);
+                if (lane == 0 && len >= 0) labels[a] = m;
+            } else
                 len = dev::wave_ia_record<C, G>(X, k, out, cap, a0, a1, a2);
         }
         if (lane == 0) {
@@ -618,6 +656,7 @@ __global__ void __launch_bounds__(64) k_cut_group(GridView g, const double* __re
                 }
                 out[0] = 0;
                 a1 = a2 = 0;
+                if (MI && labels) labels[a] = kLabelsAsk;
             }
             cnt[3 * a] = a0;
             cnt[3 * a + 1] = a1;
@@ -638,7 +677,7 @@ __global__ void __launch_bounds__(64) k_cut_huge(GridView g, const double* __res
                                                  const uint32_t* __restrict__ rec_off, uint16_t* __restrict__ rec,
                                                  uint32_t* __restrict__ cnt, uint32_t* __restrict__ errs,
                                                  uint8_t* __restrict__ ws, const uint32_t* __restrict__ rec_loc,
-                                                 uint32_t fixed_cap) {
+                                                 uint32_t fixed_cap, uint32_t* __restrict__ labels) {
     using C = CHuge;
     const uint64_t V = g.V;
     const uint64_t lane = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -679,6 +718,7 @@ __global__ void __launch_bounds__(64) k_cut_huge(GridView g, const double* __res
             a2 = X.nc;
         } else if (MI) {
             mi_counts<C>(X, a0, a1, a2);
+            labels[a] = mi_face_labels<C>(X);
         } else {
             ia_counts<C>(X, a0, a1, a2);
         }
@@ -1303,6 +1343,8 @@ constexpr int kStarShapes = 1 + 27 + 27 * 27;  // corner, edge by direction, fac
 
 struct StarArgs {
     int res;
+    int edge_shift, face_shift;  // where the edge and face ids begin in a key
+    int own;                     // a tet may hold a key more than once (its own occurrences are searched too)
     const uint64_t* okey;
     const uint32_t *oa, *act, *rank, *voff;
     const uint32_t* star_head;  // [2][kStarShapes]: first entry << 8 | entry count
@@ -1329,11 +1371,11 @@ struct StarWalk {
             a = (uint32_t)(K >> 2);
             shape = 0;
         } else if (type == 1) {
-            const uint64_t x = K >> 8;
+            const uint64_t x = K >> A.edge_shift;
             a = (uint32_t)(x / 27);
             shape = 1 + (uint32_t)(x % 27);
         } else {
-            const uint64_t fc = K >> 14;
+            const uint64_t fc = K >> A.face_shift;
             a = (uint32_t)(fc / 729);
             shape = 28 + (uint32_t)(fc % 729);
         }
@@ -1363,13 +1405,13 @@ struct StarWalk {
 // The first occurrence of key K, held by tet t at occurrence o, among the
 // star's tets after the lowest (which does not hold it) and up to t.
 __device__ __forceinline__ uint32_t star_walk_first(const StarArgs& A, uint32_t NA, uint32_t NO, uint64_t K, uint32_t t,
-                                                 uint32_t o) {
+                                                    uint32_t oa, uint32_t o) {
     const uint32_t R = (uint32_t)A.res;
     StarWalk S(A, R + 1, K);
     (void)S.next(A, R);
     for (;;) {
         const uint64_t ts = S.next(A, R);
-        if (ts >= t) return o;
+        if (ts >= t) break;
         const uint32_t a = A.rank[ts];
         if (a >= NA || A.act[a] != (uint32_t)ts) continue;
         uint32_t hi = a + 1 < NA ? A.voff[a + 1] : NO;
@@ -1377,6 +1419,10 @@ __device__ __forceinline__ uint32_t star_walk_first(const StarArgs& A, uint32_t 
         for (uint32_t p = A.voff[a]; p < hi; ++p)
             if (A.okey[p] == K) return p;
     }
+    if (A.own)
+        for (uint32_t p = A.voff[oa]; p < o; ++p)
+            if (A.okey[p] == K) return p;
+    return o;
 }
 
 __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
@@ -1406,8 +1452,9 @@ __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
 #pragma unroll
     for (int u = 0; u < kDedupU; ++u) {
         // interior keys, and keys whose lowest star tet is this one, are first here
-        found[u] = ((K[u] & 3) == 3 || ts[u] == t[u]) ? o[u] : ~0u;
-        as[u] = (found[u] == ~0u && ts[u] != ~0ull) ? A.rank[ts[u]] : ~0u;
+        // (with `own`, after a look at this one's earlier occurrences)
+        found[u] = ((K[u] & 3) == 3 || (ts[u] == t[u] && !A.own)) ? o[u] : ~0u;
+        as[u] = (found[u] == ~0u && ts[u] != ~0ull) ? (ts[u] == t[u] ? oa[u] : A.rank[ts[u]]) : ~0u;
     }
 #pragma unroll
     for (int u = 0; u < kDedupU; ++u) {
@@ -1432,7 +1479,7 @@ __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
 #pragma unroll
     for (int u = 0; u < kDedupU; ++u) {
         const bool in = o[u] < NO;
-        if (in && found[u] == ~0u) found[u] = star_walk_first(A, NA, NO, K[u], t[u], o[u]);
+        if (in && found[u] == ~0u) found[u] = star_walk_first(A, NA, NO, K[u], t[u], oa[u], o[u]);
         if (in) {
             A.first[o[u]] = found[u] == o[u];
             A.mo[o[u]] = found[u];
@@ -1723,13 +1770,6 @@ __global__ void k_dedup_assign(Count n, const uint32_t* __restrict__ mo, const u
 
 // vertex records and coordinates (src/extract_mesh.cpp:95-228, 1446-1538)
 // off: CSR offsets by tet (per_rank false) or by active rank (per_rank true)
-// the values themselves, or where a captured path's run left them
-struct ValsRef {
-    const double* p;
-    const double* const* at;
-    __device__ const double* get() const { return at ? *at : p; }
-};
-
 struct VertFieldArgs {
     GridView g;
     ValsRef vals;

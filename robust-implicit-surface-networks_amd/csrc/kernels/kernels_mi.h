@@ -73,6 +73,7 @@ struct MI2Entry {
     uint16_t off, len;   // record words in the table's word array
     uint32_t cnt[3];     // interface vertices, faces, face corners
     uint32_t cut[3];     // vertices, faces, cells of the complex
+    uint32_t labels;     // mi_face_labels
 };
 
 // 3 materials a < b < c: the complex of a and b is one of the 81 patterns
@@ -91,7 +92,7 @@ struct MITablesDev {
     const MI2Entry* e2 = nullptr;
     const uint16_t* w2 = nullptr;
     const MI3Pat* pat3 = nullptr;
-    const uint32_t *off3 = nullptr, *cnt3 = nullptr, *cut3 = nullptr;
+    const uint32_t *off3 = nullptr, *cnt3 = nullptr, *cut3 = nullptr, *lab3 = nullptr;
     const uint16_t* w3 = nullptr;
     const uint32_t* snap_off3 = nullptr;  // complexes after three materials (MI3Snap)
     const uint8_t* snap3 = nullptr;
@@ -105,6 +106,7 @@ inline MITablesDev mi_tables_view(const MITablesRaw& r) {
     d.off3 = (const uint32_t*)r.off3;
     d.cnt3 = (const uint32_t*)r.cnt3;
     d.cut3 = (const uint32_t*)r.cut3;
+    d.lab3 = (const uint32_t*)r.lab3;
     d.w3 = (const uint16_t*)r.w3;
     d.snap_off3 = (const uint32_t*)r.snap_off3;
     d.snap3 = (const uint8_t*)r.snap3;
@@ -117,15 +119,16 @@ inline MITablesDev mi_tables_view(const MITablesRaw& r) {
 // general cut (CNT_RETRY).  rec_loc (optional): the record words hold the two
 // tables' words at base2 and base3, and the tet's record location becomes the
 // table record's instead of a copy into its slot.
-__global__ void __launch_bounds__(256) k_mi_table(GridView g, const double* __restrict__ vals,
+__global__ void __launch_bounds__(256) k_mi_table(GridView g, ValsRef vref,
                                                   const uint32_t* __restrict__ act,
                                                   const uint32_t* __restrict__ csr_off, const uint8_t* __restrict__ fit,
                                                   const uint32_t* __restrict__ list, uint64_t n,
                                                   const uint32_t* __restrict__ n_dev, uint32_t flags,
                                                   const uint32_t* __restrict__ rec_off, uint16_t* __restrict__ rec,
                                                   uint32_t* __restrict__ cnt, uint32_t* __restrict__ errs,
-                                                  MITablesDev T, uint32_t* __restrict__ rec_loc, uint32_t base2,
-                                                  uint32_t base3) {
+                                                  MITablesDev T, uint32_t* __restrict__ labels,
+                                                  uint32_t* __restrict__ rec_loc, uint32_t base2, uint32_t base3) {
+    const double* __restrict__ vals = vref.get();
     __shared__ MI3Pat pats[81];
     for (int i = threadIdx.x; i < 81 * (int)sizeof(MI3Pat) / 4; i += blockDim.x)
         reinterpret_cast<uint32_t*>(pats)[i] = reinterpret_cast<const uint32_t*>(T.pat3)[i];
@@ -147,12 +150,13 @@ __global__ void __launch_bounds__(256) k_mi_table(GridView g, const double* __re
         int pat = 0;
         for (int c = 0, w = 1; c < 4; ++c, w *= 3) pat += (P[1][c] > P[0][c] ? 2 : (P[1][c] < P[0][c] ? 0 : 1)) * w;
         const uint16_t* src = nullptr;
-        uint32_t len = 0, c3[3], at_table = 0;
+        uint32_t len = 0, c3[3], at_table = 0, lab = 0;
         if (k == 2) {
             const MI2Entry E = T.e2[pat];
             src = T.w2 + E.off;
             at_table = base2 + E.off;
             len = E.len;
+            lab = E.labels;
             const uint32_t* cc = (flags & RUN_CUT_ONLY) ? E.cut : E.cnt;
             c3[0] = cc[0];
             c3[1] = cc[1];
@@ -170,6 +174,7 @@ __global__ void __launch_bounds__(256) k_mi_table(GridView g, const double* __re
                 src = T.w3 + off;
                 at_table = base3 + off;
                 len = src[6];
+                lab = T.lab3[slot];
                 const uint32_t pk = (flags & RUN_CUT_ONLY) ? T.cut3[slot] : T.cnt3[slot];
                 c3[0] = pk & 0xFF;
                 c3[1] = (pk >> 8) & 0xFF;
@@ -182,8 +187,10 @@ __global__ void __launch_bounds__(256) k_mi_table(GridView g, const double* __re
             cnt[3 * (uint64_t)a] = CNT_RETRY;
             cnt[3 * (uint64_t)a + 1] = cnt[3 * (uint64_t)a + 2] = 0;
             rec[at] = 0;
+            labels[a] = kLabelsAsk;
             continue;
         }
+        labels[a] = lab;
         if (rec_loc)
             rec_loc[a] = at_table;
         else
@@ -311,6 +318,7 @@ __device__ inline bool mi_bface_emits(const MIArgs& A, const MITet& M, uint64_t 
     uint64_t k3[3];
     bool have_k3 = false;
     const MITet N(A.g, A.rec + A.rec_loc[r2], t2, A.csr_off[t2]);
+    if (N.R.r[0] != 2) return false;  // its cut failed (and with it the run)
     const uint16_t* G = N.R.faces();
     for (int f = 0; f < N.R.nf; ++f) {
         const int n = G[3];
@@ -337,22 +345,6 @@ __device__ inline bool mi_bface_emits(const MIArgs& A, const MITet& M, uint64_t 
     return false;
 }
 
-// interface-vertex mask of a tet (vertices of faces with positive label > 3)
-__device__ inline void mi_iface_mask(const Rec& R, uint64_t m[kMaskWords]) {
-    for (int w = 0; w < kMaskWords; ++w) m[w] = 0;
-    const uint16_t* F = R.faces();
-    for (int f = 0; f < R.nf; ++f) {
-        const int n = F[3];
-        if (F[0] > 3)
-            for (int q = 0; q < n; ++q) m[F[4 + q] >> 6] |= 1ull << (F[4 + q] & 63);
-        F += 4 + n;
-    }
-}
-__device__ inline uint32_t mask_rank(const uint64_t m[kMaskWords], int j) {
-    uint32_t r = 0;
-    for (int w = 0; w < (j >> 6); ++w) r += __popcll(m[w]);
-    return r + __popcll(m[j >> 6] & ((1ull << (j & 63)) - 1));
-}
 __device__ inline bool is_corner(const Rec& R, int j) {
     const uint16_t* L4 = R.vert(j);
     return L4[2] <= 3;  // sorted labels: three tet faces
@@ -368,108 +360,74 @@ __device__ inline int corner_of(const Rec& R, int j) {
 // Which tet-boundary faces of each active tet become interface faces here
 // (the reference's two-map pairing): bit f for face f < 63; bit 63 marks a
 // tet with more faces, whose faces from 63 on are tested where they are used.
-// The faces' keys are computed once: per active tet its face count (k_mi_nf),
-// a scan gives each tet's first face slot, k_mi_face_keys writes every face's
-// tet face, corner count, record word offset and (boundary faces) its
-// (min, second-min, max) vertex-key triple, and k_mi_bface compares a
-// boundary face's triple with those of the neighbour's faces on the shared
-// tet face.  kBfaceLanes lanes per tet (adjacent lanes of one wave) take
-// faces f = lane, lane + kBfaceLanes, ...
-constexpr int kBfaceLanes = 8;
+//
+// A face emits when its copy in the lower neighbour carries other materials.
+// In each tet a material without coincident ones has one face on a tet face,
+// the region where it is the highest there, so when the neighbour has a face
+// of the same material on the shared tet face, that is the copy (or the copy's
+// corners are named differently and there is none) and nothing emits.  So a
+// tet's labels on its tet faces against its lower neighbours' decide nearly
+// every tet with a few loads; only tets whose materials do not all recur, or
+// with coincident materials, compare the faces themselves (mi_bface_emits).
+// Writing every face's vertex-key triple, comparing those and counting again
+// took 106 us and three more launches at 65^3 vertices and 8 materials (234 us
+// at 100^3 and 18); this takes 10 us (21).
+//
+// counts: cnt holds the cut's interface vertices, faces and corners; a tet
+// that emits adds its own.
 constexpr int kBfaceBits = 63;
 
-struct MIFaceKeys {
-    const uint32_t* fb;  // first face slot of each active tet (n_active + 1 entries)
-    uint16_t* fl;        // tet face (0..3, or 0xFF inside) | corners << 8
-    uint16_t* fw;        // word offset of the face in its record
-    uint64_t* ft;        // vertex-key triple (boundary faces)
-};
-
-__global__ void k_mi_nf(MIArgs A, uint32_t* __restrict__ nf) {
+__global__ void k_mi_pair(MIArgs A, const uint32_t* __restrict__ labels, uint64_t* __restrict__ emask,
+                          uint32_t* __restrict__ cnt) {
+    const uint64_t n = count_of(A.n_active);
     GRID_STRIDE(a, A.n_active) {
-        const uint16_t* r = A.rec + A.rec_loc[a];
-        nf[a] = r[0] == 2 ? r[3] : 0u;
-    }
-}
-
-__global__ void k_mi_face_keys(MIArgs A, MIFaceKeys K) {
-    const uint64_t n = count_of(A.n_active) * kBfaceLanes;
-    GRID_STRIDE(idx, n) {
-        const uint64_t a = idx / kBfaceLanes;
-        const int l0 = (int)(idx % kBfaceLanes);
-        const uint32_t t = A.act[a];
-        const MITet M(A.g, A.rec + A.rec_loc[a], t, A.csr_off[t]);
-        if (M.R.r[0] != 2) continue;
-        const int nf = M.R.nf;
-        const uint32_t fb = K.fb[a];
-        const uint16_t* F = M.R.faces();
-        for (int f = 0; f < l0 && f < nf; ++f) F += 4 + F[3];
-        for (int f = l0; f < nf; f += kBfaceLanes) {
-            const uint32_t slot = fb + (uint32_t)f;
-            const int l = F[0];
-            K.fl[slot] = (uint16_t)((l <= 3 ? l : 0xFF) | F[3] << 8);
-            K.fw[slot] = (uint16_t)(F - M.R.r);
-            if (l <= 3) {
-                uint64_t k3[3];
-                mi_face_triple(A.g, M, A.fit, a, F, k3);
-                K.ft[3 * (uint64_t)slot] = k3[0];
-                K.ft[3 * (uint64_t)slot + 1] = k3[1];
-                K.ft[3 * (uint64_t)slot + 2] = k3[2];
-            }
-            for (int q = 0; q < kBfaceLanes && f + q + 1 < nf; ++q) F += 4 + F[3];
+        const uint32_t t = A.act[a], lm = labels[a], s0 = A.csr_off[t];
+        uint32_t r2[4], l2[4];
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const uint32_t nb = A.nbr[4 * (uint64_t)t + l], t2 = nb >> 2;
+            l2[l] = nb & 3;
+            r2[l] = nb != NO_NBR && t2 < t ? A.rank[t2] : ~0u;
+            if (r2[l] < n && A.act[r2[l]] != t2) r2[l] = ~0u;
         }
-    }
-}
-
-__global__ void k_mi_bface(MIArgs A, MIFaceKeys K, uint64_t* __restrict__ emask) {
-    const uint64_t n = count_of(A.n_active) * kBfaceLanes;
-    GRID_STRIDE(idx, n) {
-        const uint64_t a = idx / kBfaceLanes;
-        const int l0 = (int)(idx % kBfaceLanes);
-        const uint32_t t = A.act[a];
-        const uint16_t* r = A.rec + A.rec_loc[a];
-        uint64_t bits = 0;
-        if (r[0] == 2) {
-            const int nf = r[3], nt = nf < kBfaceBits ? nf : kBfaceBits;
-            const uint32_t fb = K.fb[a];
-            for (int f = l0; f < nt; f += kBfaceLanes) {
-                const uint32_t slot = fb + (uint32_t)f;
-                const uint16_t fl = K.fl[slot];
-                const uint32_t l = fl & 0xFFu;
-                if (l > 3) continue;
-                const uint32_t nb = A.nbr[4 * (uint64_t)t + l];
-                if (nb == NO_NBR) continue;
-                const uint32_t t2 = nb >> 2, l2 = nb & 3;
-                if (t2 >= t) continue;
-                const uint32_t r2 = A.rank[t2];
-                if (!(r2 < count_of(A.n_active) && A.act[r2] == t2)) continue;
-                const uint64_t k0 = K.ft[3 * (uint64_t)slot], k1 = K.ft[3 * (uint64_t)slot + 1],
-                               k2 = K.ft[3 * (uint64_t)slot + 2];
-                // the copy: on the shared tet face, as many corners, same key triple
-                const uint16_t want = (uint16_t)(l2 | (fl & 0xFF00u));
-                const uint32_t g0 = K.fb[r2], g1 = K.fb[r2 + 1];
-                for (uint32_t gs = g0; gs < g1; ++gs) {
-                    if (K.fl[gs] != want) continue;
-                    if (K.ft[3 * (uint64_t)gs] != k0 || K.ft[3 * (uint64_t)gs + 1] != k1 ||
-                        K.ft[3 * (uint64_t)gs + 2] != k2)
-                        continue;
-                    const MITet M(A.g, r, t, A.csr_off[t]);
-                    const MITet N(A.g, A.rec + A.rec_loc[r2], t2, A.csr_off[t2]);
-                    const uint16_t* G = N.R.r + K.fw[gs];
-                    const uint16_t* F = M.R.r + K.fw[slot];
-                    bool share = false;
-                    mi_side_each(N, A.fit, G[1], [&](uint8_t x) {
-                        mi_side_each(M, A.fit, F[1], [&](uint8_t y) { share |= x == y; });
-                    });
-                    if (!share) bits |= 1ull << f;
-                    break;
+        bool ask = false;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            if (r2[l] >= n) continue;
+            const uint32_t lo = labels[r2[l]];
+            if (lm == kLabelsAsk || lo == kLabelsAsk) {
+                ask = true;
+                continue;
+            }
+            const uint32_t s2 = A.csr_off[A.act[r2[l]]];
+            uint64_t theirs = 0;
+            for (uint32_t m = lo >> (8 * l2[l]) & 255u; m; m &= m - 1) theirs |= 1ull << A.fit[s2 + __builtin_ctz(m)];
+            for (uint32_t m = lm >> (8 * l) & 255u; m; m &= m - 1) ask |= !(theirs >> A.fit[s0 + __builtin_ctz(m)] & 1);
+        }
+        uint64_t em = 0;
+        if (ask) {
+            const MITet M(A.g, A.rec + A.rec_loc[a], t, s0);
+            if (M.R.r[0] == 2) {
+                uint32_t nv = cnt[3 * a], nf = cnt[3 * a + 1], nfv = cnt[3 * a + 2];
+                const uint16_t* F = M.R.faces();
+                for (int f = 0; f < M.R.nf; ++f) {
+                    const int c = F[3];
+                    uint8_t other;
+                    if (F[0] <= 3 && mi_bface_emits(A, M, a, F, other)) {
+                        if (f < kBfaceBits) em |= 1ull << f;
+                        ++nf;
+                        nfv += c;
+                        for (int q = 0; q < c; ++q) nv += is_corner(M.R, F[4 + q]);
+                    }
+                    F += 4 + c;
                 }
+                if (M.R.nf > kBfaceBits) em |= 1ull << kBfaceBits;
+                cnt[3 * a] = nv;
+                cnt[3 * a + 1] = nf;
+                cnt[3 * a + 2] = nfv;
             }
-            if (nf > kBfaceBits) bits |= 1ull << kBfaceBits;
         }
-        // the lanes of one tet are adjacent and leave the loop together
-        for (int d = 1; d < kBfaceLanes; d <<= 1) bits |= __shfl_xor(bits, d, 64);
-        if (l0 == 0) emask[a] = bits;
+        emask[a] = em;
     }
 }
 
@@ -481,40 +439,69 @@ __device__ inline bool mi_emits(const MIArgs& A, const MITet& M, uint64_t a, con
         // rare: the scan again for the first copy's material
         return mi_bface_emits(A, M, a, F, other);
     }
-    return mi_bface_emits(A, M, a, F, other);
+    return (em >> kBfaceBits) && mi_bface_emits(A, M, a, F, other);
 }
 
-// per active tet: vertex occurrences (phase 0 + phase 1), faces, face corners
-__global__ void k_mi_count(MIArgs A, const uint64_t* __restrict__ emask, uint32_t* __restrict__ cnt) {
-    GRID_STRIDE(a, A.n_active) {
-        const uint32_t t = A.act[a];
-        const MITet M(A.g, A.rec + A.rec_loc[a], t, A.csr_off[t]);
-        uint32_t nv = 0, nf = 0, nfv = 0;
-        if (M.R.r[0] == 2) {
-            const uint64_t em = emask[a];
-            uint64_t m[kMaskWords];
-            mi_iface_mask(M.R, m);
-            for (int w = 0; w < kMaskWords; ++w) nv += __popcll(m[w]);
-            const uint16_t* F = M.R.faces();
-            for (int f = 0; f < M.R.nf; ++f) {
-                const int n = F[3];
-                if (F[0] > 3) {
-                    ++nf;
-                    nfv += n;
-                } else if (f < kBfaceBits ? ((em >> f) & 1) != 0 : [&] {
-                               uint8_t other;
-                               return mi_bface_emits(A, M, a, F, other);
-                           }()) {
-                    ++nf;
-                    nfv += n;
-                    for (int q = 0; q < n; ++q) nv += is_corner(M.R, F[4 + q]);
+// One tet's occurrences and face rows.  W words of vertex mask: one for the
+// tables' and nearly every other complex, held in registers (the sixteen of
+// any record, indexed, live in scratch memory and cost every lane: 55 us at
+// 65^3 vertices and 8 materials against 43, 86 at 100^3 and 18 against 60).
+template <int W>
+__device__ inline void mi_extract_tet(const MIArgs& A, const MITet& M, uint64_t a, uint64_t em, uint32_t vb, uint32_t q,
+                                      uint32_t e, uint64_t* __restrict__ okey, uint32_t* __restrict__ oa,
+                                      uint16_t* __restrict__ oj, uint32_t* __restrict__ fq_a,
+                                      uint16_t* __restrict__ fq_l, uint8_t* __restrict__ fq_m,
+                                      uint32_t* __restrict__ fq_vs, uint32_t* __restrict__ fve) {
+    uint64_t m[W];
+    for (int w = 0; w < W; ++w) m[w] = 0;
+    const uint16_t* F = M.R.faces();
+    for (int f = 0; f < M.R.nf; ++f) {
+        const int n = F[3];
+        if (F[0] > 3)
+            for (int i = 0; i < n; ++i) m[W == 1 ? 0 : F[4 + i] >> 6] |= 1ull << (F[4 + i] & 63);
+        F += 4 + n;
+    }
+    uint32_t o = vb;
+    auto put = [&](int j) {
+        int nb;
+        okey[o] = mi_vkey(A.g, M, A.fit, a, j, nb);
+        oa[o] = (uint32_t)a;
+        oj[o] = (uint16_t)j;
+        ++o;
+    };
+    for (int w = 0; w < W; ++w)
+        for (uint64_t b = m[w]; b; b &= b - 1) put(64 * w + __builtin_ctzll(b));
+    auto rank = [&](int j) {
+        uint32_t r = 0;
+        for (int w = 0; w < W && W > 1; ++w) r += w < (j >> 6) ? (uint32_t)__popcll(m[w]) : 0u;
+        return r + (uint32_t)__popcll(m[W == 1 ? 0 : j >> 6] & ((1ull << (j & 63)) - 1));
+    };
+    F = M.R.faces();
+    for (int f = 0; f < M.R.nf; ++f) {
+        const int n = F[3];
+        uint8_t other = 0xFF;
+        const bool iface = F[0] > 3;
+        if (iface || mi_emits(A, M, a, F, f, em, other)) {
+            fq_a[q] = (uint32_t)a;
+            fq_l[q] = (uint16_t)f;
+            fq_m[2 * q] = iface ? A.fit[M.s0 + F[0] - 4] : other;
+            fq_m[2 * q + 1] = A.fit[M.s0 + F[1] - 4];
+            fq_vs[q] = e;
+            for (int i = 0; i < n; ++i) {
+                const int j = F[4 + i];
+                if (!iface && is_corner(M.R, j)) {
+                    // phase 1: the corner is created here if it is new
+                    okey[o] = key_corner(M.vc(corner_of(M.R, j)));
+                    oa[o] = (uint32_t)a;
+                    oj[o] = (uint16_t)j;
+                    fve[e++] = o++;
+                } else {
+                    fve[e++] = vb + rank(j);
                 }
-                F += 4 + n;
             }
+            ++q;
         }
-        cnt[3 * a] = nv;
-        cnt[3 * a + 1] = nf;
-        cnt[3 * a + 2] = nfv;
+        F += 4 + n;
     }
 }
 
@@ -528,58 +515,22 @@ __global__ void __launch_bounds__(256) k_mi_extract(MIArgs A, const uint64_t* __
         const uint32_t t = A.act[a];
         const MITet M(A.g, A.rec + A.rec_loc[a], t, A.csr_off[t]);
         if (M.R.r[0] != 2) continue;
-        uint64_t m[kMaskWords];
-        mi_iface_mask(M.R, m);
-        const uint32_t vb = voff[a];
-        uint32_t o = vb;
-        for (int j = 0; j < M.R.nv; ++j) {
-            if (!((m[j >> 6] >> (j & 63)) & 1)) continue;
-            int nb;
-            okey[o] = mi_vkey(A.g, M, A.fit, a, j, nb);
-            oa[o] = (uint32_t)a;
-            oj[o] = (uint16_t)j;
-            ++o;
-        }
-        uint32_t q = foff[a], e = fvoff[a];
-        const uint64_t em = emask[a];
-        const uint16_t* F = M.R.faces();
-        for (int f = 0; f < M.R.nf; ++f) {
-            const int n = F[3];
-            uint8_t other = 0xFF;
-            const bool iface = F[0] > 3;
-            if (iface || mi_emits(A, M, a, F, f, em, other)) {
-                fq_a[q] = (uint32_t)a;
-                fq_l[q] = (uint16_t)f;
-                fq_m[2 * q] = iface ? A.fit[M.s0 + F[0] - 4] : other;
-                fq_m[2 * q + 1] = A.fit[M.s0 + F[1] - 4];
-                fq_vs[q] = e;
-                for (int i = 0; i < n; ++i) {
-                    const int j = F[4 + i];
-                    if (!iface && is_corner(M.R, j)) {
-                        // phase 1: the corner is created here if it is new
-                        okey[o] = key_corner(M.vc(corner_of(M.R, j)));
-                        oa[o] = (uint32_t)a;
-                        oj[o] = (uint16_t)j;
-                        fve[e++] = o++;
-                    } else {
-                        fve[e++] = vb + mask_rank(m, j);
-                    }
-                }
-                ++q;
-            }
-            F += 4 + n;
-        }
+        if (M.R.nv <= 64)
+            mi_extract_tet<1>(A, M, a, emask[a], voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_m, fq_vs, fve);
+        else
+            mi_extract_tet<kMaskWords>(A, M, a, emask[a], voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_m,
+                                       fq_vs, fve);
     }
 }
-
 // vertex records and coordinates (src/extract_mesh.cpp:640-815, 1541-1637)
-__global__ void k_vert_fields_mi(GridView g, const double* __restrict__ vals, const uint32_t* __restrict__ act,
+__global__ void k_vert_fields_mi(GridView g, ValsRef vref, const uint32_t* __restrict__ act,
                                  const uint32_t* __restrict__ csr_off, const uint8_t* __restrict__ fit,
                                  const uint32_t* __restrict__ rec_loc, const uint16_t* __restrict__ rec,
                                  const uint32_t* __restrict__ first_occ, const uint32_t* __restrict__ oa,
                                  const uint16_t* __restrict__ oj, Count nverts, uint32_t* __restrict__ v_tet,
                                  uint16_t* __restrict__ v_j, uint8_t* __restrict__ v_ss, uint32_t* __restrict__ v_sv,
                                  uint8_t* __restrict__ v_fn, double* __restrict__ xyz) {
+    const double* __restrict__ vals = vref.get();
     const uint64_t V = g.V;
     GRID_STRIDE(i, nverts) {
         const uint32_t o = first_occ[i];
@@ -691,11 +642,12 @@ __global__ void k_vert_fields_mi(GridView g, const double* __restrict__ vals, co
     }
 }
 
-// faces are never merged: face q is occurrence q
+// faces are never merged: face q is occurrence q (mo: the ids are kept at
+// first occurrences, and this gives each occurrence's)
 __global__ void k_mi_face_out(Count nf, const uint32_t* __restrict__ act, const uint32_t* __restrict__ fq_a,
                               const uint16_t* __restrict__ fq_l, const uint8_t* __restrict__ fq_m,
                               const uint32_t* __restrict__ fq_vs, const uint32_t* __restrict__ fve,
-                              const uint32_t* __restrict__ vid_of_occ, Count nfv_c, uint32_t* __restrict__ f_vstart,
+                              const uint32_t* __restrict__ vid_of_occ, const uint32_t* __restrict__ mo, Count nfv_c, uint32_t* __restrict__ f_vstart,
                               uint32_t* __restrict__ f_verts, uint32_t* __restrict__ f_tfstart,
                               uint32_t* __restrict__ f_tf_tet, uint16_t* __restrict__ f_tf_local,
                               uint8_t* __restrict__ f_func) {
@@ -703,7 +655,7 @@ __global__ void k_mi_face_out(Count nf, const uint32_t* __restrict__ act, const 
     GRID_STRIDE(q, nf) {
         const uint32_t b = fq_vs[q], e = (q + 1 < n) ? fq_vs[q + 1] : (uint32_t)nfv;
         f_vstart[q] = b;
-        for (uint32_t i = b; i < e; ++i) f_verts[i] = vid_of_occ[fve[i]];
+        for (uint32_t i = b; i < e; ++i) f_verts[i] = vid_of_occ[mo ? mo[fve[i]] : fve[i]];
         f_tfstart[q] = (uint32_t)q;
         f_tf_tet[q] = act[fq_a[q]];
         f_tf_local[q] = fq_l[q];

@@ -156,7 +156,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& v, uint32_t flags
 // device, uploaded once per process and device; plain pointers (the kernels'
 // view of them is MITablesDev in kernels_mi.h)
 struct MITablesRaw {
-    const void *e2, *w2, *pat3, *off3, *cnt3, *cut3, *w3, *snap_off3, *snap3;
+    const void *e2, *w2, *pat3, *off3, *cnt3, *cut3, *lab3, *w3, *snap_off3, *snap3;
     uint64_t n_w2, n_w3;  // record words of the two- and three-material tables
 };
 MITablesRaw mi_tables_device(hipStream_t s);
@@ -168,6 +168,9 @@ constexpr uint64_t kNoallocValues = 2u << 20;
 void* noalloc_scratch_address();
 void eval_points_noalloc(void* scratch_dev, const double* pts, uint64_t n, const FuncDesc* funcs, uint32_t F,
                          double* rowmajor, hipStream_t s);
+
+// the star tables of regular grids (StarWalk in kernels_ia.h) on the device (batched.hip)
+void upload_star_tables(DevMem& m, DBuf<uint32_t>& head, DBuf<uint8_t>& ent, hipStream_t s);
 
 // batched form of the material interface (batched_mi.hip): the plain form's
 // stages with device-side counts and capacities, captured as one graph per

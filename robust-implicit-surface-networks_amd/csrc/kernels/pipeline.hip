@@ -97,6 +97,7 @@ const MI2Table& mi2_table() {
             E.cut[0] = (uint32_t)X.nv;
             E.cut[1] = (uint32_t)X.nf;
             E.cut[2] = (uint32_t)X.nc;
+            E.labels = mi_face_labels<CMed>(X);
         }
     });
     return T;
@@ -108,7 +109,7 @@ const MI2Table& mi2_table() {
 struct MI3Table {
     MI3Pat pat[81];
     uint32_t nslots = 0;
-    std::vector<uint32_t> off, cnt, cut;
+    std::vector<uint32_t> off, cnt, cut, lab;
     std::vector<uint16_t> words;
     // the complex after the three materials, per slot (byte offset, or
     // MI3_NONE; equal complexes stored once): the state the lane-group cut of
@@ -150,6 +151,7 @@ const MI3Table& mi3_table() {
         T.off.assign(base, MI3_NONE);
         T.cnt.assign(base, 0);
         T.cut.assign(base, 0);
+        T.lab.assign(base, 0);
         T.snap_off.assign(base, MI3_NONE);
         std::map<std::vector<uint16_t>, uint32_t> seen;
         std::map<std::vector<uint8_t>, uint32_t> seen_snap;
@@ -183,6 +185,7 @@ const MI3Table& mi3_table() {
                 T.off[K.base + sv] = off;
                 T.cnt[K.base + sv] = a0 | a1 << 8 | a2 << 16;
                 T.cut[K.base + sv] = (uint32_t)X2.nv | (uint32_t)X2.nf << 8 | (uint32_t)X2.nc << 16;
+                T.lab[K.base + sv] = mi_face_labels<CMed>(X2);
                 static_assert(CMed::MP == 8 && CMed::MFV == 8, "3-material snapshot layout");
                 std::vector<uint8_t> sn = {(uint8_t)X2.nv, (uint8_t)X2.nf, (uint8_t)X2.nc, (uint8_t)X2.dup};
                 for (int p = 0; p < 8; ++p) sn.push_back(X2.grp[p]);
@@ -237,6 +240,7 @@ MITablesRaw mi_tables_device(hipStream_t s) {
     D.off3 = up(T3.off.data(), 4 * T3.off.size());
     D.cnt3 = up(T3.cnt.data(), 4 * T3.cnt.size());
     D.cut3 = up(T3.cut.data(), 4 * T3.cut.size());
+    D.lab3 = up(T3.lab.data(), 4 * T3.lab.size());
     D.w3 = up(T3.words.data(), 2 * T3.words.size());
     D.snap_off3 = up(T3.snap_off.data(), 4 * T3.snap_off.size());
     D.snap3 = up(T3.snap.data(), T3.snap.size());
@@ -302,7 +306,8 @@ namespace {
 
 // material-interface extraction and coordinates (src/extract_mesh.cpp:569-986,
 // 1541-1637); faces are never merged, so they need no sort
-void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, Timer& tm, hipStream_t s) {
+void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, DBuf<uint32_t>& cnt,
+                const DBuf<uint32_t>& labels, Timer& tm, hipStream_t s) {
     const uint64_t NA = out.n_active;
     ensure_nbr(mem, g, s);
     MIArgs A;
@@ -315,27 +320,10 @@ void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, Time
     A.fit = out.fit.p;
     A.rec = out.rec.p;
     A.n_active = Count(NA);
-    DBuf<uint32_t> cnt(mem, 3 * NA + 3), cv(mem, NA + 1), cf(mem, NA + 1), cfv(mem, NA + 1);
+    DBuf<uint32_t> cv(mem, NA + 1), cf(mem, NA + 1), cfv(mem, NA + 1);
     DBuf<uint64_t> emask(mem, NA + 1);
-    if (NA) {
-        // every face's keys once, then the boundary-face pairing from them
-        DBuf<uint32_t> fb(mem, NA + 1);
-        hipLaunchKernelGGL(k_mi_nf, dim3(nblk(NA)), dim3(256), 0, s, A, fb.p);
-        scan_u32(mem, fb.p, fb.p, NA, fb.p + NA, s);
-        const uint64_t NFT = read1(fb.p + NA, s);
-        DBuf<uint16_t> fl(mem, NFT + 1), fw(mem, NFT + 1);
-        DBuf<uint64_t> ft(mem, 3 * NFT + 3);
-        MIFaceKeys K;
-        K.fb = fb.p;
-        K.fl = fl.p;
-        K.fw = fw.p;
-        K.ft = ft.p;
-        hipLaunchKernelGGL(k_mi_face_keys, dim3(nblk(NA * kBfaceLanes)), dim3(256), 0, s, A, K);
-        hipLaunchKernelGGL(k_mi_bface, dim3(nblk(NA * kBfaceLanes)), dim3(256), 0, s, A, K, emask.p);
-        RIN_HIP(hipGetLastError());
-        RIN_HIP(hipStreamSynchronize(s));  // the face-key buffers return to the pool
-        hipLaunchKernelGGL(k_mi_count, dim3(nblk(NA)), dim3(256), 0, s, A, (const uint64_t*)emask.p, cnt.p);
-    }
+    if (NA)
+        hipLaunchKernelGGL(k_mi_pair, dim3(nblk(NA)), dim3(256), 0, s, A, (const uint32_t*)labels.p, emask.p, cnt.p);
     hipLaunchKernelGGL(k_split3, dim3(nblk(NA)), dim3(256), 0, s, Count(NA), (const uint32_t*)cnt.p, cv.p, cf.p,
                        cfv.p);
     scan_u32(mem, cv.p, cv.p, NA, cv.p + NA, s);
@@ -369,9 +357,9 @@ void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, Time
     out.v_sv.alloc(mem, 4 * NV + 4);
     out.v_fn.alloc(mem, 4 * NV + 4);
     out.xyz.alloc(mem, 3 * NV + 3);
-    hipLaunchKernelGGL(k_vert_fields_mi, dim3(nblk(NV)), dim3(256), 0, s, g.view, (const double*)val.vals.p,
-                       (const uint32_t*)out.act.p, (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p,
-                       (const uint32_t*)out.rec_loc.p, (const uint16_t*)out.rec.p, (const uint32_t*)d.first_occ.p,
+    hipLaunchKernelGGL(k_vert_fields_mi, dim3(nblk(NV)), dim3(256), 0, s, g.view,
+                       ValsRef{(const double*)val.vals.p, nullptr}, (const uint32_t*)out.act.p,
+                       (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p, (const uint32_t*)out.rec_loc.p, (const uint16_t*)out.rec.p, (const uint32_t*)d.first_occ.p,
                        (const uint32_t*)oa.p, (const uint16_t*)oj.p, Count(NV), out.v_tet.p, out.v_j.p, out.v_ss.p,
                        out.v_sv.p, out.v_fn.p, out.xyz.p);
     RIN_HIP(hipGetLastError());
@@ -387,7 +375,7 @@ void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, Time
     out.f_func.alloc(mem, 2 * NF + 2);
     hipLaunchKernelGGL(k_mi_face_out, dim3(nblk(NF)), dim3(256), 0, s, Count(NF), (const uint32_t*)out.act.p,
                        (const uint32_t*)fq_a.p, (const uint16_t*)fq_l.p, (const uint8_t*)fq_m.p,
-                       (const uint32_t*)fq_vs.p, (const uint32_t*)fve.p, (const uint32_t*)d.vid.p, Count(NFV),
+                       (const uint32_t*)fq_vs.p, (const uint32_t*)fve.p, (const uint32_t*)d.vid.p, (const uint32_t*)nullptr, Count(NFV),
                        out.f_vstart.p, out.f_verts.p, out.f_tfstart.p, out.f_tf_tet.p, out.f_tf_local.p,
                        out.f_func.p);
     fill_u32(out.f_vstart.p + NF, (uint32_t)NFV, 1, s);
@@ -578,7 +566,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     } else {
         DBuf<uint64_t> hm(mem, V);
         hipLaunchKernelGGL(k_highest_mi, dim3(nblk(V)), dim3(256), 0, s, (const double*)val.vals.p, V, F, hm.p,
-                           vflag.p, (uint32_t*)nullptr);
+                           vflag.p, (uint32_t*)nullptr, (const double**)nullptr);
         tm.mark("highest func");
         hipLaunchKernelGGL(k_filter_mi, dim3(nblk(T)), dim3(256), 0, s, g.view, (const double*)val.vals.p, F,
                            (const uint64_t*)hm.p, amask.p, kcnt.p, isact.p);
@@ -655,7 +643,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     }
     const uint64_t nwords = read1(out.rec_off.p + NA, s);
     out.rec.alloc(mem, nwords + 1);
-    DBuf<uint32_t> cnt(mem, 3 * NA + 3);
+    DBuf<uint32_t> cnt(mem, 3 * NA + 3), labels(mem, MI ? NA + 1 : 1);
     if (bcnt[0] && !MI) {
         table_cut_plain(g.view, (const double*)val.vals.p, (const uint32_t*)out.act.p, (const uint8_t*)out.act_k.p,
                         (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p, (const uint32_t*)blist[0],
@@ -663,10 +651,12 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     } else if (bcnt[0]) {
         // two- and three-material tets by table
         const MITablesDev TT = mi_tables_dev(s);
-        hipLaunchKernelGGL(k_mi_table, dim3(nblk(bcnt[0])), dim3(256), 0, s, g.view, (const double*)val.vals.p,
+        hipLaunchKernelGGL(k_mi_table, dim3(nblk(bcnt[0])), dim3(256), 0, s, g.view,
+                           ValsRef{(const double*)val.vals.p, nullptr},
                            (const uint32_t*)out.act.p, (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p,
                            (const uint32_t*)blist[0], (uint64_t)bcnt[0], (const uint32_t*)nullptr, flags,
-                           (const uint32_t*)out.rec_off.p, out.rec.p, cnt.p, errs.p, TT, (uint32_t*)nullptr, 0u, 0u);
+                           (const uint32_t*)out.rec_off.p, out.rec.p, cnt.p, errs.p, TT, labels.p,
+                           (uint32_t*)nullptr, 0u, 0u);
         RIN_HIP(hipGetLastError());
     }
     // the cuts beyond the tables: lane groups with the complex in LDS (the
@@ -696,11 +686,11 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         if (!nl) continue;
         auto go = [&](auto kernel, int per_wave, auto snap) {
             const unsigned blocks = (unsigned)std::min<uint64_t>((nl + per_wave - 1) / per_wave, 4096);
-            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, s, g.view, (const double*)val.vals.p,
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, s, g.view, ValsRef{(const double*)val.vals.p, nullptr},
                                (const uint32_t*)out.act.p, (const uint8_t*)out.act_k.p,
                                (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p,
                                (const uint32_t*)blist[1 + q], Count(nl), (const uint32_t*)out.rec_off.p, out.rec.p,
-                               cnt.p, errs.p, 1, flags, snap);
+                               cnt.p, errs.p, 1, flags, labels.p, snap);
         };
         if (q == 0)
             MI ? go(k_cut_group<CMed, 64, true>, 1, m3s) : go(k_cut_group<CMed, 16, false>, 4, k2s);
@@ -720,7 +710,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
             hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, s, g.view, (const double*)val.vals.p,
                                (const uint32_t*)out.act.p, (const uint8_t*)out.act_k.p, (const uint32_t*)out.csr_off.p,
                                (const uint8_t*)out.fit.p, list, Count(nl), flags, (const uint32_t*)out.rec_off.p, out.rec.p,
-                               cnt.p, errs.p, wsp, loc, fixed_cap);
+                               cnt.p, errs.p, wsp, loc, fixed_cap, labels.p);
         };
         MI ? go(k_cut_huge<true>) : go(k_cut_huge<false>);
         RIN_HIP(hipGetLastError());
@@ -779,7 +769,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         return;
     }
     if (MI) {
-        extract_mi(mem, g, val, out, tm, s);
+        extract_mi(mem, g, val, out, cnt, labels, tm, s);
         tm.finish(out.times);
         if (!(flags & RUN_KEEP_RECORDS)) out.rec.reset();
         out.set_views_from_buffers();

@@ -29,3 +29,33 @@ def test_zero_values_batched(ctx, res, F, zeros):
     dev.release()
     v.release()
     g.release()
+
+
+# One of these inputs differs from the oracle by one boundary face (276 for
+# 275), in the plain and the batched form, and did so with every face compared
+# by its vertex keys as well; why is not established.
+KNOWN = pytest.mark.xfail(reason="one boundary face more than the oracle", strict=True)
+
+
+@pytest.mark.parametrize("res,F,levels", [(1, 2, 2), (1, 5, 3), (2, 3, 2), pytest.param(3, 4, 4, marks=KNOWN), (5, 6, 5),
+                                          (8, 3, 3), (6, 12, 40)])
+@pytest.mark.parametrize("regular", [True, False])
+def test_tied_materials(ctx, res, F, levels, regular):
+    """Few distinct values: materials tie at vertices, along edges, on whole
+    tet faces and tets, so boundary faces pair with other materials, corners
+    are created lazily and more than once in a tet, and keys miss the star's
+    lowest tets."""
+    import rin
+
+    rng = np.random.default_rng(7000 + 100 * res + F)
+    pts, tets = S.grid(res)
+    vals = rng.integers(0, levels, (len(pts), F)).astype(np.float64)
+    ref = S.OracleRun(1, pts, tets, vals)
+    g = ctx.grid_regular(res) if regular else ctx.grid_explicit(pts, tets)
+    v = g.upload(vals)
+    for flags in (rin.FLAG_BATCHED, rin.FLAG_BATCHED, 0):
+        dev = v.run(rin.FLAG_MI | flags)
+        _compare(dev, ref)
+        dev.release()
+    v.release()
+    g.release()
