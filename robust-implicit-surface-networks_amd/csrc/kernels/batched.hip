@@ -364,13 +364,68 @@ const K2Plans& k2_plans() {
 
 // kbig: the most functions the last bucket takes (8, or kMaxHuge once a value
 // set has shown tets of more)
+// Sign masks of a vertex (bit j: function j), positive and negative side by
+// side, in the narrowest words that hold F bits: the count and fill passes
+// read eight vertices a cube, so they move a quarter of the bytes at 8
+// functions and half at 20, in one load a vertex.  At 201^3 vertices and 8
+// functions two arrays of 64-bit masks took 118 us in the signs pass, 155 in
+// the count pass and 209 in the fill pass (with a dense rank a tet); now 93,
+// 106 and 178.  At 101^3 and 20: 37, 28 and 41; now 31, 20 and 32.
+template <class T>
+struct alignas(2 * sizeof(T)) MaskPair {
+    T pos, neg;
+};
+inline int mask_width(uint32_t F) { return F <= 8 ? 1 : (F <= 16 ? 2 : (F <= 32 ? 4 : 8)); }
+// calls fn with a value of the mask word type for F functions
+template <class Fn>
+void with_mask_type(uint32_t F, Fn&& fn) {
+    switch (mask_width(F)) {
+        case 1: fn(uint8_t(0)); break;
+        case 2: fn(uint16_t(0)); break;
+        case 4: fn(uint32_t(0)); break;
+        default: fn(uint64_t(0));
+    }
+}
+// the masks where a kernel reads few of them (the width is uniform)
+struct MaskRef {
+    const void* p;
+    int width;
+    template <class T>
+    __device__ void load(uint32_t v, uint64_t& pos, uint64_t& neg) const {
+        const MaskPair<T> m = static_cast<const MaskPair<T>*>(p)[v];
+        pos = m.pos;
+        neg = m.neg;
+    }
+    __device__ void get(uint32_t v, uint64_t& pos, uint64_t& neg) const {
+        if (width == 1)
+            load<uint8_t>(v, pos, neg);
+        else if (width == 2)
+            load<uint16_t>(v, pos, neg);
+        else if (width == 4)
+            load<uint32_t>(v, pos, neg);
+        else
+            load<uint64_t>(v, pos, neg);
+    }
+    // the functions active in a tet of corners v
+    __device__ uint64_t active(const uint32_t* v, uint64_t full) const {
+        uint64_t ap = ~0ull, an = ~0ull;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            uint64_t p, q;
+            get(v[c], p, q);
+            ap &= p;
+            an &= q;
+        }
+        return full & ~(ap | an);
+    }
+};
+
 __device__ inline int bucket_of(int k, int kbig) {
     return k <= 1 ? 0 : (k == 2 ? 1 : (k <= 4 ? 2 : (k <= kbig ? 3 : 4)));
 }
 
 // per tet: active count and bucket histogram
-__global__ void k_filter_count(GridView g, const uint64_t* __restrict__ pos, const uint64_t* __restrict__ neg,
-                               uint64_t full, int kbig, uint32_t* __restrict__ kcnt, uint32_t* __restrict__ isact,
+__global__ void k_filter_count(GridView g, MaskRef masks, uint64_t full, int kbig, uint32_t* __restrict__ kcnt, uint32_t* __restrict__ isact,
                                uint32_t* __restrict__ ctr) {
     __shared__ uint32_t hist[8];
     if (threadIdx.x < 8) hist[threadIdx.x] = 0;
@@ -378,9 +433,7 @@ __global__ void k_filter_count(GridView g, const uint64_t* __restrict__ pos, con
     GRID_STRIDE(t, g.T) {
         uint32_t v[4];
         dev::tet_corners(g, t, v);
-        const uint64_t ap = pos[v[0]] & pos[v[1]] & pos[v[2]] & pos[v[3]];
-        const uint64_t an = neg[v[0]] & neg[v[1]] & neg[v[2]] & neg[v[3]];
-        const uint64_t m = full & ~(ap | an);
+        const uint64_t m = masks.active(v, full);
         const uint32_t k = (uint32_t)__popcll(m);
         kcnt[t] = k;
         isact[t] = k != 0;
@@ -393,10 +446,11 @@ __global__ void k_filter_count(GridView g, const uint64_t* __restrict__ pos, con
 
 struct FillArgs {
     GridView g;
-    const uint64_t *pos, *neg;
+    MaskRef masks;
     uint64_t full;
-    const uint32_t *csr_off, *rank;
-    uint32_t *csr_off_w, *rank_w;  // written by the cube form
+    const uint32_t *csr_off, *rank;  // explicit meshes
+    uint32_t* csr_off_w;             // written by the cube form
+    uint2* blocks;                   // written by the cube form (RankOf)
     uint8_t* fit;
     uint32_t *act, *rec_loc, *cnt;
     uint32_t* act_off;  // CSR offset by active rank
@@ -427,9 +481,7 @@ __global__ void k_fill_batched(FillArgs A) {
         uint32_t v[4] = {0, 0, 0, 0};
         if (t < T) {
             dev::tet_corners(A.g, t, v);
-            const uint64_t ap = A.pos[v[0]] & A.pos[v[1]] & A.pos[v[2]] & A.pos[v[3]];
-            const uint64_t an = A.neg[v[0]] & A.neg[v[1]] & A.neg[v[2]] & A.neg[v[3]];
-            m = A.full & ~(ap | an);
+            m = A.masks.active(v, A.full);
         }
         const int k = __popcll(m);
         int b = -1;
@@ -450,7 +502,9 @@ __global__ void k_fill_batched(FillArgs A) {
                     const uint32_t f = __ffsll((unsigned long long)m) - 1;
                     int pat = 0, w = 1;
                     for (int c = 0; c < 4; ++c, w *= 3) {
-                        const int s = ((A.pos[v[c]] >> f) & 1) ? 2 : (((A.neg[v[c]] >> f) & 1) ? 0 : 1);
+                        uint64_t mp, mn;
+                        A.masks.get(v[c], mp, mn);
+                        const int s = ((mp >> f) & 1) ? 2 : (((mn >> f) & 1) ? 0 : 1);
                         pat += s * w;
                     }
                     const K1Entry& E = tab[pat];
@@ -491,8 +545,10 @@ __global__ void k_fill_batched(FillArgs A) {
 // (1024 lanes a workgroup: on the 101^3-vertex, 20-function grid with cold
 // caches 37.6 us against 40.6 us at 256; streaming loads, as ordinary loads
 // took 72 us when the caches held other kernels' dirty lines)
-__global__ void __launch_bounds__(1024) k_signs_count(const double* __restrict__ vals, uint64_t V, uint32_t F, uint64_t* __restrict__ pos,
-                              uint64_t* __restrict__ neg, uint32_t* __restrict__ ctr, const double** __restrict__ slot) {
+template <class T>
+__global__ void __launch_bounds__(1024) k_signs_count(const double* __restrict__ vals, uint64_t V, uint32_t F,
+                                                      MaskPair<T>* __restrict__ masks, uint32_t* __restrict__ ctr,
+                                                      const double** __restrict__ slot) {
     // the later kernels, captured once per workspace, find the values here
     if (blockIdx.x == 0 && threadIdx.x == 0) *slot = vals;
     uint32_t z = 0;
@@ -512,8 +568,7 @@ __global__ void __launch_bounds__(1024) k_signs_count(const double* __restrict__
                 z += x[u] == 0;
             }
         }
-        pos[v] = p;
-        neg[v] = n;
+        masks[v] = MaskPair<T>{(T)p, (T)n};
     }
     for (int d = 32; d > 0; d >>= 1) z += __shfl_xor(z, d, 64);
     if ((threadIdx.x & 63) == 0 && z) atomicAdd(&ctr[C_DEGEN], z);
@@ -534,9 +589,9 @@ constexpr int kCubeTile = 512;  // the default
 
 // pat (optional): per tet with one active function, its corner sign pattern
 // (sum of s_c 3^c, s_c = 0 negative, 1 zero, 2 positive), else 0
-__device__ inline void cube_masks(const GridView& g, uint32_t cube, const uint64_t* __restrict__ pos,
-                                  const uint64_t* __restrict__ neg, uint64_t full, uint32_t c[8], uint64_t m[5],
-                                  bool& even, uint8_t* pat = nullptr) {
+template <class T, class M>
+__device__ inline void cube_masks(const GridView& g, uint32_t cube, const MaskPair<T>* __restrict__ masks, M full,
+                                  uint32_t c[8], M m[5], bool& even, uint8_t* pat = nullptr) {
     const uint32_t R = (uint32_t)g.res, N = R + 1;
     const uint32_t i = cube / (R * R), rem = cube - i * (R * R), j = rem / R, k = rem - j * R;
     const uint32_t b = i * N * N + j * N + k;
@@ -546,15 +601,16 @@ __device__ inline void cube_masks(const GridView& g, uint32_t cube, const uint64
     c[3] = b + N;
     for (int a = 0; a < 4; ++a) c[4 + a] = c[a] + 1;
     even = ((i + j + k) & 1u) == 0;
-    uint64_t P[8], Q[8];
+    M P[8], Q[8];
     for (int a = 0; a < 8; ++a) {
-        P[a] = pos[c[a]];
-        Q[a] = neg[c[a]];
+        const MaskPair<T> x = masks[c[a]];
+        P[a] = x.pos;
+        Q[a] = x.neg;
     }
     for (int q = 0; q < 5; ++q) {
         const uint8_t* t = even ? dev::kCubeTetEven[q] : dev::kCubeTetOdd[q];
-        const uint64_t ap = P[t[0]] & P[t[1]] & P[t[2]] & P[t[3]];
-        const uint64_t an = Q[t[0]] & Q[t[1]] & Q[t[2]] & Q[t[3]];
+        const M ap = P[t[0]] & P[t[1]] & P[t[2]] & P[t[3]];
+        const M an = Q[t[0]] & Q[t[1]] & Q[t[2]] & Q[t[3]];
         m[q] = full & ~(ap | an);
         if (pat) {
             pat[q] = 0;
@@ -596,22 +652,22 @@ struct EarlyEntry {
 // wavefront of the cut mostly holds tets of one k (two insertions past the
 // two-plane start, or one) and the longer ones start first.  A tile's entries
 // are contiguous and in tet order (the back part reversed).
-template <int TILE>
-__global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const uint64_t* __restrict__ pos,
-                                                          const uint64_t* __restrict__ neg, uint64_t full, int kbig,
-                                                          TileSums* __restrict__ tile_sums, EarlyEntry* early3,
-                                                          EarlyEntry* early5, uint32_t early_cap3,
-                                                          uint32_t early_cap5, uint32_t* ctr) {
+template <int TILE, class T>
+__global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<T>* __restrict__ masks, uint64_t full,
+                                                     int kbig, TileSums* __restrict__ tile_sums, EarlyEntry* early3,
+                                                     EarlyEntry* early5, uint32_t early_cap3, uint32_t early_cap5,
+                                                     uint32_t* ctr) {
+    using M = typename std::conditional<sizeof(T) == 8, uint64_t, uint32_t>::type;
     const uint32_t ncubes = (uint32_t)(g.T / 5);
     const uint32_t tile = blockIdx.x;
     const uint32_t cube = tile * TILE + threadIdx.x;
     uint32_t v[kTileFields] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint64_t m[5] = {0, 0, 0, 0, 0};
+    M m[5] = {0, 0, 0, 0, 0};
     uint32_t n4 = 0;  // k = 4 tets (of the k = 3..4 bucket)
     if (cube < ncubes) {
         uint32_t c[8];
         bool even;
-        cube_masks(g, cube, pos, neg, full, c, m, even);
+        cube_masks<T, M>(g, cube, masks, (M)full, c, m, even);
         for (int q = 0; q < 5; ++q) {
             const int k = __popcll(m[q]);
             v[TF_FIT] += (uint32_t)k;
@@ -767,12 +823,16 @@ __global__ void __launch_bounds__(kTileScanThreads) k_tile_scan(TileSums* __rest
 }
 
 // tile_sums: exclusive prefixes (k_tile_scan)
-template <int TILE>
+template <int TILE, class T>
 __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* __restrict__ tile_sums) {
+    using M = typename std::conditional<sizeof(T) == 8, uint64_t, uint32_t>::type;
     __shared__ K1Entry tab[81];
     __shared__ uint32_t wsum[TILE / 64];
     __shared__ uint32_t wbk[TILE / 64];  // per-wave bucket counts, 10 bits per list
-    __shared__ uint32_t s_off[5 * TILE], s_rank[5 * TILE];  // per-tet CSR entries of the tile
+    __shared__ uint32_t s_off[5 * TILE];                         // per-tet CSR offsets of the tile
+    __shared__ uint32_t s_bits[5 * TILE / 32], s_pre[5 * TILE / 32];  // its rank blocks
+    static_assert(5 * TILE % 32 == 0, "a tile holds whole rank blocks");
+    if (threadIdx.x < 5 * TILE / 32) s_bits[threadIdx.x] = 0;
     for (int i = threadIdx.x; i < 81; i += blockDim.x) tab[i] = A.k1[i];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t tile = blockIdx.x;
@@ -780,10 +840,11 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     const uint32_t ncubes = (uint32_t)(A.g.T / 5);
     const uint32_t cube = tile * TILE + threadIdx.x;
     uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint64_t m[5] = {0, 0, 0, 0, 0};
+    M m[5] = {0, 0, 0, 0, 0};
     bool even = true;
     uint8_t pat[5] = {0, 0, 0, 0, 0};
-    if (cube < ncubes) cube_masks(A.g, cube, A.pos, A.neg, A.full, c, m, even, pat);
+    if (cube < ncubes)
+        cube_masks<T, M>(A.g, cube, static_cast<const MaskPair<T>*>(A.masks.p), (M)A.full, c, m, even, pat);
     // per lane: active functions, active tets, and tets per bucket list
     // (k = 2, 3..4, 5..8), packed ks << 11 | as and 10 bits per bucket
     uint32_t ks = 0, as = 0, bp = 0;
@@ -824,11 +885,13 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     }
     for (int q = 0; q < 5; ++q) {
         const uint64_t t = (uint64_t)cube * 5 + q;
-        const uint64_t mq = m[q];
+        const M mq = m[q];
         const int k = __popcll(mq);
-        s_off[5 * threadIdx.x + q] = o;
-        s_rank[5 * threadIdx.x + q] = r;
+        const uint32_t local = 5 * threadIdx.x + q;
+        s_off[local] = o;
+        if ((local & 31u) == 0) s_pre[local >> 5] = r;
         if (k) {
+            atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
             if (r >= A.cap_active || o + (uint32_t)k > A.cap_fit) {
                 A.errs[lane] |= ERR_OVERFLOW;
                 A.ctr[C_ABORT] = 1;
@@ -837,7 +900,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
                 A.act_k[r] = (uint8_t)k;
                 A.act_off[r] = o;
                 uint32_t oo = o;
-                for (uint64_t mm = mq; mm; mm &= mm - 1) A.fit[oo++] = (uint8_t)(__ffsll((unsigned long long)mm) - 1);
+                for (M mm = mq; mm; mm &= mm - 1) A.fit[oo++] = (uint8_t)(__ffsll((unsigned long long)mm) - 1);
                 if (k == 1) {
                     const K1Entry& E = tab[pat[q]];
                     A.cnt[3 * r] = E.niv;
@@ -865,12 +928,11 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     }
     // the tile's per-tet CSR entries, coalesced
     __syncthreads();
-    const uint64_t t0 = (uint64_t)tile * (5 * TILE), T = A.g.T;
+    const uint64_t t0 = (uint64_t)tile * (5 * TILE), NT = A.g.T;
     for (int i = threadIdx.x; i < 5 * TILE; i += TILE)
-        if (t0 + i < T) {
-            A.csr_off_w[t0 + i] = s_off[i];
-            A.rank_w[t0 + i] = s_rank[i];
-        }
+        if (t0 + i < NT) A.csr_off_w[t0 + i] = s_off[i];
+    if (threadIdx.x < 5 * TILE / 32 && t0 + 32 * threadIdx.x < NT)
+        A.blocks[t0 / 32 + threadIdx.x] = make_uint2(s_bits[threadIdx.x], s_pre[threadIdx.x]);
 }
 
 struct CutArgs {
@@ -895,7 +957,7 @@ struct CutArgs {
     const EarlyEntry* early;
     const uint32_t *n_early, *n_back;  // the list's front and back parts (n_back nullable)
     const TileSums* tiles;
-    const uint64_t *pos, *neg;
+    MaskRef masks;
     uint64_t full;
     uint32_t rec_base, cap_active;
     int tf;
@@ -989,8 +1051,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
         rec_at = A.rec_base + slot * A.slot;
         uint32_t v[4];
         dev::tet_corners(A.g, e.t, v);
-        const uint64_t m = A.full & ~((A.pos[v[0]] & A.pos[v[1]] & A.pos[v[2]] & A.pos[v[3]]) |
-                                      (A.neg[v[0]] & A.neg[v[1]] & A.neg[v[2]] & A.neg[v[3]]));
+        const uint64_t m = A.masks.active(v, A.full);
         k = __popcll(m);
         if (k < A.kmin || k > A.kmax) return;
         for (int e4 = lane; e4 < 4 * (C::MP - 4); e4 += G) {
@@ -1056,7 +1117,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
 struct K2Args {
     GridView g;
     const double* const* vals;  // where the signs pass left the run's values
-    const uint64_t *pos, *neg;
+    MaskRef masks;
     uint64_t full;  // the functions' bits
     const uint32_t *act, *csr_off, *list;
     const uint64_t* lts;  // per slot: CSR offset << 32 | tet
@@ -1074,13 +1135,13 @@ struct K2Args {
 // fa < fb: the first plane's sign pattern picks the pattern, the second
 // plane's signs at the corners and at the first plane's edge points the
 // slot; K2_NONE when a sign pattern or point falls outside the table
-__device__ __forceinline__ uint32_t k2_table_slot(const K2Args& A, const K2Pat* pats, const uint32_t* v, uint32_t fa,
-                                                  uint32_t fb) {
+__device__ __forceinline__ uint32_t k2_table_slot(const K2Args& A, const K2Pat* pats, const uint32_t* v,
+                                                  const uint64_t* mp, const uint64_t* mn, uint32_t fa, uint32_t fb) {
     const uint64_t V = A.g.V;
     const double* __restrict__ vals = *A.vals;
     int pa = 0, sB[4];
     for (int c = 0, w = 1; c < 4; ++c, w *= 3) {
-        const uint64_t p = A.pos[v[c]], q = A.neg[v[c]];
+        const uint64_t p = mp[c], q = mn[c];
         pa += (((p >> fa) & 1) ? 2 : (((q >> fa) & 1) ? 0 : 1)) * w;
         sB[c] = ((p >> fb) & 1) ? 1 : (((q >> fb) & 1) ? -1 : 0);
     }
@@ -1133,11 +1194,13 @@ __global__ void k_k2_lookup(K2Args A) {
         dev::tet_corners(A.g, t, v);
         // the two active functions from the corner masks (the CSR's order,
         // one dependent load fewer than reading the CSR)
-        const uint64_t m = A.full & ~((A.pos[v[0]] & A.pos[v[1]] & A.pos[v[2]] & A.pos[v[3]]) |
-                                      (A.neg[v[0]] & A.neg[v[1]] & A.neg[v[2]] & A.neg[v[3]]));
+        uint64_t mp[4], mn[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) A.masks.get(v[c], mp[c], mn[c]);
+        const uint64_t m = A.full & ~((mp[0] & mp[1] & mp[2] & mp[3]) | (mn[0] & mn[1] & mn[2] & mn[3]));
         const uint32_t fa = (uint32_t)(__ffsll((unsigned long long)m) - 1);
         const uint32_t fb = (uint32_t)(__ffsll((unsigned long long)(m & (m - 1))) - 1);
-        const uint32_t slot = k2_table_slot(A, pats, v, fa, fb);
+        const uint32_t slot = k2_table_slot(A, pats, v, mp, mn, fa, fb);
         if (!k2_point(A, slot, r)) A.rec[A.rec_loc[r]] = 0;
     }
 }
@@ -1728,7 +1791,8 @@ struct Workspace {
     bool wide = false;
     bool wave_cut[3] = {false, false, false};  // bucket cut by the wave form (records carry face offsets)
     DBuf<const double*> vals_at;  // the run's values, left by its signs pass for the captured kernels
-    DBuf<uint64_t> pos, neg;
+    DBuf<uint8_t> masks;        // MaskPair by vertex
+    DBuf<uint2> blocks;         // regular grids: rank blocks (RankOf)
     DBuf<uint32_t> kcnt, isact, csr_off, rank, act, rec_loc, cnt, list[3];
     DBuf<uint64_t> lts[3];  // per bucket slot: CSR offset << 32 | tet
     DBuf<uint32_t> act_off;  // CSR offset of each active tet, by active rank
@@ -1783,8 +1847,8 @@ struct Workspace {
     hipGraphExec_t whole = nullptr;
     // side branches of the whole graph (the cut kernels beside each other and
     // beside the fill pass): streams to capture them on, fork and join events
-    hipStream_t side = nullptr, side2 = nullptr, side3 = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr, join3 = nullptr;
+    hipStream_t side = nullptr, side2 = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr;
     // pinned, device-mapped summary the closing kernel of a run writes (counters
     // and error flags), read by the host after the stream synchronises
     uint32_t* pub_h = nullptr;
@@ -1816,8 +1880,6 @@ struct Workspace {
         if (fork) (void)hipEventDestroy(fork);
         if (join) (void)hipEventDestroy(join);
         if (join2) (void)hipEventDestroy(join2);
-        if (join3) (void)hipEventDestroy(join3);
-        if (side3) (void)hipStreamDestroy(side3);
         if (side2) (void)hipStreamDestroy(side2);
         if (side) (void)hipStreamDestroy(side);
         if (pub_h) (void)hipHostFree(pub_h);
@@ -1929,23 +1991,23 @@ unsigned cube_tiles(const Grid& g, int tile = kCubeTile) {
     return (unsigned)std::max<uint64_t>(1, (cubes + tile - 1) / tile);
 }
 
-void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
+void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream_t s) {
     W.cap = c;
     W.slot[2] = W.wide ? rec_words<CWide>() : rec_words<CBig>();
     DevMem& m = W.mem;
     const uint64_t V = g.view.V, T = g.view.T;
     W.vals_at.alloc(m, 1);
-    W.pos.alloc(m, V);
-    W.neg.alloc(m, V);
+    W.masks.alloc(m, 2 * (size_t)mask_width(F) * V);
     if (g.view.regular) {
+        W.blocks.alloc(m, T / 32 + 1);
         W.tile_sums.alloc(m, cube_tiles(g, 256) + 1);  // the smallest tile has the most tiles
         for (int q = 1; q < 3; ++q) W.early[q].alloc(m, c.b[q] + 1);
     } else {
         W.kcnt.alloc(m, T + 1);
         W.isact.alloc(m, T + 1);
+        W.rank.alloc(m, T + 1);
     }
     W.csr_off.alloc(m, T + 1);
-    W.rank.alloc(m, T + 1);
     W.act.alloc(m, c.active + 1);
     W.act_k.alloc(m, c.active + 1);
     W.act_off.alloc(m, c.active + 1);
@@ -2048,8 +2110,11 @@ void alloc_ws(Workspace& W, const Grid& g, const Caps_& c, hipStream_t s) {
 // early3, early5: list the k = 3..4 / 5..8 tets for launch_cut_early (regular grids)
 void stage_signs(Workspace& W, const Grid& g, const Values& val, hipStream_t s, bool zero) {
     if (zero) hipLaunchKernelGGL(k_zero_ctr, dim3(1), dim3(64), 0, s, W.ctr.p, (int)C_N, W.errs.p);
-    hipLaunchKernelGGL(k_signs_count, dim3(nblk(g.view.V, 1024)), dim3(1024), 0, s, (const double*)val.vals.p, g.view.V,
-                       val.F, W.pos.p, W.neg.p, W.ctr.p, W.vals_at.p);
+    with_mask_type(val.F, [&](auto t) {
+        using T = decltype(t);
+        hipLaunchKernelGGL(k_signs_count<T>, dim3(nblk(g.view.V, 1024)), dim3(1024), 0, s, (const double*)val.vals.p,
+                           g.view.V, val.F, reinterpret_cast<MaskPair<T>*>(W.masks.p), W.ctr.p, W.vals_at.p);
+    });
 }
 
 void stage_filter(Workspace& W, const Grid& g, const Values& val, hipStream_t s, bool early3 = false,
@@ -2060,23 +2125,27 @@ void stage_filter(Workspace& W, const Grid& g, const Values& val, hipStream_t s,
     const int kbig = W.wide ? kMaxHuge : 8;
     if (g.view.regular) {
         const int tile = W.cube_tile;
-        auto count = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, g.view, (const uint64_t*)W.pos.p,
-                               (const uint64_t*)W.neg.p, full, kbig, W.tile_sums.p, early3 ? W.early[1].p : nullptr,
-                               early5 ? W.early[2].p : nullptr, W.cap.b[1], W.cap.b[2], W.ctr.p);
-        };
-        if (tile == 256)
-            count(k_cube_count<256>);
-        else if (tile == 1024)
-            count(k_cube_count<1024>);
-        else
-            count(k_cube_count<512>);
+        with_mask_type(F, [&](auto t) {
+            using M = decltype(t);
+            auto count = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, g.view,
+                                   reinterpret_cast<const MaskPair<M>*>(W.masks.p), full, kbig, W.tile_sums.p,
+                                   early3 ? W.early[1].p : nullptr, early5 ? W.early[2].p : nullptr, W.cap.b[1],
+                                   W.cap.b[2], W.ctr.p);
+            };
+            if (tile == 256)
+                count(k_cube_count<256, M>);
+            else if (tile == 1024)
+                count(k_cube_count<1024, M>);
+            else
+                count(k_cube_count<512, M>);
+        });
         hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(kTileScanThreads), 0, s, W.tile_sums.p, cube_tiles(g, tile),
                            W.ctr.p);
         return;
     }
-    hipLaunchKernelGGL(k_filter_count, dim3(nblk(T)), dim3(256), 0, s, g.view, (const uint64_t*)W.pos.p,
-                       (const uint64_t*)W.neg.p, full, kbig, W.kcnt.p, W.isact.p, W.ctr.p);
+    hipLaunchKernelGGL(k_filter_count, dim3(nblk(T)), dim3(256), 0, s, g.view, MaskRef{W.masks.p, mask_width(F)}, full,
+                       kbig, W.kcnt.p, W.isact.p, W.ctr.p);
     scan_u32(W.mem, W.kcnt.p, W.csr_off.p, Count(T), W.ctr.p + C_FIT, s);
     scan_u32(W.mem, W.isact.p, W.rank.p, Count(T), W.ctr.p + C_ACTIVE, s);
 }
@@ -2092,8 +2161,7 @@ K2Args k2_args(Workspace& W, const Grid& g, const Values& val) {
     K2Args K = {};
     K.g = g.view;
     K.vals = W.vals_at.p;
-    K.pos = W.pos.p;
-    K.neg = W.neg.p;
+    K.masks = MaskRef{W.masks.p, mask_width(val.F)};
     K.full = (val.F == 64) ? ~0ull : ((1ull << val.F) - 1);
     K.act = W.act.p;
     K.csr_off = W.csr_off.p;
@@ -2199,8 +2267,7 @@ void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int
     A.n_early = W.ctr.p + (q == 1 ? C_E3 : C_E5);
     A.n_back = q == 1 ? W.ctr.p + C_E3B : nullptr;
     A.tiles = W.tile_sums.p;
-    A.pos = W.pos.p;
-    A.neg = W.neg.p;
+    A.masks = MaskRef{W.masks.p, mask_width(val.F)};
     A.full = (val.F == 64) ? ~0ull : ((1ull << val.F) - 1);
     A.rec_base = W.rec_base[q];
     A.cap_active = W.cap.active;
@@ -2228,8 +2295,7 @@ void stage_fill(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
     const uint32_t F = val.F;
     FillArgs A;
     A.g = g.view;
-    A.pos = W.pos.p;
-    A.neg = W.neg.p;
+    A.masks = MaskRef{W.masks.p, mask_width(F)};
     A.full = (F == 64) ? ~0ull : ((1ull << F) - 1);
     A.csr_off = W.csr_off.p;
     A.rank = W.rank.p;
@@ -2253,16 +2319,22 @@ void stage_fill(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
     A.cap_active = W.cap.active;
     A.cap_fit = W.cap.fit;
     A.csr_off_w = W.csr_off.p;
-    A.rank_w = W.rank.p;
+    A.blocks = W.blocks.p;
     if (g.view.regular) {
         const int tile = W.cube_tile;
         const TileSums* ts = W.tile_sums.p;
-        if (tile == 256)
-            hipLaunchKernelGGL(k_cube_fill<256>, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, A, ts);
-        else if (tile == 1024)
-            hipLaunchKernelGGL(k_cube_fill<1024>, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, A, ts);
-        else
-            hipLaunchKernelGGL(k_cube_fill<512>, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, A, ts);
+        with_mask_type(F, [&](auto t) {
+            using M = decltype(t);
+            auto fill = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, A, ts);
+            };
+            if (tile == 256)
+                fill(k_cube_fill<256, M>);
+            else if (tile == 1024)
+                fill(k_cube_fill<1024, M>);
+            else
+                fill(k_cube_fill<512, M>);
+        });
         return;
     }
     hipLaunchKernelGGL(k_fill_batched, dim3(nblk(T)), dim3(256), 0, s, A);
@@ -2372,7 +2444,7 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
             S.okey = W.okey.p;
             S.oa = W.oa.p;
             S.act = W.act.p;
-            S.rank = W.rank.p;
+            S.rank = RankOf{nullptr, W.act.p, W.blocks.p};
             S.voff = W.cv.p;
             S.star_head = W.star_head.p;
             S.star_ent = W.star_ent.p;
@@ -2432,7 +2504,7 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
         FA.mo = W.mo.p;
         FA.vrank = W.vrank.p;
         FA.act = W.act.p;
-        FA.rank = W.rank.p;
+        FA.rank = RankOf{W.rank.p, W.act.p, W.blocks.p};
         FA.foff = W.cf.p;
         FA.nbr = g.nbr.p;
         FA.fq_bnd = W.fq_bnd.p;
@@ -2579,10 +2651,6 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         RIN_HIP(hipStreamCreateWithFlags(&w.side2, hipStreamNonBlocking));
         RIN_HIP(hipEventCreateWithFlags(&w.join2, hipEventDisableTiming));
     }
-    if (w.wide && !w.side3) {
-        RIN_HIP(hipStreamCreateWithFlags(&w.side3, hipStreamNonBlocking));
-        RIN_HIP(hipEventCreateWithFlags(&w.join3, hipEventDisableTiming));
-    }
     hipGraph_t gr = nullptr;
     RIN_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
     // regular grids with lane-group cuts start them right after the counts,
@@ -2602,20 +2670,15 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
             RIN_HIP(hipStreamWaitEvent(w.side, w.fork, 0));
             launch_cut_early(w, g, val, 2, w.grid[2], w.side);
             RIN_HIP(hipEventRecord(w.join, w.side));
-            if (w.wide) {
-                RIN_HIP(hipStreamWaitEvent(w.side3, w.fork, 0));
-                launch_cut_early(w, g, val, 2, w.grid[2], w.side3, true);
-                RIN_HIP(hipEventRecord(w.join3, w.side3));
-            }
         }
         RIN_HIP(hipStreamWaitEvent(w.side2, w.fork, 0));
         stage_fill(w, g, val, w.side2);
         if (!e5 && w.cap.b[2]) launch_cut<CBig>(w, g, val, 2, w.grid[2], w.side2);
         if (!e3 && w.cap.b[1]) launch_cut<CMed>(w, g, val, 1, w.grid[1], w.side2);
         if (w.cap.b[0]) launch_cut<CK2>(w, g, val, 0, w.grid[0], w.side2);
+        if (e5 && w.wide) launch_cut_early(w, g, val, 2, w.grid[2], w.side2, true);
         RIN_HIP(hipEventRecord(w.join2, w.side2));
         if (e5) RIN_HIP(hipStreamWaitEvent(s, w.join, 0));
-        if (e5 && w.wide) RIN_HIP(hipStreamWaitEvent(s, w.join3, 0));
         RIN_HIP(hipStreamWaitEvent(s, w.join2, 0));
     } else {
         stage_fill(w, g, val, s);
@@ -2728,7 +2791,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
                 tiny.active = tiny.fit = 64;
                 for (int q = 0; q < 3; ++q) tiny.b[q] = 64;
                 tiny.vo = tiny.fo = tiny.fv = 64;
-                alloc_ws(w, g, tiny, s);
+                alloc_ws(w, g, val.F, tiny, s);
             }
             stage_count(w, g, val, s);
             read_back(true);
@@ -2752,7 +2815,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
                 grow.vo = more(w.cap.vo, need.vo);
                 grow.fo = more(w.cap.fo, need.fo);
                 grow.fv = more(w.cap.fv, need.fv);
-                alloc_ws(w, g, grow, s);
+                alloc_ws(w, g, val.F, grow, s);
                 stage_count(w, g, val, s);
             }
             stage_fill(w, g, val, s);
@@ -2929,6 +2992,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
     vw.csr_off = w.csr_off.p;
     vw.act = w.act.p;
     vw.rank_of_tet = w.rank.p;
+    vw.rank_blocks = w.blocks.p;
     vw.rec = w.rec.p;
     vw.rec_loc = w.rec_loc.p;
     vw.k1_rec = w.k1_words.p;

@@ -377,6 +377,48 @@ __global__ void __launch_bounds__(kMiLanes) k_mi_fill_tiles(uint64_t T, const ui
         }
 }
 
+// The tables and the lane-group cuts of four and of five to eight materials
+// in one launch of wavefronts, the longest first: the lists share no output,
+// and each cut's time is the latency of its longest tet (59 + 65 us one after
+// the other at 65^3 vertices and 8 materials, and 34 us of tables; together
+// 72 us).  One launch rather than graph branches: kernels with this much
+// private memory stay on one queue.
+struct MICutArgs {
+    GridView g;
+    ValsRef vals;
+    const uint32_t* act;
+    const uint8_t* act_k;
+    const uint32_t* csr_off;
+    const uint8_t* fit;
+    const uint32_t* list[3];
+    Count n[3];
+    const uint32_t* rec_off;
+    uint32_t* rec_loc;
+    uint16_t* rec;
+    uint32_t *cnt, *errs, *labels;
+    MITablesDev tables;
+    uint32_t base2, base3;
+    MI3Snap snap;
+};
+__global__ void __launch_bounds__(64) k_mi_cuts(MICutArgs A, uint32_t nb5, uint32_t nb4, uint32_t nbt) {
+    __shared__ union U {
+        dev::WaveMI<CBig> big;
+        dev::WaveMI<CMed> med;
+        MI3Pat pats[81];
+        __device__ U() {}
+    } u;
+    const uint32_t b = blockIdx.x;
+    if (b < nb5)
+        cut_group_role<CBig, 64, true>(&u.big, b, nb5, A.g, A.vals, A.act, A.act_k, A.csr_off, A.fit, A.list[2], A.n[2],
+                                       A.rec_off, A.rec, A.cnt, A.errs, 0, 0u, A.labels, A.snap);
+    else if (b < nb5 + nb4)
+        cut_group_role<CMed, 64, true>(&u.med, b - nb5, nb4, A.g, A.vals, A.act, A.act_k, A.csr_off, A.fit, A.list[1],
+                                       A.n[1], A.rec_off, A.rec, A.cnt, A.errs, 0, 0u, A.labels, A.snap);
+    else
+        mi_table_role(u.pats, b - nb5 - nb4, nbt, A.g, A.vals, A.act, A.csr_off, A.fit, A.list[0], count_of(A.n[0]),
+                      nullptr, 0u, A.rec_off, A.rec, A.cnt, A.errs, A.tables, A.labels, A.rec_loc, A.base2, A.base3);
+}
+
 // closes the face arrays, publishes the counters and the union of the error
 // flags into pinned host memory, and clears both for the next run
 __global__ void k_mi_close(uint32_t* ctr, uint32_t* errs, uint32_t cap_fo, uint32_t* f_vstart, uint32_t* f_tfstart,
@@ -451,9 +493,6 @@ struct MIWorkspace {
     uint32_t* pub_d = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    // side branches of the graph: the cuts run beside each other
-    hipStream_t side[3] = {nullptr, nullptr, nullptr};
-    hipEvent_t fork = nullptr, join[3] = {nullptr, nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool ctr_clear = false;  // counters and error flags are zero (left so by the last run)
     void drop_graph() {
@@ -464,11 +503,6 @@ struct MIWorkspace {
     }
     ~MIWorkspace() {
         drop_graph();
-        for (int q = 0; q < 3; ++q) {
-            if (join[q]) (void)hipEventDestroy(join[q]);
-            if (side[q]) (void)hipStreamDestroy(side[q]);
-        }
-        if (fork) (void)hipEventDestroy(fork);
         for (auto e : ev)
             if (e) (void)hipEventDestroy(e);
         if (pub_h) (void)hipHostFree(pub_h);
@@ -611,55 +645,54 @@ void mi_path(MIWorkspace& W, const Grid& g, uint32_t F, const MITablesDev& TT, h
                        (const MITile*)W.tiles.p, abort, tables, W.csr_off.p, W.rank.p, W.fit.p, W.act.p, W.act_k.p,
                        W.rec_off.p, W.rec_loc.p, bl[0], bl[1], bl[2], bl[3]);
     const Count NA(ctr + M_ACTIVE, c.active, abort);
-    // The cuts beside each other, each list on a branch of its own: the
-    // tables (table tets point at the table's record), four materials, five
-    // to eight, more.  One after another they took 59 + 65 + 34 us at 65^3
-    // vertices and 8 materials, each the latency of its longest tet.
-    RIN_HIP(hipEventRecord(W.fork, s));
-    for (int q = 0; q < (W.wide ? 3 : 2); ++q) RIN_HIP(hipStreamWaitEvent(W.side[q], W.fork, 0));
-    hipLaunchKernelGGL(k_mi_table, dim3(blocks_for(c.active)), dim3(256), 0, s, G, vals, (const uint32_t*)W.act.p,
-                       (const uint32_t*)W.csr_off.p, (const uint8_t*)W.fit.p, (const uint32_t*)bl[0],
-                       (uint64_t)c.active, (const uint32_t*)(ctr + M_LIST), (uint32_t)0, (const uint32_t*)W.rec_off.p,
-                       W.rec.p, W.cnt.p, W.errs.p, TT, W.labels.p, W.rec_loc.p, W.tab_base2, W.tab_base3);
     const Count n1(ctr + M_LIST + 1, c.active, abort), n2(ctr + M_LIST + 2, c.active, abort);
+    // the cuts start from the 3-material table's complex after three
+    // materials (RIN_MI3_START=0: from the tet)
+    const char* ms = std::getenv("RIN_MI3_START");
+    MICutArgs U;
+    U.g = G;
+    U.vals = vals;
+    U.act = W.act.p;
+    U.act_k = W.act_k.p;
+    U.csr_off = W.csr_off.p;
+    U.fit = W.fit.p;
+    for (int q = 0; q < 3; ++q) U.list[q] = bl[q];
+    U.n[0] = Count(ctr + M_LIST, c.active, abort);
+    U.n[1] = n1;
+    U.n[2] = n2;
+    U.rec_off = W.rec_off.p;
+    U.rec_loc = W.rec_loc.p;
+    U.rec = W.rec.p;
+    U.cnt = W.cnt.p;
+    U.errs = W.errs.p;
+    U.labels = W.labels.p;
+    U.tables = TT;
+    U.base2 = W.tab_base2;
+    U.base3 = W.tab_base3;
+    U.snap = (ms && !std::strcmp(ms, "0")) ? MI3Snap{nullptr, nullptr, nullptr}
+                                           : MI3Snap{TT.pat3, TT.snap_off3, TT.snap3};
     if (all_thread) {
-        hipLaunchKernelGGL((k_cut_lds<CMed, true, 2>), dim3(W.cut_blocks[0]), dim3(2), 0, W.side[0], G, vals,
+        hipLaunchKernelGGL((k_cut_lds<CMed, true, 2>), dim3(W.cut_blocks[0]), dim3(2), 0, s, G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, n1, 1, 4, (uint32_t)0, (const uint32_t*)W.rec_off.p, W.rec.p,
                            W.cnt.p, W.errs.p, (const uint32_t*)bl[1], W.labels.p);
-        hipLaunchKernelGGL((k_cut_lds<CBig, true, 1>), dim3(W.cut_blocks[1]), dim3(1), 0, W.side[1], G, vals,
+        hipLaunchKernelGGL((k_cut_lds<CBig, true, 1>), dim3(W.cut_blocks[1]), dim3(1), 0, s, G, vals,
                            (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
                            (const uint8_t*)W.fit.p, n2, 5, 8, (uint32_t)0, (const uint32_t*)W.rec_off.p, W.rec.p,
                            W.cnt.p, W.errs.p, (const uint32_t*)bl[2], W.labels.p);
     } else {
-        // a wavefront per tet: these lists are short and each tet's latency
-        // is the kernel's time; the cuts start from the 3-material table's
-        // complex after three materials (RIN_MI3_START=0: from the tet)
-        const char* ms = std::getenv("RIN_MI3_START");
-        const MI3Snap m3s = (ms && !std::strcmp(ms, "0")) ? MI3Snap{nullptr, nullptr, nullptr}
-                                                          : MI3Snap{TT.pat3, TT.snap_off3, TT.snap3};
-        const unsigned g1 = (unsigned)std::min<uint64_t>(c.active + 1, 2048);
-        const unsigned g2 = (unsigned)std::min<uint64_t>(c.active + 1, 1024);
-        hipLaunchKernelGGL((k_cut_group<CMed, 64, true>), dim3(g1), dim3(64), 0, W.side[0], G, vals,
-                           (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
-                           (const uint8_t*)W.fit.p, (const uint32_t*)bl[1], n1, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, 0, (uint32_t)0, W.labels.p, m3s);
-        hipLaunchKernelGGL((k_cut_group<CBig, 64, true>), dim3(g2), dim3(64), 0, W.side[1], G, vals,
-                           (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p, (const uint32_t*)W.csr_off.p,
-                           (const uint8_t*)W.fit.p, (const uint32_t*)bl[2], n2, (const uint32_t*)W.rec_off.p, W.rec.p,
-                           W.cnt.p, W.errs.p, 0, (uint32_t)0, W.labels.p, m3s);
+        const unsigned nb5 = (unsigned)std::min<uint64_t>(c.active + 1, 1024);
+        const unsigned nb4 = (unsigned)std::min<uint64_t>(c.active + 1, 2048);
+        const unsigned nbt = (unsigned)std::min<uint64_t>((c.active + 63) / 64 + 1, 16384);
+        hipLaunchKernelGGL(k_mi_cuts, dim3(nb5 + nb4 + nbt), dim3(64), 0, s, U, nb5, nb4, nbt);
     }
     if (W.wide) {
         const MI3Snap none{nullptr, nullptr, nullptr};
         hipLaunchKernelGGL((k_cut_group<CWideMI, 64, true>), dim3((unsigned)std::min<uint64_t>(c.active + 1, 512)),
-                           dim3(64), 0, W.side[2], G, vals, (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p,
+                           dim3(64), 0, s, G, vals, (const uint32_t*)W.act.p, (const uint8_t*)W.act_k.p,
                            (const uint32_t*)W.csr_off.p, (const uint8_t*)W.fit.p, (const uint32_t*)bl[3],
                            Count(ctr + M_LIST + 3, c.active, abort), (const uint32_t*)W.rec_off.p, W.rec.p, W.cnt.p,
                            W.errs.p, 0, (uint32_t)0, W.labels.p, none);
-    }
-    for (int q = 0; q < (W.wide ? 3 : 2); ++q) {
-        RIN_HIP(hipEventRecord(W.join[q], W.side[q]));
-        RIN_HIP(hipStreamWaitEvent(s, W.join[q], 0));
     }
     // extraction (src/extract_mesh.cpp:569-986): boundary-face pairing, then
     // occurrences in the reference's creation order
@@ -700,7 +733,7 @@ void mi_path(MIWorkspace& W, const Grid& g, uint32_t F, const MITablesDev& TT, h
         S.okey = W.okey.p;
         S.oa = W.oa.p;
         S.act = W.act.p;
-        S.rank = W.rank.p;
+        S.rank = RankOf{W.rank.p, W.act.p, nullptr};
         S.voff = W.cv.p;
         S.star_head = W.star_head.p;
         S.star_ent = W.star_ent.p;
@@ -810,14 +843,8 @@ void run_batched_mi(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t 
             const int kbits = 2 + std::max({bits_of(g.view.V), bits_of(g.view.n_edge_ids) + 12,
                                             bits_of(g.view.n_face_ids) + 18, bits_of(w.cap.active) + 10});
             if (kbits > 63) throw NeedsPlainForm("simplex keys exceed 63 bits for this mesh");
-            if (!w.fork) {
-                RIN_HIP(hipEventCreateWithFlags(&w.fork, hipEventDisableTiming));
-                for (int q = 0; q < 3; ++q) {
-                    RIN_HIP(hipStreamCreateWithFlags(&w.side[q], hipStreamNonBlocking));
-                    RIN_HIP(hipEventCreateWithFlags(&w.join[q], hipEventDisableTiming));
-                }
-                for (auto& e : w.ev) RIN_HIP(hipEventCreate(&e));
-            }
+            for (auto& e : w.ev)
+                if (!e) RIN_HIP(hipEventCreate(&e));
             hipGraph_t gr = nullptr;
             RIN_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
             try {

@@ -584,24 +584,28 @@ __device__ __forceinline__ bool mi3_start(dev::WaveMI<C>& X, const MI3Snap& S, i
 // in descending order): at 50^3 vertices and 8 functions one pass of that
 // check takes 0.25 ms of cuts, and took 4.7 ms a lane a tet, 1.4 ms of them
 // for a single tet of five functions.
+template <class C, bool MI>
+using GroupComplex = typename std::conditional<MI, dev::WaveMI<C>, dev::WaveIA<C>>::type;
+template <bool MI>
+using GroupSnap = typename std::conditional<MI, MI3Snap, K2Snap>::type;
+
+// as a workgroup role (64 lanes): blk of nblk workgroups, Xs one complex a group
 template <class C, int G, bool MI>
-__global__ void __launch_bounds__(64) k_cut_group(GridView g, ValsRef vref,
-                                                  const uint32_t* __restrict__ act, const uint8_t* __restrict__ act_k,
-                                                  const uint32_t* __restrict__ csr_off,
-                                                  const uint8_t* __restrict__ fit, const uint32_t* __restrict__ list,
-                                                  Count nlist, const uint32_t* __restrict__ rec_off,
-                                                  uint16_t* __restrict__ rec, uint32_t* __restrict__ cnt,
-                                                  uint32_t* __restrict__ errs, int retry, uint32_t flags,
-                                                  uint32_t* __restrict__ labels, typename std::conditional<MI, MI3Snap, K2Snap>::type snap) {
+__device__ __forceinline__ void cut_group_role(GroupComplex<C, MI>* Xs, uint32_t blk, uint32_t nblk, const GridView& g,
+                                               ValsRef vref, const uint32_t* __restrict__ act,
+                                               const uint8_t* __restrict__ act_k, const uint32_t* __restrict__ csr_off,
+                                               const uint8_t* __restrict__ fit, const uint32_t* __restrict__ list,
+                                               Count nlist, const uint32_t* __restrict__ rec_off,
+                                               uint16_t* __restrict__ rec, uint32_t* __restrict__ cnt,
+                                               uint32_t* __restrict__ errs, int retry, uint32_t flags,
+                                               uint32_t* __restrict__ labels, const GroupSnap<MI>& snap) {
     const double* __restrict__ vals = vref.get();
     constexpr int NG = 64 / G;
-    using Cx = typename std::conditional<MI, dev::WaveMI<C>, dev::WaveIA<C>>::type;
-    __shared__ Cx Xs[NG];
     const int gid = threadIdx.x / G, lane = threadIdx.x & (G - 1);
-    Cx& X = Xs[gid];
+    GroupComplex<C, MI>& X = Xs[gid];
     const uint64_t n = count_of(nlist);
     const uint64_t V = g.V;
-    for (uint64_t i = (uint64_t)blockIdx.x * NG + gid; i < n; i += (uint64_t)gridDim.x * NG) {
+    for (uint64_t i = (uint64_t)blk * NG + gid; i < n; i += (uint64_t)nblk * NG) {
         const uint32_t a = list[i];
         const int k = act_k[a];
         const uint32_t t = act[a], s0 = csr_off[t];
@@ -664,6 +668,20 @@ __global__ void __launch_bounds__(64) k_cut_group(GridView g, ValsRef vref,
         }
         __syncthreads();  // the group's complex is reused by its next tet
     }
+}
+
+template <class C, int G, bool MI>
+__global__ void __launch_bounds__(64) k_cut_group(GridView g, ValsRef vref, const uint32_t* __restrict__ act,
+                                                  const uint8_t* __restrict__ act_k,
+                                                  const uint32_t* __restrict__ csr_off,
+                                                  const uint8_t* __restrict__ fit, const uint32_t* __restrict__ list,
+                                                  Count nlist, const uint32_t* __restrict__ rec_off,
+                                                  uint16_t* __restrict__ rec, uint32_t* __restrict__ cnt,
+                                                  uint32_t* __restrict__ errs, int retry, uint32_t flags,
+                                                  uint32_t* __restrict__ labels, GroupSnap<MI> snap) {
+    __shared__ GroupComplex<C, MI> Xs[64 / G];
+    cut_group_role<C, G, MI>(Xs, blockIdx.x, gridDim.x, g, vref, act, act_k, csr_off, fit, list, nlist, rec_off, rec,
+                             cnt, errs, retry, flags, labels, snap);
 }
 
 // active tets with more than 8 functions, and tets a bucket kernel could not
@@ -1230,6 +1248,8 @@ __global__ void __launch_bounds__(kPatchLanes) k_patch_walk(const uint32_t* __re
                     if (adj[o] != ~0u) atomicMin(&claim[adj[o]], (unsigned long long)(i + 1) << 16 | (o - b));
             }
         }
+        // the minima are done, not only issued, before any lane reads a claim
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         uint32_t next = tail;
         for (uint32_t i0 = head; i0 < tail; i0 += kPatchLanes) {
@@ -1339,6 +1359,27 @@ __device__ inline void hash_insert_one(uint32_t o, const uint64_t* __restrict__ 
     hslot[o] = 0;
 }
 
+// The active rank of a tet, or ~0 when it is not active: by the scan of the
+// active flags (dense, one word a tet), or on regular grids by blocks of 32
+// tets (active bits, active tets before the block): a thirty-second of the
+// dense ranks to write, and a look-up that rarely leaves the L2 and need not
+// check the rank's tet.
+struct RankOf {
+    const uint32_t* dense;
+    const uint32_t* act;
+    const uint2* blocks;
+    __device__ uint32_t operator()(uint64_t t, uint32_t n_active) const {
+        if (blocks) {
+            const uint2 b = blocks[t >> 5];
+            const uint32_t bit = 1u << (t & 31);
+            const uint32_t r = b.y + (uint32_t)__popc(b.x & (bit - 1));
+            return (b.x & bit) && r < n_active ? r : ~0u;
+        }
+        const uint32_t r = dense[t];
+        return r < n_active && act[r] == (uint32_t)t ? r : ~0u;
+    }
+};
+
 constexpr int kStarShapes = 1 + 27 + 27 * 27;  // corner, edge by direction, face by two directions
 
 struct StarArgs {
@@ -1346,7 +1387,8 @@ struct StarArgs {
     int edge_shift, face_shift;  // where the edge and face ids begin in a key
     int own;                     // a tet may hold a key more than once (its own occurrences are searched too)
     const uint64_t* okey;
-    const uint32_t *oa, *act, *rank, *voff;
+    const uint32_t *oa, *act, *voff;
+    RankOf rank;
     const uint32_t* star_head;  // [2][kStarShapes]: first entry << 8 | entry count
     const uint8_t* star_ent;    // (di+1) | (dj+1) << 2 | (dk+1) << 4 with di.. in {-1, 0}, then q
     uint32_t *first, *mo;
@@ -1412,8 +1454,8 @@ __device__ __forceinline__ uint32_t star_walk_first(const StarArgs& A, uint32_t 
     for (;;) {
         const uint64_t ts = S.next(A, R);
         if (ts >= t) break;
-        const uint32_t a = A.rank[ts];
-        if (a >= NA || A.act[a] != (uint32_t)ts) continue;
+        const uint32_t a = A.rank(ts, NA);
+        if (a == ~0u) continue;
         uint32_t hi = a + 1 < NA ? A.voff[a + 1] : NO;
         hi = hi < NO ? hi : NO;
         for (uint32_t p = A.voff[a]; p < hi; ++p)
@@ -1454,11 +1496,11 @@ __global__ void __launch_bounds__(256) k_dedup_star(Count n, StarArgs A) {
         // interior keys, and keys whose lowest star tet is this one, are first here
         // (with `own`, after a look at this one's earlier occurrences)
         found[u] = ((K[u] & 3) == 3 || (ts[u] == t[u] && !A.own)) ? o[u] : ~0u;
-        as[u] = (found[u] == ~0u && ts[u] != ~0ull) ? (ts[u] == t[u] ? oa[u] : A.rank[ts[u]]) : ~0u;
+        as[u] = (found[u] == ~0u && ts[u] != ~0ull) ? (ts[u] == t[u] ? oa[u] : A.rank(ts[u], NA)) : ~0u;
     }
 #pragma unroll
     for (int u = 0; u < kDedupU; ++u) {
-        const bool ok = as[u] < NA && A.act[as[u]] == (uint32_t)ts[u];
+        const bool ok = as[u] < NA;
         lo[u] = ok ? A.voff[as[u]] : 0u;
         hi[u] = ok ? (as[u] + 1 < NA ? A.voff[as[u] + 1] : NO) : 0u;
         hi[u] = hi[u] < NO ? hi[u] : NO;
@@ -2069,7 +2111,8 @@ constexpr int kFaceU = 4;
 constexpr uint32_t kFaceTile = 256u * kFaceU;
 
 struct FaceTileArgs {
-    const uint32_t *fq_a, *fq_vs, *fve, *act, *rank, *foff, *nbr;
+    const uint32_t *fq_a, *fq_vs, *fve, *act, *foff, *nbr;
+    RankOf rank;
     const uint32_t *mo, *vrank;  // vertex id of occurrence o: vrank[mo[o]]
     const uint8_t* fq_bnd;
     const uint16_t* fq_l;
@@ -2139,8 +2182,8 @@ __device__ inline void face_first_role(const FaceTileArgs& A, uint32_t blk) {
             const uint32_t a = A.fq_a[q], t = A.act[a], l = A.fq_bnd[q] - 1u;
             const uint32_t nb = A.nbr[4 * (uint64_t)t + l];
             if (nb != 0xFFFFFFFFu) {
-                const uint32_t t2 = nb >> 2, l2 = nb & 3u, r2 = A.rank[t2];
-                if (r2 < NA && A.act[r2] == t2) {
+                const uint32_t t2 = nb >> 2, l2 = nb & 3u, r2 = A.rank(t2, NA);
+                if (r2 < NA) {
                     const uint32_t q0 = A.foff[r2];
                     const uint32_t q1 = (r2 + 1 < NA) ? A.foff[r2 + 1] : clamp_count(A.nfo_total, A.nfo_cap);
                     for (uint32_t p = q0; p < q1; ++p) {

@@ -119,7 +119,8 @@ inline MITablesDev mi_tables_view(const MITablesRaw& r) {
 // general cut (CNT_RETRY).  rec_loc (optional): the record words hold the two
 // tables' words at base2 and base3, and the tet's record location becomes the
 // table record's instead of a copy into its slot.
-__global__ void __launch_bounds__(256) k_mi_table(GridView g, ValsRef vref,
+// as a workgroup role: blk of nblk workgroups, pats in LDS
+__device__ __forceinline__ void mi_table_role(MI3Pat* pats, uint32_t blk, uint32_t nblk, const GridView& g, ValsRef vref,
                                                   const uint32_t* __restrict__ act,
                                                   const uint32_t* __restrict__ csr_off, const uint8_t* __restrict__ fit,
                                                   const uint32_t* __restrict__ list, uint64_t n,
@@ -129,13 +130,12 @@ __global__ void __launch_bounds__(256) k_mi_table(GridView g, ValsRef vref,
                                                   MITablesDev T, uint32_t* __restrict__ labels,
                                                   uint32_t* __restrict__ rec_loc, uint32_t base2, uint32_t base3) {
     const double* __restrict__ vals = vref.get();
-    __shared__ MI3Pat pats[81];
     for (int i = threadIdx.x; i < 81 * (int)sizeof(MI3Pat) / 4; i += blockDim.x)
         reinterpret_cast<uint32_t*>(pats)[i] = reinterpret_cast<const uint32_t*>(T.pat3)[i];
     __syncthreads();
     if (n_dev) n = *n_dev < n ? *n_dev : n;
     const uint64_t V = g.V;
-    GRID_STRIDE(i, n) {
+    for (uint64_t i = (uint64_t)blk * blockDim.x + threadIdx.x; i < n; i += (uint64_t)nblk * blockDim.x) {
         const uint32_t a = list[i];
         const uint32_t t = act[a];
         uint32_t v[4];
@@ -197,6 +197,19 @@ __global__ void __launch_bounds__(256) k_mi_table(GridView g, ValsRef vref,
             for (uint32_t q = 0; q < len; ++q) rec[at + q] = src[q];
         for (int q = 0; q < 3; ++q) cnt[3 * (uint64_t)a + q] = c3[q];
     }
+}
+
+__global__ void __launch_bounds__(256) k_mi_table(GridView g, ValsRef vref,
+                                                  const uint32_t* __restrict__ act,
+                                                  const uint32_t* __restrict__ csr_off, const uint8_t* __restrict__ fit,
+                                                  const uint32_t* __restrict__ list, uint64_t n,
+                                                  const uint32_t* __restrict__ n_dev, uint32_t flags,
+                                                  const uint32_t* __restrict__ rec_off, uint16_t* __restrict__ rec,
+                                                  uint32_t* __restrict__ cnt, uint32_t* __restrict__ errs,
+                                                  MITablesDev T, uint32_t* __restrict__ labels,
+                                                  uint32_t* __restrict__ rec_loc, uint32_t base2, uint32_t base3) {
+    __shared__ MI3Pat pats[81];
+    mi_table_role(pats, blockIdx.x, gridDim.x, g, vref, act, csr_off, fit, list, n, n_dev, flags, rec_off, rec, cnt, errs, T, labels, rec_loc, base2, base3);
 }
 
 // ------------------------------------------------------------------ per-tet helpers

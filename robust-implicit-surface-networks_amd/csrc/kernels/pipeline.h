@@ -95,6 +95,7 @@ struct RunOut {
     struct View {
         const uint8_t* fit = nullptr;
         const uint32_t *csr_off = nullptr, *act = nullptr, *rank_of_tet = nullptr, *rec_off = nullptr;
+        const uint2* rank_blocks = nullptr;      // instead of rank_of_tet: batched IA on regular grids
         const uint16_t* rec = nullptr;
         const uint32_t* rec_loc = nullptr;       // batched: word offset, or 0x80000000|pattern for k=1
         const uint16_t* k1_rec = nullptr;        // batched: k=1 records by pattern

@@ -999,7 +999,7 @@ __global__ void __launch_bounds__(64) k_debug_cut_wave(const double* rows, const
 // record lookup for a list of tets: source word offset (bit 63: k=1 table)
 // and length, 0 for inactive tets
 __global__ void k_rec_lookup(const uint32_t* __restrict__ tets, uint64_t n, uint64_t T, uint64_t n_active,
-                             const uint32_t* __restrict__ rank, const uint32_t* __restrict__ act,
+                             RankOf rank,
                              const uint32_t* __restrict__ rec_loc, const uint16_t* __restrict__ rec,
                              const uint16_t* __restrict__ k1_rec, const uint32_t* __restrict__ k1_off,
                              uint64_t* __restrict__ src, uint32_t* __restrict__ len) {
@@ -1008,8 +1008,8 @@ __global__ void k_rec_lookup(const uint32_t* __restrict__ tets, uint64_t n, uint
         uint32_t L = 0;
         uint64_t o = 0;
         if (t < T) {
-            const uint32_t rk = rank[t];
-            if (rk < n_active && act[rk] == t) {
+            const uint32_t rk = rank(t, (uint32_t)n_active);
+            if (rk != ~0u) {
                 const uint32_t loc = rec_loc ? rec_loc[rk] : 0u;
                 if (rec_loc && (loc & 0x80000000u)) {
                     o = (1ull << 63) | k1_off[loc & 0x7FFFFFFFu];
@@ -1051,7 +1051,7 @@ void gather_records(DevMem& mem, const RunOut& r, const uint64_t* tets, uint64_t
     DBuf<uint64_t> dsrc(mem, n);
     RIN_HIP(hipMemcpyAsync(dt.p, t32.data(), 4 * n, hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_rec_lookup, dim3(nblk(n)), dim3(256), 0, s, (const uint32_t*)dt.p, n, r.T, r.n_active,
-                       vw.rank_of_tet, vw.act, vw.rec_loc, vw.rec, vw.k1_rec, vw.k1_rec_off, dsrc.p, dlen.p);
+                       RankOf{vw.rank_of_tet, vw.act, vw.rank_blocks}, vw.rec_loc, vw.rec, vw.k1_rec, vw.k1_rec_off, dsrc.p, dlen.p);
     std::vector<uint32_t> len(n);
     RIN_HIP(hipMemcpyAsync(len.data(), dlen.p, 4 * n, hipMemcpyDeviceToHost, s));
     RIN_HIP(hipStreamSynchronize(s));
