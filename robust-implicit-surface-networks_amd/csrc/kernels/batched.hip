@@ -451,6 +451,7 @@ struct FillArgs {
     const uint32_t *csr_off, *rank;  // explicit meshes
     uint32_t* csr_off_w;             // written by the cube form
     uint2* blocks;                   // written by the cube form (RankOf)
+    const uint64_t* busy;            // cube form: per 64 cubes, which hold an active tet
     uint8_t* fit;
     uint32_t *act, *rec_loc, *cnt;
     uint32_t* act_off;  // CSR offset by active rank
@@ -582,46 +583,62 @@ __global__ void __launch_bounds__(1024) k_signs_count(const double* __restrict__
 // tets and bucket sizes, one workgroup scans those, and each fill workgroup
 // places its tets in the CSR, the active list and the bucket lists from its
 // tile's prefixes, in tet order and without atomics.
+//
+// Both passes are bound by instructions and waits, not by memory (their masks
+// stay in L2; the fill writes 4 bytes a tet, 30 a row).  What counts is what a
+// wave without an active tet (the most, on a fine grid) has to do: the masks
+// come two corners a load, one AND over the cube ends an inactive one, the
+// wave sums are two packed words (7 before), and the count leaves which cubes
+// are active for the fill.  The fill lists its active tets in LDS and writes
+// their rows a lane each.  200^3 cubes, 8 functions: count 106 -> 57 us, fill
+// 178 -> 128 us (31 us are its bytes); 100^3, 20 functions: 20 -> 14 us and
+// 32 -> 30 us.
 
 // cubes per tile (one workgroup): 256, 512 or 1024, picked per plan by the
 // autotuner (the results do not depend on it)
 constexpr int kCubeTile = 512;  // the default
 
-// pat (optional): per tet with one active function, its corner sign pattern
-// (sum of s_c 3^c, s_c = 0 negative, 1 zero, 2 positive), else 0
 template <class T, class M>
 __device__ inline void cube_masks(const GridView& g, uint32_t cube, const MaskPair<T>* __restrict__ masks, M full,
-                                  uint32_t c[8], M m[5], bool& even, uint8_t* pat = nullptr) {
+                                  M m[5]) {
     const uint32_t R = (uint32_t)g.res, N = R + 1;
     const uint32_t i = cube / (R * R), rem = cube - i * (R * R), j = rem / R, k = rem - j * R;
     const uint32_t b = i * N * N + j * N + k;
-    c[0] = b;
-    c[1] = b + N * N;
-    c[2] = b + N * N + N;
-    c[3] = b + N;
-    for (int a = 0; a < 4; ++a) c[4 + a] = c[a] + 1;
-    even = ((i + j + k) & 1u) == 0;
+    const uint32_t c[4] = {b, b + N * N, b + N * N + N, b + N};
+    const bool even = ((i + j + k) & 1u) == 0;
     M P[8], Q[8];
-    for (int a = 0; a < 8; ++a) {
-        const MaskPair<T> x = masks[c[a]];
-        P[a] = x.pos;
-        Q[a] = x.neg;
+    // the corners c[a] and c[a + 4] = c[a] + 1 lie side by side: one load each
+    // (from an element's alignment; global loads take any)
+    struct Two {
+        MaskPair<T> lo, hi;
+    };
+    for (int a = 0; a < 4; ++a) {
+        Two x;
+        __builtin_memcpy(&x, masks + c[a], sizeof x);
+        P[a] = x.lo.pos;
+        Q[a] = x.lo.neg;
+        P[4 + a] = x.hi.pos;
+        Q[4 + a] = x.hi.neg;
     }
+    // a function of one sign over the cube's corners is active in none of its
+    // tets: most cubes of a fine grid end here, and many waves with them
+    if (!(full & ~((P[0] & P[1] & P[2] & P[3] & P[4] & P[5] & P[6] & P[7]) |
+                   (Q[0] & Q[1] & Q[2] & Q[3] & Q[4] & Q[5] & Q[6] & Q[7])))) {
+        for (int q = 0; q < 5; ++q) m[q] = 0;
+        return;
+    }
+    // both parities' tets with indices known here, then one select: an index
+    // into P and Q known only at run time is a chain of compares and selects
+    // (256 of the count pass's 900 instructions)
+#pragma unroll
     for (int q = 0; q < 5; ++q) {
-        const uint8_t* t = even ? dev::kCubeTetEven[q] : dev::kCubeTetOdd[q];
-        const M ap = P[t[0]] & P[t[1]] & P[t[2]] & P[t[3]];
-        const M an = Q[t[0]] & Q[t[1]] & Q[t[2]] & Q[t[3]];
-        m[q] = full & ~(ap | an);
-        if (pat) {
-            pat[q] = 0;
-            if (__popcll(m[q]) == 1) {
-                const uint32_t f = __ffsll((unsigned long long)m[q]) - 1;
-                int p = 0, w = 1;
-                for (int a = 0; a < 4; ++a, w *= 3)
-                    p += (((P[t[a]] >> f) & 1) ? 2 : (((Q[t[a]] >> f) & 1) ? 0 : 1)) * w;
-                pat[q] = (uint8_t)p;
-            }
-        }
+        constexpr auto& E = dev::kCubeTetEven;
+        constexpr auto& O = dev::kCubeTetOdd;
+        const M pe = P[E[q][0]] & P[E[q][1]] & P[E[q][2]] & P[E[q][3]];
+        const M ne = Q[E[q][0]] & Q[E[q][1]] & Q[E[q][2]] & Q[E[q][3]];
+        const M po = P[O[q][0]] & P[O[q][1]] & P[O[q][2]] & P[O[q][3]];
+        const M no = Q[O[q][0]] & Q[O[q][1]] & Q[O[q][2]] & Q[O[q][3]];
+        m[q] = full & ~(even ? pe | ne : po | no);
     }
 }
 
@@ -654,7 +671,8 @@ struct EarlyEntry {
 // are contiguous and in tet order (the back part reversed).
 template <int TILE, class T>
 __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<T>* __restrict__ masks, uint64_t full,
-                                                     int kbig, TileSums* __restrict__ tile_sums, EarlyEntry* early3,
+                                                     int kbig, TileSums* __restrict__ tile_sums,
+                                                     uint64_t* __restrict__ busy, EarlyEntry* early3,
                                                      EarlyEntry* early5, uint32_t early_cap3, uint32_t early_cap5,
                                                      uint32_t* ctr) {
     using M = typename std::conditional<sizeof(T) == 8, uint64_t, uint32_t>::type;
@@ -662,13 +680,12 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
     const uint32_t tile = blockIdx.x;
     const uint32_t cube = tile * TILE + threadIdx.x;
     uint32_t v[kTileFields] = {0, 0, 0, 0, 0, 0, 0, 0};
-    M m[5] = {0, 0, 0, 0, 0};
+    M m[5] = {0, 0, 0, 0, 0}, some = 0;
     uint32_t n4 = 0;  // k = 4 tets (of the k = 3..4 bucket)
     if (cube < ncubes) {
-        uint32_t c[8];
-        bool even;
-        cube_masks<T, M>(g, cube, masks, (M)full, c, m, even);
-        for (int q = 0; q < 5; ++q) {
+        cube_masks<T, M>(g, cube, masks, (M)full, m);
+        some = m[0] | m[1] | m[2] | m[3] | m[4];
+        for (int q = 0; q < 5 && some; ++q) {
             const int k = __popcll(m[q]);
             v[TF_FIT] += (uint32_t)k;
             v[TF_ACTIVE] += k != 0;
@@ -681,6 +698,8 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
         }
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t bl = __ballot(some != 0);
+    if (lane == 0) busy[cube >> 6] = bl;
     // tiles holding listed tets rank them inside the tile: exclusive scans of
     // (active functions, active tets) packed as in the fill pass, and of the
     // listed counts in 16-bit fields (k = 4 | k = 3 << 16 | k = 5..8 << 32;
@@ -748,10 +767,28 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
             lr += k != 0;
         }
     }
+    // the wave's sums: a wave holds at most 320 tets and 64 functions a tet, so
+    // five fields fit one 64-bit word and two another; a wave without an
+    // active tet (most, on a fine grid) has none to add
     __shared__ uint32_t red[TILE / 64][kTileFields];
-    for (int x = 0; x < kTileFields - 1; ++x) {
-        for (int d = 32; d > 0; d >>= 1) v[x] += __shfl_xor(v[x], d, 64);
-        if (lane == 0) red[wave][x] = v[x];
+    uint64_t p0 = 0;
+    uint32_t p1 = 0;
+    if (bl) {
+        p0 = (uint64_t)v[TF_FIT] | (uint64_t)v[TF_ACTIVE] << 16 | (uint64_t)v[TF_B1] << 28 | (uint64_t)v[TF_B2] << 40 |
+             (uint64_t)v[TF_B3] << 52;
+        p1 = v[TF_B5] | v[TF_BX] << 16;
+        for (int d = 32; d > 0; d >>= 1) p0 += __shfl_xor(p0, d, 64);
+        if (__any(p1 != 0))
+            for (int d = 32; d > 0; d >>= 1) p1 += __shfl_xor(p1, d, 64);
+    }
+    if (lane == 0) {
+        red[wave][TF_FIT] = (uint32_t)p0 & 0xffffu;
+        red[wave][TF_ACTIVE] = (uint32_t)(p0 >> 16) & 0xfffu;
+        red[wave][TF_B1] = (uint32_t)(p0 >> 28) & 0xfffu;
+        red[wave][TF_B2] = (uint32_t)(p0 >> 40) & 0xfffu;
+        red[wave][TF_B3] = (uint32_t)(p0 >> 52);
+        red[wave][TF_B5] = p1 & 0xffffu;
+        red[wave][TF_BX] = p1 >> 16;
     }
     __syncthreads();
     if (threadIdx.x < kTileFields) {
@@ -832,19 +869,22 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     __shared__ uint32_t s_off[5 * TILE];                         // per-tet CSR offsets of the tile
     __shared__ uint32_t s_bits[5 * TILE / 32], s_pre[5 * TILE / 32];  // its rank blocks
     static_assert(5 * TILE % 32 == 0, "a tile holds whole rank blocks");
+    // the tile's active tets in order: index in the tile | k << 13 | the
+    // function (k = 1) << 20
+    __shared__ uint32_t s_act[5 * TILE];
+    static_assert(5 * TILE <= (1 << 13), "13 bits of the index in the tile");
     if (threadIdx.x < 5 * TILE / 32) s_bits[threadIdx.x] = 0;
     for (int i = threadIdx.x; i < 81; i += blockDim.x) tab[i] = A.k1[i];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t tile = blockIdx.x;
     const TileSums pre = tile_sums[tile];
-    const uint32_t ncubes = (uint32_t)(A.g.T / 5);
     const uint32_t cube = tile * TILE + threadIdx.x;
-    uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const MaskPair<T>* masks = static_cast<const MaskPair<T>*>(A.masks.p);
     M m[5] = {0, 0, 0, 0, 0};
-    bool even = true;
-    uint8_t pat[5] = {0, 0, 0, 0, 0};
-    if (cube < ncubes)
-        cube_masks<T, M>(A.g, cube, static_cast<const MaskPair<T>*>(A.masks.p), (M)A.full, c, m, even, pat);
+    // only the cubes that the count pass found an active tet in
+    const uint64_t busy = A.busy[tile * (TILE / 64) + wave];
+    if (busy >> lane & 1)
+        cube_masks<T, M>(A.g, cube, masks, (M)A.full, m);
     // per lane: active functions, active tets, and tets per bucket list
     // (k = 2, 3..4, 5..8), packed ks << 11 | as and 10 bits per bucket
     uint32_t ks = 0, as = 0, bp = 0;
@@ -857,10 +897,11 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     // bucket slots: the tile's prefix, the waves before this one, the lanes
     // before this one (a wave holds at most 320 tets of a list)
     uint32_t binc = bp;
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(binc, d, 64);
-        if (lane >= d) binc += o;
-    }
+    if (__any(bp != 0))
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(binc, d, 64);
+            if (lane >= d) binc += o;
+        }
     if (lane == 63) wbk[wave] = binc;
     // block exclusive scan of (ks, as) packed as ks << kAsBits | as (a tile
     // holds at most 5 TILE active tets and 64 times as many functions)
@@ -868,23 +909,23 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     static_assert(5 * TILE < (1 << kAsBits) && 5 * 64 * TILE < (1 << (32 - kAsBits)), "tile packing");
     const uint32_t packed = ks << kAsBits | as;
     uint32_t inc = packed;
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += o;
-    }
+    if (busy)
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += o;
+        }
     if (lane == 63) wsum[wave] = inc;
     __syncthreads();
     uint32_t ex = inc - packed;
     for (int w = 0; w < wave; ++w) ex += wsum[w];
     uint32_t o = pre.v[TF_FIT] + (ex >> kAsBits), r = pre.v[TF_ACTIVE] + (ex & ((1u << kAsBits) - 1u));
-    uint32_t bnext[3];
-    for (int qq = 0; qq < 3; ++qq) {
+    uint32_t bnext[3] = {0, 0, 0};
+    for (int qq = 0; qq < 3 && busy; ++qq) {
         uint32_t b = pre.v[TF_B2 + qq] + (((binc - bp) >> (10 * qq)) & 1023u);
         for (int w = 0; w < wave; ++w) b += (wbk[w] >> (10 * qq)) & 1023u;
         bnext[qq] = b;
     }
     for (int q = 0; q < 5; ++q) {
-        const uint64_t t = (uint64_t)cube * 5 + q;
         const M mq = m[q];
         const int k = __popcll(mq);
         const uint32_t local = 5 * threadIdx.x + q;
@@ -892,27 +933,18 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
         if ((local & 31u) == 0) s_pre[local >> 5] = r;
         if (k) {
             atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
-            if (r >= A.cap_active || o + (uint32_t)k > A.cap_fit) {
-                A.errs[lane] |= ERR_OVERFLOW;
-                A.ctr[C_ABORT] = 1;
-            } else {
-                A.act[r] = (uint32_t)t;
-                A.act_k[r] = (uint8_t)k;
-                A.act_off[r] = o;
+            s_act[r - pre.v[TF_ACTIVE]] =
+                local | (uint32_t)k << 13 | (uint32_t)(__ffsll((unsigned long long)mq) - 1) << 20;
+            // the few tets of more functions: their functions and list slots
+            if (k > 1 && r < A.cap_active && o + (uint32_t)k <= A.cap_fit) {
                 uint32_t oo = o;
                 for (M mm = mq; mm; mm &= mm - 1) A.fit[oo++] = (uint8_t)(__ffsll((unsigned long long)mm) - 1);
-                if (k == 1) {
-                    const K1Entry& E = tab[pat[q]];
-                    A.cnt[3 * r] = E.niv;
-                    A.cnt[3 * r + 1] = E.nif;
-                    A.cnt[3 * r + 2] = E.nfv;
-                    A.rec_loc[r] = K1_FLAG | (uint32_t)pat[q];
-                } else if (k <= A.kbig) {
+                if (k <= A.kbig) {
                     const int qq = k == 2 ? 0 : (k <= 4 ? 1 : 2);
                     const uint32_t slot = bnext[qq]++;
                     if (slot < A.cap[qq]) {
                         A.list[qq][slot] = r;
-                        A.lts[qq][slot] = (uint64_t)o << 32 | (uint32_t)t;
+                        A.lts[qq][slot] = (uint64_t)o << 32 | (cube * 5 + q);
                         A.rec_loc[r] = A.rec_base[qq] + slot * A.slot[qq];
                     } else {
                         A.errs[lane] |= ERR_OVERFLOW;
@@ -926,9 +958,41 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
         o += (uint32_t)k;
         r += k != 0;
     }
-    // the tile's per-tet CSR entries, coalesced
+    __shared__ uint32_t s_n;
+    if (threadIdx.x == TILE - 1) s_n = r - pre.v[TF_ACTIVE];
     __syncthreads();
+    // the active tets' rows, a lane each (they are few and far between in the
+    // loop above, where each store would carry a few lanes)
     const uint64_t t0 = (uint64_t)tile * (5 * TILE), NT = A.g.T;
+    for (uint32_t i = threadIdx.x; i < s_n; i += TILE) {
+        const uint32_t e = s_act[i], local = e & 0x1fffu, k = (e >> 13) & 127u, f = e >> 20;
+        const uint32_t off = s_off[local], row = pre.v[TF_ACTIVE] + i;
+        if (row >= A.cap_active || off + k > A.cap_fit) {
+            A.errs[lane] |= ERR_OVERFLOW;
+            A.ctr[C_ABORT] = 1;
+            continue;
+        }
+        A.act[row] = (uint32_t)t0 + local;
+        A.act_k[row] = (uint8_t)k;
+        A.act_off[row] = off;
+        if (k == 1) {
+            A.fit[off] = (uint8_t)f;
+            // the corner sign pattern: sum of s_c 3^c, s_c = 0 negative, 1 zero, 2 positive
+            uint32_t v[4], p = 0;
+            dev::regular_tet(A.g.res, t0 + local, v);
+#pragma unroll
+            for (int a = 3; a >= 0; --a) {
+                const MaskPair<T> x = masks[v[a]];
+                p = 3 * p + ((x.pos >> f & 1) ? 2u : ((x.neg >> f & 1) ? 0u : 1u));
+            }
+            const K1Entry& E = tab[p];
+            A.cnt[3 * row] = E.niv;
+            A.cnt[3 * row + 1] = E.nif;
+            A.cnt[3 * row + 2] = E.nfv;
+            A.rec_loc[row] = K1_FLAG | p;
+        }
+    }
+    // the tile's per-tet CSR entries, coalesced
     for (int i = threadIdx.x; i < 5 * TILE; i += TILE)
         if (t0 + i < NT) A.csr_off_w[t0 + i] = s_off[i];
     if (threadIdx.x < 5 * TILE / 32 && t0 + 32 * threadIdx.x < NT)
@@ -1793,6 +1857,7 @@ struct Workspace {
     DBuf<const double*> vals_at;  // the run's values, left by its signs pass for the captured kernels
     DBuf<uint8_t> masks;        // MaskPair by vertex
     DBuf<uint2> blocks;         // regular grids: rank blocks (RankOf)
+    DBuf<uint64_t> busy;        // regular grids: per 64 cubes, which hold an active tet
     DBuf<uint32_t> kcnt, isact, csr_off, rank, act, rec_loc, cnt, list[3];
     DBuf<uint64_t> lts[3];  // per bucket slot: CSR offset << 32 | tet
     DBuf<uint32_t> act_off;  // CSR offset of each active tet, by active rank
@@ -2000,6 +2065,7 @@ void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream
     W.masks.alloc(m, 2 * (size_t)mask_width(F) * V);
     if (g.view.regular) {
         W.blocks.alloc(m, T / 32 + 1);
+        W.busy.alloc(m, (size_t)cube_tiles(g, 1024) * 16);  // whole tiles, of every size
         W.tile_sums.alloc(m, cube_tiles(g, 256) + 1);  // the smallest tile has the most tiles
         for (int q = 1; q < 3; ++q) W.early[q].alloc(m, c.b[q] + 1);
     } else {
@@ -2130,7 +2196,7 @@ void stage_filter(Workspace& W, const Grid& g, const Values& val, hipStream_t s,
             auto count = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, g.view,
                                    reinterpret_cast<const MaskPair<M>*>(W.masks.p), full, kbig, W.tile_sums.p,
-                                   early3 ? W.early[1].p : nullptr, early5 ? W.early[2].p : nullptr, W.cap.b[1],
+                                   W.busy.p, early3 ? W.early[1].p : nullptr, early5 ? W.early[2].p : nullptr, W.cap.b[1],
                                    W.cap.b[2], W.ctr.p);
             };
             if (tile == 256)
@@ -2320,6 +2386,7 @@ void stage_fill(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
     A.cap_fit = W.cap.fit;
     A.csr_off_w = W.csr_off.p;
     A.blocks = W.blocks.p;
+    A.busy = W.busy.p;
     if (g.view.regular) {
         const int tile = W.cube_tile;
         const TileSums* ts = W.tile_sums.p;

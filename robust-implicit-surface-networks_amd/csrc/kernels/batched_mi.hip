@@ -114,9 +114,14 @@ __global__ void __launch_bounds__(kMiLanes) k_mi_count_tiles(GridView g, const d
 #pragma unroll
             for (int q = 0; q < 8; ++q) h[q] = hm[c[q]];
             const bool even = ((i + j + k) & 1u) == 0;
+            // both parities' tets with indices known here, then one select
+#pragma unroll
             for (int q = 0; q < 5; ++q) {
-                const uint8_t* t = even ? dev::kCubeTetEven[q] : dev::kCubeTetOdd[q];
-                put(5 * tid + q, h[t[0]] | h[t[1]] | h[t[2]] | h[t[3]]);
+                constexpr auto& E = dev::kCubeTetEven;
+                constexpr auto& O = dev::kCubeTetOdd;
+                const uint64_t e = h[E[q][0]] | h[E[q][1]] | h[E[q][2]] | h[E[q][3]];
+                const uint64_t o = h[O[q][0]] | h[O[q][1]] | h[O[q][2]] | h[O[q][3]];
+                put(5 * tid + q, even ? e : o);
             }
         }
     } else {

@@ -32,6 +32,20 @@ namespace dev {
 constexpr uint8_t kCubeTetEven[5][4] = {{4, 6, 1, 3}, {6, 3, 4, 7}, {1, 3, 0, 4}, {3, 1, 2, 6}, {4, 1, 6, 5}};
 constexpr uint8_t kCubeTetOdd[5][4] = {{7, 0, 2, 5}, {2, 3, 0, 7}, {5, 7, 0, 4}, {7, 2, 6, 5}, {0, 1, 2, 5}};
 
+// the same tables in one word each, 12 bits per tet: per corner its offset
+// bits di | dj << 1 | dk << 2.  A tet's corners are then shifts and masked
+// adds; an array of the cube's corners indexed by the byte tables costs a
+// chain of compares and selects per corner.
+constexpr uint64_t cube_tet_words(const uint8_t (&tab)[5][4]) {
+    uint64_t w = 0;
+    for (int q = 0; q < 5; ++q)
+        for (int a = 0; a < 4; ++a) {
+            const uint64_t c = tab[q][a], di = (c & 3) == 1 || (c & 3) == 2, dj = (c & 3) >= 2, dk = c >> 2;
+            w |= (di | dj << 1 | dk << 2) << (12 * q + 3 * a);
+        }
+    return w;
+}
+
 __host__ __device__ inline void regular_tet(int res, uint64_t t, uint32_t v[4]) {
     // 32-bit index arithmetic: a regular grid has fewer than 2^32 / 27
     // vertices, so its cube and vertex indices fit
@@ -40,9 +54,12 @@ __host__ __device__ inline void regular_tet(int res, uint64_t t, uint32_t v[4]) 
     const int q = (int)(t32 - cube * 5u);
     const uint32_t i = cube / (R * R), rem = cube - i * (R * R), j = rem / R, k = rem - j * R;
     const uint32_t b = i * N * N + j * N + k;
-    const uint32_t c[8] = {b, b + N * N, b + N * N + N, b + N, b + 1, b + N * N + 1, b + N * N + N + 1, b + N + 1};
-    const bool ev = ((i + j + k) & 1u) == 0;
-    for (int a = 0; a < 4; ++a) v[a] = c[ev ? kCubeTetEven[q][a] : kCubeTetOdd[q][a]];
+    constexpr uint64_t even = cube_tet_words(kCubeTetEven), odd = cube_tet_words(kCubeTetOdd);
+    const uint32_t w = (uint32_t)(((((i + j + k) & 1u) == 0) ? even : odd) >> (12 * q));
+    for (int a = 0; a < 4; ++a) {
+        const uint32_t o = w >> (3 * a);
+        v[a] = b + ((0u - (o & 1u)) & (N * N)) + ((0u - (o >> 1 & 1u)) & N) + (o >> 2 & 1u);
+    }
 }
 
 __host__ __device__ inline void tet_corners(const GridView& g, uint64_t t, uint32_t v[4]) {
