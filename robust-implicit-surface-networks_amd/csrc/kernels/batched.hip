@@ -30,7 +30,6 @@ namespace rin {
 
 namespace {
 
-using CK2 = dev::Caps<16, 24, 6, 6>;
 // CMed (k 3..4) and CBig (k 5..8) come from kernels_ia.h
 
 // words of a record slot: the largest record a bucket's capacity allows

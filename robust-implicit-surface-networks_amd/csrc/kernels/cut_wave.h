@@ -73,11 +73,11 @@ struct WaveIA {
     int nv, nf, nc, dup, err;
 };
 
-// Lane-group primitives: a group of G lanes (16, 32 or the whole 64-lane
+// Lane-group primitives: a group of G lanes (8, 16, 32 or the whole 64-lane
 // wavefront) works on one tet, so a wavefront can carry 64 / G tets.
 template <int G>
 struct Grp {
-    static_assert(G == 16 || G == 32 || G == 64, "group size");
+    static_assert(G == 8 || G == 16 || G == 32 || G == 64, "group size");
     __device__ static int lane() { return threadIdx.x & (G - 1); }
     __device__ static bool any(bool p) {
         const uint64_t b = __ballot(p);

@@ -12,6 +12,7 @@ namespace rin {
 namespace {
 
 using dev::Complex;
+using CK2 = dev::Caps<16, 24, 6, 6>;    // up to 2 active functions
 using CMed = dev::Caps<40, 64, 8, 8>;      // up to 4 active functions
 using CBig = dev::Caps<132, 284, 10, 12>;  // up to 8 active functions
 // more than 8 active functions (ties, coincident functions; many functions on
@@ -671,7 +672,7 @@ __device__ __forceinline__ void cut_group_role(GroupComplex<C, MI>* Xs, uint32_t
 }
 
 template <class C, int G, bool MI>
-__global__ void __launch_bounds__(64) k_cut_group(GridView g, ValsRef vref, const uint32_t* __restrict__ act,
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MI ? 1 : 3))) k_cut_group(GridView g, ValsRef vref, const uint32_t* __restrict__ act,
                                                   const uint8_t* __restrict__ act_k,
                                                   const uint32_t* __restrict__ csr_off,
                                                   const uint8_t* __restrict__ fit, const uint32_t* __restrict__ list,
@@ -809,7 +810,92 @@ __device__ inline bool ia_face_is_iso(const Rec& R, const uint16_t* F) {
     return false;
 }
 
-__global__ void k_extract_ia(GridView g, const uint32_t* __restrict__ act, const uint32_t* __restrict__ csr_off,
+// W: words of the tet's vertex mask.  One word (64 vertices, nearly every tet)
+// stays in registers; an array indexed by vertex lies in scratch memory, which
+// took a quarter of the pass, and a load per 16-bit word another part: 446000
+// tets, nearly all of one or two functions, 310 -> 216 us.  What is left is
+// the walk of a record by one lane.
+template <int W>
+__device__ inline void ia_extract_tet(const GridView& g, uint64_t a, uint32_t t, const Rec& R, uint32_t s0,
+                                      const uint8_t* __restrict__ fit, uint32_t vb, uint32_t q, uint32_t e,
+                                      uint64_t* __restrict__ okey, uint32_t* __restrict__ oa,
+                                      uint16_t* __restrict__ oj, uint32_t* __restrict__ fq_a,
+                                      uint16_t* __restrict__ fq_l, uint8_t* __restrict__ fq_fn,
+                                      uint8_t* __restrict__ fq_bnd, uint32_t* __restrict__ fq_vs,
+                                      uint32_t* __restrict__ fve) {
+    uint32_t v[4];
+    dev::tet_corners(g, t, v);
+    // four words of the record in one load (rows of four faces' fields, a
+    // vertex, up to four of a face's vertices; the buffer is padded for the
+    // words past the last record)
+    auto four = [](const uint16_t* p) {
+        uint64_t x;
+        __builtin_memcpy(&x, p, 8);
+        return x;
+    };
+    uint64_t iso[W];
+    for (int w = 0; w < W; ++w) iso[w] = 0;
+    const uint16_t* F = R.faces();
+    for (int f = 0; f < R.nf; ++f) {
+        const uint64_t h = four(F);
+        const int n = (int)(h >> 48);
+        if ((h & 0xffffu) > 3 || (R.dup && ia_face_is_iso(R, F)))
+            for (int i = 0; i < n; i += 4) {
+                uint64_t r = four(F + 4 + i);
+                for (int x = i; x < n && x < i + 4; ++x, r >>= 16)
+                    iso[W == 1 ? 0 : (r & 0xffffu) >> 6] |= 1ull << (r & 63);
+            }
+        F += 4 + n;
+    }
+    // vertex occurrences in local order
+    uint32_t o = vb;
+    for (int w = 0; w < W; ++w)
+        for (uint64_t b = iso[w]; b; b &= b - 1) {
+            const int j = 64 * w + __builtin_ctzll(b);
+            const uint64_t T3 = four(R.vert(j));
+            okey[o] = ia_vertex_key(g, t, v, a, j, (int)(T3 & 0xffffu), (int)(T3 >> 16 & 0xffffu),
+                                    (int)(T3 >> 32 & 0xffffu), fit, s0);
+            oa[o] = (uint32_t)a;
+            oj[o] = (uint16_t)j;
+            ++o;
+        }
+    // face occurrences in local order; vertex slots point at occurrences
+    F = R.faces();
+    for (int f = 0; f < R.nf; ++f) {
+        const uint64_t h = four(F);
+        const int n = (int)(h >> 48);
+        if ((h & 0xffffu) > 3 || (R.dup && ia_face_is_iso(R, F))) {
+            int sp = (int)(h & 0xffffu);
+            if (sp <= 3) {
+                // a tet face coinciding with implicit planes: the smallest of them
+                const uint16_t* grp = R.groups_ia();
+                for (int p = 4; p < R.L; ++p)
+                    if (grp[p] == grp[sp]) {
+                        sp = p;
+                        break;
+                    }
+            }
+            fq_a[q] = (uint32_t)a;
+            fq_l[q] = (uint16_t)f;
+            fq_fn[q] = fit[s0 + sp - 4];
+            fq_bnd[q] = (h >> 32 & 0xffffu) == 0xffffu ? (uint8_t)(1 + (h & 0xffffu)) : 0;
+            fq_vs[q] = e;
+            uint64_t r = 0;
+            for (int i = 0; i < n; ++i, r >>= 16) {
+                if ((i & 3) == 0) r = four(F + 4 + i);
+                const int j = (int)(r & 0xffffu);
+                uint32_t rank = 0;
+                for (int w = 0; w < W && W > 1; ++w) rank += w < (j >> 6) ? (uint32_t)__popcll(iso[w]) : 0u;
+                rank += (uint32_t)__popcll(iso[W == 1 ? 0 : j >> 6] & ((1ull << (j & 63)) - 1));
+                fve[e++] = vb + rank;
+            }
+            ++q;
+        }
+        F += 4 + n;
+    }
+}
+
+__global__ void __launch_bounds__(256) k_extract_ia(GridView g, const uint32_t* __restrict__ act, const uint32_t* __restrict__ csr_off,
                              const uint8_t* __restrict__ fit, Count n_active, const uint32_t* __restrict__ rec_loc,
                              const uint16_t* __restrict__ rec, const uint32_t* __restrict__ voff,
                              const uint32_t* __restrict__ foff, const uint32_t* __restrict__ fvoff,
@@ -817,66 +903,15 @@ __global__ void k_extract_ia(GridView g, const uint32_t* __restrict__ act, const
                              uint32_t* __restrict__ fq_a, uint16_t* __restrict__ fq_l, uint8_t* __restrict__ fq_fn,
                              uint8_t* __restrict__ fq_bnd, uint32_t* __restrict__ fq_vs, uint32_t* __restrict__ fve) {
     GRID_STRIDE(a, n_active) {
-        const uint32_t t = act[a];
         const Rec R(rec + rec_loc[a]);
         if (R.r[0] != 1) continue;
-        uint32_t v[4];
-        dev::tet_corners(g, t, v);
-        const uint32_t s0 = csr_off[t];
-        uint64_t iso[kMaskWords];
-        for (int w = 0; w < kMaskWords; ++w) iso[w] = 0;
-        const uint16_t* F = R.faces();
-        for (int f = 0; f < R.nf; ++f) {
-            const int n = F[3];
-            if (ia_face_is_iso(R, F))
-                for (int q = 0; q < n; ++q) iso[F[4 + q] >> 6] |= 1ull << (F[4 + q] & 63);
-            F += 4 + n;
-        }
-        // vertex occurrences in local order
-        uint32_t o = voff[a];
-        for (int j = 0; j < R.nv; ++j) {
-            if (!((iso[j >> 6] >> (j & 63)) & 1)) continue;
-            const uint16_t* T3 = R.vert(j);
-            const uint64_t key =
-                ia_vertex_key(g, t, v, a, j, T3[0], T3[1], T3[2], fit, s0);
-            okey[o] = key;
-            oa[o] = (uint32_t)a;
-            oj[o] = (uint16_t)j;
-            ++o;
-        }
-        // face occurrences in local order; vertex slots point at occurrences
-        uint32_t q = foff[a], e = fvoff[a];
-        const uint32_t vb = voff[a];
-        F = R.faces();
-        for (int f = 0; f < R.nf; ++f) {
-            const int n = F[3];
-            if (ia_face_is_iso(R, F)) {
-                int sp = F[0];
-                if (sp <= 3) {
-                    // a tet face coinciding with implicit planes: the smallest of them
-                    const uint16_t* grp = R.groups_ia();
-                    for (int p = 4; p < R.L; ++p)
-                        if (grp[p] == grp[sp]) {
-                            sp = p;
-                            break;
-                        }
-                }
-                fq_a[q] = (uint32_t)a;
-                fq_l[q] = (uint16_t)f;
-                fq_fn[q] = fit[s0 + sp - 4];
-                fq_bnd[q] = F[2] == 0xFFFF ? (uint8_t)(1 + F[0]) : 0;
-                fq_vs[q] = e;
-                for (int i = 0; i < n; ++i) {
-                    const int j = F[4 + i];
-                    uint32_t rank = 0;
-                    for (int w = 0; w < (j >> 6); ++w) rank += __popcll(iso[w]);
-                    rank += __popcll(iso[j >> 6] & ((1ull << (j & 63)) - 1));
-                    fve[e++] = vb + rank;
-                }
-                ++q;
-            }
-            F += 4 + n;
-        }
+        const uint32_t t = act[a], s0 = csr_off[t];
+        if (R.nv <= 64)
+            ia_extract_tet<1>(g, a, t, R, s0, fit, voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_fn, fq_bnd,
+                              fq_vs, fve);
+        else
+            ia_extract_tet<kMaskWords>(g, a, t, R, s0, fit, voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_fn,
+                                       fq_bnd, fq_vs, fve);
     }
 }
 
@@ -1590,8 +1625,8 @@ __global__ void __launch_bounds__(1024) k_dedup_tile_scan(Count n, uint32_t* __r
 }
 
 // Plain form: the active tets' cut lists by active-function count, built on
-// the device in active-rank order.  List 0: MI two-material table, 1: up to
-// 4 functions, 2: 5..8, 3: more.  Per chunk of kBucketChunk active tets,
+// the device in active-rank order.  List 0: MI table tets, IA tets of one and
+// two functions (by table, or by groups of 8 lanes), 1: up to 4 functions, 2: 5..8, 3: more.  Per chunk of kBucketChunk active tets,
 // kBucketWords words: list sizes [0..4), the reference's bucket histogram
 // [4..7) (IA: 1, 2, >= 3 functions; MI: 2, 3, >= 4), tets with 3..4 and
 // 5..8 functions [7], [8], the largest count [9] (k_bucket_count).  One
@@ -1601,9 +1636,9 @@ __global__ void __launch_bounds__(1024) k_dedup_tile_scan(Count n, uint32_t* __r
 constexpr uint32_t kBucketChunk = 2048;
 constexpr int kBucketWords = 10;
 
-// table2: the material-interface tables take two- and three-material tets
 // table2: 1 material interfaces (two and three materials by table), 2
-// implicit arrangements (one and two functions by table), 0 no tables
+// implicit arrangements (one and two functions), 0 material interfaces
+// without tables
 __device__ inline int bucket_of_k(int k, int table2) {
     const bool tab = (table2 == 1 && (k == 2 || k == 3)) || (table2 == 2 && k <= 2);
     return k > 8 ? 3 : (k > 4 ? 2 : (tab ? 0 : 1));

@@ -604,7 +604,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     // (the IA table kernel writes output counts, so the -R check's complex
     // counts take the general cut)
     const bool use_tables = !(flags & (RUN_REVERSE | RUN_NO_LOOKUP)) && (MI || !(flags & RUN_CUT_ONLY));
-    const int table_mode = use_tables ? (MI ? 1 : 2) : 0;
+    const int table_mode = MI ? (use_tables ? 1 : 0) : 2;
     DBuf<uint32_t> blists(mem, 4 * (NA + 1));
     uint32_t* blist[4];
     for (int q = 0; q < 4; ++q) blist[q] = blists.p + (uint64_t)q * (NA + 1);
@@ -642,13 +642,13 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         scan_u32(mem, b.p, out.rec_off.p, NA, out.rec_off.p + NA, s);
     }
     const uint64_t nwords = read1(out.rec_off.p + NA, s);
-    out.rec.alloc(mem, nwords + 1);
+    out.rec.alloc(mem, nwords + 4);  // k_extract_ia reads four words at a time
     DBuf<uint32_t> cnt(mem, 3 * NA + 3), labels(mem, MI ? NA + 1 : 1);
-    if (bcnt[0] && !MI) {
+    if (bcnt[0] && !MI && use_tables) {
         table_cut_plain(g.view, (const double*)val.vals.p, (const uint32_t*)out.act.p, (const uint8_t*)out.act_k.p,
                         (const uint32_t*)out.csr_off.p, (const uint8_t*)out.fit.p, (const uint32_t*)blist[0],
                         (uint64_t)bcnt[0], (const uint32_t*)out.rec_off.p, out.rec.p, cnt.p, errs.p, s);
-    } else if (bcnt[0]) {
+    } else if (bcnt[0] && MI) {
         // two- and three-material tets by table
         const MITablesDev TT = mi_tables_dev(s);
         hipLaunchKernelGGL(k_mi_table, dim3(nblk(bcnt[0])), dim3(256), 0, s, g.view,
@@ -681,7 +681,12 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     // list 3 (more than 8 functions) by a wavefront a tet as well: a lane a
     // tet took 6 to 45 ms for some hundred tets of 9..13 functions (33^3
     // vertices, 32 functions), this takes 0.2 ms
-    for (int q = 2; q >= 0 && NA; --q) {
+    // list 0 without the tables (lookups off, the -R check; implicit
+    // arrangements only): groups of 8 lanes with the smallest complex.  A cut
+    // of one or two planes is a chain of short steps that 16 lanes do not fill,
+    // so tets in flight count: 446000 of them in groups of 16 with room for
+    // four functions took 1077 us, this takes 584 us
+    for (int q = 2; q >= (use_tables ? 0 : -1) && NA; --q) {
         const uint64_t nl = bcnt[1 + q];
         if (!nl) continue;
         auto go = [&](auto kernel, int per_wave, auto snap) {
@@ -692,7 +697,9 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
                                (const uint32_t*)blist[1 + q], Count(nl), (const uint32_t*)out.rec_off.p, out.rec.p,
                                cnt.p, errs.p, 1, flags, labels.p, snap);
         };
-        if (q == 0)
+        if (q < 0)
+            go(k_cut_group<CK2, 8, false>, 8, k2s);
+        else if (q == 0)
             MI ? go(k_cut_group<CMed, 64, true>, 1, m3s) : go(k_cut_group<CMed, 16, false>, 4, k2s);
         else if (q == 1)
             MI ? go(k_cut_group<CBig, 64, true>, 1, m3s) : go(k_cut_group<CBig, 64, false>, 1, k2s);
@@ -742,7 +749,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         constexpr uint32_t slot = 8 + 4 * CHuge::MV + CHuge::MF * (4 + CHuge::MFV) + 2 * CHuge::MP;
         const uint64_t total = nwords + (uint64_t)slot * retry.size();
         if (total >= (1ull << 31)) throw std::runtime_error("record buffer exceeds 2^31 words");
-        DBuf<uint16_t> rec2(mem, total + 1);
+        DBuf<uint16_t> rec2(mem, total + 4);
         RIN_HIP(hipMemcpyAsync(rec2.p, out.rec.p, 2 * nwords, hipMemcpyDeviceToDevice, s));
         for (size_t i = 0; i < retry.size(); ++i) hl[retry[i]] = (uint32_t)(nwords + slot * i);
         RIN_HIP(hipMemcpyAsync(out.rec_loc.p, hl.data(), 4 * NA, hipMemcpyHostToDevice, s));
