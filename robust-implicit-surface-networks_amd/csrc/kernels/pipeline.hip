@@ -35,6 +35,27 @@ T read1(const T* d, hipStream_t s) {
     return h;
 }
 
+struct Words {
+    const uint32_t* p[3];
+};
+
+__global__ void k_gather(Words w, uint32_t* __restrict__ out) {
+    if (threadIdx.x < 3) out[threadIdx.x] = *w.p[threadIdx.x];
+}
+
+// three words from three places in one read-back (each one waits for the
+// queue and costs about 48 us with the gap that it leaves behind it)
+struct Read3 {
+    uint32_t v[3];
+    Read3(DevMem& mem, const uint32_t* a, const uint32_t* b, const uint32_t* c, hipStream_t s) {
+        DBuf<uint32_t> d(mem, 3);
+        hipLaunchKernelGGL(k_gather, dim3(1), dim3(64), 0, s, Words{{a, b, c}}, d.p);
+        RIN_HIP(hipGetLastError());
+        RIN_HIP(hipMemcpyAsync(v, d.p, sizeof(v), hipMemcpyDeviceToHost, s));
+        RIN_HIP(hipStreamSynchronize(s));
+    }
+};
+
 struct Timer {
     hipStream_t s;
     std::vector<std::pair<std::string, hipEvent_t>> ev;
@@ -329,7 +350,8 @@ void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, DBuf
     scan_u32(mem, cv.p, cv.p, NA, cv.p + NA, s);
     scan_u32(mem, cf.p, cf.p, NA, cf.p + NA, s);
     scan_u32(mem, cfv.p, cfv.p, NA, cfv.p + NA, s);
-    const uint64_t NVO = read1(cv.p + NA, s), NF = read1(cf.p + NA, s), NFV = read1(cfv.p + NA, s);
+    const Read3 tot(mem, cv.p + NA, cf.p + NA, cfv.p + NA, s);
+    const uint64_t NVO = tot.v[0], NF = tot.v[1], NFV = tot.v[2];
     out.n_vert_occ = NVO;
     out.n_face_occ = NF;
     out.n_face_occ_verts = NFV;
@@ -572,15 +594,14 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
                            (const uint64_t*)hm.p, amask.p, kcnt.p, isact.p);
     }
     RIN_HIP(hipGetLastError());
-    {
-        DBuf<uint32_t> vsum(mem, 1);
-        scan_u32(mem, vflag.p, vflag.p, V, vsum.p, s);
-        out.num_degenerate = read1(vsum.p, s);  // IA: zero entries; MI: tied vertices
-    }
+    DBuf<uint32_t> vsum(mem, 1);
+    scan_u32(mem, vflag.p, vflag.p, V, vsum.p, s);
     scan_u32(mem, kcnt.p, out.csr_off.p, T, out.csr_off.p + T, s);
     scan_u32(mem, isact.p, out.rank_of_tet.p, T, tot.p, s);
-    out.n_fit = read1(out.csr_off.p + T, s);
-    out.n_active = read1(tot.p, s);
+    const Read3 sizes(mem, vsum.p, out.csr_off.p + T, tot.p, s);
+    out.num_degenerate = sizes.v[0];  // IA: zero entries; MI: tied vertices
+    out.n_fit = sizes.v[1];
+    out.n_active = sizes.v[2];
     out.num_intersecting = out.n_active;
     const uint64_t NA = out.n_active;
     out.fit.alloc(mem, out.n_fit + 1);
@@ -608,8 +629,16 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     DBuf<uint32_t> blists(mem, 4 * (NA + 1));
     uint32_t* blist[4];
     for (int q = 0; q < 4; ++q) blist[q] = blists.p + (uint64_t)q * (NA + 1);
-    uint32_t bcnt[4] = {0, 0, 0, 0};  // list sizes: two-material table, up to 4, 5..8, more
+    uint32_t bcnt[4] = {0, 0, 0, 0};  // list sizes: one and two functions (MI: by table), up to 4, 5..8, more
+    uint64_t nwords = 0;
+    out.rec_off.alloc(mem, NA + 1);
     if (NA) {
+        {
+            DBuf<uint32_t> b(mem, NA + 1);
+            hipLaunchKernelGGL(k_rec_bound, dim3(nblk(NA)), dim3(256), 0, s, NA, (const uint8_t*)out.act_k.p, (int)MI,
+                               b.p);
+            scan_u32(mem, b.p, out.rec_off.p, NA, out.rec_off.p + NA, s);
+        }
         const uint32_t nch = (uint32_t)((NA + kBucketChunk - 1) / kBucketChunk);
         DBuf<uint32_t> bc(mem, (uint64_t)kBucketWords * nch + kBucketWords), bo(mem, 16);
         hipLaunchKernelGGL(k_bucket_count, dim3(nch), dim3(256), 0, s, Count(NA), (const uint8_t*)out.act_k.p, (int)MI,
@@ -617,12 +646,14 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, s, nch, bc.p, bo.p);
         hipLaunchKernelGGL(k_bucket_fill, dim3(nch), dim3(256), 0, s, Count(NA), (const uint8_t*)out.act_k.p, table_mode,
                            (const uint32_t*)bc.p, blist[0], blist[1], blist[2], blist[3]);
+        copy_u32(bo.p + 15, out.rec_off.p + NA, Count(1), s);
         RIN_HIP(hipGetLastError());
         uint32_t hb[16];
         RIN_HIP(hipMemcpyAsync(hb, bo.p, sizeof(hb), hipMemcpyDeviceToHost, s));
         RIN_HIP(hipStreamSynchronize(s));
         for (int q = 0; q < 4; ++q) bcnt[q] = hb[q];
         for (int q = 0; q < 3; ++q) out.nb[q] = hb[4 + q];
+        nwords = hb[15];
         out.n_cut34 = hb[7];
         out.n_cut58 = hb[8];
         if ((int)hb[9] > kMaxHuge) {
@@ -631,17 +662,11 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
                                      " active functions; the device cut supports at most " +
                                      std::to_string(kMaxHuge));
         }
+    } else {
+        fill_u32(out.rec_off.p, 0, 1, s);
     }
 
     // ---- per-tet cut
-    out.rec_off.alloc(mem, NA + 1);
-    {
-        DBuf<uint32_t> b(mem, NA + 1);
-        hipLaunchKernelGGL(k_rec_bound, dim3(nblk(NA)), dim3(256), 0, s, NA, (const uint8_t*)out.act_k.p, (int)MI,
-                           b.p);
-        scan_u32(mem, b.p, out.rec_off.p, NA, out.rec_off.p + NA, s);
-    }
-    const uint64_t nwords = read1(out.rec_off.p + NA, s);
     out.rec.alloc(mem, nwords + 4);  // k_extract_ia reads four words at a time
     DBuf<uint32_t> cnt(mem, 3 * NA + 3), labels(mem, MI ? NA + 1 : 1);
     if (bcnt[0] && !MI && use_tables) {
@@ -789,7 +814,8 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
     scan_u32(mem, cv.p, cv.p, NA, cv.p + NA, s);
     scan_u32(mem, cf.p, cf.p, NA, cf.p + NA, s);
     scan_u32(mem, cfv.p, cfv.p, NA, cfv.p + NA, s);
-    const uint64_t NVO = read1(cv.p + NA, s), NFO = read1(cf.p + NA, s), NFV = read1(cfv.p + NA, s);
+    const Read3 occ(mem, cv.p + NA, cf.p + NA, cfv.p + NA, s);
+    const uint64_t NVO = occ.v[0], NFO = occ.v[1], NFV = occ.v[2];
     out.n_vert_occ = NVO;
     out.n_face_occ = NFO;
     out.n_face_occ_verts = NFV;
