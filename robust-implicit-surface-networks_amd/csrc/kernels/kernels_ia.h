@@ -1006,10 +1006,10 @@ __global__ void k_edge_fill(Count n, const uint32_t* __restrict__ sidx, const ui
 // two occurrences), seeded at its smallest face and listed in breadth-first
 // order (queue order, neighbours in edge order).  Components come from
 // union-find (a root hooks under the smaller root, so each component's root
-// is its smallest face); the breadth-first order from level-synchronous
-// expansion where each newly reached face keeps the smallest (position of
-// its parent in the frontier, edge index) that reaches it, exactly the queue
-// order of one search per patch.
+// is its smallest face); the breadth-first order from one workgroup per
+// patch (k_patch_walk), level by level: each newly reached face keeps the
+// smallest (position of its parent in the frontier, edge index) that reaches
+// it, exactly the queue order of one search per patch.
 
 // the face across face corner position o's edge, or ~0u when the edge is
 // not manifold
