@@ -2055,9 +2055,15 @@ unsigned cube_tiles(const Grid& g, int tile = kCubeTile) {
     return (unsigned)std::max<uint64_t>(1, (cubes + tile - 1) / tile);
 }
 
+// W.cap says what the buffers hold: it is empty from the first change to them
+// until the last has its size, so a growth that fails midway (no memory) leaves
+// a workspace that the next run allocates anew
 void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream_t s) {
-    W.cap = c;
     W.slot[2] = W.wide ? rec_words<CWide>() : rec_words<CBig>();
+    uint64_t words = 0;
+    for (int q = 0; q < 3; ++q) words += (uint64_t)c.b[q] * W.slot[q];
+    if (words >= record_limit(1ull << 31)) throw std::runtime_error("record workspace exceeds capacity");
+    W.cap = Caps_{};
     DevMem& m = W.mem;
     const uint64_t V = g.view.V, T = g.view.T;
     W.vals_at.alloc(m, 1);
@@ -2079,14 +2085,13 @@ void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream
     W.rec_loc.alloc(m, c.active + 1);
     W.cnt.alloc(m, 3 * (uint64_t)c.active + 3);
     W.fit.alloc(m, c.fit + 1);
-    uint64_t words = 0;
+    words = 0;
     for (int q = 0; q < 3; ++q) {
         W.list[q].alloc(m, c.b[q] + 1);
         W.lts[q].alloc(m, c.b[q] + 1);
         W.rec_base[q] = (uint32_t)words;
         words += (uint64_t)c.b[q] * W.slot[q];
     }
-    if (words >= (1ull << 31)) throw std::runtime_error("record workspace exceeds capacity");
     W.rec.alloc(m, words + 1);
     W.cv.alloc(m, c.active + 1);
     W.cf.alloc(m, c.active + 1);
@@ -2165,6 +2170,7 @@ void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream
     // legacy stream, which another thread's graph capture forbids); `off`
     // lives until they are done
     RIN_HIP(hipStreamSynchronize(s));
+    W.cap = c;
 }
 
 // stage 1 (also run eagerly to size the workspace): signs, filter, and
@@ -2852,7 +2858,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         if (!w.exec) {
             w.ctr_clear = false;  // the eager passes below use the counters
             // size the workspace from an eager counting pass
-            if (!w.ctr.p) {
+            if (!w.cap.active) {
                 Caps_ tiny;
                 tiny.active = tiny.fit = 64;
                 for (int q = 0; q < 3; ++q) tiny.b[q] = 64;

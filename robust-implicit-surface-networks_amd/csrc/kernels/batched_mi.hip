@@ -534,12 +534,18 @@ std::shared_ptr<void> make_mi_plan_cache() { return std::make_shared<MIPlanCache
 
 namespace {
 
+// W.cap says what the buffers hold: it is empty from the first change to them
+// until the last has its size, so a growth that fails midway (no memory) leaves
+// a workspace that the next run allocates anew
 void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     DevMem& m = W.mem;
     W.drop_graph();
     const uint64_t V = g.view.V, T = g.view.T;
-    W.cap = c;
-    if (!W.hm.p) {
+    const MITablesRaw TR = mi_tables_device(s);
+    if ((uint64_t)c.words + 1 + TR.n_w2 + TR.n_w3 >= record_limit(1ull << 32))
+        throw std::runtime_error("material-interface record words exceed 32-bit offsets");
+    W.cap = MICaps{};
+    if (!W.errs.p) {
         W.hm.alloc(m, V);
         W.amask.alloc(m, T);
         W.vals_at.alloc(m, 1);
@@ -558,9 +564,6 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     W.rec_loc.alloc(m, A + 2);
     {
         // the slots, then the two tables' record words (copied once per allocation)
-        const MITablesRaw TR = mi_tables_device(s);
-        if ((uint64_t)c.words + 1 + TR.n_w2 + TR.n_w3 >= (1ull << 32))
-            throw std::runtime_error("material-interface record words exceed 32-bit offsets");
         W.tab_base2 = (uint32_t)c.words + 1;
         W.tab_base3 = W.tab_base2 + (uint32_t)TR.n_w2;
         W.rec.alloc(m, (uint64_t)W.tab_base3 + TR.n_w3 + 1);
@@ -619,6 +622,7 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
                               hipHostMallocMapped | hipHostMallocCoherent));
         RIN_HIP(hipHostGetDevicePointer((void**)&W.pub_d, W.pub_h, 0));
     }
+    W.cap = c;
 }
 
 // the whole path on stream s; every launch is sized by capacities and reads
@@ -832,7 +836,7 @@ void run_batched_mi(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t 
     uint32_t pub[kMiPub + 1];
     bool ok = false;
     for (int attempt = 0; attempt < 8 && !ok; ++attempt) {
-        if (!w.ctr.p) {
+        if (!w.cap.active) {
             MICaps c0;
             c0.active = (uint32_t)std::min<uint64_t>(T, 1024 + T / 16);
             c0.fit = 3 * c0.active;

@@ -3,7 +3,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstdlib>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -140,6 +142,13 @@ void values_upload(DevMem& mem, const Grid& g, const double* rowmajor, uint32_t 
 void eval_points(DevMem& mem, const double* pts, uint64_t n, const FuncDesc* funcs, uint32_t F, double* rowmajor,
                  hipStream_t s);
 void run_pipeline(DevMem& mem, const Grid& g, const Values& v, uint32_t flags, RunOut& out, hipStream_t s);
+
+// record words that a run may take: `most`, or fewer where RIN_RECORD_WORDS
+// says so (small inputs then reach the limit)
+inline uint64_t record_limit(uint64_t most) {
+    const char* e = std::getenv("RIN_RECORD_WORDS");
+    return e ? std::min<uint64_t>(most, std::strtoull(e, nullptr, 10)) : most;
+}
 
 // thrown by the batched form when a tet needs more than its buckets hold
 // (more than 8 active functions, or a complex beyond the bucket capacities);
