@@ -55,7 +55,8 @@ __host__ __device__ inline uint32_t spread_at(int counter, uint32_t slot) {
 }
 enum Ctr : int {
     C_ACTIVE = 0, C_FIT, C_VO, C_FO, C_FV, C_VERTS, C_FACES, C_FACEVERTS, C_B1, C_B2, C_B3, C_B5, C_BX, C_DEGEN,
-    C_Q2, C_Q3, C_Q5, C_ABORT, C_TETFACES, C_RECW, C_CUTK3, C_CUTW3, C_CUTK5, C_CUTW5, C_E3, C_E5, C_E3B, C_N
+    C_Q2, C_Q3, C_Q5, C_QX, C_ABORT, C_TETFACES, C_RECW, C_CUTK3, C_CUTW3, C_CUTK5, C_CUTW5, C_E3, C_E5, C_E3B, C_EX,
+    C_N
 };
 
 struct K1Entry {
@@ -361,8 +362,6 @@ const K2Plans& k2_plans() {
     return P;
 }
 
-// kbig: the most functions the last bucket takes (8, or kMaxHuge once a value
-// set has shown tets of more)
 // Sign masks of a vertex (bit j: function j), positive and negative side by
 // side, in the narrowest words that hold F bits: the count and fill passes
 // read eight vertices a cube, so they move a quarter of the bytes at 8
@@ -419,13 +418,14 @@ struct MaskRef {
     }
 };
 
-__device__ inline int bucket_of(int k, int kbig) {
-    return k <= 1 ? 0 : (k == 2 ? 1 : (k <= 4 ? 2 : (k <= kbig ? 3 : 4)));
+// the buckets: 1, 2, 3..4, 5..8, 9..kMaxHuge functions (5: more than the device cut takes)
+__device__ inline int bucket_of(int k) {
+    return k <= 1 ? 0 : (k == 2 ? 1 : (k <= 4 ? 2 : (k <= 8 ? 3 : (k <= kMaxHuge ? 4 : 5))));
 }
 
 // per tet: active count and bucket histogram
-__global__ void k_filter_count(GridView g, MaskRef masks, uint64_t full, int kbig, uint32_t* __restrict__ kcnt, uint32_t* __restrict__ isact,
-                               uint32_t* __restrict__ ctr) {
+__global__ void k_filter_count(GridView g, MaskRef masks, uint64_t full, uint32_t* __restrict__ kcnt,
+                               uint32_t* __restrict__ isact, uint32_t* __restrict__ ctr) {
     __shared__ uint32_t hist[8];
     if (threadIdx.x < 8) hist[threadIdx.x] = 0;
     __syncthreads();
@@ -436,8 +436,7 @@ __global__ void k_filter_count(GridView g, MaskRef masks, uint64_t full, int kbi
         const uint32_t k = (uint32_t)__popcll(m);
         kcnt[t] = k;
         isact[t] = k != 0;
-        if (k) atomicAdd(&hist[bucket_of((int)k, kbig)], 1u);
-        if (k > 8 && k <= (uint32_t)kbig) atomicAdd(&hist[4], 1u);  // the last field counts every tet of more than 8
+        if (k) atomicAdd(&hist[bucket_of((int)k)], 1u);
     }
     __syncthreads();
     if (threadIdx.x < 5 && hist[threadIdx.x]) atomicAdd(&ctr[C_B1 + threadIdx.x], hist[threadIdx.x]);
@@ -456,12 +455,11 @@ struct FillArgs {
     uint32_t* act_off;  // CSR offset by active rank
     uint8_t* act_k;
     const K1Entry* k1;
-    int kbig;
-    uint32_t* list[3];      // buckets k=2, 3..4, 5..kbig
-    uint64_t* lts[3];       // per slot: CSR offset << 32 | tet
-    uint32_t cap[3];
-    uint32_t rec_base[3];   // word offsets of each bucket's slots
-    uint32_t slot[3];       // words per slot
+    uint32_t* list[4];      // buckets k=2, 3..4, 5..8, 9..kMaxHuge
+    uint64_t* lts[4];       // per slot: CSR offset << 32 | tet
+    uint32_t cap[4];
+    uint32_t rec_base[4];   // word offsets of each bucket's slots
+    uint32_t slot[4];       // words per slot
     uint32_t* ctr;
     uint32_t* errs;
     uint32_t cap_active, cap_fit;
@@ -513,13 +511,13 @@ __global__ void k_fill_batched(FillArgs A) {
                     A.cnt[3 * r + 2] = E.nfv;
                     A.rec_loc[r] = K1_FLAG | (uint32_t)pat;
                 } else {
-                    b = k == 2 ? 0 : (k <= 4 ? 1 : (k <= A.kbig ? 2 : -1));
+                    b = k <= kMaxHuge ? bucket_of(k) - 1 : -1;
                     if (b < 0) A.errs[lane] |= 1;  // more active functions than the device cut supports
                 }
             }
         }
         // wave-aggregated appends to the bucket lists
-        for (int q = 0; q < 3; ++q) {
+        for (int q = 0; q < 4; ++q) {
             const uint64_t mask = __ballot(b == q);
             if (!mask) continue;
             const int leader = __ffsll((unsigned long long)mask) - 1;
@@ -642,9 +640,9 @@ __device__ inline void cube_masks(const GridView& g, uint32_t cube, const MaskPa
 }
 
 // Per tile of cubes: active functions, active tets and tets per bucket
-// (k = 1, 2, 3..4, 5..kbig; and every tet with k > 8).  No atomics: the tile scan below turns the
-// tile sums into prefixes (the CSR offsets and the bucket-list slots of each
-// tile) and writes the totals, so the bucket lists come out in tet order.
+// (k = 1, 2, 3..4, 5..8, 9..kMaxHuge).  No atomics: the tile scan below turns
+// the tile sums into prefixes (the CSR offsets and the bucket-list slots of
+// each tile) and writes the totals, so the bucket lists come out in tet order.
 constexpr int kTileFields = 8;
 enum TileField { TF_FIT = 0, TF_ACTIVE, TF_B1, TF_B2, TF_B3, TF_B5, TF_BX };
 struct TileSums {
@@ -661,18 +659,18 @@ struct EarlyEntry {
     uint32_t lrb;  // active tets before it | tets of its bucket list before it << 16
 };
 
-// early3, early5 (nullable): lists of the k = 3..4 and 5..8 tets, at most
-// early_cap3 / early_cap5 entries, counted in ctr[C_E3] / ctr[C_E5] (zero at
-// the start of a run).  The k = 3..4 list holds the k = 4 tets from its front
+// early3, early5, earlyx (nullable): lists of the k = 3..4, 5..8 and 9.. tets,
+// at most early_cap3 / early_cap5 / early_capx entries, counted in ctr[C_E3],
+// ctr[C_E5] and ctr[C_EX] (zero at the start of a run).  The k = 3..4 list holds the k = 4 tets from its front
 // (ctr[C_E3] of them) and the k = 3 tets from its back (ctr[C_E3B]), so that a
 // wavefront of the cut mostly holds tets of one k (two insertions past the
 // two-plane start, or one) and the longer ones start first.  A tile's entries
 // are contiguous and in tet order (the back part reversed).
 template <int TILE, class T>
 __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<T>* __restrict__ masks, uint64_t full,
-                                                     int kbig, TileSums* __restrict__ tile_sums,
-                                                     uint64_t* __restrict__ busy, EarlyEntry* early3,
-                                                     EarlyEntry* early5, uint32_t early_cap3, uint32_t early_cap5,
+                                                     TileSums* __restrict__ tile_sums, uint64_t* __restrict__ busy,
+                                                     EarlyEntry* early3, EarlyEntry* early5, EarlyEntry* earlyx,
+                                                     uint32_t early_cap3, uint32_t early_cap5, uint32_t early_capx,
                                                      uint32_t* ctr) {
     using M = typename std::conditional<sizeof(T) == 8, uint64_t, uint32_t>::type;
     const uint32_t ncubes = (uint32_t)(g.T / 5);
@@ -691,8 +689,8 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
             v[TF_B1] += k == 1;
             v[TF_B2] += k == 2;
             v[TF_B3] += k == 3 || k == 4;
-            v[TF_B5] += k >= 5 && k <= kbig;
-            v[TF_BX] += k > 8;
+            v[TF_B5] += k >= 5 && k <= 8;
+            v[TF_BX] += k > 8 && k <= kMaxHuge;
             n4 += k == 4;
         }
     }
@@ -701,13 +699,13 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
     if (lane == 0) busy[cube >> 6] = bl;
     // tiles holding listed tets rank them inside the tile: exclusive scans of
     // (active functions, active tets) packed as in the fill pass, and of the
-    // listed counts in 16-bit fields (k = 4 | k = 3 << 16 | k = 5..8 << 32;
-    // a tile holds at most 5 TILE tets); one atomic add per list part and
-    // tile reserves the tile's entries
+    // listed counts in 16-bit fields (k = 4 | k = 3 << 16 | k = 5..8 << 32 |
+    // k = 9.. << 48; a tile holds at most 5 TILE tets); one atomic add per list
+    // part and tile reserves the tile's entries
     const uint64_t want = (early3 ? (uint64_t)n4 | (uint64_t)(v[TF_B3] - n4) << 16 : 0ull) |
-                          (early5 ? (uint64_t)v[TF_B5] << 32 : 0ull);
+                          (early5 ? (uint64_t)v[TF_B5] << 32 : 0ull) | (earlyx ? (uint64_t)v[TF_BX] << 48 : 0ull);
     if ((early3 || early5) && __syncthreads_or(want != 0)) {
-        __shared__ uint32_t esum[TILE / 64], ebase[3];
+        __shared__ uint32_t esum[TILE / 64], ebase[4];
         __shared__ uint64_t ebk[TILE / 64];
         constexpr int kAsBits = 13;
         const uint32_t packed = v[TF_FIT] << kAsBits | v[TF_ACTIVE];
@@ -730,10 +728,11 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
             uint64_t tot = 0;
             for (int w = 0; w < TILE / 64; ++w) tot += ebk[w];
             const uint32_t t4 = (uint32_t)tot & 0xffffu, t3 = (uint32_t)(tot >> 16) & 0xffffu,
-                           t5 = (uint32_t)(tot >> 32);
+                           t5 = (uint32_t)(tot >> 32) & 0xffffu, tx = (uint32_t)(tot >> 48);
             ebase[0] = t4 ? atomicAdd(ctr + C_E3, t4) : 0u;
             ebase[1] = t5 ? atomicAdd(ctr + C_E5, t5) : 0u;
             ebase[2] = t3 ? atomicAdd(ctr + C_E3B, t3) : 0u;
+            ebase[3] = tx ? atomicAdd(ctr + C_EX, tx) : 0u;
         }
         uint32_t ex = inc - packed;
         uint64_t bx = binc - want;
@@ -743,8 +742,9 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
         }
         __syncthreads();
         uint32_t lo = ex >> kAsBits, lr = ex & ((1u << kAsBits) - 1u);
-        // the tile's k = 4, k = 3 and k = 5..8 tets before this one
-        uint32_t b4 = (uint32_t)bx & 0xffffu, b3 = (uint32_t)(bx >> 16) & 0xffffu, b5 = (uint32_t)(bx >> 32);
+        // the tile's k = 4, k = 3, k = 5..8 and k = 9.. tets before this one
+        uint32_t b4 = (uint32_t)bx & 0xffffu, b3 = (uint32_t)(bx >> 16) & 0xffffu,
+                 b5 = (uint32_t)(bx >> 32) & 0xffffu, b9 = (uint32_t)(bx >> 48);
         for (int q = 0; q < 5; ++q) {
             const int k = __popcll(m[q]);
             const uint32_t t = cube * 5u + (uint32_t)q;
@@ -757,10 +757,14 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
                     const uint32_t back = ebase[2] + b3++;
                     if (back < early_cap3) early3[early_cap3 - 1 - back] = {t, tile, lo, lr | rank << 16};
                 }
-            } else if (k >= 5 && k <= kbig && early5) {
+            } else if (k >= 5 && k <= 8 && early5) {
                 const uint32_t at = ebase[1] + b5;
                 if (at < early_cap5) early5[at] = {t, tile, lo, lr | b5 << 16};
                 ++b5;
+            } else if (k > 8 && k <= kMaxHuge && earlyx) {
+                const uint32_t at = ebase[3] + b9;
+                if (at < early_capx) earlyx[at] = {t, tile, lo, lr | b9 << 16};
+                ++b9;
             }
             lo += (uint32_t)k;
             lr += k != 0;
@@ -855,6 +859,7 @@ __global__ void __launch_bounds__(kTileScanThreads) k_tile_scan(TileSums* __rest
         ctr[C_Q2] = carry[TF_B2];
         ctr[C_Q3] = carry[TF_B3];
         ctr[C_Q5] = carry[TF_B5];
+        ctr[C_QX] = carry[TF_BX];
     }
 }
 
@@ -865,6 +870,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     __shared__ K1Entry tab[81];
     __shared__ uint32_t wsum[TILE / 64];
     __shared__ uint32_t wbk[TILE / 64];  // per-wave bucket counts, 10 bits per list
+    __shared__ uint32_t wbx[TILE / 64];  // the same of the last list
     __shared__ uint32_t s_off[5 * TILE];                         // per-tet CSR offsets of the tile
     __shared__ uint32_t s_bits[5 * TILE / 32], s_pre[5 * TILE / 32];  // its rank blocks
     static_assert(5 * TILE % 32 == 0, "a tile holds whole rank blocks");
@@ -885,13 +891,14 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     if (busy >> lane & 1)
         cube_masks<T, M>(A.g, cube, masks, (M)A.full, m);
     // per lane: active functions, active tets, and tets per bucket list
-    // (k = 2, 3..4, 5..8), packed ks << 11 | as and 10 bits per bucket
-    uint32_t ks = 0, as = 0, bp = 0;
+    // (k = 2, 3..4, 5..8: 10 bits per bucket; bx: k = 9..)
+    uint32_t ks = 0, as = 0, bp = 0, bx = 0;
     for (int q = 0; q < 5; ++q) {
         const int k = __popcll(m[q]);
         ks += (uint32_t)k;
         as += k != 0;
-        if (k >= 2 && k <= A.kbig) bp += 1u << (10 * (k == 2 ? 0 : (k <= 4 ? 1 : 2)));
+        if (k >= 2 && k <= 8) bp += 1u << (10 * (k == 2 ? 0 : (k <= 4 ? 1 : 2)));
+        bx += k > 8 && k <= kMaxHuge;
     }
     // bucket slots: the tile's prefix, the waves before this one, the lanes
     // before this one (a wave holds at most 320 tets of a list)
@@ -901,7 +908,16 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
             const uint32_t o = __shfl_up(binc, d, 64);
             if (lane >= d) binc += o;
         }
-    if (lane == 63) wbk[wave] = binc;
+    uint32_t xinc = bx;
+    if (__any(bx != 0))
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(xinc, d, 64);
+            if (lane >= d) xinc += o;
+        }
+    if (lane == 63) {
+        wbk[wave] = binc;
+        wbx[wave] = xinc;
+    }
     // block exclusive scan of (ks, as) packed as ks << kAsBits | as (a tile
     // holds at most 5 TILE active tets and 64 times as many functions)
     constexpr int kAsBits = 13;
@@ -918,11 +934,16 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     uint32_t ex = inc - packed;
     for (int w = 0; w < wave; ++w) ex += wsum[w];
     uint32_t o = pre.v[TF_FIT] + (ex >> kAsBits), r = pre.v[TF_ACTIVE] + (ex & ((1u << kAsBits) - 1u));
-    uint32_t bnext[3] = {0, 0, 0};
+    uint32_t bnext[4] = {0, 0, 0, 0};
     for (int qq = 0; qq < 3 && busy; ++qq) {
         uint32_t b = pre.v[TF_B2 + qq] + (((binc - bp) >> (10 * qq)) & 1023u);
         for (int w = 0; w < wave; ++w) b += (wbk[w] >> (10 * qq)) & 1023u;
         bnext[qq] = b;
+    }
+    if (bx) {
+        uint32_t b = pre.v[TF_BX] + xinc - bx;
+        for (int w = 0; w < wave; ++w) b += wbx[w];
+        bnext[3] = b;
     }
     for (int q = 0; q < 5; ++q) {
         const M mq = m[q];
@@ -938,8 +959,8 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
             if (k > 1 && r < A.cap_active && o + (uint32_t)k <= A.cap_fit) {
                 uint32_t oo = o;
                 for (M mm = mq; mm; mm &= mm - 1) A.fit[oo++] = (uint8_t)(__ffsll((unsigned long long)mm) - 1);
-                if (k <= A.kbig) {
-                    const int qq = k == 2 ? 0 : (k <= 4 ? 1 : 2);
+                if (k <= kMaxHuge) {
+                    const int qq = k == 2 ? 0 : (k <= 4 ? 1 : (k <= 8 ? 2 : 3));
                     const uint32_t slot = bnext[qq]++;
                     if (slot < A.cap[qq]) {
                         A.list[qq][slot] = r;
@@ -1024,7 +1045,6 @@ struct CutArgs {
     uint64_t full;
     uint32_t rec_base, cap_active;
     int tf;
-    int kmin, kmax;  // the tets of the list that this launch cuts
     K2Snap k2s;  // lane-group forms: the complexes after two planes (off null: none)
 };
 
@@ -1043,7 +1063,6 @@ __global__ void __launch_bounds__(64) k_cut_bucket(CutArgs A) {
         if (i >= n) continue;
         const uint32_t r = A.list[i];
         const int k = A.act_k[r];
-        if (k < A.kmin || k > A.kmax) continue;
         const uint32_t t = A.act[r];
         uint32_t v[4];
         dev::tet_corners(A.g, t, v);
@@ -1116,7 +1135,6 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
         dev::tet_corners(A.g, e.t, v);
         const uint64_t m = A.masks.active(v, A.full);
         k = __popcll(m);
-        if (k < A.kmin || k > A.kmax) return;
         for (int e4 = lane; e4 < 4 * (C::MP - 4); e4 += G) {
             // row q: the q-th active function (rows past k load function 0, unused)
             uint64_t mm = m;
@@ -1131,7 +1149,6 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_
         r = A.list[i];
         const uint64_t ts = A.lts[i];
         k = A.act_k[r];
-        if (k < A.kmin || k > A.kmax) return;
         rec_at = 0;
         // corner values: the loads need not wait for k (rows past the tet's
         // functions read the CSR's next entries, inside its head-room of 64,
@@ -1391,11 +1408,11 @@ struct ExtractArgs {
     uint16_t* fq_l;
     uint8_t *fq_fn, *fq_bnd;
     uint32_t *fq_vs, *fve, *errs;
-    const uint32_t* list[3];  // bucket lists (k = 2, 3..4, 5..8) of active ranks
-    const uint64_t* lts[3];   // per slot: CSR offset << 32 | tet
-    uint32_t list_cap[3];
-    uint32_t slot_words[3];   // words per record slot of each bucket
-    uint32_t fo_table[3];     // 1: the bucket's cut leaves face offsets after a record that fits
+    const uint32_t* list[4];  // bucket lists (k = 2, 3..4, 5..8, 9..) of active ranks
+    const uint64_t* lts[4];   // per slot: CSR offset << 32 | tet
+    uint32_t list_cap[4];
+    uint32_t slot_words[4];   // words per record slot of each bucket
+    uint32_t fo_table[4];     // 1: the bucket's cut leaves face offsets after a record that fits
     const uint32_t* plan_off;  // k = 2 table records: extraction plans (k2_plans)
     const uint8_t* plan;
     uint32_t n_plans;
@@ -1585,12 +1602,13 @@ __device__ inline void extract_wave_role(const ExtractArgs& A, WaveExtractLds& S
     uint32_t* isov = S.isov;
     uint8_t* isof = S.isof;
     if (!extract_guard(A)) return;
-    const uint32_t n2 = min(A.ctr[C_Q5], A.list_cap[2]), n1 = min(A.ctr[C_Q3], A.list_cap[1]);
+    const uint32_t n3 = min(A.ctr[C_QX], A.list_cap[3]), n2 = min(A.ctr[C_Q5], A.list_cap[2]),
+                   n1 = min(A.ctr[C_Q3], A.list_cap[1]);
     const uint32_t i = blk;
-    if (i >= n1 + n2) return;
+    if (i >= n1 + n2 + n3) return;
     // the larger complexes first
-    const int bq = i < n2 ? 2 : 1;
-    const uint32_t a = bq == 2 ? A.list[2][i] : A.list[1][i - n2];
+    const int bq = i < n3 ? 3 : (i < n3 + n2 ? 2 : 1);
+    const uint32_t a = bq == 3 ? A.list[3][i] : (bq == 2 ? A.list[2][i - n3] : A.list[1][i - n3 - n2]);
     const int lane = threadIdx.x;
     const uint32_t loc = A.rec_loc[a];
     const uint16_t* W = (loc & K1_FLAG) ? A.tab + A.tab_off[loc & ~K1_FLAG] : A.rec + loc;
@@ -1837,32 +1855,31 @@ void table_cut_plain(const GridView& g, const double* vals, const uint32_t* act,
 // ------------------------------------------------------------------ plan
 
 struct Caps_ {
-    uint32_t active = 0, fit = 0, b[3] = {0, 0, 0}, vo = 0, fo = 0, fv = 0;
+    // b[3] (tets of more than 8 functions): 0 until a value set has shown one
+    uint32_t active = 0, fit = 0, b[4] = {0, 0, 0, 0}, vo = 0, fo = 0, fv = 0;
 };
 
 struct Workspace {
     DevMem mem;  // every buffer (and every temporary of the captured launches) lives here
     Caps_ cap;
-    uint32_t rec_base[3] = {0, 0, 0};
+    uint32_t rec_base[4] = {0, 0, 0, 0};
     // words per record slot: the largest record a bucket's capacity allows
-    // (header, vertices, faces with their cycles, coincidence groups)
-    uint32_t slot[3] = {rec_words<CK2>(), rec_words<CMed>(), rec_words<CBig>()};
-    // value sets of this plan have tets of more than 8 functions: they join
-    // the last bucket, whose slots grow, and the wide cut takes them (such a
-    // run was handed to the plain form: 3.9 ms against 2.8 ms for a job of 32
-    // functions at 33^3 vertices, 1.9 ms of either the copies to the host)
-    bool wide = false;
-    bool wave_cut[3] = {false, false, false};  // bucket cut by the wave form (records carry face offsets)
+    // (header, vertices, faces with their cycles, coincidence groups).  Tets of
+    // more than 8 functions have a bucket of their own: in the 5..8 bucket
+    // they made every slot there three times as large (13248 words for 4536),
+    // and that bucket reached 2^31 words at 144,000 tets for 420,000
+    const uint32_t slot[4] = {rec_words<CK2>(), rec_words<CMed>(), rec_words<CBig>(), rec_words<CWide>()};
+    bool wave_cut[4] = {false, false, false, true};  // bucket cut by the wave form (records carry face offsets)
     DBuf<const double*> vals_at;  // the run's values, left by its signs pass for the captured kernels
     DBuf<uint8_t> masks;        // MaskPair by vertex
     DBuf<uint2> blocks;         // regular grids: rank blocks (RankOf)
     DBuf<uint64_t> busy;        // regular grids: per 64 cubes, which hold an active tet
-    DBuf<uint32_t> kcnt, isact, csr_off, rank, act, rec_loc, cnt, list[3];
-    DBuf<uint64_t> lts[3];  // per bucket slot: CSR offset << 32 | tet
+    DBuf<uint32_t> kcnt, isact, csr_off, rank, act, rec_loc, cnt, list[4];
+    DBuf<uint64_t> lts[4];  // per bucket slot: CSR offset << 32 | tet
     DBuf<uint32_t> act_off;  // CSR offset of each active tet, by active rank
     DBuf<TileSums> tile_sums;  // regular grids: per tile of cubes
     int cube_tile = kCubeTile;  // cubes per tile of the count and fill passes
-    DBuf<EarlyEntry> early[3];  // regular grids: the k = 3..4 and 5..8 tets ([1], [2]), listed by the count pass
+    DBuf<EarlyEntry> early[4];  // regular grids: the tets of the lists from k = 3..4 on, listed by the count pass
     DBuf<uint8_t> fit, act_k;
     DBuf<uint16_t> rec;
     DBuf<uint32_t> cv, cf, cfv;
@@ -1955,8 +1972,6 @@ struct Plan {
     std::vector<std::shared_ptr<Workspace>> ws;
     int blocks_per_cu[3] = {0, 0, 0};  // autotuned grid of each bucket's cut kernel
     int cube_tile = 0;                  // autotuned cube tile of the count and fill passes (0: not yet)
-    bool wide = false;                  // new workspaces start wide
-    uint32_t hint_b[5] = {0, 0, 0, 0, 0};
 };
 
 // one plan per (mode, function count) of a grid
@@ -2059,10 +2074,9 @@ unsigned cube_tiles(const Grid& g, int tile = kCubeTile) {
 // until the last has its size, so a growth that fails midway (no memory) leaves
 // a workspace that the next run allocates anew
 void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream_t s) {
-    W.slot[2] = W.wide ? rec_words<CWide>() : rec_words<CBig>();
     uint64_t words = 0;
-    for (int q = 0; q < 3; ++q) words += (uint64_t)c.b[q] * W.slot[q];
-    if (words >= record_limit(1ull << 31)) throw std::runtime_error("record workspace exceeds capacity");
+    for (int q = 0; q < 4; ++q) words += (uint64_t)c.b[q] * W.slot[q];
+    if (words >= record_limit(1ull << 31)) throw NeedsPlainForm("the record slots exceed 2^31 words");
     W.cap = Caps_{};
     DevMem& m = W.mem;
     const uint64_t V = g.view.V, T = g.view.T;
@@ -2072,7 +2086,7 @@ void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream
         W.blocks.alloc(m, T / 32 + 1);
         W.busy.alloc(m, (size_t)cube_tiles(g, 1024) * 16);  // whole tiles, of every size
         W.tile_sums.alloc(m, cube_tiles(g, 256) + 1);  // the smallest tile has the most tiles
-        for (int q = 1; q < 3; ++q) W.early[q].alloc(m, c.b[q] + 1);
+        for (int q = 1; q < 4; ++q) W.early[q].alloc(m, c.b[q] + 1);
     } else {
         W.kcnt.alloc(m, T + 1);
         W.isact.alloc(m, T + 1);
@@ -2086,7 +2100,7 @@ void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream
     W.cnt.alloc(m, 3 * (uint64_t)c.active + 3);
     W.fit.alloc(m, c.fit + 1);
     words = 0;
-    for (int q = 0; q < 3; ++q) {
+    for (int q = 0; q < 4; ++q) {
         W.list[q].alloc(m, c.b[q] + 1);
         W.lts[q].alloc(m, c.b[q] + 1);
         W.rec_base[q] = (uint32_t)words;
@@ -2178,7 +2192,7 @@ void alloc_ws(Workspace& W, const Grid& g, uint32_t F, const Caps_& c, hipStream
 // signs pass is launched for each run, before the path's graph: it is the one
 // kernel that is given the values, and runs while the host launches the
 // graph; zero: clear the counters first (a whole run leaves them clear)
-// early3, early5: list the k = 3..4 / 5..8 tets for launch_cut_early (regular grids)
+// early3, early5: list the k = 3..4 / 5.. tets for launch_cut_early (regular grids)
 void stage_signs(Workspace& W, const Grid& g, const Values& val, hipStream_t s, bool zero) {
     if (zero) hipLaunchKernelGGL(k_zero_ctr, dim3(1), dim3(64), 0, s, W.ctr.p, (int)C_N, W.errs.p);
     with_mask_type(val.F, [&](auto t) {
@@ -2193,16 +2207,16 @@ void stage_filter(Workspace& W, const Grid& g, const Values& val, hipStream_t s,
     const uint64_t T = g.view.T;
     const uint32_t F = val.F;
     const uint64_t full = (F == 64) ? ~0ull : ((1ull << F) - 1);
-    const int kbig = W.wide ? kMaxHuge : 8;
     if (g.view.regular) {
         const int tile = W.cube_tile;
         with_mask_type(F, [&](auto t) {
             using M = decltype(t);
             auto count = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3(cube_tiles(g, tile)), dim3(tile), 0, s, g.view,
-                                   reinterpret_cast<const MaskPair<M>*>(W.masks.p), full, kbig, W.tile_sums.p,
-                                   W.busy.p, early3 ? W.early[1].p : nullptr, early5 ? W.early[2].p : nullptr, W.cap.b[1],
-                                   W.cap.b[2], W.ctr.p);
+                                   reinterpret_cast<const MaskPair<M>*>(W.masks.p), full, W.tile_sums.p, W.busy.p,
+                                   early3 ? W.early[1].p : nullptr, early5 ? W.early[2].p : nullptr,
+                                   early5 && W.cap.b[3] ? W.early[3].p : nullptr, W.cap.b[1], W.cap.b[2], W.cap.b[3],
+                                   W.ctr.p);
             };
             if (tile == 256)
                 count(k_cube_count<256, M>);
@@ -2216,7 +2230,7 @@ void stage_filter(Workspace& W, const Grid& g, const Values& val, hipStream_t s,
         return;
     }
     hipLaunchKernelGGL(k_filter_count, dim3(nblk(T)), dim3(256), 0, s, g.view, MaskRef{W.masks.p, mask_width(F)}, full,
-                       kbig, W.kcnt.p, W.isact.p, W.ctr.p);
+                       W.kcnt.p, W.isact.p, W.ctr.p);
     scan_u32(W.mem, W.kcnt.p, W.csr_off.p, Count(T), W.ctr.p + C_FIT, s);
     scan_u32(W.mem, W.isact.p, W.rank.p, Count(T), W.ctr.p + C_ACTIVE, s);
 }
@@ -2272,18 +2286,9 @@ void launch_cut(Workspace& W, const Grid& g, const Values& val, int q, int grid,
     A.cnt = W.cnt.p;
     A.errs = W.errs.p;
     A.ctr = W.ctr.p;
-    A.kmin = 0;
-    A.kmax = q == 2 ? 8 : kMaxHuge;
     A.stat_k = q == 1 ? SP_CUTK3 : (q == 2 ? SP_CUTK5 : -1);
     A.stat_w = q == 1 ? SP_CUTW3 : (q == 2 ? SP_CUTW5 : -1);
     A.k2s = W.k2_start ? K2Snap{W.k2pat.p, W.k2snap_off.p, W.k2snap.p} : K2Snap{nullptr, nullptr, nullptr};
-    if (W.wide && q == 2) {  // the list's tets of more than 8 functions
-        CutArgs B = A;
-        B.kmin = 9;
-        B.kmax = kMaxHuge;
-        B.stat_k = B.stat_w = -1;
-        hipLaunchKernelGGL((k_cut_wave<CWide, 64>), dim3(W.cap.b[q]), dim3(64), 0, s, B);
-    }
     if (grid == -2) {  // k = 2 table
         K2Args K = k2_args(W, g, val);
         K.n = A.n;
@@ -2305,21 +2310,21 @@ void launch_cut(Workspace& W, const Grid& g, const Values& val, int q, int grid,
         hipLaunchKernelGGL((k_cut_wave<C, G>), dim3((W.cap.b[q] + 64 / G - 1) / (64 / G)), dim3(64), 0, s, A);
         return;
     }
-    fill_u32(W.ctr.p + kQueueBase + q, 0, 1, s);
-    // the complexes of the thread form live in the workspace (grown outside
-    // capture: the autotuner launches every candidate eagerly first)
-    const size_t need = LaneCut<C>::stride * 64 * (size_t)grid;
-    if (W.ws_thread[q].n < need) W.ws_thread[q].alloc(W.mem, need);
-    A.ws = W.ws_thread[q].p;
-    hipLaunchKernelGGL(k_cut_bucket<C>, dim3(grid), dim3(64), 0, s, A);
+    if constexpr (!std::is_same<C, CWide>::value) {  // (tets of more than 8 functions: the wave form only)
+        fill_u32(W.ctr.p + kQueueBase + q, 0, 1, s);
+        // the complexes of the thread form live in the workspace (grown outside
+        // capture: the autotuner launches every candidate eagerly first)
+        const size_t need = LaneCut<C>::stride * 64 * (size_t)grid;
+        if (W.ws_thread[q].n < need) W.ws_thread[q].alloc(W.mem, need);
+        A.ws = W.ws_thread[q].p;
+        hipLaunchKernelGGL(k_cut_bucket<C>, dim3(grid), dim3(64), 0, s, A);
+    }
 }
 
-// the k = 3..4 (q = 1) or 5..8 (q = 2) cut from the count pass's list,
-// beside the fill pass (regular grids, lane-group forms: grid -1, or -3 for
-// four tets a wavefront)
-// wide: the tets of the last list with more than 8 functions
-void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int grid, hipStream_t s,
-                      bool wide = false) {
+// the k = 3..4 (q = 1), 5..8 (q = 2) or 9.. (q = 3) cut from the count pass's
+// list, beside the fill pass (regular grids, lane-group forms: grid -1, or -3
+// for four tets a wavefront)
+void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int grid, hipStream_t s) {
     CutArgs A = {};
     A.g = g.view;
     A.vals = W.vals_at.p;
@@ -2330,22 +2335,20 @@ void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int
     A.cnt = W.cnt.p;
     A.errs = W.errs.p;
     A.ctr = W.ctr.p;
-    A.kmin = wide ? 9 : 0;
-    A.kmax = wide ? kMaxHuge : 8;
-    A.stat_k = wide ? -1 : (q == 1 ? SP_CUTK3 : SP_CUTK5);
-    A.stat_w = wide ? -1 : (q == 1 ? SP_CUTW3 : SP_CUTW5);
+    A.stat_k = q == 1 ? SP_CUTK3 : (q == 2 ? SP_CUTK5 : -1);
+    A.stat_w = q == 1 ? SP_CUTW3 : (q == 2 ? SP_CUTW5 : -1);
     A.early = W.early[q].p;
-    A.n_early = W.ctr.p + (q == 1 ? C_E3 : C_E5);
+    A.n_early = W.ctr.p + (q == 1 ? C_E3 : (q == 2 ? C_E5 : C_EX));
     A.n_back = q == 1 ? W.ctr.p + C_E3B : nullptr;
     A.tiles = W.tile_sums.p;
     A.masks = MaskRef{W.masks.p, mask_width(val.F)};
     A.full = (val.F == 64) ? ~0ull : ((1ull << val.F) - 1);
     A.rec_base = W.rec_base[q];
     A.cap_active = W.cap.active;
-    A.tf = q == 1 ? TF_B3 : TF_B5;
+    A.tf = q == 1 ? TF_B3 : (q == 2 ? TF_B5 : TF_BX);
     A.k2s = W.k2_start ? K2Snap{W.k2pat.p, W.k2snap_off.p, W.k2snap.p} : K2Snap{nullptr, nullptr, nullptr};
     const uint32_t cap = W.cap.b[q];
-    if (wide)
+    if (q == 3)
         hipLaunchKernelGGL((k_cut_wave<CWide, 64, true>), dim3(cap), dim3(64), 0, s, A);
     else if (q == 2)
         hipLaunchKernelGGL((k_cut_wave<CBig, 64, true>), dim3(cap), dim3(64), 0, s, A);
@@ -2377,8 +2380,7 @@ void stage_fill(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
     A.cnt = W.cnt.p;
     A.act_k = W.act_k.p;
     A.k1 = W.k1.p;
-    A.kbig = W.wide ? kMaxHuge : 8;
-    for (int q = 0; q < 3; ++q) {
+    for (int q = 0; q < 4; ++q) {
         A.list[q] = W.list[q].p;
         A.lts[q] = W.lts[q].p;
         A.cap[q] = W.cap.b[q];
@@ -2473,7 +2475,7 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
         E.fq_vs = W.fq_vs.p;
         E.fve = W.fve.p;
         E.errs = W.errs.p;
-        for (int q = 0; q < 3; ++q) {
+        for (int q = 0; q < 4; ++q) {
             E.list[q] = W.list[q].p;
             E.lts[q] = W.lts[q].p;
             E.list_cap[q] = c.b[q];
@@ -2488,14 +2490,15 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
             // tet at 101^3: 0.375 ms/step against 0.381 with 8192)
             const uint32_t ecap = 16384u;
             const uint32_t nb_rec = std::min<uint32_t>((c.b[0] + 63) / 64, ecap) + 1;
-            const uint32_t nb_wave = std::max(1u, c.b[1] + c.b[2]);
+            const uint32_t nb_wave = std::max(1u, c.b[1] + c.b[2] + c.b[3]);
             const uint32_t nb_k1 = std::min<uint32_t>((c.active + 63) / 64, ecap) + 1;
             hipLaunchKernelGGL(k_extract_all, dim3(nb_rec + nb_wave + nb_k1), dim3(64), 0, s, E, nb_rec, nb_wave,
                                nb_k1);
         } else {
             if (part & REST_EXTRACT_K1) hipLaunchKernelGGL(k_extract_k1, dim3(cgrid(c.active)), dim3(256), 0, s, E);
             if (part & REST_EXTRACT_REC) {
-                hipLaunchKernelGGL(k_extract_records_wave, dim3(std::max(1u, c.b[1] + c.b[2])), dim3(64), 0, s, E);
+                hipLaunchKernelGGL(k_extract_records_wave, dim3(std::max(1u, c.b[1] + c.b[2] + c.b[3])), dim3(64),
+                                   0, s, E);
                 hipLaunchKernelGGL(k_extract_records, dim3(cgrid(c.b[0])), dim3(256), 0, s, E);
             }
         }
@@ -2618,17 +2621,18 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
 
 // conservative per-tet output bounds by active count (maxima of the cut's
 // vertex / face counts, see the capacities of the bucket kernels)
-void caps_from_counts(const uint32_t* ctr, bool wide, Caps_& c) {
-    const uint64_t b1 = ctr[C_B1], b2 = ctr[C_B2], b3 = ctr[C_B3], bx = wide ? ctr[C_BX] : 0, b5 = ctr[C_B5] - bx;
+void caps_from_counts(const uint32_t* ctr, Caps_& c) {
+    const uint64_t b1 = ctr[C_B1], b2 = ctr[C_B2], b3 = ctr[C_B3], b5 = ctr[C_B5], bx = ctr[C_BX];
     auto clamp = [](uint64_t x) -> uint32_t {
-        if (x >= (1ull << 31)) throw std::runtime_error("workspace capacity exceeds 2^31 entries");
+        if (x >= (1ull << 31)) throw NeedsPlainForm("the workspace exceeds 2^31 entries");
         return (uint32_t)x;
     };
     c.active = clamp(ctr[C_ACTIVE] + 64);
     c.fit = clamp(ctr[C_FIT] + 64);
     c.b[0] = clamp(b2 + 64);
     c.b[1] = clamp(b3 + 64);
-    c.b[2] = clamp(b5 + bx + 64);
+    c.b[2] = clamp(b5 + 64);
+    c.b[3] = bx ? clamp(bx + 64) : 0u;
     c.vo = clamp(4 * b1 + 16 * b2 + 40 * b3 + 132 * b5 + (uint64_t)CWide::MV * bx + 64);
     c.fo = clamp(1 * b1 + 24 * b2 + 64 * b3 + 284 * b5 + (uint64_t)CWide::MF * bx + 64);
     c.fv = clamp(4 * b1 + 24 * 6 * b2 + 64 * 8 * b3 + 284 * 10 * b5 + (uint64_t)CWide::MF * CWide::MFV * bx + 64);
@@ -2636,7 +2640,8 @@ void caps_from_counts(const uint32_t* ctr, bool wide, Caps_& c) {
 
 bool caps_ok(const Caps_& have, const Caps_& need) {
     return have.active >= need.active && have.fit >= need.fit && have.b[0] >= need.b[0] && have.b[1] >= need.b[1] &&
-           have.b[2] >= need.b[2] && have.vo >= need.vo && have.fo >= need.fo && have.fv >= need.fv;
+           have.b[2] >= need.b[2] && have.b[3] >= need.b[3] && have.vo >= need.vo && have.fo >= need.fo &&
+           have.fv >= need.fv;
 }
 
 float time_ms(hipStream_t s, const std::function<void()>& f) {
@@ -2748,7 +2753,8 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         if (!e5 && w.cap.b[2]) launch_cut<CBig>(w, g, val, 2, w.grid[2], w.side2);
         if (!e3 && w.cap.b[1]) launch_cut<CMed>(w, g, val, 1, w.grid[1], w.side2);
         if (w.cap.b[0]) launch_cut<CK2>(w, g, val, 0, w.grid[0], w.side2);
-        if (e5 && w.wide) launch_cut_early(w, g, val, 2, w.grid[2], w.side2, true);
+        if (e5 && w.cap.b[3]) launch_cut_early(w, g, val, 3, -1, w.side2);
+        if (!e5 && w.cap.b[3]) launch_cut<CWide>(w, g, val, 3, -1, w.side2);
         RIN_HIP(hipEventRecord(w.join2, w.side2));
         if (e5) RIN_HIP(hipStreamWaitEvent(s, w.join, 0));
         RIN_HIP(hipStreamWaitEvent(s, w.join2, 0));
@@ -2756,6 +2762,7 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         stage_fill(w, g, val, s);
         RIN_HIP(hipEventRecord(w.fork, s));
         RIN_HIP(hipStreamWaitEvent(w.side, w.fork, 0));
+        if (w.cap.b[3]) launch_cut<CWide>(w, g, val, 3, -1, w.side);
         if (w.cap.b[2]) launch_cut<CBig>(w, g, val, 2, w.grid[2], w.side);
         if (w.cap.b[0]) launch_cut<CK2>(w, g, val, 0, w.grid[0], w.side);
         RIN_HIP(hipEventRecord(w.join, w.side));
@@ -2794,6 +2801,7 @@ void record_parts(Workspace& w, const Grid& g, const Values& val, const Plan& P,
     if (w.cap.b[0]) capture(cut_label("cut k=2", w, P, 0), [&] { launch_cut<CK2>(w, g, val, 0, w.grid[0], s); });
     if (w.cap.b[1]) capture(cut_label("cut k=3..4", w, P, 1), [&] { launch_cut<CMed>(w, g, val, 1, w.grid[1], s); });
     if (w.cap.b[2]) capture(cut_label("cut k=5..8", w, P, 2), [&] { launch_cut<CBig>(w, g, val, 2, w.grid[2], s); });
+    if (w.cap.b[3]) capture("cut k=9.. (wave per tet)", [&] { launch_cut<CWide>(w, g, val, 3, -1, s); });
     capture("extract: per-tet output scans", [&] { stage_rest(w, g, val, s, REST_SCANS); });
     capture("extract k=1 occurrences (k_extract_k1)", [&] { stage_rest(w, g, val, s, REST_EXTRACT_K1); });
     capture("extract record occurrences (k_extract_records)", [&] { stage_rest(w, g, val, s, REST_EXTRACT_REC); });
@@ -2831,7 +2839,6 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         }
     if (!W) {
         W = std::make_shared<Workspace>();
-        W->wide = P.wide;
         P.ws.push_back(W);
     }
     Workspace& w = *W;
@@ -2854,7 +2861,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
     };
     auto errors = [&] { return herr; };
     bool ran = false;
-    for (int attempt = 0; attempt < 4 && !ran; ++attempt) {
+    for (int attempt = 0; attempt < 3 && !ran; ++attempt) {
         if (!w.exec) {
             w.ctr_clear = false;  // the eager passes below use the counters
             // size the workspace from an eager counting pass
@@ -2867,15 +2874,8 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             }
             stage_count(w, g, val, s);
             read_back(true);
-            if (hctr[C_BX] && !w.wide) {
-                // larger slots for the last bucket, and the counts with it
-                w.wide = P.wide = true;
-                w.cap = Caps_{};
-                stage_count(w, g, val, s);
-                read_back(true);
-            }
             Caps_ need;
-            caps_from_counts(hctr, w.wide, need);
+            caps_from_counts(hctr, need);
             if (!caps_ok(w.cap, need)) {
                 // grow with head-room; what is there already stays, so that
                 // value sets that alternate settle on one capacity
@@ -2883,7 +2883,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
                 Caps_ grow;
                 grow.active = more(w.cap.active, need.active);
                 grow.fit = more(w.cap.fit, need.fit);
-                for (int q = 0; q < 3; ++q) grow.b[q] = more(w.cap.b[q], need.b[q]);
+                for (int q = 0; q < 4; ++q) grow.b[q] = more(w.cap.b[q], need.b[q]);
                 grow.vo = more(w.cap.vo, need.vo);
                 grow.fo = more(w.cap.fo, need.fo);
                 grow.fv = more(w.cap.fv, need.fv);
@@ -3010,11 +3010,6 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             w.exec = false;
             continue;
         }
-        if (e && hctr[C_BX] && !w.wide) {  // the first value set with tets of more than 8 functions
-            w.drop_graphs();
-            w.exec = false;
-            continue;
-        }
         if (e) {
             out.err = e;
             throw NeedsPlainForm("a complex exceeds the bucket capacities or the predicate range");
@@ -3044,7 +3039,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
     out.n_fit = hctr[C_FIT];
     out.nb[0] = hctr[C_B1];
     out.nb[1] = hctr[C_B2];
-    out.nb[2] = hctr[C_B3] + hctr[C_B5];
+    out.nb[2] = hctr[C_B3] + hctr[C_B5] + hctr[C_BX];
     out.n_verts = hctr[C_VERTS];
     out.n_faces = hctr[C_FACES];
     out.n_face_verts = hctr[C_FACEVERTS];
@@ -3053,7 +3048,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
     out.n_face_occ = hctr[C_FO];
     out.n_face_occ_verts = hctr[C_FV];
     out.n_cut34 = hctr[C_B3];
-    out.n_cut58 = hctr[C_B5] - (w.wide ? hctr[C_BX] : 0u);
+    out.n_cut58 = hctr[C_B5];
     out.n_rec_words = hctr[C_RECW];
     out.cut_k_sum[0] = hctr[C_CUTK3];
     out.cut_k_sum[1] = hctr[C_CUTK5];

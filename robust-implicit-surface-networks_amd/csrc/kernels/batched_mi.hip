@@ -543,7 +543,7 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     const uint64_t V = g.view.V, T = g.view.T;
     const MITablesRaw TR = mi_tables_device(s);
     if ((uint64_t)c.words + 1 + TR.n_w2 + TR.n_w3 >= record_limit(1ull << 32))
-        throw std::runtime_error("material-interface record words exceed 32-bit offsets");
+        throw NeedsPlainForm("the record slots exceed 2^32 words");
     W.cap = MICaps{};
     if (!W.errs.p) {
         W.hm.alloc(m, V);

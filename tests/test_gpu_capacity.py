@@ -27,7 +27,8 @@ def _values(mi, F, n, pts):
 @pytest.mark.parametrize("mi,F", [(0, 8), (1, 20)])
 @pytest.mark.parametrize("regular", [True, False])
 def test_runs_after_a_growth_that_failed(ctx, monkeypatch, mi, F, regular):
-    """A workspace that could not grow is not used as if it had."""
+    """A run past the limit takes the plain form, and a workspace that could not
+    grow is not used as if it had."""
     import rin
 
     pts, tets = S.grid(3)
@@ -37,19 +38,56 @@ def test_runs_after_a_growth_that_failed(ctx, monkeypatch, mi, F, regular):
     refs = [S.OracleRun(mi, pts, tets, v) for v in sets]
     few, many = [g.upload(v) for v in sets]
 
-    def check(v, ref):
+    def check(v, ref, path="batched path (one graph)"):
         dev = v.run(flags)
         _compare(dev, ref)
-        assert dev.stage_times()[0][0] == "batched path (one graph)"
+        assert dev.stage_times()[0][0].startswith(path)
         dev.release()
 
     check(few, refs[0])
     monkeypatch.setenv("RIN_RECORD_WORDS", "1000")
-    with pytest.raises(rin.RinError):
-        many.run(flags)
+    check(many, refs[1], "batched form fell back")
     check(few, refs[0])
     monkeypatch.delenv("RIN_RECORD_WORDS")
     check(many, refs[1])
     check(few, refs[0])
     for x in (few, many, g):
         x.release()
+
+
+# record words of a slot by the tet's functions: 2, 3..4, 5..8, 9..28
+SLOTS = ((2, 2, 324), (3, 4, 952), (5, 8, 4536), (9, 28, 13248))
+
+
+@pytest.mark.parametrize("regular", [True, False])
+def test_wide_tets_leave_the_other_slots_alone(ctx, monkeypatch, regular):
+    """A value set with tets of nine functions, then one of five to eight in most
+    tets, under a limit that both fit when only the former have large slots."""
+    import rin
+
+    pts, tets = S.grid(5)
+    g = ctx.grid_regular(5) if regular else ctx.grid_explicit(pts, tets)
+    rng = np.random.default_rng(3)
+    fs = W.FuncSet()
+    for _ in range(9):
+        fs.plane(rng.uniform(-0.02, 0.02, 3) + [0.1, 0.05, 0.0], rng.standard_normal(3))
+    wide = S.evaluate(*fs.arrays(), pts)
+    many = rng.integers(1, 4, (len(pts), 9)) * rng.choice([-1.0, 1.0], (len(pts), 9))
+    many[:, 8] = 1.0
+    refs = [S.OracleRun(0, pts, tets, v) for v in (wide, many)]
+    k = [np.diff(r.start_index.astype(np.int64)) for r in refs]
+    assert k[0].max() == 9 and k[1].max() == 8
+    n = [max(int(((x >= lo) & (x <= hi)).sum()) for x in k) for lo, hi, _ in SLOTS]
+    assert n[3] < 20 and n[2] > 400
+    need = sum((x + 64) * 9 // 8 * w for x, (_, _, w) in zip(n, SLOTS))
+    assert (n[2] + 64) * 9 // 8 * SLOTS[3][2] > 1.5 * need  # as one list with the larger slots
+    monkeypatch.setenv("RIN_RECORD_WORDS", str(int(1.1 * need)))
+    values = [g.upload(v) for v in (wide, many)]
+    for i in (0, 1, 0, 1):
+        dev = values[i].run(rin.FLAG_BATCHED)
+        _compare(dev, refs[i])
+        assert dev.stage_times()[0][0] == "batched path (one graph)"
+        dev.release()
+    for v in values:
+        v.release()
+    g.release()
