@@ -898,7 +898,6 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
         ks += (uint32_t)k;
         as += k != 0;
         if (k >= 2 && k <= 8) bp += 1u << (10 * (k == 2 ? 0 : (k <= 4 ? 1 : 2)));
-        bx += k > 8 && k <= kMaxHuge;
     }
     // bucket slots: the tile's prefix, the waves before this one, the lanes
     // before this one (a wave holds at most 320 tets of a list)
@@ -908,12 +907,15 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
             const uint32_t o = __shfl_up(binc, d, 64);
             if (lane >= d) binc += o;
         }
-    uint32_t xinc = bx;
-    if (__any(bx != 0))
+    uint32_t xinc = 0;
+    if (__any(ks > 8)) {
+        for (int q = 0; q < 5; ++q) bx += __popcll(m[q]) > 8 && __popcll(m[q]) <= kMaxHuge;
+        xinc = bx;
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t o = __shfl_up(xinc, d, 64);
             if (lane >= d) xinc += o;
         }
+    }
     if (lane == 63) {
         wbk[wave] = binc;
         wbx[wave] = xinc;
@@ -934,16 +936,15 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     uint32_t ex = inc - packed;
     for (int w = 0; w < wave; ++w) ex += wsum[w];
     uint32_t o = pre.v[TF_FIT] + (ex >> kAsBits), r = pre.v[TF_ACTIVE] + (ex & ((1u << kAsBits) - 1u));
-    uint32_t bnext[4] = {0, 0, 0, 0};
+    uint32_t bnext[3] = {0, 0, 0}, xnext = 0;
     for (int qq = 0; qq < 3 && busy; ++qq) {
         uint32_t b = pre.v[TF_B2 + qq] + (((binc - bp) >> (10 * qq)) & 1023u);
         for (int w = 0; w < wave; ++w) b += (wbk[w] >> (10 * qq)) & 1023u;
         bnext[qq] = b;
     }
     if (bx) {
-        uint32_t b = pre.v[TF_BX] + xinc - bx;
-        for (int w = 0; w < wave; ++w) b += wbx[w];
-        bnext[3] = b;
+        xnext = pre.v[TF_BX] + xinc - bx;
+        for (int w = 0; w < wave; ++w) xnext += wbx[w];
     }
     for (int q = 0; q < 5; ++q) {
         const M mq = m[q];
@@ -959,9 +960,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
             if (k > 1 && r < A.cap_active && o + (uint32_t)k <= A.cap_fit) {
                 uint32_t oo = o;
                 for (M mm = mq; mm; mm &= mm - 1) A.fit[oo++] = (uint8_t)(__ffsll((unsigned long long)mm) - 1);
-                if (k <= kMaxHuge) {
-                    const int qq = k == 2 ? 0 : (k <= 4 ? 1 : (k <= 8 ? 2 : 3));
-                    const uint32_t slot = bnext[qq]++;
+                auto put = [&](int qq, uint32_t slot) {
                     if (slot < A.cap[qq]) {
                         A.list[qq][slot] = r;
                         A.lts[qq][slot] = (uint64_t)o << 32 | (cube * 5 + q);
@@ -970,6 +969,12 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
                         A.errs[lane] |= ERR_OVERFLOW;
                         A.ctr[C_ABORT] = 1;
                     }
+                };
+                if (k <= 8) {
+                    const int qq = k == 2 ? 0 : (k <= 4 ? 1 : 2);
+                    put(qq, bnext[qq]++);
+                } else if (k <= kMaxHuge) {
+                    put(3, xnext++);
                 } else {
                     A.errs[lane] |= 1;  // more active functions than the device cut supports
                 }
