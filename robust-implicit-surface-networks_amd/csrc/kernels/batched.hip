@@ -54,7 +54,8 @@ __host__ __device__ inline uint32_t spread_at(int counter, uint32_t slot) {
     return kSpreadBase + ((uint32_t)counter * kSpread + slot % kSpread) * kSpreadStride;
 }
 enum Ctr : int {
-    C_ACTIVE = 0, C_FIT, C_VO, C_FO, C_FV, C_VERTS, C_FACES, C_FACEVERTS, C_B1, C_B2, C_B3, C_B5, C_BX, C_DEGEN,
+    C_ACTIVE = 0, C_FIT, C_VO, C_FO, C_FV, C_VERTS, C_FACES, C_FACEVERTS, C_B1, C_B2, C_B3, C_B5, C_BX, C_BH,
+    C_DEGEN,
     C_Q2, C_Q3, C_Q5, C_QX, C_ABORT, C_TETFACES, C_RECW, C_CUTK3, C_CUTW3, C_CUTK5, C_CUTW5, C_E3, C_E5, C_E3B, C_EX,
     C_N
 };
@@ -418,7 +419,8 @@ struct MaskRef {
     }
 };
 
-// the buckets: 1, 2, 3..4, 5..8, 9..kMaxHuge functions (5: more than the device cut takes)
+// the buckets: 1, 2, 3..4, 5..8, 9..kMaxHuge functions; 5: more than the device
+// cut takes (a run that counts one goes to the plain form, which reports it)
 __device__ inline int bucket_of(int k) {
     return k <= 1 ? 0 : (k == 2 ? 1 : (k <= 4 ? 2 : (k <= 8 ? 3 : (k <= kMaxHuge ? 4 : 5))));
 }
@@ -439,7 +441,7 @@ __global__ void k_filter_count(GridView g, MaskRef masks, uint64_t full, uint32_
         if (k) atomicAdd(&hist[bucket_of((int)k)], 1u);
     }
     __syncthreads();
-    if (threadIdx.x < 5 && hist[threadIdx.x]) atomicAdd(&ctr[C_B1 + threadIdx.x], hist[threadIdx.x]);
+    if (threadIdx.x < 6 && hist[threadIdx.x]) atomicAdd(&ctr[C_B1 + threadIdx.x], hist[threadIdx.x]);
 }
 
 struct FillArgs {
@@ -512,7 +514,10 @@ __global__ void k_fill_batched(FillArgs A) {
                     A.rec_loc[r] = K1_FLAG | (uint32_t)pat;
                 } else {
                     b = k <= kMaxHuge ? bucket_of(k) - 1 : -1;
-                    if (b < 0) A.errs[lane] |= 1;  // more active functions than the device cut supports
+                    if (b < 0) {  // its row is not written: the later stages have nothing to read
+                        A.errs[lane] |= ERR_CAPACITY;
+                        A.ctr[C_ABORT] = 1;
+                    }
                 }
             }
         }
@@ -640,11 +645,11 @@ __device__ inline void cube_masks(const GridView& g, uint32_t cube, const MaskPa
 }
 
 // Per tile of cubes: active functions, active tets and tets per bucket
-// (k = 1, 2, 3..4, 5..8, 9..kMaxHuge).  No atomics: the tile scan below turns
+// (k = 1, 2, 3..4, 5..8, 9..kMaxHuge, more).  No atomics: the tile scan below turns
 // the tile sums into prefixes (the CSR offsets and the bucket-list slots of
 // each tile) and writes the totals, so the bucket lists come out in tet order.
 constexpr int kTileFields = 8;
-enum TileField { TF_FIT = 0, TF_ACTIVE, TF_B1, TF_B2, TF_B3, TF_B5, TF_BX };
+enum TileField { TF_FIT = 0, TF_ACTIVE, TF_B1, TF_B2, TF_B3, TF_B5, TF_BX, TF_BH };
 struct TileSums {
     uint32_t v[kTileFields];
 };
@@ -691,6 +696,7 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
             v[TF_B3] += k == 3 || k == 4;
             v[TF_B5] += k >= 5 && k <= 8;
             v[TF_BX] += k > 8 && k <= kMaxHuge;
+            v[TF_BH] += k > kMaxHuge;
             n4 += k == 4;
         }
     }
@@ -771,7 +777,7 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
         }
     }
     // the wave's sums: a wave holds at most 320 tets and 64 functions a tet, so
-    // five fields fit one 64-bit word and two another; a wave without an
+    // five fields fit one 64-bit word and three another; a wave without an
     // active tet (most, on a fine grid) has none to add
     __shared__ uint32_t red[TILE / 64][kTileFields];
     uint64_t p0 = 0;
@@ -779,7 +785,7 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
     if (bl) {
         p0 = (uint64_t)v[TF_FIT] | (uint64_t)v[TF_ACTIVE] << 16 | (uint64_t)v[TF_B1] << 28 | (uint64_t)v[TF_B2] << 40 |
              (uint64_t)v[TF_B3] << 52;
-        p1 = v[TF_B5] | v[TF_BX] << 16;
+        p1 = v[TF_B5] | v[TF_BX] << 10 | v[TF_BH] << 20;
         for (int d = 32; d > 0; d >>= 1) p0 += __shfl_xor(p0, d, 64);
         if (__any(p1 != 0))
             for (int d = 32; d > 0; d >>= 1) p1 += __shfl_xor(p1, d, 64);
@@ -790,14 +796,14 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
         red[wave][TF_B1] = (uint32_t)(p0 >> 28) & 0xfffu;
         red[wave][TF_B2] = (uint32_t)(p0 >> 40) & 0xfffu;
         red[wave][TF_B3] = (uint32_t)(p0 >> 52);
-        red[wave][TF_B5] = p1 & 0xffffu;
-        red[wave][TF_BX] = p1 >> 16;
+        red[wave][TF_B5] = p1 & 1023u;
+        red[wave][TF_BX] = p1 >> 10 & 1023u;
+        red[wave][TF_BH] = p1 >> 20;
     }
     __syncthreads();
     if (threadIdx.x < kTileFields) {
         uint32_t t = 0;
-        if (threadIdx.x < kTileFields - 1)
-            for (int w = 0; w < TILE / 64; ++w) t += red[w][threadIdx.x];
+        for (int w = 0; w < TILE / 64; ++w) t += red[w][threadIdx.x];
         tile_sums[tile].v[threadIdx.x] = t;
     }
 }
@@ -856,6 +862,7 @@ __global__ void __launch_bounds__(kTileScanThreads) k_tile_scan(TileSums* __rest
         ctr[C_B3] = carry[TF_B3];
         ctr[C_B5] = carry[TF_B5];
         ctr[C_BX] = carry[TF_BX];
+        ctr[C_BH] = carry[TF_BH];
         ctr[C_Q2] = carry[TF_B2];
         ctr[C_Q3] = carry[TF_B3];
         ctr[C_Q5] = carry[TF_B5];
@@ -975,8 +982,9 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
                     put(qq, bnext[qq]++);
                 } else if (k <= kMaxHuge) {
                     put(3, xnext++);
-                } else {
-                    A.errs[lane] |= 1;  // more active functions than the device cut supports
+                } else {  // its row is not written: the later stages have nothing to read
+                    A.errs[lane] |= ERR_CAPACITY;
+                    A.ctr[C_ABORT] = 1;
                 }
             }
         }
@@ -2865,6 +2873,9 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         herr = w.pub_h[32];
     };
     auto errors = [&] { return herr; };
+    auto too_many = [&] {
+        if (hctr[C_BH]) throw NeedsPlainForm("a tet has more active functions than the device cut takes");
+    };
     bool ran = false;
     for (int attempt = 0; attempt < 3 && !ran; ++attempt) {
         if (!w.exec) {
@@ -2879,6 +2890,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
             }
             stage_count(w, g, val, s);
             read_back(true);
+            too_many();
             Caps_ need;
             caps_from_counts(hctr, need);
             if (!caps_ok(w.cap, need)) {
@@ -3010,6 +3022,7 @@ void run_batched(DevMem& ctx_mem, const Grid& g, const Values& val, uint32_t fla
         w.ctr_clear = true;  // the run's closing kernel cleared them
         const uint32_t e = errors();
         if (e && w.hkey.p) w.hash_dirty = true;
+        too_many();
         if (e & ERR_OVERFLOW) {
             w.drop_graphs();
             w.exec = false;

@@ -91,3 +91,41 @@ def test_wide_tets_leave_the_other_slots_alone(ctx, monkeypatch, regular):
     for v in values:
         v.release()
     g.release()
+
+
+@pytest.mark.parametrize("regular", [True, False])
+def test_more_functions_than_the_cut_takes(ctx, regular):
+    """Value sets of one plan in turn: tets of 9..28 functions, of at most 8, and
+    of more than 28; the last give the plain form's error each time."""
+    import rin
+
+    pts, tets = S.grid(4)
+    g = ctx.grid_regular(4) if regular else ctx.grid_explicit(pts, tets)
+    rng = np.random.default_rng(5)
+    fs = W.FuncSet()
+    for _ in range(32):
+        fs.plane([0.1, 0.05, 0.0], rng.standard_normal(3))
+    too_many = S.evaluate(*fs.arrays(), pts)
+    wide, few = too_many.copy(), too_many.copy()
+    wide[:, 9:] = 1.0
+    few[:, 7:] = 1.0
+    active = [(~((v[tets.astype(int)] > 0).all(1) | (v[tets.astype(int)] < 0).all(1))).sum(1).max()
+              for v in (too_many, wide, few)]
+    assert active[0] > 28 and 8 < active[1] <= 28 and 4 < active[2] <= 8
+    values = {n: g.upload(v) for n, v in (("wide", wide), ("few", few), ("too many", too_many))}
+    refs = {"wide": S.OracleRun(0, pts, tets, wide), "few": S.OracleRun(0, pts, tets, few)}
+    with pytest.raises(rin.RinError) as plain:
+        values["too many"].run(0)
+    for n in ("too many", "few", "too many", "wide", "too many", "few", "wide"):
+        if n == "too many":
+            with pytest.raises(rin.RinError) as e:
+                values[n].run(rin.FLAG_BATCHED)
+            assert str(e.value) == str(plain.value)
+            continue
+        dev = values[n].run(rin.FLAG_BATCHED)
+        _compare(dev, refs[n])
+        assert dev.stage_times()[0][0] == "batched path (one graph)"
+        dev.release()
+    for v in values.values():
+        v.release()
+    g.release()
