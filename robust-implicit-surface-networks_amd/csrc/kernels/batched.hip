@@ -693,11 +693,13 @@ __global__ void __launch_bounds__(TILE) k_cube_count(GridView g, const MaskPair<
             v[TF_ACTIVE] += k != 0;
             v[TF_B1] += k == 1;
             v[TF_B2] += k == 2;
-            v[TF_B3] += k == 3 || k == 4;
-            v[TF_B5] += k >= 5 && k <= 8;
-            v[TF_BX] += k > 8 && k <= kMaxHuge;
-            v[TF_BH] += k > kMaxHuge;
-            n4 += k == 4;
+            if (k > 2) {  // few lanes, in few waves
+                v[TF_B3] += k <= 4;
+                n4 += k == 4;
+                v[TF_B5] += k >= 5 && k <= 8;
+                v[TF_BX] += k > 8 && k <= kMaxHuge;
+                v[TF_BH] += k > kMaxHuge;
+            }
         }
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -876,8 +878,7 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     using M = typename std::conditional<sizeof(T) == 8, uint64_t, uint32_t>::type;
     __shared__ K1Entry tab[81];
     __shared__ uint32_t wsum[TILE / 64];
-    __shared__ uint32_t wbk[TILE / 64];  // per-wave bucket counts, 10 bits per list
-    __shared__ uint32_t wbx[TILE / 64];  // the same of the last list
+    __shared__ uint2 wbk[TILE / 64];  // per-wave bucket counts, 10 bits per list; of the last list
     __shared__ uint32_t s_off[5 * TILE];                         // per-tet CSR offsets of the tile
     __shared__ uint32_t s_bits[5 * TILE / 32], s_pre[5 * TILE / 32];  // its rank blocks
     static_assert(5 * TILE % 32 == 0, "a tile holds whole rank blocks");
@@ -908,25 +909,22 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     }
     // bucket slots: the tile's prefix, the waves before this one, the lanes
     // before this one (a wave holds at most 320 tets of a list)
-    uint32_t binc = bp;
-    if (__any(bp != 0))
+    uint32_t binc = bp, xinc = 0;
+    if (__any(ks > as)) {  // a tet of two functions or more
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t o = __shfl_up(binc, d, 64);
             if (lane >= d) binc += o;
         }
-    uint32_t xinc = 0;
-    if (__any(ks > 8)) {
-        for (int q = 0; q < 5; ++q) bx += __popcll(m[q]) > 8 && __popcll(m[q]) <= kMaxHuge;
-        xinc = bx;
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t o = __shfl_up(xinc, d, 64);
-            if (lane >= d) xinc += o;
+        if (__any(ks > 8)) {
+            for (int q = 0; q < 5; ++q) bx += __popcll(m[q]) > 8 && __popcll(m[q]) <= kMaxHuge;
+            xinc = bx;
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t o = __shfl_up(xinc, d, 64);
+                if (lane >= d) xinc += o;
+            }
         }
     }
-    if (lane == 63) {
-        wbk[wave] = binc;
-        wbx[wave] = xinc;
-    }
+    if (lane == 63) wbk[wave] = make_uint2(binc, xinc);
     // block exclusive scan of (ks, as) packed as ks << kAsBits | as (a tile
     // holds at most 5 TILE active tets and 64 times as many functions)
     constexpr int kAsBits = 13;
@@ -946,12 +944,12 @@ __global__ void __launch_bounds__(TILE) k_cube_fill(FillArgs A, const TileSums* 
     uint32_t bnext[3] = {0, 0, 0}, xnext = 0;
     for (int qq = 0; qq < 3 && busy; ++qq) {
         uint32_t b = pre.v[TF_B2 + qq] + (((binc - bp) >> (10 * qq)) & 1023u);
-        for (int w = 0; w < wave; ++w) b += (wbk[w] >> (10 * qq)) & 1023u;
+        for (int w = 0; w < wave; ++w) b += (wbk[w].x >> (10 * qq)) & 1023u;
         bnext[qq] = b;
     }
     if (bx) {
         xnext = pre.v[TF_BX] + xinc - bx;
-        for (int w = 0; w < wave; ++w) xnext += wbx[w];
+        for (int w = 0; w < wave; ++w) xnext += wbk[w].y;
     }
     for (int q = 0; q < 5; ++q) {
         const M mq = m[q];
