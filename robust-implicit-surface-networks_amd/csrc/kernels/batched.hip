@@ -2726,11 +2726,15 @@ std::string cut_label(const char* base, const Workspace& w, const Plan& P, int q
 
 // the whole path as one graph: the k = 5..8 cut (few tets, long serial
 // insertions) and the k = 2 table lookups on a branch beside the k = 3..4 cut
-// (the cut kernels share no outputs; on regular grids the k = 3..4 and 5..8
-// cuts start beside the fill pass, from the count pass's lists); the three
-// extraction passes write
-// disjoint rows and run as one launch, and so do coordinates and the first
-// face pass
+// (the cut kernels share no outputs; on regular grids the cuts of three
+// functions and more start beside the fill pass, from the count pass's lists).
+// The cut of more than 8 functions follows that of 3..4 on its branch: at most
+// two kernels with lane-group cuts, whose exact predicates need 2.6 KB of
+// scratch a lane, are in flight at once, and the shorter of the two branches
+// takes it (a job of 32 functions at 33^3 vertices: 81 + 215 us beside 195;
+// 1.55 ms a job, and 1.72 with it behind the 5..8 cut).  The three extraction
+// passes write disjoint rows and run as one launch, and so do coordinates and
+// the first face pass
 void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s) {
     if (!w.side) {
         RIN_HIP(hipStreamCreateWithFlags(&w.side, hipStreamNonBlocking));
@@ -2754,6 +2758,7 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         // (tens of wavefronts) and the fill pass follow on side streams
         RIN_HIP(hipEventRecord(w.fork, s));
         if (e3) launch_cut_early(w, g, val, 1, w.grid[1], s);
+        if (e5 && w.cap.b[3]) launch_cut_early(w, g, val, 3, -1, s);
         if (e5) {
             RIN_HIP(hipStreamWaitEvent(w.side, w.fork, 0));
             launch_cut_early(w, g, val, 2, w.grid[2], w.side);
@@ -2764,7 +2769,6 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         if (!e5 && w.cap.b[2]) launch_cut<CBig>(w, g, val, 2, w.grid[2], w.side2);
         if (!e3 && w.cap.b[1]) launch_cut<CMed>(w, g, val, 1, w.grid[1], w.side2);
         if (w.cap.b[0]) launch_cut<CK2>(w, g, val, 0, w.grid[0], w.side2);
-        if (e5 && w.cap.b[3]) launch_cut_early(w, g, val, 3, -1, w.side2);
         if (!e5 && w.cap.b[3]) launch_cut<CWide>(w, g, val, 3, -1, w.side2);
         RIN_HIP(hipEventRecord(w.join2, w.side2));
         if (e5) RIN_HIP(hipStreamWaitEvent(s, w.join, 0));
@@ -2773,11 +2777,11 @@ void record_whole(Workspace& w, const Grid& g, const Values& val, hipStream_t s)
         stage_fill(w, g, val, s);
         RIN_HIP(hipEventRecord(w.fork, s));
         RIN_HIP(hipStreamWaitEvent(w.side, w.fork, 0));
-        if (w.cap.b[3]) launch_cut<CWide>(w, g, val, 3, -1, w.side);
         if (w.cap.b[2]) launch_cut<CBig>(w, g, val, 2, w.grid[2], w.side);
         if (w.cap.b[0]) launch_cut<CK2>(w, g, val, 0, w.grid[0], w.side);
         RIN_HIP(hipEventRecord(w.join, w.side));
         if (w.cap.b[1]) launch_cut<CMed>(w, g, val, 1, w.grid[1], s);
+        if (w.cap.b[3]) launch_cut<CWide>(w, g, val, 3, -1, s);
         RIN_HIP(hipStreamWaitEvent(s, w.join, 0));
     }
     stage_rest(w, g, val, s, REST_SCANS);
