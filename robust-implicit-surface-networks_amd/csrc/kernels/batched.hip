@@ -32,13 +32,6 @@ namespace {
 
 // CMed (k 3..4) and CBig (k 5..8) come from kernels_ia.h
 
-// words of a record slot: the largest record a bucket's capacity allows
-// (header, vertices, faces with their cycles, coincidence groups)
-template <class C>
-constexpr uint32_t rec_words() {
-    return 8 + 4 * C::MV + C::MF * (4 + C::MFV) + 2 * C::MP;
-}
-
 constexpr uint32_t K1_FLAG = 0x80000000u;
 constexpr uint32_t ERR_OVERFLOW = 8;
 

@@ -74,12 +74,6 @@ struct MITile {
     uint32_t v[MT_N];
 };
 
-// a tet's place among the cut lists (bucket_of_k) and its slot's words
-__device__ inline uint32_t mi_slot_words(int k) {
-    constexpr uint32_t wide = 8 + 4 * CWideMI::MV + CWideMI::MF * (4 + CWideMI::MFV) + 2 * CWideMI::MP;
-    return k > 8 ? wide : rec_bound(1, k);
-}
-
 // The highest materials at a tet's corners are active; so is every material
 // above the lowest of those at two corners or more
 // (src/material_interface.cpp:94-152).  Few tets have two materials among
@@ -175,7 +169,7 @@ __global__ void __launch_bounds__(kMiLanes) k_mi_count_tiles(GridView g, const d
         const int b = bucket_of_k(k, tables);
 #pragma unroll
         for (int z = 0; z < 4; ++z) s[MT_LIST + z] += b == z;
-        s[MT_WORDS] += mi_slot_words(k);
+        s[MT_WORDS] += rec_bound(1, k);
         s[MT_HIST] += k == 2;
         s[MT_HIST + 1] += k == 3;
         s[MT_HIST + 2] += k > 3;
@@ -239,9 +233,11 @@ __global__ void __launch_bounds__(1024) k_mi_tile_scan(MITile* __restrict__ ts, 
     constexpr int P = 1024 + 1024 / 16;  // a pad word every 16 against bank conflicts
     __shared__ uint32_t sm[MT_N][P];
     __shared__ uint32_t tot[MT_N];
+    __shared__ uint32_t wrapped;  // tot[MT_WORDS] has passed 2^32
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     static_assert(MT_N == 16, "a wavefront a field");
     if (threadIdx.x < MT_N) tot[threadIdx.x] = 0;
+    if (threadIdx.x == 0) wrapped = 0;
     for (uint32_t base = 0; base < n; base += 1024) {
         const uint32_t i = base + threadIdx.x;
         const int pi = threadIdx.x + threadIdx.x / 16;
@@ -255,10 +251,16 @@ __global__ void __launch_bounds__(1024) k_mi_tile_scan(MITile* __restrict__ ts, 
             for (int e = 0; e < 16; ++e) sum = f == MT_KMAX ? max(sum, sm[f][p0 + e]) : sum + sm[f][p0 + e];
             if (f < kMiPrefixes) {
                 uint32_t inc = sum;
+                bool wrap = false;
                 for (int d = 1; d < 64; d <<= 1) {
                     const uint32_t o = __shfl_up(inc, d, 64);
-                    if (lane >= d) inc += o;
+                    if (lane >= d) {
+                        inc += o;
+                        wrap |= inc < o;
+                    }
                 }
+                wrap |= tot[f] + inc < inc;
+                if (f == MT_WORDS && wrap) wrapped = 1;
                 uint32_t run = tot[f] + inc - sum;
                 for (int e = 0; e < 16; ++e) {
                     const uint32_t v = sm[f][p0 + e];
@@ -287,7 +289,7 @@ __global__ void __launch_bounds__(1024) k_mi_tile_scan(MITile* __restrict__ ts, 
         ctr[M_LIST + 7] = tot[MT_N34];
         ctr[M_LIST + 8] = tot[MT_N58];
         ctr[M_LIST + 9] = tot[MT_KMAX];
-        ctr[M_WORDS] = tot[MT_WORDS];
+        ctr[M_WORDS] = wrapped ? 0xFFFFFFFFu : tot[MT_WORDS];  // (past any capacity)
         csr_off[T] = tot[MT_FIT];
         mi_check(ctr, c, errs);
         if (!ctr[M_ABORT]) rec_off[tot[MT_ACTIVE]] = tot[MT_WORDS];
@@ -322,7 +324,7 @@ __global__ void __launch_bounds__(kMiLanes) k_mi_fill_tiles(uint64_t T, const ui
         if (k < 2) continue;
         a += (uint64_t)k | 1ull << 32;
         b += 1ull << (16 * bucket_of_k(k, tables));
-        w += mi_slot_words(k);
+        w += rec_bound(1, k);
     }
     uint64_t ia = a, ib = b;
     uint32_t iw = w;
@@ -372,7 +374,7 @@ __global__ void __launch_bounds__(kMiLanes) k_mi_fill_tiles(uint64_t T, const ui
         for (uint32_t x = o; m; m &= m - 1) fit[x++] = (uint8_t)(__ffsll((unsigned long long)m) - 1);
         o += (uint32_t)k;
         ++r;
-        at += mi_slot_words(k);
+        at += rec_bound(1, k);
     }
     __syncthreads();
     for (uint32_t q = tid; q < kMiTile; q += kMiLanes)

@@ -249,13 +249,19 @@ __global__ void k_fill(uint64_t T, const uint64_t* __restrict__ amask, const uin
     }
 }
 
-// record slot bound per active count
+// words of the largest record that a complex's capacity allows (header,
+// vertices, faces with their cycles, coincidence groups)
+template <class C>
+__host__ __device__ constexpr uint32_t rec_words() {
+    return 8 + 4 * C::MV + C::MF * (4 + C::MFV) + 2 * C::MP;
+}
+
+// record slot bound per active count; beyond 8 what the lane-group cut holds
+// (a complex beyond that gets a slot behind the others)
 __device__ inline uint32_t rec_bound(int mi, int k) {
     const uint32_t ia[9] = {0, 128, 256, 448, 768, 1280, 1920, 2560, 3200};
     const uint32_t m[9] = {0, 64, 128, 256, 320, 400, 480, 560, 640};
-    // beyond 8: everything a CHuge complex can hold
-    constexpr uint32_t huge = 8 + 4 * CHuge::MV + CHuge::MF * (4 + CHuge::MFV) + 2 * CHuge::MP;
-    return (k < 0 || k > 8) ? huge : (mi ? m[k] : ia[k]);
+    return (k < 0 || k > 8) ? (mi ? rec_words<CWideMI>() : rec_words<CWide>()) : (mi ? m[k] : ia[k]);
 }
 
 __global__ void k_rec_bound(Count n, const uint8_t* __restrict__ act_k, int mi, uint32_t* __restrict__ b) {
@@ -1629,12 +1635,13 @@ __global__ void __launch_bounds__(1024) k_dedup_tile_scan(Count n, uint32_t* __r
 // two functions (by table, or by groups of 8 lanes), 1: up to 4 functions, 2: 5..8, 3: more.  Per chunk of kBucketChunk active tets,
 // kBucketWords words: list sizes [0..4), the reference's bucket histogram
 // [4..7) (IA: 1, 2, >= 3 functions; MI: 2, 3, >= 4), tets with 3..4 and
-// 5..8 functions [7], [8], the largest count [9] (k_bucket_count).  One
+// 5..8 functions [7], [8], the largest count [9], the words of their record
+// slots [10] (k_bucket_count).  One
 // workgroup turns the list sizes into each chunk's list offsets and writes
 // the totals (k_bucket_scan); each chunk then writes its entries
 // (k_bucket_fill).  No atomics.
 constexpr uint32_t kBucketChunk = 2048;
-constexpr int kBucketWords = 10;
+constexpr int kBucketWords = 11;
 
 // table2: 1 material interfaces (two and three materials by table), 2
 // implicit arrangements (one and two functions), 0 material interfaces
@@ -1650,7 +1657,7 @@ __global__ void __launch_bounds__(256) k_bucket_count(Count nc, const uint8_t* _
     const uint64_t base = (uint64_t)blockIdx.x * kBucketChunk;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lo = mi ? 2 : 1;
-    uint32_t w[kBucketWords] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    uint32_t w[kBucketWords] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (uint32_t i = threadIdx.x; i < kBucketChunk; i += 256) {
         const uint64_t a = base + i;
         if (a >= n) break;
@@ -1666,6 +1673,7 @@ __global__ void __launch_bounds__(256) k_bucket_count(Count nc, const uint8_t* _
         w[7] += k >= 3 && k <= 4;
         w[8] += k >= 5 && k <= 8;
         w[9] = max(w[9], (uint32_t)k);
+        w[10] += rec_bound(mi, k);
     }
     __shared__ uint32_t red[256 / 64][kBucketWords];
 #pragma unroll
@@ -1686,20 +1694,24 @@ __global__ void __launch_bounds__(256) k_bucket_count(Count nc, const uint8_t* _
     }
 }
 
-// one workgroup of 1024 lanes; tot: the 10 totals
+// one workgroup of 1024 lanes; tot: the totals, [10] and [11] the words' low
+// and high half (their sum can pass 32 bits)
 __global__ void __launch_bounds__(1024) k_bucket_scan(uint32_t nchunks, uint32_t* __restrict__ bc,
                                                       uint32_t* __restrict__ tot) {
     // statistics first (the scan overwrites the list sizes only)
-    __shared__ uint32_t red[16][kBucketWords];
+    constexpr int NS = kBucketWords - 5;
+    __shared__ uint32_t red[16][NS];
+    __shared__ uint64_t redw[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t w[kBucketWords - 4] = {0, 0, 0, 0, 0, 0};
-    for (uint32_t c = threadIdx.x; c < nchunks; c += 1024)
-        for (int f = 0; f < kBucketWords - 4; ++f) {
-            const uint32_t x = bc[(uint64_t)c * kBucketWords + 4 + f];
-            w[f] = f == 5 ? max(w[f], x) : w[f] + x;
-        }
+    uint32_t w[NS] = {0, 0, 0, 0, 0, 0};
+    uint64_t words = 0;
+    for (uint32_t c = threadIdx.x; c < nchunks; c += 1024) {
+        const uint32_t* x = bc + (uint64_t)c * kBucketWords + 4;
+        for (int f = 0; f < NS; ++f) w[f] = f == 5 ? max(w[f], x[f]) : w[f] + x[f];
+        words += x[NS];
+    }
 #pragma unroll
-    for (int f = 0; f < kBucketWords - 4; ++f) {
+    for (int f = 0; f < NS; ++f) {
         uint32_t x = w[f];
         for (int d = 32; d > 0; d >>= 1) {
             const uint32_t y = __shfl_xor(x, d, 64);
@@ -1707,12 +1719,19 @@ __global__ void __launch_bounds__(1024) k_bucket_scan(uint32_t nchunks, uint32_t
         }
         if (lane == 0) red[wave][f] = x;
     }
+    for (int d = 32; d > 0; d >>= 1) words += __shfl_xor(words, d, 64);
+    if (lane == 0) redw[wave] = words;
     __syncthreads();
-    if (threadIdx.x < kBucketWords - 4) {
+    if (threadIdx.x < NS) {
         const int f = threadIdx.x;
         uint32_t x = 0;
         for (int v = 0; v < 16; ++v) x = f == 5 ? max(x, red[v][f]) : x + red[v][f];
         tot[4 + f] = x;
+    } else if (threadIdx.x == 64) {
+        words = 0;
+        for (int v = 0; v < 16; ++v) words += redw[v];
+        tot[4 + NS] = (uint32_t)words;
+        tot[5 + NS] = (uint32_t)(words >> 32);
     }
     __syncthreads();
     const TileTotals tt = {{tot, tot + 1, tot + 2, tot + 3}};

@@ -646,14 +646,13 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, s, nch, bc.p, bo.p);
         hipLaunchKernelGGL(k_bucket_fill, dim3(nch), dim3(256), 0, s, Count(NA), (const uint8_t*)out.act_k.p, table_mode,
                            (const uint32_t*)bc.p, blist[0], blist[1], blist[2], blist[3]);
-        copy_u32(bo.p + 15, out.rec_off.p + NA, Count(1), s);
         RIN_HIP(hipGetLastError());
         uint32_t hb[16];
         RIN_HIP(hipMemcpyAsync(hb, bo.p, sizeof(hb), hipMemcpyDeviceToHost, s));
         RIN_HIP(hipStreamSynchronize(s));
         for (int q = 0; q < 4; ++q) bcnt[q] = hb[q];
         for (int q = 0; q < 3; ++q) out.nb[q] = hb[4 + q];
-        nwords = hb[15];
+        nwords = (uint64_t)hb[11] << 32 | hb[10];
         out.n_cut34 = hb[7];
         out.n_cut58 = hb[8];
         if ((int)hb[9] > kMaxHuge) {
@@ -662,6 +661,9 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
                                      " active functions; the device cut supports at most " +
                                      std::to_string(kMaxHuge));
         }
+        // the offsets are 32-bit words, and of arrangements bit 31 is k_vert_fields_ia's table flag
+        if (nwords >= (1ull << (MI ? 32 : 31)) - 4)
+            throw std::runtime_error("the record slots exceed 2^" + std::to_string(MI ? 32 : 31) + " words");
     } else {
         fill_u32(out.rec_off.p, 0, 1, s);
     }
@@ -771,7 +773,7 @@ void run_pipeline(DevMem& mem, const Grid& g, const Values& val, uint32_t flags,
         std::vector<uint32_t> retry;
         for (uint64_t a = 0; a < NA; ++a)
             if (hc[3 * a] == CNT_RETRY) retry.push_back((uint32_t)a);
-        constexpr uint32_t slot = 8 + 4 * CHuge::MV + CHuge::MF * (4 + CHuge::MFV) + 2 * CHuge::MP;
+        constexpr uint32_t slot = rec_words<CHuge>();
         const uint64_t total = nwords + (uint64_t)slot * retry.size();
         if (total >= (1ull << 31)) throw std::runtime_error("record buffer exceeds 2^31 words");
         DBuf<uint16_t> rec2(mem, total + 4);
@@ -1044,7 +1046,7 @@ __global__ void k_rec_lookup(const uint32_t* __restrict__ tets, uint64_t n, uint
             const uint32_t rk = rank(t, (uint32_t)n_active);
             if (rk != ~0u) {
                 const uint32_t loc = rec_loc ? rec_loc[rk] : 0u;
-                if (rec_loc && (loc & 0x80000000u)) {
+                if (k1_rec && (loc & 0x80000000u)) {
                     o = (1ull << 63) | k1_off[loc & 0x7FFFFFFFu];
                     L = k1_rec[k1_off[loc & 0x7FFFFFFFu] + 6];
                 } else {

@@ -129,3 +129,33 @@ def test_more_functions_than_the_cut_takes(ctx, regular):
     for v in values.values():
         v.release()
     g.release()
+
+
+@pytest.mark.parametrize("mi,F,res", [(0, 12, 50), (1, 12, 62)])
+def test_record_words_past_32_bits(ctx, mi, F, res):
+    """Most tets with more than 8 functions: their record slots' words pass 2^32,
+    and the run is refused before anything of their size is allocated."""
+    import rin
+
+    pts, tets = S.grid(res)
+    rng = np.random.default_rng(6)
+    vals = rng.uniform(-1.0, 1.0, (len(pts), F))
+    if mi:
+        vals[:, :] = rng.permuted(np.tile(np.arange(F, dtype=np.float64), (len(pts), 1)), axis=1)
+        c = vals[tets.astype(int)]  # a lower bound of a tet's materials: each corner's highest, and the rule's
+        top = c.argmax(2)
+        low = np.stack([np.take_along_axis(c[:, q], top, 1).min(1) for q in range(4)], 1)
+        active = ((c > low[:, :, None]).sum(1) > 1)
+        np.put_along_axis(active, top, True, 1)
+        k, words = active.sum(1), 7928
+    else:
+        c = vals[tets.astype(int)]
+        k, words = (~((c > 0).all(1) | (c < 0).all(1))).sum(1), 13248
+    assert k.max() <= 28 and int((k > 8).sum()) * words > 1 << 32
+    g = ctx.grid_regular(res)
+    v = g.upload(vals)
+    for flags in (rin.FLAG_BATCHED, 0, rin.FLAG_NO_LOOKUP):
+        with pytest.raises(rin.RinError, match="record slots exceed"):
+            v.run(flags | (rin.FLAG_MI if mi else 0))
+    v.release()
+    g.release()
