@@ -15,7 +15,7 @@
 
 #include <algorithm>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "../devmem.h"
@@ -164,8 +164,9 @@ void HostStage::fetch(int device, const std::vector<PackCol>& cols, hipStream_t 
     int started = 1;
     try {
         for (; started < threads; ++started) pool.emplace_back(guarded, started);
-    } catch (const std::system_error&) {
-        // no thread to be had: this one takes the rest's chunks after its own
+    } catch (...) {
+        // no thread to be had (or no memory for one; nothing may leave here
+        // while others run): this one takes the rest's chunks after its own
     }
     guarded(0);
     for (int t = started; t < threads; ++t) guarded(t);
