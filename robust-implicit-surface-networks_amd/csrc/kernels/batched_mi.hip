@@ -37,6 +37,7 @@ enum MICtr : uint32_t {
     M_VO, M_FO, M_FV,  // vertex occurrences, faces, face corners
     M_NV,          // vertices after dedup
     M_FIT,         // active (tet, material) entries: the CSR's total
+    M_EMIT,        // tet-boundary faces among the faces (MIEmits)
     M_ABORT,       // a count exceeded its capacity: later stages process nothing
     M_N
 };
@@ -473,7 +474,8 @@ struct MIWorkspace {
     DBuf<uint32_t> rec_loc;
     uint32_t tab_base2 = 0, tab_base3 = 0;
     DBuf<uint16_t> rec;
-    DBuf<uint64_t> emask;
+    DBuf<uint2> emit_at;      // MIEmits
+    DBuf<uint32_t> emit_list;
     unsigned cut_blocks[2] = {0, 0};
     bool wide = false;  // the path holds the cut of more than 8 materials, once a run needs it
     // per occurrence, face
@@ -574,7 +576,8 @@ void alloc_mi(MIWorkspace& W, const Grid& g, const MICaps& c, hipStream_t s) {
     }
     W.cnt.alloc(m, 3 * A + 3);
     W.labels.alloc(m, A + 1);
-    W.emask.alloc(m, A + 1);
+    W.emit_at.alloc(m, A + 1);
+    W.emit_list.alloc(m, c.fo + 1);
     W.cv.alloc(m, A + 2);
     W.cf.alloc(m, A + 2);
     W.cfv.alloc(m, A + 2);
@@ -717,8 +720,9 @@ void mi_path(MIWorkspace& W, const Grid& g, uint32_t F, const MITablesDev& TT, h
     A.fit = W.fit.p;
     A.rec = W.rec.p;
     A.n_active = NA;
-    hipLaunchKernelGGL(k_mi_pair, dim3(blocks_for(c.active)), dim3(256), 0, s, A, (const uint32_t*)W.labels.p,
-                       W.emask.p, W.cnt.p);
+    const MIEmits E{W.emit_at.p, W.emit_list.p, c.fo, ctr + M_EMIT};
+    hipLaunchKernelGGL(k_mi_pair, dim3(blocks_for(c.active)), dim3(256), 0, s, A, (const uint32_t*)W.labels.p, E,
+                       W.cnt.p);
     {
         const uint32_t* in[3] = {W.cnt.p, W.cnt.p + 1, W.cnt.p + 2};
         uint32_t* out[3] = {W.cv.p, W.cf.p, W.cfv.p};
@@ -726,7 +730,7 @@ void mi_path(MIWorkspace& W, const Grid& g, uint32_t F, const MITablesDev& TT, h
         scan3_u32(W.mem, in, 3, out, NA, tot, s);
     }
     hipLaunchKernelGGL(k_mi_check, dim3(1), dim3(64), 0, s, ctr, c, W.errs.p);
-    hipLaunchKernelGGL(k_mi_extract, dim3(blocks_for(c.active)), dim3(256), 0, s, A, (const uint64_t*)W.emask.p,
+    hipLaunchKernelGGL(k_mi_extract, dim3(blocks_for(c.active)), dim3(256), 0, s, A, E,
                        (const uint32_t*)W.cv.p, (const uint32_t*)W.cf.p, (const uint32_t*)W.cfv.p, W.okey.p, W.oa.p,
                        W.oj.p, W.fq_a.p, W.fq_l.p, W.fq_m.p, W.fq_vs.p, W.fve.p);
     // vertex dedup: on regular grids each key's first occurrence by its

@@ -269,44 +269,16 @@ __device__ inline uint64_t mi_vkey(const GridView& g, const MITet& M, const uint
     return key_inner(a, j);
 }
 
-// Material set on the inner side of a tet-boundary face: its negative
-// label's material, or every material of that label's coincidence group (in
-// label order).  Enumerated, not stored: an indexed local array would live in
-// scratch memory.
-template <class Fn>
-__device__ inline void mi_side_each(const MITet& M, const uint8_t* __restrict__ fit, int neg, Fn&& fn) {
+// Materials (bits) on the inner side of a tet-boundary face: its negative
+// label's, or every material of that label's coincidence group.
+__device__ inline uint64_t mi_side(const MITet& M, const uint8_t* __restrict__ fit, int neg) {
+    uint64_t m = 1ull << fit[M.s0 + neg - 4];
     if (M.R.dup) {
         const uint16_t* grp = M.groups();
-        int n = 0;
-        for (int l = 4; l < M.R.L; ++l) n += grp[l] == grp[neg];
-        if (n > 1) {
-            for (int l = 4; l < M.R.L; ++l)
-                if (grp[l] == grp[neg]) fn((uint8_t)fit[M.s0 + l - 4]);
-            return;
-        }
+        for (int l = 4; l < M.R.L; ++l)
+            if (grp[l] == grp[neg]) m |= 1ull << fit[M.s0 + l - 4];
     }
-    fn((uint8_t)fit[M.s0 + neg - 4]);
-}
-
-// (min, second-min, max) of a face's vertex keys
-__device__ inline void mi_face_triple(const GridView& g, const MITet& M, const uint8_t* __restrict__ fit, uint64_t a,
-                                      const uint16_t* F, uint64_t k3[3]) {
-    const int n = F[3];
-    uint64_t mn = ~0ull, sm = ~0ull, mx = 0;
-    for (int q = 0; q < n; ++q) {
-        int nb;
-        const uint64_t k = mi_vkey(g, M, fit, a, F[4 + q], nb);
-        if (k < mn) {
-            sm = mn;
-            mn = k;
-        } else if (k < sm) {
-            sm = k;
-        }
-        if (k > mx) mx = k;
-    }
-    k3[0] = mn;
-    k3[1] = sm;
-    k3[2] = mx;
+    return m;
 }
 
 struct MIArgs {
@@ -317,43 +289,147 @@ struct MIArgs {
     Count n_active;
 };
 
+// whether tet t2 is active with a complete record; r2 is then its active rank
+__device__ inline bool mi_active(const MIArgs& A, uint32_t t2, uint32_t& r2) {
+    r2 = A.rank[t2];
+    return r2 < count_of(A.n_active) && A.act[r2] == t2 && A.rec[A.rec_loc[r2]] == 2;  // (else its cut failed)
+}
+
+// local vertex of active tet r2 (tet t2) with key k, or -1
+__device__ inline int mi_find_vertex(const MIArgs& A, uint32_t t2, uint32_t r2, uint64_t k) {
+    const MITet N(A.g, A.rec + A.rec_loc[r2], t2, A.csr_off[t2]);
+    for (int j = 0; j < N.R.nv; ++j) {
+        int nb;
+        if (mi_vkey(A.g, N, A.fit, r2, j, nb) == k) return j;
+    }
+    return -1;
+}
+
+// The reference's order among the vertices of a tet-boundary face (by id;
+// corners as minus their vertex id, below all others): for local vertex j,
+// key k, of active tet a.  Ids are given in tet order and, in a tet, in local
+// order, so a vertex off the corners stands where the first tet that holds it
+// lists it: of the two tets at a tet face, or of those around a tet edge
+// (walked through the tet faces at the edge, both ways from an open end).
+__device__ inline int64_t mi_vertex_order(const MIArgs& A, const MITet& M, int j, uint64_t k) {
+    const uint16_t* L4 = M.R.vert(j);
+    unsigned bm = 0;  // the tet faces that it lies on
+#pragma unroll
+    for (int q = 0; q < 4; ++q) bm |= L4[q] <= 3 ? 1u << L4[q] : 0u;
+    if (__popc(bm) == 3) return -(int64_t)M.vc(__builtin_ctz(~bm & 15u)) - 1;
+    uint32_t first = M.t;
+    int at = j;
+    const unsigned em = ~bm & 15u;  // on an edge: its two corners
+    const bool edge = __popc(bm) == 2;
+    const uint32_t ea = M.vc(__builtin_ctz(em)), eb = edge ? M.vc(__builtin_ctz(em & (em - 1))) : ea;
+    bool closed = false;
+    for (unsigned way = bm; way && !closed; way &= way - 1) {
+        uint32_t t = M.t, c = (uint32_t)__builtin_ctz(way);
+        for (int step = 0; step < 4096; ++step) {  // (an edge has a few tets; the bound is for broken meshes)
+            const uint32_t nb = A.nbr[4 * (uint64_t)t + c];
+            if (nb == NO_NBR) break;
+            t = nb >> 2;
+            if (t == M.t) {
+                closed = true;
+                break;
+            }
+            uint32_t r2;
+            if (t < first && mi_active(A, t, r2)) {
+                const int q = mi_find_vertex(A, t, r2, k);
+                if (q >= 0) {
+                    first = t;
+                    at = q;
+                }
+            }
+            if (!edge) break;
+            // on through the other tet face at the edge: that opposite the
+            // corner which is neither the edge's nor opposite the way in
+            uint32_t v[4];
+            dev::tet_corners(A.g, t, v);
+            uint32_t next = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if (q != (nb & 3) && v[q] != ea && v[q] != eb) next = q;
+            c = next;
+        }
+    }
+    return (int64_t)first << 16 | at;
+}
+
+// (min, second-min, max) of a tet-boundary face's vertices in that order: their keys
+__device__ inline void mi_face_triple(const MIArgs& A, const MITet& M, uint64_t a, const uint16_t* F, uint64_t k3[3]) {
+    const int n = F[3];
+    int64_t mn = INT64_MAX, sm = INT64_MAX, mx = INT64_MIN;
+    for (int q = 0; q < n; ++q) {
+        int nb;
+        const uint64_t k = mi_vkey(A.g, M, A.fit, a, F[4 + q], nb);
+        const int64_t o = mi_vertex_order(A, M, F[4 + q], k);
+        if (o < mn) {
+            sm = mn;
+            k3[1] = k3[0];
+            mn = o;
+            k3[0] = k;
+        } else if (o < sm) {
+            sm = o;
+            k3[1] = k;
+        }
+        if (o > mx) {
+            mx = o;
+            k3[2] = k;
+        }
+    }
+}
+
+// Whether G of active tet r2 is the reference's first copy of F of active tet a
+// (both on one tet face): faces are one to it when their least, second and
+// greatest vertices are.  Those of equal vertices are; where ties name some
+// vertices after different materials, the three decide.
+__device__ inline bool mi_same_bface(const MIArgs& A, const MITet& M, uint64_t a, const uint16_t* F, const MITet& N,
+                                     uint64_t r2, const uint16_t* G) {
+    const int n = F[3], m = G[3];
+    int common = 0;
+    for (int q = 0; q < n; ++q) {
+        int nb;
+        const uint64_t k = mi_vkey(A.g, M, A.fit, a, F[4 + q], nb);
+        bool in = false;
+        for (int p = 0; p < m && !in; ++p) in = mi_vkey(A.g, N, A.fit, r2, G[4 + p], nb) == k;
+        common += in;
+        if (common + n - 1 - q < 3) return false;
+    }
+    if (common == n && common == m) return true;
+    uint64_t f3[3], g3[3];
+    mi_face_triple(A, M, a, F, f3);
+    mi_face_triple(A, N, r2, G, g3);
+    return f3[0] == g3[0] && f3[1] == g3[1] && f3[2] == g3[2];
+}
+
 // whether tet-boundary face F of active tet a becomes an interface face
-// here (the second copy); `other` is the first copy's material
+// here (the second copy); `other` is the first copy's material, the lowest.
+// A face of the neighbour with a material of F's is F's region: its copy, or
+// none is; either way F does not emit, and only where no material of F's
+// recurs do the faces themselves decide.
 __device__ inline bool mi_bface_emits(const MIArgs& A, const MITet& M, uint64_t a, const uint16_t* F,
                                       uint8_t& other) {
     const int l = F[0];
     const uint32_t nb = A.nbr[4 * (uint64_t)M.t + l];
     if (nb == NO_NBR) return false;
     const uint32_t t2 = nb >> 2, l2 = nb & 3;
-    if (t2 >= M.t) return false;
-    const uint32_t r2 = A.rank[t2];
-    if (!(r2 < count_of(A.n_active) && A.act[r2] == t2)) return false;
-    uint64_t k3[3];
-    bool have_k3 = false;
+    uint32_t r2;
+    if (t2 >= M.t || !mi_active(A, t2, r2)) return false;
     const MITet N(A.g, A.rec + A.rec_loc[r2], t2, A.csr_off[t2]);
-    if (N.R.r[0] != 2) return false;  // its cut failed (and with it the run)
+    const uint64_t mine = mi_side(M, A.fit, F[1]);
     const uint16_t* G = N.R.faces();
     for (int f = 0; f < N.R.nf; ++f) {
-        const int n = G[3];
-        // a copy lies on the shared tet face and has as many corners
-        if (G[0] == l2 && n == F[3]) {
-            if (!have_k3) {
-                mi_face_triple(A.g, M, A.fit, a, F, k3);
-                have_k3 = true;
-            }
-            uint64_t q3[3];
-            mi_face_triple(A.g, N, A.fit, r2, G, q3);
-            if (q3[0] == k3[0] && q3[1] == k3[1] && q3[2] == k3[2]) {
-                bool share = false, first = true;
-                mi_side_each(N, A.fit, G[1], [&](uint8_t x) {
-                    if (first) other = x;
-                    first = false;
-                    mi_side_each(M, A.fit, F[1], [&](uint8_t y) { share |= x == y; });
-                });
-                return !share;
-            }
+        if (G[0] == l2 && (mi_side(N, A.fit, G[1]) & mine)) return false;
+        G += 4 + G[3];
+    }
+    G = N.R.faces();
+    for (int f = 0; f < N.R.nf; ++f) {
+        if (G[0] == l2 && mi_same_bface(A, M, a, F, N, r2, G)) {
+            other = (uint8_t)__builtin_ctzll(mi_side(N, A.fit, G[1]));
+            return true;
         }
-        G += 4 + n;
+        G += 4 + G[3];
     }
     return false;
 }
@@ -371,9 +447,15 @@ __device__ inline int corner_of(const Rec& R, int j) {
 }
 
 // Which tet-boundary faces of each active tet become interface faces here
-// (the reference's two-map pairing): bit f for face f < 63; bit 63 marks a
-// tet with more faces, whose faces from 63 on are tested where they are used.
-//
+// (the reference's two-map pairing), listed per tet in face order with the
+// first copy's material, so that the extraction compares no faces.
+struct MIEmits {
+    uint2* at;       // per active tet: its first entry and how many
+    uint32_t* list;  // face | material << 16
+    uint32_t cap;    // entries there is room for (past it the faces' capacity stops the run as well)
+    uint32_t* n;
+};
+
 // A face emits when its copy in the lower neighbour carries other materials.
 // In each tet a material without coincident ones has one face on a tet face,
 // the region where it is the highest there, so when the neighbour has a face
@@ -388,10 +470,8 @@ __device__ inline int corner_of(const Rec& R, int j) {
 //
 // counts: cnt holds the cut's interface vertices, faces and corners; a tet
 // that emits adds its own.
-constexpr int kBfaceBits = 63;
-
-__global__ void k_mi_pair(MIArgs A, const uint32_t* __restrict__ labels, uint64_t* __restrict__ emask,
-                          uint32_t* __restrict__ cnt) {
+__global__ void __launch_bounds__(256) k_mi_pair(MIArgs A, const uint32_t* __restrict__ labels, MIEmits E,
+                                                 uint32_t* __restrict__ cnt) {
     const uint64_t n = count_of(A.n_active);
     GRID_STRIDE(a, A.n_active) {
         const uint32_t t = A.act[a], lm = labels[a], s0 = A.csr_off[t];
@@ -417,42 +497,35 @@ __global__ void k_mi_pair(MIArgs A, const uint32_t* __restrict__ labels, uint64_
             for (uint32_t m = lo >> (8 * l2[l]) & 255u; m; m &= m - 1) theirs |= 1ull << A.fit[s2 + __builtin_ctz(m)];
             for (uint32_t m = lm >> (8 * l) & 255u; m; m &= m - 1) ask |= !(theirs >> A.fit[s0 + __builtin_ctz(m)] & 1);
         }
-        uint64_t em = 0;
+        uint2 em = make_uint2(0, 0);
         if (ask) {
             const MITet M(A.g, A.rec + A.rec_loc[a], t, s0);
             if (M.R.r[0] == 2) {
-                uint32_t nv = cnt[3 * a], nf = cnt[3 * a + 1], nfv = cnt[3 * a + 2];
-                const uint16_t* F = M.R.faces();
-                for (int f = 0; f < M.R.nf; ++f) {
-                    const int c = F[3];
-                    uint8_t other;
-                    if (F[0] <= 3 && mi_bface_emits(A, M, a, F, other)) {
-                        if (f < kBfaceBits) em |= 1ull << f;
-                        ++nf;
-                        nfv += c;
-                        for (int q = 0; q < c; ++q) nv += is_corner(M.R, F[4 + q]);
+                // counted, then (few tets) listed
+                for (int pass = 0; pass < 2; ++pass) {
+                    uint32_t ne = 0, nv = 0, nfv = 0;
+                    const uint16_t* F = M.R.faces();
+                    for (int f = 0; f < M.R.nf; ++f) {
+                        const int c = F[3];
+                        uint8_t other;
+                        if (F[0] <= 3 && mi_bface_emits(A, M, a, F, other)) {
+                            if (pass && em.x + ne < E.cap) E.list[em.x + ne] = (uint32_t)f | (uint32_t)other << 16;
+                            ++ne;
+                            nfv += c;
+                            for (int q = 0; q < c; ++q) nv += is_corner(M.R, F[4 + q]);
+                        }
+                        F += 4 + c;
                     }
-                    F += 4 + c;
+                    if (!ne || pass) break;
+                    em = make_uint2(atomicAdd(E.n, ne), ne);
+                    cnt[3 * a] += nv;
+                    cnt[3 * a + 1] += ne;
+                    cnt[3 * a + 2] += nfv;
                 }
-                if (M.R.nf > kBfaceBits) em |= 1ull << kBfaceBits;
-                cnt[3 * a] = nv;
-                cnt[3 * a + 1] = nf;
-                cnt[3 * a + 2] = nfv;
             }
         }
-        emask[a] = em;
+        E.at[a] = em;
     }
-}
-
-// whether tet-boundary face f (record words F) emits here, from the mask
-__device__ inline bool mi_emits(const MIArgs& A, const MITet& M, uint64_t a, const uint16_t* F, int f, uint64_t em,
-                                uint8_t& other) {
-    if (f < kBfaceBits) {
-        if (!((em >> f) & 1)) return false;
-        // rare: the scan again for the first copy's material
-        return mi_bface_emits(A, M, a, F, other);
-    }
-    return (em >> kBfaceBits) && mi_bface_emits(A, M, a, F, other);
 }
 
 // One tet's occurrences and face rows.  W words of vertex mask: one for the
@@ -460,8 +533,9 @@ __device__ inline bool mi_emits(const MIArgs& A, const MITet& M, uint64_t a, con
 // any record, indexed, live in scratch memory and cost every lane: 55 us at
 // 65^3 vertices and 8 materials against 43, 86 at 100^3 and 18 against 60).
 template <int W>
-__device__ inline void mi_extract_tet(const MIArgs& A, const MITet& M, uint64_t a, uint64_t em, uint32_t vb, uint32_t q,
-                                      uint32_t e, uint64_t* __restrict__ okey, uint32_t* __restrict__ oa,
+__device__ inline void mi_extract_tet(const MIArgs& A, const MITet& M, uint64_t a, const uint2 em,
+                                      const uint32_t* __restrict__ emits, uint32_t vb, uint32_t q, uint32_t e,
+                                      uint64_t* __restrict__ okey, uint32_t* __restrict__ oa,
                                       uint16_t* __restrict__ oj, uint32_t* __restrict__ fq_a,
                                       uint16_t* __restrict__ fq_l, uint8_t* __restrict__ fq_m,
                                       uint32_t* __restrict__ fq_vs, uint32_t* __restrict__ fve) {
@@ -490,14 +564,15 @@ __device__ inline void mi_extract_tet(const MIArgs& A, const MITet& M, uint64_t 
         return r + (uint32_t)__popcll(m[W == 1 ? 0 : j >> 6] & ((1ull << (j & 63)) - 1));
     };
     F = M.R.faces();
+    uint32_t ne = em.x;
+    uint32_t next = em.y ? emits[ne] : 0xFFFFu;  // the next face that emits, its first copy's material
     for (int f = 0; f < M.R.nf; ++f) {
         const int n = F[3];
-        uint8_t other = 0xFF;
         const bool iface = F[0] > 3;
-        if (iface || mi_emits(A, M, a, F, f, em, other)) {
+        if (iface || (next & 0xFFFFu) == (uint32_t)f) {
             fq_a[q] = (uint32_t)a;
             fq_l[q] = (uint16_t)f;
-            fq_m[2 * q] = iface ? A.fit[M.s0 + F[0] - 4] : other;
+            fq_m[2 * q] = iface ? A.fit[M.s0 + F[0] - 4] : (uint8_t)(next >> 16);
             fq_m[2 * q + 1] = A.fit[M.s0 + F[1] - 4];
             fq_vs[q] = e;
             for (int i = 0; i < n; ++i) {
@@ -512,13 +587,14 @@ __device__ inline void mi_extract_tet(const MIArgs& A, const MITet& M, uint64_t 
                     fve[e++] = vb + rank(j);
                 }
             }
+            if (!iface) next = ++ne < em.x + em.y ? emits[ne] : 0xFFFFu;
             ++q;
         }
         F += 4 + n;
     }
 }
 
-__global__ void __launch_bounds__(256) k_mi_extract(MIArgs A, const uint64_t* __restrict__ emask, const uint32_t* __restrict__ voff,
+__global__ void __launch_bounds__(256) k_mi_extract(MIArgs A, MIEmits E, const uint32_t* __restrict__ voff,
                              const uint32_t* __restrict__ foff, const uint32_t* __restrict__ fvoff,
                              uint64_t* __restrict__ okey,
                              uint32_t* __restrict__ oa, uint16_t* __restrict__ oj, uint32_t* __restrict__ fq_a,
@@ -528,10 +604,12 @@ __global__ void __launch_bounds__(256) k_mi_extract(MIArgs A, const uint64_t* __
         const uint32_t t = A.act[a];
         const MITet M(A.g, A.rec + A.rec_loc[a], t, A.csr_off[t]);
         if (M.R.r[0] != 2) continue;
+        uint2 em = E.at[a];
+        if ((uint64_t)em.x + em.y > E.cap) em.y = 0;
         if (M.R.nv <= 64)
-            mi_extract_tet<1>(A, M, a, emask[a], voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_m, fq_vs, fve);
+            mi_extract_tet<1>(A, M, a, em, E.list, voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_m, fq_vs, fve);
         else
-            mi_extract_tet<kMaskWords>(A, M, a, emask[a], voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_m,
+            mi_extract_tet<kMaskWords>(A, M, a, em, E.list, voff[a], foff[a], fvoff[a], okey, oa, oj, fq_a, fq_l, fq_m,
                                        fq_vs, fve);
     }
 }

@@ -342,9 +342,14 @@ void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, DBuf
     A.rec = out.rec.p;
     A.n_active = Count(NA);
     DBuf<uint32_t> cv(mem, NA + 1), cf(mem, NA + 1), cfv(mem, NA + 1);
-    DBuf<uint64_t> emask(mem, NA + 1);
+    // a material has at most one face on a tet face: room for every one that can emit
+    const uint32_t emit_cap = (uint32_t)std::min<uint64_t>(4 * out.n_fit, 0xFFFFFFFFu);
+    DBuf<uint2> emit_at(mem, NA + 1);
+    DBuf<uint32_t> emit_list(mem, (uint64_t)emit_cap + 1), n_emit(mem, 1);
+    const MIEmits E{emit_at.p, emit_list.p, emit_cap, n_emit.p};
+    fill_u32(n_emit.p, 0, 1, s);
     if (NA)
-        hipLaunchKernelGGL(k_mi_pair, dim3(nblk(NA)), dim3(256), 0, s, A, (const uint32_t*)labels.p, emask.p, cnt.p);
+        hipLaunchKernelGGL(k_mi_pair, dim3(nblk(NA)), dim3(256), 0, s, A, (const uint32_t*)labels.p, E, cnt.p);
     hipLaunchKernelGGL(k_split3, dim3(nblk(NA)), dim3(256), 0, s, Count(NA), (const uint32_t*)cnt.p, cv.p, cf.p,
                        cfv.p);
     scan_u32(mem, cv.p, cv.p, NA, cv.p + NA, s);
@@ -360,8 +365,7 @@ void extract_mi(DevMem& mem, const Grid& g, const Values& val, RunOut& out, DBuf
     DBuf<uint16_t> oj(mem, NVO + 1), fq_l(mem, NF + 1);
     DBuf<uint8_t> fq_m(mem, 2 * NF + 2);
     if (NA)
-        hipLaunchKernelGGL(k_mi_extract, dim3(nblk(NA)), dim3(256), 0, s, A, (const uint64_t*)emask.p,
-                           (const uint32_t*)cv.p,
+        hipLaunchKernelGGL(k_mi_extract, dim3(nblk(NA)), dim3(256), 0, s, A, E, (const uint32_t*)cv.p,
                            (const uint32_t*)cf.p, (const uint32_t*)cfv.p, okey.p, oa.p, oj.p, fq_a.p, fq_l.p, fq_m.p,
                            fq_vs.p, fve.p);
     RIN_HIP(hipGetLastError());
