@@ -4,7 +4,7 @@
 //    never runs the cut: its complex depends only on the four corner signs,
 //    so an 81-entry table built from the cut itself gives counts, iso
 //    vertices, iso faces and the record; each block stages the table in LDS.
-//  * k = 2 goes by a sign-vector table; 3..4 and 5..8 run per-bucket cut
+//  * k = 2 goes by a sign-vector table; 3..4, 5..8 and 9..28 run per-bucket cut
 //    kernels sized for that bucket: lane groups per tet with the complex in
 //    LDS, or one lane per tet (persistent grids pulling 64-tet chunks from a
 //    work queue); a small autotuner times the candidates on the run's own
@@ -2362,12 +2362,6 @@ void launch_cut_early(Workspace& W, const Grid& g, const Values& val, int q, int
         hipLaunchKernelGGL((k_cut_wave<CMed, 32, true>), dim3((cap + 1) / 2), dim3(64), 0, s, A);
 }
 
-void stage_cut(Workspace& W, const Grid& g, const Values& val, const int* grid, hipStream_t s) {
-    if (W.cap.b[0]) launch_cut<CK2>(W, g, val, 0, grid[0], s);
-    if (W.cap.b[1]) launch_cut<CMed>(W, g, val, 1, grid[1], s);
-    if (W.cap.b[2]) launch_cut<CBig>(W, g, val, 2, grid[2], s);
-}
-
 void stage_fill(Workspace& W, const Grid& g, const Values& val, hipStream_t s) {
     const uint64_t T = g.view.T;
     const uint32_t F = val.F;
@@ -2427,8 +2421,7 @@ enum RestPart {
     REST_DEDUP = 4,
     REST_XYZ = 8,
     REST_FACES = 16,
-    REST_EXTRACT_REC = 32,
-    REST_ALL = 63
+    REST_EXTRACT_REC = 32
 };
 
 // grid of a grid-stride kernel whose element count lives on the device:
@@ -2538,15 +2531,14 @@ void stage_rest(Workspace& W, const Grid& g, const Values& val, hipStream_t s, i
             hipLaunchKernelGGL(k_dedup_rank, dim3(tgrid), dim3(256), 0, s, NVO, (const uint32_t*)W.first.p,
                                (const uint32_t*)W.tile_first.p, W.vrank.p, W.first_occ.p);
         } else {
-            const uint32_t* list = nullptr;
-            hipLaunchKernelGGL(k_hash_insert, dim3(nblk(c.vo)), dim3(256), 0, s, NVO, list, (const uint64_t*)W.okey.p,
+            hipLaunchKernelGGL(k_hash_insert, dim3(nblk(c.vo)), dim3(256), 0, s, NVO, (const uint64_t*)W.okey.p,
                                W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p);
-            hipLaunchKernelGGL(k_hash_first, dim3(nblk(c.vo)), dim3(256), 0, s, NVO, list, (const uint32_t*)W.hslot.p,
+            hipLaunchKernelGGL(k_hash_first, dim3(nblk(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.hslot.p,
                                (const uint32_t*)W.hmx.p, W.first.p, W.mo.p);
             scan_u32(m, W.first.p, W.vrank.p, NVO, ctr + C_VERTS, s);
             hipLaunchKernelGGL(k_dedup_assign, dim3(cgrid(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.mo.p,
-                               (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p, NVO,
-                               list, (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p, true);
+                               (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p,
+                               (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p);
         }
     }
     VertFieldArgs VF;

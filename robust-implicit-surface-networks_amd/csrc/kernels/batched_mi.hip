@@ -48,7 +48,7 @@ static_assert(M_N <= kMiPub, "published counters");
 
 struct MICaps {
     uint32_t active = 0, fit = 0, words = 0, vo = 0, fo = 0, fv = 0;
-    uint32_t huge = 0;  // the captured path holds the large-capacity cut
+    uint32_t huge = 0;  // the captured path holds the wide cut
 };
 
 __global__ void k_mi_zero(uint32_t* ctr, uint32_t* errs) {
@@ -763,14 +763,14 @@ void mi_path(MIWorkspace& W, const Grid& g, uint32_t F, const MITablesDev& TT, h
         vid = W.vrank.p;
         mo = W.mo.p;
     } else {
-        hipLaunchKernelGGL(k_hash_insert, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)nullptr,
-                           (const uint64_t*)W.okey.p, W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p);
-        hipLaunchKernelGGL(k_hash_first, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)nullptr,
-                           (const uint32_t*)W.hslot.p, (const uint32_t*)W.hmx.p, W.first.p, W.mo.p);
+        hipLaunchKernelGGL(k_hash_insert, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint64_t*)W.okey.p,
+                           W.hkey.p, W.hmx.p, W.hbits, W.hslot.p, W.errs.p);
+        hipLaunchKernelGGL(k_hash_first, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.hslot.p,
+                           (const uint32_t*)W.hmx.p, W.first.p, W.mo.p);
         scan_u32(W.mem, W.first.p, W.vrank.p, NVO, ctr + M_NV, s);
         hipLaunchKernelGGL(k_dedup_assign, dim3(blocks_for(c.vo)), dim3(256), 0, s, NVO, (const uint32_t*)W.mo.p,
-                           (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p, NVO,
-                           (const uint32_t*)nullptr, (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p, true);
+                           (const uint32_t*)W.first.p, (const uint32_t*)W.vrank.p, W.vid.p, W.first_occ.p,
+                           (const uint32_t*)W.hslot.p, W.hkey.p, W.hmx.p);
     }
     // coordinates and faces
     const Count NV(ctr + M_NV, c.vo, abort), NF(ctr + M_FO, c.fo, abort), NFV(ctr + M_FV, c.fv, abort);

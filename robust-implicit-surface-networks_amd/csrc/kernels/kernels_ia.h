@@ -1593,8 +1593,7 @@ struct TileTotals {
     uint32_t* p[4];
 };
 
-// one workgroup of 1024 lanes; the counts are read with device-scope loads,
-// so that counts other workgroups of this kernel added atomically are seen
+// one workgroup of 1024 lanes
 __device__ inline void scan_tiles_block(uint32_t nt, uint32_t* __restrict__ x, int stride, int nfield,
                                         const TileTotals& total) {
     __shared__ uint32_t wsum[16];
@@ -1607,9 +1606,7 @@ __device__ inline void scan_tiles_block(uint32_t nt, uint32_t* __restrict__ x, i
             const uint32_t i0 = base + 4 * threadIdx.x;
             uint32_t v[4];
             for (int q = 0; q < 4; ++q)
-                v[q] = i0 + q < nt ? __hip_atomic_load(&x[(uint64_t)(i0 + q) * stride + f], __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT)
-                                   : 0u;
+                v[q] = i0 + q < nt ? x[(uint64_t)(i0 + q) * stride + f] : 0u;
             const uint32_t sum = v[0] + v[1] + v[2] + v[3];
             uint32_t inc = sum;
             for (int d = 1; d < 64; d <<= 1) {
@@ -1642,12 +1639,12 @@ __global__ void __launch_bounds__(1024) k_dedup_tile_scan(Count n, uint32_t* __r
 
 // Plain form: the active tets' cut lists by active-function count, built on
 // the device in active-rank order.  List 0: MI table tets, IA tets of one and
-// two functions (by table, or by groups of 8 lanes), 1: up to 4 functions, 2: 5..8, 3: more.  Per chunk of kBucketChunk active tets,
-// kBucketWords words: list sizes [0..4), the reference's bucket histogram
-// [4..7) (IA: 1, 2, >= 3 functions; MI: 2, 3, >= 4), tets with 3..4 and
-// 5..8 functions [7], [8], the largest count [9], the words of their record
-// slots [10] (k_bucket_count).  One
-// workgroup turns the list sizes into each chunk's list offsets and writes
+// two functions (by table, or by groups of 8 lanes), 1: up to 4 functions, 2:
+// 5..8, 3: more.  Per chunk of kBucketChunk active tets, kBucketWords words:
+// list sizes [0..4), the reference's bucket histogram [4..7) (IA: 1, 2, >= 3
+// functions; MI: 2, 3, >= 4), tets with 3..4 and 5..8 functions [7], [8], the
+// largest count [9], the words of their record slots [10] (k_bucket_count).
+// One workgroup turns the list sizes into each chunk's list offsets and writes
 // the totals (k_bucket_scan); each chunk then writes its entries
 // (k_bucket_fill).  No atomics.
 constexpr uint32_t kBucketChunk = 2048;
@@ -1835,38 +1832,32 @@ __global__ void __launch_bounds__(256) k_dedup_rank(Count n, const uint32_t* __r
     }
 }
 
-// hash path over occurrences list[0..n) (all occurrences when list is null)
-__global__ void k_hash_insert(Count n, const uint32_t* __restrict__ list, const uint64_t* __restrict__ okey,
-                              unsigned long long* __restrict__ hkey, uint32_t* __restrict__ hmx, int bits,
-                              uint32_t* __restrict__ hslot, uint32_t* __restrict__ errs) {
-    GRID_STRIDE(i, n) hash_insert_one(list ? list[i] : (uint32_t)i, okey, hkey, hmx, bits, hslot, errs);
+// hash path over the occurrences
+__global__ void k_hash_insert(Count n, const uint64_t* __restrict__ okey, unsigned long long* __restrict__ hkey,
+                              uint32_t* __restrict__ hmx, int bits, uint32_t* __restrict__ hslot,
+                              uint32_t* __restrict__ errs) {
+    GRID_STRIDE(o, n) hash_insert_one((uint32_t)o, okey, hkey, hmx, bits, hslot, errs);
 }
 
-__global__ void k_hash_first(Count n, const uint32_t* __restrict__ list, const uint32_t* __restrict__ hslot,
-                             const uint32_t* __restrict__ hmx, uint32_t* __restrict__ first, uint32_t* __restrict__ mo) {
-    GRID_STRIDE(i, n) {
-        const uint32_t o = list ? list[i] : (uint32_t)i;
+__global__ void k_hash_first(Count n, const uint32_t* __restrict__ hslot, const uint32_t* __restrict__ hmx,
+                             uint32_t* __restrict__ first, uint32_t* __restrict__ mo) {
+    GRID_STRIDE(o, n) {
         const uint32_t m = ~hmx[hslot[o]];
-        first[o] = m == o;
+        first[o] = m == (uint32_t)o;
         mo[o] = m;
     }
 }
 
-// vrank: exclusive scan of `first`.  The hash slots the run used (those of
-// list[0..n_hash), or of every occurrence when list is null) are cleared here.
+// vrank: exclusive scan of `first`.  The hash slots the run used are cleared here.
 __global__ void k_dedup_assign(Count n, const uint32_t* __restrict__ mo, const uint32_t* __restrict__ first,
                                const uint32_t* __restrict__ vrank, uint32_t* __restrict__ id_of_occ,
-                               uint32_t* __restrict__ first_occ, Count n_hash, const uint32_t* __restrict__ list,
-                               const uint32_t* __restrict__ hslot, unsigned long long* __restrict__ hkey,
-                               uint32_t* __restrict__ hmx, bool set_first_occ) {
+                               uint32_t* __restrict__ first_occ, const uint32_t* __restrict__ hslot,
+                               unsigned long long* __restrict__ hkey, uint32_t* __restrict__ hmx) {
     GRID_STRIDE(o, n) {
         const uint32_t id = vrank[mo[o]];
         id_of_occ[o] = id;
-        if (set_first_occ && first[o]) first_occ[id] = (uint32_t)o;
-    }
-    GRID_STRIDE(i, n_hash) {
-        const uint32_t o = list ? list[i] : (uint32_t)i;
         if (first[o]) {
+            first_occ[id] = (uint32_t)o;
             const uint32_t h = hslot[o];
             hkey[h] = 0;
             hmx[h] = 0;

@@ -18,7 +18,6 @@
 namespace rin {
 
 constexpr uint32_t kMaxFuncs = 64;   // function ids are packed in 6 bits
-constexpr uint32_t kMaxActive = 10;  // active functions per tet on the device path
 
 struct PlanCache;  // batched form: workspaces and captured graphs per function count (batched.hip)
 std::shared_ptr<PlanCache> make_plan_cache();
@@ -150,9 +149,10 @@ inline uint64_t record_limit(uint64_t most) {
     return e ? std::min<uint64_t>(most, std::strtoull(e, nullptr, 10)) : most;
 }
 
-// thrown by the batched form when a tet needs more than its buckets hold
-// (more than 8 active functions, or a complex beyond the bucket capacities);
-// the caller runs the plain form, which handles those tets
+// thrown by the batched forms when a tet needs more than their buckets hold (a
+// complex beyond the capacities, more than 28 functions) or the run needs more
+// than a workspace addresses; the caller runs the plain form, which handles
+// the former and says what it cannot hold
 struct NeedsPlainForm : std::runtime_error {
     using std::runtime_error::runtime_error;
 };
