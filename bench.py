@@ -285,7 +285,7 @@ def pmc_summary(fetch_csv, write_csv, trace_csv, copy_bytes, command):
         durs.setdefault(_short(r["Kernel_Name"]), []).append(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
     os.makedirs(os.path.join(ROOT, "profiles"), exist_ok=True)
     lines = ["# HBM traffic per dispatch (rocprofv3 FETCH_SIZE / WRITE_SIZE), %s" % WORKLOAD, "",
-             "Commands (from the repository root on the GPU box):", "",
+             "Commands (from the repository root, on an MI355X):", "",
              "    " + command.replace("COUNTER", "FETCH_SIZE"), "    " + command.replace("COUNTER", "WRITE_SIZE"), "",
              "Copy probe (k_copy_u64, %d bytes read + %d written per dispatch): FETCH_SIZE reads %.0f KiB, "
              "WRITE_SIZE %.0f KiB -> scale factors %.4f (fetch), %.4f (write)." % (
@@ -320,7 +320,7 @@ def _replay_timeline(trace_csv):
     trace (segments start at k_signs_count; the most common kernel count
     marks a whole-path replay): (start us, duration us, queue, kernel)."""
     rows = sorted(csv.DictReader(open(trace_csv)), key=lambda r: int(r["Start_Timestamp"]))
-    starts = [i for i, r in enumerate(rows) if _short(r["Kernel_Name"]) == "k_signs_count"]
+    starts = [i for i, r in enumerate(rows) if _short(r["Kernel_Name"]).startswith("k_signs_count")]
     segs = [rows[a:b] for a, b in zip(starts, starts[1:] + [len(rows)])]
     # whole-path runs end with the faces' closing kernel (the autotuner's
     # timing passes start with the signs pass too, and stop early)
@@ -356,7 +356,7 @@ def trace_summary(stats_csv, command, title, out_name):
             durs.setdefault(_short(r["Kernel_Name"]), []).append(
                 int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
         med = {k: sorted(v)[len(v) // 2] / 1e3 for k, v in durs.items()}
-    lines = ["# Kernel trace: %s" % title, "", "Command (from the repository root on the GPU box):", "",
+    lines = ["# Kernel trace: %s" % title, "", "Command (from the repository root, on an MI355X):", "",
              "    " + command, "",
              "Durations in microseconds over every dispatch of the run; totals and means include one-time work "
              "(first-run counting pass, autotuning candidates, tet adjacency), medians mostly do not.", "",

@@ -585,9 +585,9 @@ __global__ void __launch_bounds__(1024) k_signs_count(const double* __restrict__
 // come two corners a load, one AND over the cube ends an inactive one, the
 // wave sums are two packed words (7 before), and the count leaves which cubes
 // are active for the fill.  The fill lists its active tets in LDS and writes
-// their rows a lane each.  200^3 cubes, 8 functions: count 106 -> 57 us, fill
-// 178 -> 128 us (31 us are its bytes); 100^3, 20 functions: 20 -> 14 us and
-// 32 -> 30 us.
+// their rows a lane each.  200^3 cubes, 8 functions, tiles of 512 cubes: count
+// 106 -> 49 us, fill 178 -> 111 us (31 us are its bytes); 100^3, 20 functions:
+// 20 -> 15 us and 32 -> 30 us.
 
 // cubes per tile (one workgroup): 256, 512 or 1024, picked per plan by the
 // autotuner (the results do not depend on it)

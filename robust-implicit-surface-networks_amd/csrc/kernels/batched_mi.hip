@@ -389,7 +389,7 @@ __global__ void __launch_bounds__(kMiLanes) k_mi_fill_tiles(uint64_t T, const ui
 // in one launch of wavefronts, the longest first: the lists share no output,
 // and each cut's time is the latency of its longest tet (59 + 65 us one after
 // the other at 65^3 vertices and 8 materials, and 34 us of tables; together
-// 72 us).  One launch rather than graph branches: kernels with this much
+// 66 us).  One launch rather than graph branches: kernels with this much
 // private memory stay on one queue.
 struct MICutArgs {
     GridView g;
