@@ -88,6 +88,10 @@ def test_wide_tets_leave_the_other_slots_alone(ctx, monkeypatch, regular):
         _compare(dev, refs[i])
         assert dev.stage_times()[0][0] == "batched path (one graph)"
         dev.release()
+        dev = values[i].run(rin.FLAG_BATCHED | rin.FLAG_STAGE_TIMES)  # the same launches, a graph a stage
+        _compare(dev, refs[i])
+        assert "cut k=9.. (wave per tet)" in [n for n, _ in dev.stage_times()]
+        dev.release()
     for v in values:
         v.release()
     g.release()
